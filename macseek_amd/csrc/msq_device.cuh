@@ -398,6 +398,12 @@ __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
   asm volatile("" ::: "memory");
 }
+// Waits for the wave's LDS operations: in front of a load that writes LDS where earlier reads were served from.
+__device__ __forceinline__ void wait_lgkm0() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+  asm volatile("" ::: "memory");
+}
 // A piece of a prologue copy by loads that write LDS themselves (no registers in between, so the requests can be issued
 // ahead of everything else a kernel asks memory for and cost nothing until the data is needed): the whole groups of 64
 // items of the piece, dealt over the waves; item `slot` of the LDS region comes from src[perm(slot)] (a wave's load

@@ -58,4 +58,8 @@ void prefill_side_stream_setup();  // msq_prefill.hip: creates the current devic
 int matvec_tok(hipStream_t st, int t, const uint8_t* W, int rows, int cols, const float* X, float* Y, int n, int accumulate,
                int groups, const MsqMvCfg* cfg = nullptr, const float* norm_w = nullptr, float eps = 0.f);
 
+// few-token product over block formats on the matrix cores (msq_rows.hip); MSQ_ERR_UNSUPPORTED, without a message, when
+// another kernel serves the call
+int matvec_rows(hipStream_t st, int t, const uint8_t* W, int rows, int cols, const float* X, float* Y, int n, int accumulate, int groups);
+
 }  // namespace msq

@@ -41,6 +41,14 @@ __device__ __forceinline__ uint32_t bf16_rne(float f) {
   return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 
+// fp16(scale * payload + add) for both halves of a payload word: fp32 arithmetic on the fp16 payloads, one rounding
+__device__ __forceinline__ uint32_t scale_round_h2(uint32_t h, float scale, float add) {
+  uint32_t r;
+  asm("v_fma_mixlo_f16 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(scale), "v"(add));
+  asm("v_fma_mixhi_f16 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(r) : "v"(h), "v"(scale), "v"(add));
+  return r;
+}
+
 // ================================================================================================ fragments
 // Interface of a fragment decoder F (one K step = 32 matrix columns, chunk q = l / 16 of the step, 8 positions p):
 //   BF16_MATH          payloads are bf16 (activations are then split into two bf16 terms) instead of fp16

@@ -60,14 +60,6 @@ struct FragBF16H {
   }
 };
 
-// fp16(scale * payload + add) for both halves of a payload word: fp32 arithmetic on the fp16 payloads, one rounding
-__device__ __forceinline__ uint32_t scale_round_h2(uint32_t h, float scale, float add) {
-  uint32_t r;
-  asm("v_fma_mixlo_f16 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(scale), "v"(add));
-  asm("v_fma_mixhi_f16 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(r) : "v"(h), "v"(scale), "v"(add));
-  return r;
-}
-
 constexpr int kMmKStage = 128, kMmPitch = kMmKStage * 2 + 16;  // bytes per staged token row
 
 // WV waves (16 weight rows each) x TM token tiles per workgroup
