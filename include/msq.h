@@ -253,7 +253,7 @@ typedef struct MsqMoePrefillArgs {
 } MsqMoePrefillArgs;
 
 /* reference: ms::q::moe_prefill_scratch_bytes (quant.hpp:117, quant.mm:427-431). Layout (caller-owned device memory):
- * header (expert pointer table, offsets, token-tile table) | Xg fp16[(total+n) x dim] | H fp16[(total+n) x inter] |
+ * header (expert pointer table, offsets, work items) | Xg fp16[(total+n) x dim] | H fp16[(total+n) x inter] |
  * Z f32[(total+n) x dim]. The header is written by small kernels that carry it in their arguments, so unlike the
  * reference the scratch may still be in use by earlier work on the same stream. */
 size_t msq_moe_prefill_scratch_bytes(int total_entries, int n_tokens, int n_exp, int dim, int inter);
@@ -261,10 +261,11 @@ size_t msq_moe_prefill_scratch_bytes(int total_entries, int n_tokens, int n_exp,
 /* reference: ms::q::encode_moe_prefill (quant.hpp:118, quant.mm:433-612). Enqueues gather, grouped gate/up GEMM +
  * SwiGLU, grouped down GEMM and the ordered reduction into Y. Activations and H are staged as fp16 and weights enter
  * the matrix instructions as fp16 like the reference's tiles (IQ1_S / IQ2_XXS: the sub-block scale is rounded to fp16 and
- * its product with the grid value is rounded again, where the reference rounds the fp32 product once). The call only enqueues
- * (no host copy, no wait, no allocation) and can be captured in a HIP graph. Two of its launches are independent and
- * run side by side: one is forked onto a stream that the library owns (one per device, created by msq_init() or by the
- * first call outside a capture) and joined back before the call's later launches, all through events, so the caller
+ * its product with the grid value is rounded again, where the reference rounds the fp32 product once; a Q6_K / Q8_0 shared
+ * expert keeps exact payloads and fp32 scales). The call only enqueues
+ * (no host copy, no wait, no allocation) and can be captured in a HIP graph. With a shared expert its launches are
+ * forked onto a stream that the library owns (one per device, created by msq_init() or by the
+ * first call outside a capture) and joined back before the reduction, all through events, so the caller
  * sees the ordering of a single stream (MSQ_MOEP_ONE_STREAM=1 in the environment turns the fork off); `offs` (host memory) is read at call time and
  * travels to the device inside kernel arguments. The result is bit-identical from run to run. n_tokens <= 0 returns MSQ_OK and
  * does nothing (quant.mm:435). */

@@ -1,4 +1,4 @@
-// MFMA building blocks for the multi-token paths (small-N matvec_n and the prefill grouped MoE GEMM).
+// MFMA building blocks for the multi-token paths (small-N matvec_n, the prefill matmul and the prefill MoE GEMMs).
 //
 // v_mfma_f32_16x16x32_{f16,bf16}: D[16 x 16] += A[16 x 32] . B[32 x 16], one wave.
 //   A operand: lane l holds row  (l % 16), eight K positions 8 * (l / 16) .. + 7   (activations: row = token)
@@ -17,7 +17,6 @@ namespace msq {
 
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
 
-constexpr int kMvnMaxSteps = 16;  // K steps (of 32 columns) whose activations one wave of the token-tile GEMM keeps in registers
 constexpr int kMvnSubSteps = 8;   // K steps a wave of the small-N matvec fetches and multiplies at a time
 
 __device__ __forceinline__ f4_t mfma_f16(const uint32_t a[4], const uint32_t b[4], f4_t c) {

@@ -7,175 +7,14 @@
 //   down   : Z[i][c] = H_e[i] . Wd[c]   (fp32, one row per entry)
 //   reduce : Y[t] += Z[total + t] + sum_k Z[slot_of[t][k]]   in that fixed order
 //
-// GEMM work item = (token tile of up to 16 entries of one expert, chunk of weight-row tiles). A workgroup is up to 16
-// waves that split K; each wave keeps the token tile's activations of its K steps in registers as MFMA A fragments,
-// and the workgroup walks the 16-row weight tiles of its chunk. A tile's raw block bytes (16 contiguous rows) are
-// copied into LDS with fully coalesced 128-bit loads, one tile ahead through registers, and decoded from there into
-// B fragments; weights stay exact (fp16 payloads, fp32 scales applied to the MFMA result). The K-split partial tiles
-// meet in LDS and are added in wave order, so results do not depend on scheduling.
+// The routed experts and a shared expert of a codebook type go through the block GEMM below, a K-quant / Q8_0 shared
+// expert through the dense tile kernel of msq_prefill_tile.cuh.
 #pragma once
 #include <type_traits>
 
 #include "msq_mfma.cuh"
 
 namespace msq {
-
-struct PfArgs {
-  const uint16_t* A;        // activations fp16 [(total + n) x K]: Xg (gate/up) or H (down)
-  uint16_t* H;              // gate/up output fp16 [(total + n) x inter]
-  float* Z;                 // down output fp32 [(total + n) x dim]
-  const float* wt;          // routing weight per entry [total]
-  const uint64_t* ptrs;     // (n_exp + 1) x {gate, up, down} device addresses (the shared expert is entry n_exp)
-  const uint32_t* offs;     // n_exp + 2 entry offsets
-  const uint32_t* tiles;    // token tiles: pairs {expert index, first entry of the tile inside the expert}
-  uint32_t ntiles;          // token tiles this launch covers
-  uint32_t total;           // routed entries: entries at or beyond use weight 1 (shared expert)
-  uint32_t K, N;            // gate/up: K = dim, N = inter; down: K = inter, N = dim
-  uint32_t row_bytes;
-  uint32_t nsteps, steps_per_wave;
-  uint32_t chunk_tiles;     // weight-row tiles per work item
-  uint32_t nchunks;         // ceil(N / 16 / chunk_tiles)
-  uint32_t staged;          // 1: weight tiles go through LDS staging
-};
-
-constexpr int kPfStageGranules = 3;  // 16-byte granules per thread per matrix the staging path can hold (48 KiB / 1024 threads)
-
-template <class F, bool GU, bool STAGED>
-__global__ __launch_bounds__(1024) void moe_pf_gemm_kernel(const PfArgs a) {
-  constexpr int NM = GU ? 2 : 1;
-  extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
-  uint32_t* tbl = smem;
-  float* red = (float*)(smem + F::LDS_WORDS);  // [NM][wave][token][17]
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, nthreads = blockDim.x;
-  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), nwaves = nthreads >> 6;
-  uint8_t* stage = (uint8_t*)(red + NM * nwaves * 16 * 17);  // [NM][tile window]
-  const uint32_t m16 = lane & 15u, q = lane >> 4;
-  const uint32_t S = a.steps_per_wave, s0 = wave * S;
-  const uint32_t tile_bytes = 16u * a.row_bytes;
-  const uint32_t window = (tile_bytes + 15u + 15u) & ~15u;  // staged window per matrix, rounded to granules
-
-  F::fill_lds(tbl, (int)tid, (int)nthreads);
-
-  const uint32_t item = blockIdx.x;
-  const uint32_t mt = item / a.nchunks, rc = item - mt * a.nchunks;
-  const uint32_t e = a.tiles[2 * mt], t0 = a.tiles[2 * mt + 1];
-  const uint32_t base = a.offs[e] + t0;                       // first entry (row of A / H / Z) of the token tile
-  const uint32_t mtok = min(16u, a.offs[e + 1] - base);
-  gptr_t W[NM];
-  if (GU) { W[0] = as_global((const void*)a.ptrs[3 * e]); W[NM - 1] = as_global((const void*)a.ptrs[3 * e + 1]); }
-  else W[0] = as_global((const void*)a.ptrs[3 * e + 2]);
-
-  // A fragments of this wave's K steps: token m16 of the tile, chunk q
-  uint32_t xa[kMvnMaxSteps][4];
-#pragma unroll
-  for (int i = 0; i < kMvnMaxSteps; i++) {
-    const uint32_t step = s0 + i;
-    uint4 v = {0u, 0u, 0u, 0u};
-    if ((uint32_t)i < S && step < a.nsteps && m16 < mtok) {
-      const uint16_t* xs = a.A + (size_t)(base + m16) * a.K + 32u * step;
-      v = *(const uint4*)(xs + 8u * q);  // every format used here keeps the natural column order (col_of = 8 q + p)
-    }
-    xa[i][0] = v.x; xa[i][1] = v.y; xa[i][2] = v.z; xa[i][3] = v.w;
-  }
-
-  const uint32_t ntile_rows = (a.N + 15u) / 16u;
-  const uint32_t tile_first = rc * a.chunk_tiles, tile_last = min(ntile_rows, tile_first + a.chunk_tiles);
-  // staging: thread i owns granules i, i + nthreads, ... of each matrix' aligned window
-  uint4 pf[NM][kPfStageGranules];
-  auto issue = [&](uint32_t tile) {
-#pragma unroll
-    for (int m = 0; m < NM; m++) {
-      const gptr_t start = W[m] + (size_t)tile * tile_bytes;
-      const uint32_t shift = (uint32_t)((uintptr_t)start & 15u);
-      // the last tile of a matrix may be short: never read beyond the last row's granule
-      const uint32_t rows_here = min(16u, a.N - tile * 16u);
-      const uint32_t valid = shift + rows_here * a.row_bytes;
-#pragma unroll
-      for (int g = 0; g < kPfStageGranules; g++) {
-        const uint32_t gi = tid + g * nthreads;
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (16u * gi < valid) v = *(const MSQ_GLOBAL u32x4*)(start - shift + 16u * gi);
-        pf[m][g] = uint4{v.x, v.y, v.z, v.w};
-      }
-    }
-  };
-  if (STAGED && tile_first < tile_last) issue(tile_first);
-  __syncthreads();  // tables ready
-
-  const uint32_t ones[4] = {0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
-  for (uint32_t tile = tile_first; tile < tile_last; tile++) {
-    std::conditional_t<STAGED, const uint8_t*, gptr_t> wr[NM];
-    if constexpr (STAGED) {
-#pragma unroll
-      for (int m = 0; m < NM; m++) {
-#pragma unroll
-        for (int g = 0; g < kPfStageGranules; g++) {
-          const uint32_t gi = tid + g * nthreads;
-          if (16u * gi < window) ((uint4*)(stage + (size_t)m * window))[gi] = pf[m][g];
-        }
-        const uint32_t shift = (uint32_t)((uintptr_t)(W[m] + (size_t)tile * tile_bytes) & 15u);
-        wr[m] = stage + (size_t)m * window + shift + m16 * a.row_bytes;
-      }
-      if (tile + 1 < tile_last) issue(tile + 1);  // next tile's bytes travel while this one is decoded
-      __syncthreads();
-    } else {
-      const uint32_t row = min(tile * 16u + m16, a.N - 1);
-#pragma unroll
-      for (int m = 0; m < NM; m++) wr[m] = W[m] + (size_t)row * a.row_bytes;
-    }
-    f4_t acc[NM];
-#pragma unroll
-    for (int m = 0; m < NM; m++) acc[m] = f4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < kMvnMaxSteps; i++) {
-      const uint32_t step = s0 + i;
-      if ((uint32_t)i < S && step < a.nsteps) {  // wave-uniform
-        const f4_t zero = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int m = 0; m < NM; m++) {
-          const FragOut f = F::get(wr[m], step, q, tbl);
-          if constexpr (requires(float& s) { F::get_scales(wr[m], step, s, s); }) {
-            float sa, sb;
-            F::get_scales(wr[m], step, sa, sb);
-            uint32_t ha[4], hb[4];
-#pragma unroll
-            for (int p = 0; p < 4; p++) { ha[p] = q < 2 ? f.h[p] : 0u; hb[p] = q < 2 ? 0u : f.h[p]; }
-            acc[m] += sa * mfma_f16(xa[i], ha, zero) + sb * mfma_f16(xa[i], hb, zero);
-          } else {
-            acc[m] += f.scale * mfma_f16(xa[i], f.h, zero);
-            if constexpr (F::HAS_ADD) acc[m] += f.add * mfma_f16(xa[i], ones, zero);
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < NM; m++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) red[((m * nwaves + wave) * 16u + 4u * q + i) * 17u + m16] = acc[m][i];
-    __syncthreads();
-    for (uint32_t idx = tid; idx < 16u * mtok; idx += nthreads) {
-      const uint32_t t = idx >> 4, r = idx & 15u, orow = tile * 16u + r;
-      if (orow < a.N) {
-        float s[NM];
-#pragma unroll
-        for (int m = 0; m < NM; m++) {
-          s[m] = 0.f;
-          for (uint32_t w = 0; w < nwaves; w++) s[m] += red[((m * nwaves + w) * 16u + t) * 17u + r];
-        }
-        const uint32_t entry = base + t;
-        if constexpr (GU) {
-          float g = fminf(s[0], 10.f), u = fminf(fmaxf(s[NM - 1], -10.f), 10.f);
-          const float w = entry < a.total ? a.wt[entry] : 1.f;
-          const float h = g / (1.f + expf(-g)) * u * w;
-          a.H[(size_t)entry * a.N + orow] = __builtin_bit_cast(uint16_t, (_Float16)h);
-        } else {
-          a.Z[(size_t)entry * a.N + orow] = s[0];
-        }
-      }
-    }
-    __syncthreads();
-  }
-}
 
 // ------------------------------------------------------------------------------------------------ block GEMM
 // Grouped GEMM for the 256-weight codebook formats (block fragments, see msq_mfma.cuh). A work item is one expert's
@@ -466,8 +305,7 @@ __global__ __launch_bounds__(64 * pf_blk_waves(T)) void moe_pf_block_kernel(cons
 }
 
 // ------------------------------------------------------------------------------------------------ scratch header
-// The header of the prefill scratch (expert addresses, entry offsets, the shared expert's token tiles, the work items
-// of the block GEMM) is built on the device. What only the host knows travels in kernel arguments: a raw image
+// The header of the prefill scratch (expert addresses, entry offsets, the work items of the block GEMM) is built on the device. What only the host knows travels in kernel arguments: a raw image
 //   word 0 n_exp | 1 has_shared | 2 n_tokens | 3 total | 4, 5 base address | 6 address mode | 7 unused
 //   words 8 .. 8 + n_exp: entry offsets offs[0 .. n_exp]
 //   then 3 addresses per expert (gate, up, down; the shared expert last): mode 0 one word each, (address - base) / 4;
@@ -483,7 +321,6 @@ struct HdrBuild {
   uint32_t* raw;        // the image, behind the header
   uint64_t* ptrs;       // (n_exp + 1) x {gate, up, down}
   uint32_t* offs;       // n_exp + 2
-  uint32_t* tiles;      // shared expert: {n_exp, first token} per 16 tokens
   uint32_t* items;      // routed items, then the shared expert's
   uint32_t build;       // 1: this launch holds the image's last piece and expands it
 };
@@ -527,8 +364,6 @@ __global__ __launch_bounds__(kHdrThreads) void moe_pf_header_kernel(const HdrBui
     b.ptrs[i] = mode ? ((uint64_t)rp[2 * i] | ((uint64_t)rp[2 * i + 1] << 32)) : base + 4ull * rp[i];
   for (uint32_t i = tid; i <= ne; i += kHdrThreads) b.offs[i] = roffs[i];
   if (tid == 0) b.offs[ne + 1] = total + n;
-  if (has_shared)
-    for (uint32_t i = tid; i < (n + 15u) / 16u; i += kHdrThreads) { b.tiles[2 * i] = ne; b.tiles[2 * i + 1] = 16u * i; }
   // routed items: this thread's experts [j0, j1)
   const uint32_t per = (ne + kHdrThreads - 1) / kHdrThreads, j0 = min(ne, tid * per), j1 = min(ne, j0 + per);
   uint32_t cnt[7] = {0, 0, 0, 0, 0, 0, 0};

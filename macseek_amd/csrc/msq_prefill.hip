@@ -9,22 +9,21 @@
 
 #include "msq_host.h"
 #include "msq_prefill.cuh"
+#include "msq_prefill_tile.cuh"
 
 namespace msq {
 namespace {
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
-// header: addresses | offsets | the shared expert's token tiles | work items | raw image (see moe_pf_header_kernel)
-struct HdrLayout { size_t ptrs, offs, tiles, items, raw, bytes; };
+// header: addresses | offsets | work items | raw image (see moe_pf_header_kernel)
+struct HdrLayout { size_t ptrs, offs, items, raw, bytes; };
 HdrLayout header_layout(int total, int n, int n_exp) {
   HdrLayout h;
-  const size_t tiles = (size_t)n / 16 + 2;                                          // the shared expert's
   const size_t items = 2 * ((size_t)n_exp + 1) + (size_t)total / kPfBigTokens + (size_t)n / kPfBigTokens;  // m / 112 blocks + a rest per expert
   const size_t raw_words = kHdrRawHead + ((size_t)n_exp + 1) + 6 * ((size_t)n_exp + 1);
   h.ptrs = 0;
   h.offs = 24 * (size_t)(n_exp + 1);
-  h.tiles = h.offs + 4 * (size_t)(n_exp + 2);
-  h.items = h.tiles + 8 * tiles;
+  h.items = h.offs + 4 * (size_t)(n_exp + 2);
   h.raw = h.items + 12 * items;
   h.bytes = align256(h.raw + 4 * raw_words);
   return h;
@@ -33,30 +32,20 @@ size_t header_bytes(int total, int n, int n_exp) { return header_layout(total, n
 bool routed_ok(int t) { return t == MSQ_IQ1_S || t == MSQ_IQ2_XXS; }
 bool shared_ok(int t) { return t == MSQ_Q6_K || t == MSQ_Q8_0 || t == MSQ_IQ2_XXS || t == MSQ_IQ1_S; }
 
-template <class F, bool GU>
-int launch_gemm_t(hipStream_t st, PfArgs a, int cus) {
-  const uint32_t waves = (a.nsteps + a.steps_per_wave - 1) / a.steps_per_wave;
-  const uint32_t threads = 64 * waves;
-  constexpr int NM = GU ? 2 : 1;
-  const size_t window = ((size_t)16 * a.row_bytes + 30) & ~(size_t)15;
-  const size_t base_lds = (size_t)F::LDS_WORDS * 4 + (size_t)NM * waves * 16 * 17 * 4;
-  a.staged = (window <= (size_t)threads * kPfStageGranules * 16 && base_lds + NM * window <= 150 * 1024) ? 1u : 0u;
-  const size_t lds = base_lds + (a.staged ? NM * window : 0);
-  const uint32_t ntile_rows = (a.N + 15) / 16;
-  // enough work items to fill the chip a few times, at least 8 weight tiles per item to amortise the A fragments
-  uint32_t nchunks = std::max<uint32_t>(1, std::min<uint32_t>((4u * (uint32_t)cus + a.ntiles - 1) / a.ntiles, (ntile_rows + 7) / 8));
-  a.chunk_tiles = (ntile_rows + nchunks - 1) / nchunks;
-  a.nchunks = (ntile_rows + a.chunk_tiles - 1) / a.chunk_tiles;
-  static bool attr_set = false;  // per instantiation: allow more than 64 KiB of dynamic LDS
-  if (!attr_set) {
-    MSQ_HIP(hipFuncSetAttribute((const void*)moe_pf_gemm_kernel<F, GU, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    MSQ_HIP(hipFuncSetAttribute((const void*)moe_pf_gemm_kernel<F, GU, false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    attr_set = true;
-  }
-  if (a.staged) hipLaunchKernelGGL((moe_pf_gemm_kernel<F, GU, true>), dim3(a.ntiles * a.nchunks), dim3(threads), lds, st, a);
-  else hipLaunchKernelGGL((moe_pf_gemm_kernel<F, GU, false>), dim3(a.ntiles * a.nchunks), dim3(threads), lds, st, a);
+template <class D, bool GU>
+int launch_tile_t(hipStream_t st, PfTileArgs a) {
+  const size_t lds = 4 * (size_t)kPfTileBuf + 2 * (size_t)kPfTileRows * D::GROUPS * 4;
+  const int rc = allow_large_lds(moe_pf_tile_kernel<D, GU>, lds);
+  if (rc != MSQ_OK) return rc;
+  a.row_chunks = a.N / (GU ? kPfTileRows / 2 : kPfTileRows);  // (N is a multiple of 256)
+  a.token_blocks = (a.cnt + kPfTileTok - 1) / kPfTileTok;
+  hipLaunchKernelGGL((moe_pf_tile_kernel<D, GU>), dim3(a.row_chunks * a.token_blocks), dim3(kPfTileThreads), lds, st, a);
   MSQ_HIP(hipGetLastError());
   return MSQ_OK;
+}
+template <bool GU>
+int launch_tile(int t, hipStream_t st, const PfTileArgs& a) {
+  return t == MSQ_Q6_K ? launch_tile_t<TileQ6K, GU>(st, a) : launch_tile_t<TileQ8_0, GU>(st, a);
 }
 template <class B, bool GU, int T>
 int launch_block_tt(hipStream_t st, PfBlkArgs a) {
@@ -81,12 +70,12 @@ int launch_block_tt(hipStream_t st, PfBlkArgs a) {
   MSQ_HIP(hipGetLastError());
   return MSQ_OK;
 }
-// A second stream of the library's own, per device, and the two events that fork work onto it and join it back. The
-// routed experts' work falls into two classes that never meet before the final reduction: the popular experts' blocks
-// (gate/up, then down of the same entries) and the small items (likewise). Each launch has one workgroup per CU and
-// ends in a round that leaves CUs idle (the blocks' last round fills less than half of them); as two pipelines on two
-// streams, each class starts on the CUs the other leaves idle, and no class waits for the other's gate/up before its
-// own down. Fork and join are event dependencies, so a stream capture records them like any other (the objects are created
+// A second stream of the library's own, per device, and the two events that fork work onto it and join it back: the
+// shared expert's two products run beside the routed experts', which they only meet in the reduction. With few tokens
+// the shared expert has too few workgroups to fill the chip and its K loop is a chain of latencies (37 tokens, dim 5120:
+// 115 us that are hidden, the call 774 -> 659 us); with many it changes nothing. (The popular experts' blocks and the small
+// items stay on one stream: each takes a whole CU's LDS, side by side they measured 2.73 ms against 2.70 in turn.)
+// Fork and join are event dependencies, so a stream capture records them like any other (the objects are created
 // outside of captures: by msq_init() or by the first call that is not being captured; until then calls stay on one stream).
 struct SideStream { hipStream_t stream = nullptr; hipEvent_t fork = nullptr, join = nullptr; bool ok = false; };
 std::mutex g_side_mu;
@@ -122,35 +111,24 @@ SideStream* side_stream(hipStream_t st) {
 }
 
 // items are sorted by size, largest first: n6 blocks of more than 48 entries, n3 items of three token tiles, n2 of two,
-// then the one-tile items; which: kBig (the blocks), kSmall (everything up to three tiles, one launch: one tail of
-// half-idle CUs instead of two) or both; skip: profiling mask (see msq_moe_prefill)
-enum { kBig = 1, kSmall = 2 };
+// then the one-tile items: the blocks in one launch, everything up to three tiles in another (one tail of half-idle CUs
+// instead of two); skip: profiling mask (see msq_moe_prefill)
 template <class B, bool GU>
-int launch_block_t(hipStream_t st, PfBlkArgs a, uint32_t n6, uint32_t n3, uint32_t n2, int skip, int which) {
+int launch_block_t(hipStream_t st, PfBlkArgs a, uint32_t n6, uint32_t n3, uint32_t n2, int skip) {
   const uint32_t* items = a.items;
   const uint32_t n = a.nitems;
   int rc;
   a.items = items; a.nitems = n6;
-  if ((which & kBig) && !(skip & 256) && (rc = launch_block_tt<B, GU, kPfBigTiles>(st, a))) return rc;
-  if (!(which & kSmall)) return MSQ_OK;
+  if (!(skip & 256) && (rc = launch_block_tt<B, GU, kPfBigTiles>(st, a))) return rc;
   const uint32_t lo = (skip & 128) ? n6 + n3 + n2 : n6, hi = (skip & 64) ? n6 + n3 + n2 : n;
   a.items = items + 3 * (size_t)lo; a.nitems = hi > lo ? hi - lo : 0u;
   return launch_block_tt<B, GU, 3>(st, a);
 }
 bool block_path(int t) { return t == MSQ_IQ1_S || t == MSQ_IQ2_XXS; }
 template <bool GU>
-int launch_block(int t, hipStream_t st, const PfBlkArgs& a, uint32_t n6, uint32_t n3, uint32_t n2, int skip, int which) {
-  return t == MSQ_IQ1_S ? launch_block_t<BlkIQ1S, GU>(st, a, n6, n3, n2, skip, which)
-                        : launch_block_t<BlkIQ2XXS, GU>(st, a, n6, n3, n2, skip, which);
-}
-
-template <bool GU>
-int launch_gemm(int t, hipStream_t st, const PfArgs& a, int cus) {
-  switch (t) {  // the codebook formats never come here (block_path)
-    case MSQ_Q6_K: return launch_gemm_t<FragQ6K, GU>(st, a, cus);
-    case MSQ_Q8_0: return launch_gemm_t<FragQ8_0, GU>(st, a, cus);
-  }
-  return unsupported("moe_prefill types", t, 0, 0);
+int launch_block(int t, hipStream_t st, const PfBlkArgs& a, uint32_t n6, uint32_t n3, uint32_t n2, int skip) {
+  return t == MSQ_IQ1_S ? launch_block_t<BlkIQ1S, GU>(st, a, n6, n3, n2, skip)
+                        : launch_block_t<BlkIQ2XXS, GU>(st, a, n6, n3, n2, skip);
 }
 
 }  // namespace
@@ -212,7 +190,6 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: moe_prefill: shared expert missing or too small");
 
   hipStream_t st = (hipStream_t)stream;
-  const int cus = device_info().cus;
   // PROFILING ONLY (wrong output): MSQ_MOEP_SKIP bit mask 1 gather, 2 routed gate/up, 4 shared gate/up, 8 routed down,
   // 16 shared down, 32 reduce; of the block GEMMs' work 64 the one-tile items, 128 the two- and three-tile
   // items, 256 the blocks of the popular experts -- read on every call (reference: MACSEEK_MOEP_SKIP,
@@ -223,7 +200,6 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   // on the device from a raw image that travels in kernel arguments (moe_pf_header_kernel): nothing is read from host
   // memory after this call returns, the call never waits for the stream, and a stream capture records the values.
   const HdrLayout hl = header_layout(total, n, ne);
-  const uint32_t nt_shared = p->has_shared ? (uint32_t)((n + 15) / 16) : 0u;
   uint32_t ni_routed = 0, ni_shared = 0;
   uint32_t nc_routed[3] = {0, 0, 0}, nc_shared[3] = {0, 0, 0};  // items of more than 48 entries / three tiles / two tiles
   auto count = [](int m, uint32_t& ni, uint32_t* nc) {  // an expert of m entries: m / 112 blocks of 112 and one of m % 112
@@ -264,7 +240,7 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
     }
     HdrBuild hb{};
     hb.raw = (uint32_t*)(sc + hl.raw); hb.ptrs = (uint64_t*)(sc + hl.ptrs); hb.offs = (uint32_t*)(sc + hl.offs);
-    hb.tiles = (uint32_t*)(sc + hl.tiles); hb.items = (uint32_t*)(sc + hl.items);
+    hb.items = (uint32_t*)(sc + hl.items);
     for (size_t w0 = 0; w0 < raw.size(); w0 += kHdrChunkWords) {
       HdrChunk c;
       const uint32_t nw = (uint32_t)std::min<size_t>(kHdrChunkWords, raw.size() - w0);
@@ -281,7 +257,6 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   float* Z = (float*)((uint8_t*)H + align256(rows * inter * 2));
   const uint64_t* d_ptrs = (const uint64_t*)(sc + hl.ptrs);
   const uint32_t* d_offs = (const uint32_t*)(sc + hl.offs);
-  const uint32_t* d_tiles = (const uint32_t*)(sc + hl.tiles);
   const uint32_t* d_items = (const uint32_t*)(sc + hl.items);
   const bool any_routed = total > 0;
 
@@ -294,55 +269,52 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
     else hipLaunchKernelGGL((moe_pf_gather_kernel<false>), grid, block, 0, st, (const void*)bptr(&p->X), Xg, tok, (uint32_t)total, grows, (uint32_t)dim);
     MSQ_HIP(hipGetLastError());
   }
-  PfArgs a{};
-  a.H = H; a.Z = Z; a.wt = total > 0 ? (const float*)bptr(&p->wt) : nullptr;
-  a.ptrs = d_ptrs; a.offs = d_offs; a.total = (uint32_t)total;
-  auto steps = [&](uint32_t K) {
-    a.K = K; a.nsteps = K / 32;
-    const uint32_t ks = std::min<uint32_t>(16u, a.nsteps);
-    a.steps_per_wave = (a.nsteps + ks - 1) / ks;
-  };
   PfBlkArgs b{};
-  b.H = H; b.Z = Z; b.wt = a.wt; b.ptrs = d_ptrs; b.offs = d_offs; b.total = (uint32_t)total;
-  // one GEMM over the routed experts or over the shared expert: block kernel for the codebook formats, else the
-  // token-tile kernel
-  auto gemm = [&](auto gu_tag, int type, bool shared, const uint16_t* A, uint32_t K, uint32_t N, size_t row_bytes,
-                  hipStream_t gs, int which) -> int {
+  b.H = H; b.Z = Z; b.wt = total > 0 ? (const float*)bptr(&p->wt) : nullptr;
+  b.ptrs = d_ptrs; b.offs = d_offs; b.total = (uint32_t)total;
+  // one product over the routed experts' items
+  auto routed = [&](auto gu_tag, hipStream_t gs) -> int {
     constexpr bool GU = decltype(gu_tag)::value;
-    if (block_path(type)) {
-      b.A = A; b.K = K; b.N = N; b.nblocks = K / 256; b.row_bytes = (uint32_t)row_bytes;
-      b.items = d_items + (shared ? 3 * (size_t)ni_routed : 0); b.nitems = shared ? ni_shared : ni_routed;
-      const uint32_t* nc = shared ? nc_shared : nc_routed;
-      return launch_block<GU>(type, gs, b, nc[0], nc[1], nc[2], skip, which);
-    }
-    a.A = A; a.N = N; steps(K); a.row_bytes = (uint32_t)row_bytes;
-    // (the token-tile kernel only ever serves a Q6_K / Q8_0 shared expert: routed experts are codebook formats)
-    a.tiles = d_tiles; a.ntiles = shared ? nt_shared : 0u;
-    if (!a.ntiles) return MSQ_OK;
-    return launch_gemm<GU>(type, gs, a, cus);
+    b.A = GU ? Xg : H; b.K = (uint32_t)(GU ? dim : inter); b.N = (uint32_t)(GU ? inter : dim);
+    b.nblocks = b.K / 256; b.row_bytes = (uint32_t)(GU ? rb_gu : rb_d);
+    b.items = d_items; b.nitems = ni_routed;
+    return launch_block<GU>(GU ? p->t_gate_up : p->t_down, gs, b, nc_routed[0], nc_routed[1], nc_routed[2], skip);
   };
-  int rc;
+  // ... and one over all tokens with the shared expert's weights
+  auto shared = [&](auto gu_tag, hipStream_t gs) -> int {
+    constexpr bool GU = decltype(gu_tag)::value;
+    const uint32_t K = (uint32_t)(GU ? dim : inter), N = (uint32_t)(GU ? inter : dim), rb = (uint32_t)(GU ? rb_sgu : rb_sd);
+    if (block_path(p->t_shared)) {
+      b.A = GU ? Xg : H; b.K = K; b.N = N; b.nblocks = K / 256; b.row_bytes = rb;
+      b.items = d_items + 3 * (size_t)ni_routed; b.nitems = ni_shared;
+      return launch_block<GU>(p->t_shared, gs, b, nc_shared[0], nc_shared[1], nc_shared[2], skip);
+    }
+    PfTileArgs t{};
+    t.A = (GU ? Xg : H) + (size_t)total * K;
+    t.H = H + (size_t)total * inter; t.Z = Z + (size_t)total * dim;
+    t.W[0] = bptr(GU ? &p->shared.gate : &p->shared.down); t.W[1] = GU ? bptr(&p->shared.up) : nullptr;
+    t.cnt = (uint32_t)n; t.K = K; t.N = N; t.row_bytes = rb;
+    return launch_tile<GU>(p->t_shared, gs, t);
+  };
+  int rc = MSQ_OK;
+  using GuT = std::true_type; using DnT = std::false_type;
   const bool routed_gu = any_routed && !(skip & 2), routed_dn = any_routed && !(skip & 8);
-  const int both = kBig | kSmall;
-  // The routed experts' two item classes as two pipelines (see SideStream) when both exist and a side stream does
+  const bool shared_gu = p->has_shared && !(skip & 4), shared_dn = p->has_shared && !(skip & 16);
+  // The shared expert and the routed experts only meet in the reduction: two pipelines on two streams (see SideStream)
   bool forked = false;
-  if ((routed_gu || routed_dn) && block_path(p->t_gate_up) && block_path(p->t_down) && nc_routed[0] > 0 &&
-      ni_routed > nc_routed[0] && !(skip & 256) && (skip & (64 | 128)) != (64 | 128)) {
+  if (p->has_shared && any_routed) {
     std::lock_guard<std::mutex> lock(g_side_mu);
     SideStream* s = side_stream(st);
     if (s && hipEventRecord(s->fork, st) == hipSuccess && hipStreamWaitEvent(s->stream, s->fork, 0) == hipSuccess) {
       forked = true;
-      rc = routed_gu ? gemm(std::true_type{}, p->t_gate_up, false, Xg, (uint32_t)dim, (uint32_t)inter, rb_gu, s->stream, kBig) : MSQ_OK;
-      if (rc == MSQ_OK && routed_dn) rc = gemm(std::false_type{}, p->t_down, false, H, (uint32_t)inter, (uint32_t)dim, rb_d, s->stream, kBig);
-      // whatever happened above, the side stream is joined back before anything else can fail: a caller's capture is
-      // never left with an unjoined stream
+      if (shared_gu) rc = shared(GuT{}, s->stream);
+      if (rc == MSQ_OK && shared_dn) rc = shared(DnT{}, s->stream);
       const hipError_t ej = hipEventRecord(s->join, s->stream);
+      if (rc == MSQ_OK && routed_gu) rc = routed(GuT{}, st);
+      if (rc == MSQ_OK && routed_dn) rc = routed(DnT{}, st);
+      // whatever happened above, the side stream is joined back: a caller's capture is never left with an unjoined stream
       const hipError_t ew = ej == hipSuccess ? hipStreamWaitEvent(st, s->join, 0) : ej;
       if (rc == MSQ_OK && ew != hipSuccess) rc = hip_fail(ew, "joining the side stream");
-      if (rc == MSQ_OK && routed_gu) rc = gemm(std::true_type{}, p->t_gate_up, false, Xg, (uint32_t)dim, (uint32_t)inter, rb_gu, st, kSmall);
-      if (rc == MSQ_OK && nt_shared && !(skip & 4)) rc = gemm(std::true_type{}, p->t_shared, true, Xg, (uint32_t)dim, (uint32_t)inter, rb_sgu, st, both);
-      if (rc == MSQ_OK && routed_dn) rc = gemm(std::false_type{}, p->t_down, false, H, (uint32_t)inter, (uint32_t)dim, rb_d, st, kSmall);
-      if (rc == MSQ_OK && nt_shared && !(skip & 16)) rc = gemm(std::false_type{}, p->t_shared, true, H, (uint32_t)inter, (uint32_t)dim, rb_sd, st, both);
       if (rc != MSQ_OK) return rc;
     } else {
       (void)hipGetLastError();
@@ -350,14 +322,14 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   }
   if (!forked) {
     // 2) gate + up + SwiGLU -> H
-    if (routed_gu && (rc = gemm(std::true_type{}, p->t_gate_up, false, Xg, (uint32_t)dim, (uint32_t)inter, rb_gu, st, both))) return rc;
-    if (nt_shared && !(skip & 4) && (rc = gemm(std::true_type{}, p->t_shared, true, Xg, (uint32_t)dim, (uint32_t)inter, rb_sgu, st, both))) return rc;
+    if (routed_gu && (rc = routed(GuT{}, st))) return rc;
+    if (shared_gu && (rc = shared(GuT{}, st))) return rc;
     // 3) down -> Z
-    if (routed_dn && (rc = gemm(std::false_type{}, p->t_down, false, H, (uint32_t)inter, (uint32_t)dim, rb_d, st, both))) return rc;
-    if (nt_shared && !(skip & 16) && (rc = gemm(std::false_type{}, p->t_shared, true, H, (uint32_t)inter, (uint32_t)dim, rb_sd, st, both))) return rc;
+    if (routed_dn && (rc = routed(DnT{}, st))) return rc;
+    if (shared_dn && (rc = shared(DnT{}, st))) return rc;
   }
   // 4) ordered reduction into Y
-  if ((any_routed || nt_shared) && !(skip & 32)) {
+  if ((any_routed || p->has_shared) && !(skip & 32)) {
     const dim3 grid((dim / 4 + 255) / 256, (unsigned)n), block(256);
     hipLaunchKernelGGL(moe_pf_reduce_kernel, grid, block, 0, st, (const float*)Z, (float*)bptr_mut(&p->Y),
                        p->k_per_token > 0 ? (const int*)bptr(&p->slot_of) : nullptr, (uint32_t)n, (uint32_t)total, (uint32_t)dim,
