@@ -483,8 +483,21 @@ int msq_rmsnorm(void* stream, const MsqBuffer* x, const MsqBuffer* w, const MsqB
   if (!buf_ok(x, ((size_t)(rows - 1) * is + dim) * 4) || !buf_ok(y, ((size_t)(rows - 1) * os + dim) * 4) ||
       (has_w && !buf_ok(w, (size_t)dim * 4)))
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: rmsnorm: buffer missing or too small (rows %d dim %d)", rows, dim);
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, (const float*)bptr(x),
-                     has_w ? (const float*)bptr(w) : nullptr, (float*)bptr_mut(y), (uint32_t)dim, eps, (uint32_t)is, (uint32_t)os);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, (const float*)bptr(x),
+                       has_w ? (const float*)bptr(w) : nullptr, (float*)bptr_mut(y), (uint32_t)dim, eps, (uint32_t)is, (uint32_t)os);
+  };
+  switch ((dim + 1023) / 1024) {  // 1024 elements: four per thread
+    case 1: launch(rmsnorm_kernel<4>); break;
+    case 2: launch(rmsnorm_kernel<8>); break;
+    case 3: launch(rmsnorm_kernel<12>); break;
+    case 4: launch(rmsnorm_kernel<16>); break;
+    case 5: launch(rmsnorm_kernel<20>); break;
+    case 6: launch(rmsnorm_kernel<24>); break;
+    case 7: launch(rmsnorm_kernel<28>); break;
+    case 8: launch(rmsnorm_kernel<32>); break;
+    default: launch(rmsnorm_kernel<0>);
+  }
   MSQ_HIP(hipGetLastError());
   return MSQ_OK;
 }

@@ -57,40 +57,69 @@ __device__ __forceinline__ void load_x_row(const MvArgs& a, float* xs, const flo
 // scale = 1 / sqrt(mean(x^2) + eps) of one row, computed by a workgroup with a reduction whose order does not depend
 // on the workgroup's size: four virtual waves, virtual lane v (0..255) adds x[v], x[v + 256], ... with fused
 // multiply-adds, a DPP wave sum per virtual wave, then (s0 + s1) + (s2 + s3). The standalone norm kernel and the
-// matvec kernels with a fused norm both call this, so "norm, then matvec" and the fused call produce the same bits
+// matvec kernels with a fused norm both add in this order, so "norm, then matvec" and the fused call produce the same bits
 // (reference contract: src/kernels/quant.hpp:20-23; reduction being replayed there: src/kernels/quant_mv.metal:72-86).
-// `red` is four floats of LDS; all threads of the workgroup must call (it synchronises).
-__device__ __forceinline__ float rms_scale(const float* __restrict__ x, uint32_t dim, float eps, float* red, uint32_t lane,
-                                           uint32_t wave, uint32_t nwaves) {
-  for (uint32_t v = wave; v < 4u; v += nwaves) {
-    float ss = 0.f;
-    // eight elements are requested before the first is used (one at a time the loop is a chain of memory latencies);
-    // indices past the end repeat the last element and are left out of the sum, so the order of additions stays
-    for (uint32_t i0 = v * 64u + lane; i0 < dim; i0 += 8u * 256u) {
-      float t[8];
-#pragma unroll
-      for (int k = 0; k < 8; k++) t[k] = x[min(i0 + 256u * k, dim - 1u)];
-#pragma unroll
-      for (int k = 0; k < 8; k++)
-        if (i0 + 256u * k < dim) ss = __builtin_fmaf(t[k], t[k], ss);
-    }
-    ss = wave_sum(ss);
-    if (lane == 0) red[v] = ss;
-  }
-  __syncthreads();
+__device__ __forceinline__ float rms_of_sums(const float* red, uint32_t dim, float eps) {
   const float total = (red[0] + red[1]) + (red[2] + red[3]);
   return 1.0f / __builtin_sqrtf(total / (float)dim + eps);
+}
+// The four virtual waves of a row in device memory, by a workgroup of four waves. `red` is four floats of LDS; all threads
+// of the workgroup must call (it synchronises).
+__device__ __forceinline__ float rms_scale(const float* __restrict__ x, uint32_t dim, float eps, float* red, uint32_t lane, uint32_t wave) {
+  float ss = 0.f;
+  // eight elements are requested before the first is used (one at a time the loop is a chain of memory latencies);
+  // indices past the end repeat the last element and are left out of the sum, so the order of additions stays
+  for (uint32_t i0 = wave * 64u + lane; i0 < dim; i0 += 8u * 256u) {
+    float t[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) t[k] = x[min(i0 + 256u * k, dim - 1u)];
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      if (i0 + 256u * k < dim) ss = __builtin_fmaf(t[k], t[k], ss);
+  }
+  ss = wave_sum(ss);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  return rms_of_sums(red, dim, eps);
 }
 
 // y[row] = (x[row] * scale) * w (w may be null): reference ms::arch::encode_rmsnorm (src/kernels/arch.hpp:127-130,
 // kernel arch_rmsnorm, src/kernels/arch_sample.metal:216-233). One workgroup of 256 threads per row; y may alias x.
+// Bound by the trip to memory, not by bytes (16 rows of 5120: 0.6 MB): a thread owns the elements that its lane of the
+// reduction adds, up to 256 NV of a row, so the whole row and the weights are requested at once and each is read once.
+// NV = 0: rows longer than 8192, in pieces. Four of them among an attention layer's five products, 16 x 5120: 3.5 us
+// less per launch than in pieces of eight and a second pass over x (4 x 5120 the same).
+template <int NV>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* x, const float* __restrict__ w, float* y, uint32_t dim,
                                                       float eps, uint32_t in_stride, uint32_t out_stride) {
   __shared__ float red[4];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const float* xr = x + (size_t)blockIdx.x * in_stride;
   float* yr = y + (size_t)blockIdx.x * out_stride;
-  const float r = rms_scale(xr, dim, eps, red, lane, wave, 4u);
+  if constexpr (NV > 0) {
+    float xv[NV], wv[NV];
+#pragma unroll
+    for (int k = 0; k < NV; k++) xv[k] = xr[min(tid + 256u * k, dim - 1u)];
+    if (w) {
+#pragma unroll
+      for (int k = 0; k < NV; k++) wv[k] = w[min(tid + 256u * k, dim - 1u)];
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < NV; k++)
+      if (tid + 256u * k < dim) ss = __builtin_fmaf(xv[k], xv[k], ss);
+    ss = wave_sum(ss);
+    if (lane == 0) red[wave] = ss;
+    __syncthreads();
+    const float r = rms_of_sums(red, dim, eps);
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+      const uint32_t i = tid + 256u * k;
+      if (i < dim) { const float v = xv[k] * r; yr[i] = w ? v * wv[k] : v; }
+    }
+    return;
+  }
+  const float r = rms_scale(xr, dim, eps, red, lane, wave);
   for (uint32_t i0 = tid; i0 < dim; i0 += 4u * 256u) {  // four elements in flight per thread
     float xv[4], wv[4];
 #pragma unroll
@@ -109,25 +138,55 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* x, const floa
 
 // Prologue of the NORM matvec kernels: the normalized activations of the (single) input row go to LDS as fp32 (padded
 // layout of XLds), from where load_x() converts them exactly as it would from device memory.
+// A chain of latencies, so one trip to memory: all threads request the row and the norm's weights (kept in registers up
+// to 16 elements a thread) and the kernel's first weight rows with them (`with()`, called between the two); the
+// reduction then reads the row from LDS in its own order. Rows are 4-byte aligned. Before, four waves fetched the row in
+// pieces of eight and all waves fetched it again: Q5_K 512x7168 6.9 -> 5.4 us, Q6_K 1280x5120 + 512x5120 16.3 -> 11.5.
+template <class With>
 __device__ __forceinline__ void stage_normed_x(const MvArgs& a, uint32_t* smem, float* xs, uint32_t tid, uint32_t lane, uint32_t wave,
-                                               uint32_t nwaves) {
+                                               uint32_t nwaves, With with) {
+  typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int K = 4;
   float* red = (float*)(smem + a.norm_off);
-  const float r = rms_scale(a.x, a.cols, a.eps, red, lane, wave, nwaves);
-  const uint32_t nt = nwaves * 64u;
-  for (uint32_t i0 = tid; i0 < a.cols; i0 += 4u * nt) {  // four elements in flight per thread
-    float xv[4], wv[4];
+  const uint32_t nt = nwaves * 64u, n4 = a.cols >> 2;  // (cols is a multiple of 32)
+  const f4u *xg = (const f4u*)a.x, *wg = (const f4u*)a.norm_w;
+  auto at = [&](uint32_t i4) { return (f4_t*)(xs + 4u * i4 + (i4 >> 3) * 4u); };
+  f4_t xv[K], wv[K];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t i = min(i0 + nt * k, a.cols - 1u);
-      xv[k] = a.x[i];
-      wv[k] = a.norm_w[i];
-    }
+  for (int k = 0; k < K; k++) xv[k] = xg[min(tid + k * nt, n4 - 1u)];
+  __builtin_amdgcn_sched_barrier(0);
+  with();
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t i = i0 + nt * k;
-      if (i < a.cols) { const float v = xv[k] * r; xs[i + (i >> 5) * 4u] = v * wv[k]; }
+  for (int k = 0; k < K; k++) wv[k] = wg[min(tid + k * nt, n4 - 1u)];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < K; k++)
+    if (tid + k * nt < n4) *at(tid + k * nt) = xv[k];
+  for (uint32_t i = tid + K * nt; i < n4; i += nt) *at(i) = xg[i];
+  __syncthreads();
+  for (uint32_t v = wave; v < 4u; v += nwaves) {
+    float ss = 0.f;
+    for (uint32_t i0 = v * 64u + lane; i0 < a.cols; i0 += 8u * 256u) {
+      float t[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) { const uint32_t i = min(i0 + 256u * k, a.cols - 1u); t[k] = xs[i + (i >> 5) * 4u]; }
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        if (i0 + 256u * k < a.cols) ss = __builtin_fmaf(t[k], t[k], ss);
     }
+    ss = wave_sum(ss);
+    if (lane == 0) red[v] = ss;
   }
+  __syncthreads();
+  const float r = rms_of_sums(red, a.cols, a.eps);
+  auto normed = [&](f4_t x, f4_t w) {
+    const f4_t v = {x[0] * r, x[1] * r, x[2] * r, x[3] * r};
+    return f4_t{v[0] * w[0], v[1] * w[1], v[2] * w[2], v[3] * w[3]};
+  };
+#pragma unroll
+  for (int k = 0; k < K; k++)
+    if (tid + k * nt < n4) *at(tid + k * nt) = normed(xv[k], wv[k]);
+  for (uint32_t i = tid + K * nt; i < n4; i += nt) *at(i) = normed(*at(i), wg[i]);
   __syncthreads();
 }
 
@@ -156,8 +215,14 @@ __global__ __launch_bounds__(1024) void mv_kernel(const MvArgs a) {
   typename D::X xr[ITERS];
   uint32_t cur_group = 0xFFFFFFFFu;
   float* xs = (float*)(smem + a.xs_off);
-  if constexpr (NORM) stage_normed_x(a, smem, xs, tid, lane, wave, nwaves);  // synchronises (one group only)
-  else if (D::LDS_WORDS) __syncthreads();
+  constexpr bool FIRST = NORM && ITERS == 1;  // fused norm: the wave's first row is requested with the activations
+  [[maybe_unused]] typename D::Raw raw0;
+  if constexpr (NORM) {
+    const uint8_t* wr = a.W + (size_t)min(blockIdx.x * tile_rows + rw * a.rpw, a.rows - 1) * a.row_bytes;
+    stage_normed_x(a, smem, xs, tid, lane, wave, nwaves, [&] {  // synchronises (one group only)
+      if constexpr (FIRST) raw0 = D::load(wr, unit[0]);
+    });
+  } else if (D::LDS_WORDS) __syncthreads();
 
   for (uint32_t tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
     const uint32_t tile_row0 = tile * tile_rows;
@@ -178,7 +243,10 @@ __global__ __launch_bounds__(1024) void mv_kernel(const MvArgs a) {
       const uint8_t* wr = a.W + (size_t)row * a.row_bytes;
       typename D::Raw raw[ITERS];
 #pragma unroll
-      for (int i = 0; i < ITERS; i++) raw[i] = D::load(wr, unit[i]);
+      for (int i = 0; i < ITERS; i++) {
+        if (FIRST && j == 0 && tile == blockIdx.x) raw[i] = raw0;
+        else raw[i] = D::load(wr, unit[i]);
+      }
       float acc = 0.f;
 #pragma unroll
       for (int i = 0; i < ITERS; i++) {
@@ -438,8 +506,7 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
   typename D::X xr[T][ITERS];
   uint32_t cur_group = 0xFFFFFFFFu;
   float* xs = (float*)(smem + a.xs_off);
-  if constexpr (NORM) stage_normed_x(a, smem, xs, tid, lane, wave, nwaves);  // synchronises (one token, one group)
-  else if (D::LDS_WORDS) __syncthreads();
+  if (!NORM && D::LDS_WORDS) __syncthreads();
   const uint32_t roww = xlds_words(cols_);
 
   for (uint32_t tile = blockIdx.x; tile < ntiles_; tile += gridDim.x) {
@@ -509,11 +576,15 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
     // Half of the ring is requested ahead of the activations, the other half behind them: loads return in order, so with
     // the whole ring ahead the activations of a small matrix wait for four rows.
     constexpr int AHEAD = NR / 2;
+    auto ahead = [&] {
 #pragma unroll
-    for (int s = 0; s < AHEAD; s++) {
-      if constexpr (STAGE_W) request(s, s);
-      else fetch(ring[s], s);
-    }
+      for (int s = 0; s < AHEAD; s++) {
+        if constexpr (STAGE_W) request(s, s);
+        else fetch(ring[s], s);
+      }
+    };
+    if (NORM && cur_group == 0xFFFFFFFFu) stage_normed_x(a, smem, xs, tid, lane, wave, nwaves, ahead);  // synchronises (one token, one group)
+    else ahead();
     if (group != cur_group) {
       // tokens past the last repeat it; their results are never stored
       auto x_of = [&](int t) { return x_ + (size_t)min(t0 + t, ta.n - 1) * ta.x_stride + (size_t)group * a.x_group_stride; };

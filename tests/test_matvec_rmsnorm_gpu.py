@@ -82,3 +82,34 @@ def test_matvec_rmsnorm_misuse(dev):
         q.encode_matvec_rmsnorm(e, q.QType.Q6_K, W, 64, 1000, v, v, 1e-6, v)
     with pytest.raises(q.QuantError, match="matvec_rmsnorm unsupported"):  # wider than the LDS row
         q.encode_matvec_rmsnorm(e, q.QType.Q8_0, W, 16, 16384, v, v, 1e-6, v)
+
+
+@pytest.mark.parametrize("dim", [1, 255, 1024, 1025, 2048, 3000, 4097, 5120, 6145, 8192, 8193])
+def test_rmsnorm_row_lengths(dev, dim):
+    """Every number of elements per thread, at its longest row and one past it; rows longer than the registers hold."""
+    X, w = O.randn(3 * dim, 20 + dim, 2.0), O.randn(dim, 21)
+    Xd, wd = up(X), up(w)
+    Y = torch.full((3 * dim + 8,), 7.0, dtype=torch.float32, device=dev)
+    e = q.Enc()
+    arch.encode_rmsnorm(e, q.Buffer.of(Xd), q.Buffer.of(wd), q.Buffer.of(Y), 3, dim, 1e-6)
+    e.wait()
+    got = Y.cpu().numpy()
+    assert (got[3 * dim:] == 7.0).all()
+    for r in range(3):
+        assert np.allclose(got[r * dim:(r + 1) * dim], O.rmsnorm(X[r * dim:(r + 1) * dim], w, 1e-6), rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("t,rows,cols", [(O.Q5_K, 512, 7168), (O.Q6_K, 2048, 5120), (O.IQ4_NL, 33, 12288), (O.BF16, 600, 256)], ids=lambda v: None)
+def test_fused_norm_takes_rows_off_16_byte_boundaries(dev, t, rows, cols):
+    """Input row and norm weights 4 bytes past a boundary give the bits of aligned ones."""
+    arena, (W,) = place_in_arena([O.random_blocks(t, rows * cols, 31, 0.03)])
+    x, nw = O.randn(cols, 32, 3.0), (1.0 + 0.2 * O.randn(cols, 33)).astype(np.float32)
+    y = []
+    for off in (0, 1):
+        xd, nwd = (up(np.concatenate([np.zeros(off, np.float32), v])) for v in (x, nw))
+        o = torch.zeros(rows, dtype=torch.float32, device=dev)
+        e = q.Enc()
+        q.encode_matvec_rmsnorm(e, t, W, rows, cols, q.Buffer.of(xd[off:]), q.Buffer.of(nwd[off:]), 1e-6, q.Buffer.of(o))
+        e.wait()
+        y.append(o)
+    assert torch.equal(y[0], y[1]) and bool(y[0].any())
