@@ -311,6 +311,9 @@ __device__ __forceinline__ uint32_t pk_mul_f16(uint32_t a, uint32_t b) {
   const h2_t r = as_h2(a) * as_h2(b);
   return __builtin_bit_cast(uint32_t, r);
 }
+__device__ __forceinline__ uint32_t pk_fma_f16(uint32_t a, uint32_t b, uint32_t c) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(as_h2(a), as_h2(b), as_h2(c)));
+}
 // both halves = (fp16)v for an integer 0 <= v < 1024, without a conversion: 0x6400 | v is 1024 + v
 __device__ __forceinline__ uint32_t pk_small_int_f16(uint32_t v) {
   return pk_add_f16(0x64006400u | v | (v << 16), 0xE400E400u);
@@ -377,34 +380,51 @@ struct BlkIQ2XXS {
   }
 };
 
-struct BlkIQ1S {
-  static constexpr int LDS_WORDS = FragIQ1S::LDS_WORDS, BLOCK_BYTES = 50;
-  __device__ static void fill_lds(uint32_t* lds, int tid, int nt) { FragIQ1S::fill_lds(lds, tid, nt); }
-  struct Raw { uint32_t qs[2]; uint32_t qh; uint32_t d; };  // qs bytes 8 q .. 8 q + 7; qh[2 q] | qh[2 q + 1] << 16
-  __device__ static Raw load(gptr_t blk, uint32_t q) {
-    Raw r;
-    uint32_t qh[1];
-    ld_dwords_2aligned<2>(blk + 2 + 8 * q, r.qs);
-    ld_dwords_2aligned<1>(blk + 34 + 4 * q, qh);
-    r.qh = qh[0];
-    r.d = ld16(blk);
-    return r;
+// The grid as fp4: a trit (-1, 0, +1) is a nibble, an entry of eight one word, two conversions a word pair. Entries of 16
+// bytes (fp16) made every lookup a 16-byte read at a random place, 12 LDS cycles against 4 to 5 of one word.
+struct TblIQ1S4 { uint32_t w[MSQ_IQ1S_GRID_N]; };
+constexpr TblIQ1S4 make_iq1s4() {
+  TblIQ1S4 t{};
+  constexpr uint32_t nib[3] = {0xA, 0x0, 0x2};  // fp4 (E2M1): sign, two exponent bits (bias 1), one mantissa bit
+  for (int i = 0; i < MSQ_IQ1S_GRID_N; i++) {
+    unsigned c = msq_iq1s_code[i];
+    for (int j = 0; j < 8; j++, c /= 3) t.w[i] |= nib[c % 3] << (4 * j);
   }
-  struct Look { uint4 g; };
+  return t;
+}
+__device__ __attribute__((aligned(16))) const TblIQ1S4 g_tbl_iq1s4 = make_iq1s4();
+template <int BYTE>
+__device__ __forceinline__ uint32_t fp4_pair_to_h2(uint32_t w) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.f, BYTE));
+}
+
+struct BlkIQ1S {
+  static constexpr int LDS_WORDS = MSQ_IQ1S_GRID_N, BLOCK_BYTES = 50;
+  __device__ static void fill_lds(uint32_t* lds, int tid, int nt) { copy_words16(lds, g_tbl_iq1s4.w, LDS_WORDS, tid, nt); }
+  struct Raw { uint32_t qs[2]; uint32_t qh; uint32_t d; };  // qs bytes 8 q .. 8 q + 7; qh[2 q] | qh[2 q + 1] << 16
+  // the lane's bytes: read from LDS, where a row's 50 lie somewhere in PIECES aligned pieces. Fetched from memory in fragment
+  // order neighbouring lanes touch different rows: 290 vector cache lookups per 16 rows and block, which filled 94 % of
+  // the cycles of a launch with few tokens per expert
+  static constexpr int PIECES = 5;  // 50 + 14 bytes of misalignment fit four; an odd number spreads the rows over the banks
+  __device__ static Raw load(LdsRow b, uint32_t q) {
+    return {{ld32(b + (2u + 8u * q)), ld32(b + (6u + 8u * q))}, ld32(b + (34u + 4u * q)), ld16(b)};
+  }
+  struct Look { uint32_t g; };
   __device__ static Look lookup(const Raw& r, int j, const uint32_t* tbl, uint32_t) {
     const uint32_t qs = r.qs[j >> 2], qh = (j >> 2) ? r.qh >> 16 : r.qh & 0xFFFFu;
     const int l = j & 3;
-    return {((const uint4*)tbl)[((qs >> (8 * l)) & 0xFFu) | (((qh >> (3 * l)) & 7u) << 8)]};
+    return {tbl[((qs >> (8 * l)) & 0xFFu) | (((qh >> (3 * l)) & 7u) << 8)]};
   }
-  // weight = fp16(fp16(d (2 s + 1)) * (grid + delta)): scale rounded to fp16, product rounded again (the reference's
-  // tile rounds the fp32 product once, src/kernels/quant_moe_prefill.metal:137-147)
+  // weight = fp16(s2 * grid + s2 * delta) with s2 = fp16(d (2 s + 1)): s2 / 8 is exact (of a scale below 2^-11 it loses
+  // at most 2^-25, half a step of the smallest fp16), so the sum is rounded once, as s2 * (grid + delta) would be (the
+  // reference's tile rounds the fp32 product once, src/kernels/quant_moe_prefill.metal:137-147)
   __device__ static void finish(const Raw& r, int j, const Look& k, uint32_t (&h)[4]) {
     const uint32_t qh = (j >> 2) ? r.qh >> 16 : r.qh & 0xFFFFu;
     const uint32_t d2 = (qh & 0x8000u) ? 0xB000B000u : 0x30003000u;          // -+ 1/8 in both halves
     const float m = half_bits_to_float(r.d) * (float)(((qh >> 11) & 0xEu) | 1u);
-    const uint32_t m2 = pack_h2(m, m);
-    h[0] = pk_mul_f16(pk_add_f16(k.g.x, d2), m2); h[1] = pk_mul_f16(pk_add_f16(k.g.y, d2), m2);
-    h[2] = pk_mul_f16(pk_add_f16(k.g.z, d2), m2); h[3] = pk_mul_f16(pk_add_f16(k.g.w, d2), m2);
+    const uint32_t m2 = pack_h2(m, m), md = pk_mul_f16(m2, d2);
+    h[0] = pk_fma_f16(fp4_pair_to_h2<0>(k.g), m2, md); h[1] = pk_fma_f16(fp4_pair_to_h2<1>(k.g), m2, md);
+    h[2] = pk_fma_f16(fp4_pair_to_h2<2>(k.g), m2, md); h[3] = pk_fma_f16(fp4_pair_to_h2<3>(k.g), m2, md);
   }
 };
 

@@ -47,8 +47,13 @@ constexpr int pf_blk_waves(int T) { return T > 3 ? 12 : 16; }
 constexpr int pf_blk_rt(bool gu, int) { return gu ? 1 : 2; }
 constexpr int pf_blk_rows(bool gu, int T) { return pf_blk_waves(T) * pf_blk_rt(gu, T) * 16; }  // weight rows per work item
 // activation staging: double-buffered for up to three token tiles, a single buffer (two barriers per block) for seven
+constexpr size_t pf_blk_act_lds(int T) { return (T > 3 ? 1 : 2) * (size_t)(T > 3 ? kPfBigTokens : kPfBlkTokens) * kPfBlkPitch; }
+// A decoder with PIECES takes its bytes from LDS: a wave's block bytes of 16 rows (its R fragments: twice that) as
+// consecutive aligned 16-byte pieces, PIECES a row, by loads that write LDS themselves
 template <class B>
-constexpr size_t pf_blk_lds(int T) { return (size_t)B::LDS_WORDS * 4 + (T > 3 ? 1 : 2) * (size_t)(T > 3 ? kPfBigTokens : kPfBlkTokens) * kPfBlkPitch; }
+constexpr size_t pf_blk_raw_slot() { if constexpr (requires { B::PIECES; }) return 16 * 16 * B::PIECES; else return 0; }
+template <class B>
+constexpr size_t pf_blk_lds(int T) { return (size_t)B::LDS_WORDS * 4 + pf_blk_act_lds(T) + pf_blk_waves(T) * 2 * pf_blk_raw_slot<B>(); }
 
 // Where the 16 bytes of step j of chunk q (columns blk_col_of(q, j) .. + 7 of a block) sit in a token's staged row: the
 // chunks in the order 0, 2, 1, 3. A 16-byte LDS read serves the lanes in four groups of sixteen -- {0-7, 24-31},
@@ -100,6 +105,30 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
     woff[jt] = min(row_of[jt], a.N - 1) * a.row_bytes;
   }
   auto wrow = [&](int r, uint32_t off) { return wbase[r % NM] + (size_t)(woff[r / NM] + off); };
+  // ... or, staged: bytes off .. of the 16 rows of fragment r into the wave's slot r; lane l of piece group k fetches piece
+  // 64 k + l. Rows past the matrix's end: no traffic.
+  constexpr bool STAGED = requires { B::PIECES; };
+  uint8_t* const raw_lds = abuf + pf_blk_act_lds(T) + wave * (uint32_t)(R * pf_blk_raw_slot<B>());
+  auto request = [&](int r, uint32_t off) {
+    if constexpr (STAGED) {
+      const uint64_t b64 = (uint64_t)(uintptr_t)wbase[r % NM];  // (uniform, which an inline assembly operand has to be shown)
+      const uintptr_t base = ((uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b64 >> 32)) << 32) |
+                             (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b64);
+      const uint32_t mis = (uint32_t)base & 15u, end = mis + a.N * a.row_bytes, bytes = (end + 15u) & ~15u;  // whole aligned pieces
+      const rsrc_t rs = make_rsrc((const void*)(base - mis), bytes);
+      const uint32_t tile = ((rc0 * WAVES + wave) * RT + r / NM) * 16u;
+#pragma unroll
+      for (uint32_t p0 = 0; p0 < 16u * B::PIECES; p0 += 64u) {
+        const uint32_t p = p0 + lane, v = mis + (tile + p / B::PIECES) * a.row_bytes + off;
+        if (p < 16u * B::PIECES) lds_dma16(rs, raw_lds + r * pf_blk_raw_slot<B>() + 16u * p0, v < end ? (v & ~15u) + 16u * (p % B::PIECES) : bytes, 0u);
+      }
+    }
+  };
+  auto fetched = [&](int r, uint32_t off) {  // (the lane's row; what the slot holds of rows past the end is never stored)
+    if constexpr (STAGED)
+      return B::load(LdsRow::of(raw_lds + r * pf_blk_raw_slot<B>() + n16 * (16u * B::PIECES),
+                                ((uint32_t)(uintptr_t)wbase[r % NM] + (((rc0 * WAVES + wave) * RT + r / NM) * 16u + n16) * a.row_bytes + off) & 15u), q);
+  };
 
   // activation chunk loader: T * 512 granules of 16 bytes (token g / 32, column g % 32) over the workgroup's threads
   constexpr int AG = (T * 512 + NT - 1) / NT;
@@ -124,10 +153,16 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
 
   typename B::Raw cur[R], nxt[R];
 #pragma unroll
-  for (int r = 0; r < R; r++) cur[r] = B::load(wrow(r, 0u), q);
+  for (int r = 0; r < R; r++)
+    if constexpr (STAGED) request(r, 0u); else cur[r] = B::load(wrow(r, 0u), q);
   a_issue(0);
   B::fill_lds(tbl, (int)tid, NT);
   a_store(0);
+  if constexpr (STAGED) {
+    wait_vm<0>();
+#pragma unroll
+    for (int r = 0; r < R; r++) cur[r] = fetched(r, 0u);
+  }
   __syncthreads();
 
   uint32_t kb = 0;  // blocks done so far (double buffering: block kb sits in buffer kb % 2)
@@ -163,7 +198,12 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
         }
         if (j >= 2 && j - 2 < R) {
           __builtin_amdgcn_sched_barrier(0);
-          nxt[j - 2] = B::load(wrow(j - 2, wn), q);
+          if constexpr (STAGED) {
+            if (j == 2) wait_lgkm0();  // the slots are read: refill them
+            request(j - 2, wn);
+          } else {
+            nxt[j - 2] = B::load(wrow(j - 2, wn), q);
+          }
           __builtin_amdgcn_sched_barrier(0);
         }
         typename B::Look lk[R];
@@ -214,7 +254,12 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
       }
       if (p % 2 == 0 && p >= 2 && p / 2 - 1 < R) {
         __builtin_amdgcn_sched_barrier(0);
-        nxt[p / 2 - 1] = B::load(wrow(p / 2 - 1, wn), q);
+        if constexpr (STAGED) {
+          if (p == 2) wait_lgkm0();
+          request(p / 2 - 1, wn);
+        } else {
+          nxt[p / 2 - 1] = B::load(wrow(p / 2 - 1, wn), q);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
       if (p % PPS == 0) {  // activations of step j, read with the fragments' column mapping
@@ -247,8 +292,10 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
     // single buffer every wave has to be done with the block first)
     if (!DB) __syncthreads();
     a_store(DB ? (kb & 1u) ^ 1u : 0u);
+    if constexpr (STAGED) wait_vm<0>();
 #pragma unroll
-    for (int r = 0; r < R; r++) cur[r] = nxt[r];
+    for (int r = 0; r < R; r++)
+      if constexpr (STAGED) cur[r] = fetched(r, wn); else cur[r] = nxt[r];
     __syncthreads();
   }
 
