@@ -41,11 +41,12 @@ __device__ __forceinline__ uint32_t bf16_rne(float f) {
 }
 
 // fp16(scale * payload + add) for both halves of a payload word: fp32 arithmetic on the fp16 payloads, one rounding
+// (v_fma_mixlo_f16 / v_fma_mixhi_f16. Left to the compiler: the second reads the half that the first wrote, which wants a
+// wait state between them that it does not insert inside or around inline assembly)
 __device__ __forceinline__ uint32_t scale_round_h2(uint32_t h, float scale, float add) {
-  uint32_t r;
-  asm("v_fma_mixlo_f16 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(h), "v"(scale), "v"(add));
-  asm("v_fma_mixhi_f16 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(r) : "v"(h), "v"(scale), "v"(add));
-  return r;
+  const h2_t p = as_h2(h);
+  const h2_t r = {(_Float16)__builtin_fmaf((float)p.x, scale, add), (_Float16)__builtin_fmaf((float)p.y, scale, add)};
+  return __builtin_bit_cast(uint32_t, r);
 }
 
 // ================================================================================================ fragments
