@@ -61,5 +61,8 @@ int matvec_tok(hipStream_t st, int t, const uint8_t* W, int rows, int cols, cons
 // few-token product over block formats on the matrix cores (msq_rows.hip); MSQ_ERR_UNSUPPORTED, without a message, when
 // another kernel serves the call
 int matvec_rows(hipStream_t st, int t, const uint8_t* W, int rows, int cols, const float* X, float* Y, int n, int accumulate, int groups);
+// ... and over fp16-rounded weights (the arithmetic of msq_matmul), fp32 or fp16 activations
+int matmul_rows(hipStream_t st, int t, const uint8_t* W, int rows, int cols, const void* X, bool x_half, size_t x_stride, float* Y, int n,
+                int accumulate);
 
 }  // namespace msq

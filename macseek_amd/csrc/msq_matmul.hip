@@ -3,7 +3,8 @@
 //
 // The reference multiplies fp16 activations by weight tiles dequantized to fp16 inside its GEMM kernel and, from
 // n >= 512, dequantizes the whole matrix to fp16 once and runs a dense GEMM (quant.mm:204-221). The same two routes
-// exist here; the switch between them sits where they were measured to cross (use_fused, tile_ok below). Fused route:
+// exist here; the switch between them sits where they were measured to cross (use_fused, tile_ok below). Products of little
+// work over block formats go to the few-token kernel first (matmul_rows, msq_rows.hip). Fused route:
 // mm_fused_kernel (msq_mm.cuh) decodes each weight tile straight into matrix-core fragments -- no fp16 copy of W or X,
 // nothing allocated, the call only enqueues; for large matrices of four formats at 65 to 256 tokens mm_tile_kernel
 // does the same with both operands staged through LDS (F32 activations are first rounded to fp16 rows in a
@@ -345,6 +346,8 @@ int msq_matmul_h(void* stream, int t, const MsqBuffer* W, int rows, int cols, co
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: matmul: buffer missing, too small or misaligned (type %s rows %d cols %d n %d)",
                 msq_type_name_of(t), rows, cols, n);
   hipStream_t st = (hipStream_t)stream;
+  if (const int rc = matmul_rows(st, t, bptr(W), rows, cols, bptr(X16), true, (size_t)xs, (float*)bptr_mut(Y), n, accumulate); rc != MSQ_ERR_UNSUPPORTED)
+    return rc;
   if (tile_ok(t, n, rows, cols, (size_t)xs, bptr(X16))) {
     const MmArgs a{bptr(X16), bptr(W), (float*)bptr_mut(Y), (uint32_t)n, (uint32_t)rows, (uint32_t)cols, (uint32_t)xs,
                    (uint32_t)msq_type_row_bytes(t, cols), accumulate ? 1u : 0u};
@@ -367,6 +370,8 @@ int msq_matmul(void* stream, int t, const MsqBuffer* W, int rows, int cols, cons
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: matmul: buffer missing, too small or misaligned (type %s rows %d cols %d n %d)",
                 msq_type_name_of(t), rows, cols, n);
   hipStream_t st = (hipStream_t)stream;
+  if (const int rc = matmul_rows(st, t, bptr(W), rows, cols, bptr(X), false, (size_t)cols, (float*)bptr_mut(Y), n, accumulate); rc != MSQ_ERR_UNSUPPORTED)
+    return rc;
   if (tile_ok(t, n, rows, cols, (size_t)cols, nullptr)) {
     // the activations as fp16 rows first (one pass over X; every workgroup of the tile kernel then fetches half the bytes)
     const size_t xbytes = (size_t)n * cols * 2;

@@ -17,13 +17,15 @@
 // before -> after, us): Q6_K 32768x1280 at 4 / 8 / 16 tokens 18.7 / 28.4 / 22.8 -> 12.6 / 13.0 / 14.8, 5120x8192 at 16
 // 28.8 -> 20.8, IQ4_NL 16384x1536 at 16 22.5 -> 10.4, IQ1_S 7168x4096 at 4 / 16 9.9 / 20.7 -> 8.6 / 9.9.
 #pragma once
+#include <type_traits>
+
 #include "msq_mfma.cuh"
 
 namespace msq {
 
 struct RowsArgs {
   const uint8_t* W;  // raw block rows, below 4 GiB in all
-  const float* X;    // [n][x_stride] on 16-byte boundaries
+  const void* X;     // [n][x_stride]: fp32 on 16-byte boundaries, or fp16 on 8-byte ones
   float* Y;          // [n][rows]
   uint32_t n, rows, cols, x_stride, row_bytes, accumulate;
   uint32_t rows_per_group, x_group_stride;  // block-diagonal: rows per group (whole tiles), elements between the groups' inputs
@@ -78,7 +80,9 @@ __device__ __forceinline__ f4_t fma4(float s, f4_t p, f4_t c) {
   return f4_t{__builtin_fmaf(s, p[0], c[0]), __builtin_fmaf(s, p[1], c[1]), __builtin_fmaf(s, p[2], c[2]), __builtin_fmaf(s, p[3], c[3])};
 }
 
-template <class F, int BPW, int S, int NT, int UT>
+// ROUND: the arithmetic of msq_matmul -- scale times payload rounded to fp16, summed in the matrix cores -- over any number
+// of tokens, sixteen per workgroup (blockIdx.y). XH: activations in memory are fp16.
+template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false>
 __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   constexpr int P = rows_pieces<F>(), PIECES = 16 * P, NPI = (PIECES + 63) / 64, SLOT = rows_slot<F>();
   constexpr bool GROUPS = requires { F::GROUPS; };
@@ -91,6 +95,7 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   float* red = (float*)(smem + F::LDS_WORDS);                    // [2][wave][tile][token][16]
   uint8_t* mine = (uint8_t*)(red + 2u * nwaves * (256u * UT)) + wave * (uint32_t)rows_ring<F>(S);
 
+  const uint32_t m0 = ROUND ? blockIdx.y * 16u : 0u, ntok = ROUND ? min(a.n - m0, 16u) : a.n;
   const uint32_t tile0 = blockIdx.x * a.tiles_per_wg, ntile = min(a.tiles_per_wg, a.ntiles - tile0);  // (grid: tile0 < ntiles)
   const uint32_t group = (tile0 * 16u) / a.rows_per_group;
   const uint32_t ws0 = wave * BPW;
@@ -127,24 +132,30 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   uint32_t xr[BPW * 8][4];
   {
     uint8_t* xs = mine + rows_early<F>(S) * SLOT;
-    const float* xg = a.X + (size_t)group * a.x_group_stride;
+    using XT = std::conditional_t<XH, uint16_t, float>;
+    using XV = std::conditional_t<XH, uint2, f4_t>;  // four activations
+    const XT* xg = (const XT*)a.X + (size_t)group * a.x_group_stride + (size_t)m0 * a.x_stride;
     // (all of them requested at once where the registers hold them)
     constexpr int NK = NT / 2, NB = 2 * BPW, AHEAD = NB * NK <= 16 ? NB : 2;
-    f4_t raw[AHEAD][NK];
-    auto fetch = [&](int hb, f4_t (&r)[NK]) {  // half stage hb: 128 columns; lanes 0-31 even tokens, 32-63 odd ones
+    XV raw[AHEAD][NK];
+    auto fetch = [&](int hb, XV (&r)[NK]) {  // half stage hb: 128 columns; lanes 0-31 even tokens, 32-63 odd ones
       const uint32_t col = min((ws0 * 2u + hb) * 128u, a.cols - 128u) + 4u * (lane & 31u);
 #pragma unroll
-      for (int k = 0; k < NK; k++) r[k] = *(const f4_t*)(xg + (size_t)min(2u * k + (lane >> 5), a.n - 1u) * a.x_stride + col);  // tokens past n repeat the last
+      for (int k = 0; k < NK; k++) r[k] = *(const XV*)(xg + (size_t)min(2u * k + (lane >> 5), ntok - 1u) * a.x_stride + col);  // tokens past n repeat the last
     };
 #pragma unroll
     for (int hb = 0; hb < AHEAD; hb++) fetch(hb, raw[hb]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int hb = 0; hb < NB; hb++) {
-      f4_t(&r)[NK] = raw[hb % AHEAD];
+      XV(&r)[NK] = raw[hb % AHEAD];
 #pragma unroll
-      for (int k = 0; k < NK; k++)
-        *(uint2*)(xs + (2u * k + (lane >> 5)) * kRowsXPitch + 8u * (lane & 31u)) = uint2{pack_h2(r[k][0], r[k][1]), pack_h2(r[k][2], r[k][3])};
+      for (int k = 0; k < NK; k++) {
+        uint2 v;
+        if constexpr (XH) v = r[k];
+        else v = uint2{pack_h2(r[k][0], r[k][1]), pack_h2(r[k][2], r[k][3])};
+        *(uint2*)(xs + (2u * k + (lane >> 5)) * kRowsXPitch + 8u * (lane & 31u)) = v;
+      }
       asm volatile("" ::: "memory");  // (written and read through different types)
       if (hb + AHEAD < NB) fetch(hb + AHEAD, raw[hb % AHEAD]);
 #pragma unroll
@@ -203,8 +214,15 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
               const FragOut f = F::finish(F::load_raw(lrow, (uint32_t)js, q), (uint32_t)js, q, tbl);
               // (formats of 32-weight blocks: past a row that ends with half a stage the bytes are no blocks)
               const float sc = !PAIR || (ws0 + b) * 256u + 32u * js < a.cols ? f.scale : 0.f;
-              acc[u] = fma4(sc, mfma_f16(x, f.h, zero), acc[u]);
-              if constexpr (F::HAS_ADD) acc[u] = fma4(f.add, mfma_f16(x, ones, zero), acc[u]);
+              if constexpr (ROUND) {
+                uint32_t h[4];
+#pragma unroll
+                for (int p = 0; p < 4; p++) h[p] = scale_round_h2(f.h[p], sc, F::HAS_ADD ? f.add : 0.f);
+                acc[u] = mfma_f16(x, h, acc[u]);
+              } else {
+                acc[u] = fma4(sc, mfma_f16(x, f.h, zero), acc[u]);
+                if constexpr (F::HAS_ADD) acc[u] = fma4(f.add, mfma_f16(x, ones, zero), acc[u]);
+              }
             }
           }
         }
@@ -219,7 +237,7 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
 #pragma unroll
       for (int k = 0; k < 4; k++) rb[((wave * UT + u) * 16u + 4u * q + k) * 16u + n16] = acc[u][k];
     __syncthreads();  // (everyone read this buffer's last contents before the barrier between)
-    for (uint32_t idx = tid; idx < 16u * UT * a.n; idx += nthreads) {
+    for (uint32_t idx = tid; idx < 16u * UT * ntok; idx += nthreads) {
       const uint32_t t = idx / (16u * UT), r = idx % (16u * UT), u = r >> 4, orow = (tile0 + tl) * 16u + r;
       if (tl + u >= ntile || orow >= a.rows) continue;
       float s = 0.f;
@@ -230,7 +248,7 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
 #pragma unroll
         for (uint32_t k = 0; k < 8u; k++) s += w0 + k < nwaves ? v[k] : 0.f;
       }
-      float* y = a.Y + (size_t)t * a.rows + orow;
+      float* y = a.Y + (size_t)(m0 + t) * a.rows + orow;
       *y = a.accumulate ? *y + s : s;
     }
   }
