@@ -346,7 +346,8 @@ int msq_matmul_h(void* stream, int t, const MsqBuffer* W, int rows, int cols, co
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: matmul: buffer missing, too small or misaligned (type %s rows %d cols %d n %d)",
                 msq_type_name_of(t), rows, cols, n);
   hipStream_t st = (hipStream_t)stream;
-  if (const int rc = matmul_rows(st, t, bptr(W), rows, cols, bptr(X16), true, (size_t)xs, (float*)bptr_mut(Y), n, accumulate); rc != MSQ_ERR_UNSUPPORTED)
+  // (a forced switch between the fused and the materialising route leaves nothing to a third)
+  if (const int rc = fused_forced() >= 0 ? MSQ_ERR_UNSUPPORTED : matmul_rows(st, t, bptr(W), rows, cols, bptr(X16), true, (size_t)xs, (float*)bptr_mut(Y), n, accumulate); rc != MSQ_ERR_UNSUPPORTED)
     return rc;
   if (tile_ok(t, n, rows, cols, (size_t)xs, bptr(X16))) {
     const MmArgs a{bptr(X16), bptr(W), (float*)bptr_mut(Y), (uint32_t)n, (uint32_t)rows, (uint32_t)cols, (uint32_t)xs,
@@ -370,7 +371,7 @@ int msq_matmul(void* stream, int t, const MsqBuffer* W, int rows, int cols, cons
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: matmul: buffer missing, too small or misaligned (type %s rows %d cols %d n %d)",
                 msq_type_name_of(t), rows, cols, n);
   hipStream_t st = (hipStream_t)stream;
-  if (const int rc = matmul_rows(st, t, bptr(W), rows, cols, bptr(X), false, (size_t)cols, (float*)bptr_mut(Y), n, accumulate); rc != MSQ_ERR_UNSUPPORTED)
+  if (const int rc = fused_forced() >= 0 ? MSQ_ERR_UNSUPPORTED : matmul_rows(st, t, bptr(W), rows, cols, bptr(X), false, (size_t)cols, (float*)bptr_mut(Y), n, accumulate); rc != MSQ_ERR_UNSUPPORTED)
     return rc;
   if (tile_ok(t, n, rows, cols, (size_t)cols, nullptr)) {
     // the activations as fp16 rows first (one pass over X; every workgroup of the tile kernel then fetches half the bytes)
