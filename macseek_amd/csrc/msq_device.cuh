@@ -119,6 +119,7 @@ __device__ __forceinline__ gptr_t as_global(const void* p) { return (gptr_t)p; }
 // zero without touching memory. A pipelined loop can thus issue its prefetches unconditionally (an empty descriptor for
 // the rows past the end), which keeps the number of loads in flight known at every wait.
 typedef uint32_t __attribute__((ext_vector_type(4))) u32x4;
+typedef uint32_t __attribute__((ext_vector_type(2))) u32x2;
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);

@@ -304,77 +304,103 @@ struct FragDense16 {
 // 2^-12; the scale in fp32 would cost a second multiply per register), so a wave accumulates
 // all of K in the matrix cores without touching the accumulators in between. Lane (row n, chunk q) owns the sub-blocks 2 q and 2 q + 1 of its row's block
 // (16 contiguous bytes of IQ2_XXS), so no lane loads a byte twice; step j (0..7) of a block therefore covers, for chunk
-// q, the 8 columns col_of(q, j) .. + 7 of the block, and the activation operand is read with the same mapping.
-//   Raw / load(block pointer, q)    the lane's bytes of one block
-//   lookup(raw, j, tbl, col)        table reads of step j (col = lane % 16), issued ahead of their use
-//   finish(raw, j, look, h)         payloads of step j
+// q, the 8 columns 64 q + 32 (j / 4) + 8 (j % 4) .. + 7 of the block, and the activation operand is read with the same mapping.
+//   Raw / load(at, slot, sel)       the lane's bytes of one block from LDS (PIECES, piece_at, at_of: how they lie there)
+//   lane_low(lane % 16)             low byte of the lane's lookup addresses
+//   lookup<j>(raw, low)             table reads of step j, issued ahead of their use (the table starts the workgroup's LDS)
+//   scale(raw, sub)                 scale of the lane's sub-block sub (0, 1), in both halves
+//   finish(scale, look, h)          payloads of a step
 __device__ __forceinline__ uint32_t pk_mul_f16(uint32_t a, uint32_t b) {
   const h2_t r = as_h2(a) * as_h2(b);
   return __builtin_bit_cast(uint32_t, r);
 }
-// both halves = (fp16)v for an integer 0 <= v < 1024, without a conversion: 0x6400 | v is 1024 + v
-__device__ __forceinline__ uint32_t pk_small_int_f16(uint32_t v) {
-  return pk_add_f16(0x64006400u | v | (v << 16), 0xE400E400u);
-}
-// N dwords from a global address that is only 2-byte aligned, fetched with 4-byte-aligned loads: wide loads that are
-// not dword aligned run at about a third of the rate of aligned ones. N aligned dwords plus the one that follows (the
-// last one again when the address is aligned, so nothing past the data is touched), then a funnel shift.
-template <int N>
-__device__ __forceinline__ void ld_dwords_2aligned(gptr_t p, uint32_t (&out)[N]) {
-  typedef uint32_t __attribute__((ext_vector_type(N), aligned(4))) vec_t;
-  const uintptr_t a = (uintptr_t)p;
-  const uint32_t odd = (uint32_t)a & 2u;
-  const MSQ_GLOBAL uint32_t* w = (const MSQ_GLOBAL uint32_t*)(a - odd);
-  const vec_t v = *(const MSQ_GLOBAL vec_t*)w;
-  const uint32_t tail = w[odd ? N : N - 1];
-#pragma unroll
-  for (int i = 0; i < N; i++) out[i] = __builtin_amdgcn_alignbit(i + 1 < N ? v[i + 1] : tail, v[i], odd * 8u);
-}
-__device__ __forceinline__ uint32_t blk_col_of(uint32_t q, uint32_t j) { return 64u * q + 32u * (j >> 2) + 8u * (j & 3u); }
 
-// IQ2_XXS keeps 16 copies of its two small tables in LDS, copy c in the 16-byte bank column c of each 256-byte row:
-// a 16-lane group whose lanes read "their" column (c = lane % 16) touches every bank exactly once whatever the
-// entries are, so the random lookups run at the conflict-free rate.
+// A table entry's LDS address is assembled from whole bytes: v_perm puts an index byte above the low byte that the caller
+// prepared (one instruction instead of a shift, a mask and an addition). The low byte's bits must not be known to the
+// compiler, which otherwise turns the assembly back into an addition to a base.
+typedef __attribute__((address_space(3))) const uint8_t* lds_cptr_t;
+template <int BYTE>
+__device__ __forceinline__ uint32_t byte_over(uint32_t w, uint32_t low) {  // byte BYTE of w at bits 8..15, byte 0 of low below it
+  return __builtin_amdgcn_perm(w, low, 0x0c0c0000u | ((4u + BYTE) << 8));
+}
+__device__ __forceinline__ uint32_t bits_from(uint32_t mask, uint32_t a, uint32_t b) { return (mask & a) | (~mask & b); }  // v_bfi
+__device__ __forceinline__ uint32_t opaque(uint32_t v) { asm("" : "+v"(v)); return v; }
+template <class T>
+__device__ __forceinline__ T lds_at(uint32_t at, uint32_t off) {
+  typedef const __attribute__((address_space(3))) T* p_t;
+  return *(p_t)((lds_cptr_t)(uintptr_t)at + off);
+}
+
+// A row's block bytes in LDS: the whole dwords from the block's start, rounded down to a dword, on, in PIECES 16-byte pieces.
+// A block starts in the first dword's low half or in its high half: SEL_LOW picks bytes that start two bytes into a pair of
+// dwords, and ^ SEL_FLIP picks the second dword of the pair (blocks and rows are whole 16-bit words).
+constexpr uint32_t SEL_LOW = 0x05040302u, SEL_FLIP = 0x02020606u;
+__device__ __forceinline__ uint32_t halves_of(uint32_t lo, uint32_t hi, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
+
+// IQ2_XXS keeps 16 copies of its grid table in LDS, copy c in the 16-byte bank column c of each 256-byte row: a 16-lane
+// group whose lanes read "their" column (c = lane % 16) touches every bank exactly once whatever the entries are, so the
+// random lookups run at the conflict-free rate. So does the sign table (SIGNS = 16) where there is room for it; four copies
+// leave about two lanes to a bank column.
+template <int SIGNS>
 struct BlkIQ2XXS {
-  static constexpr int LDS_WORDS = (MSQ_IQ2XXS_GRID_N + 128) * 16 * 4, BLOCK_BYTES = 66;
-  // the sign table comes first: both table bases then fit the 16-bit offset field of the LDS instructions (signs at 0,
-  // grid at 32 KB), and a lookup address is one v_and_or of the entry index and the lane's column
-  static constexpr uint32_t GRID_AT = 128u * 256u;
+  // the sign table comes first: both table bases then fit the 16-bit offset field of the LDS instructions, and a lookup
+  // address is the entry index above the lane's column
+  static constexpr uint32_t GRID_AT = 128u * 16u * SIGNS;
+  static constexpr int LDS_WORDS = GRID_AT / 4 + MSQ_IQ2XXS_GRID_N * 16 * 4, BLOCK_BYTES = 66;
   __device__ static void fill_lds(uint32_t* lds, int tid, int nt) {
     const uint4* grid = (const uint4*)g_tbl_iq2xxs.w;
     const uint4* sign = (const uint4*)g_tbl_sign.w;
     uint4* dst = (uint4*)lds;
-    for (int i = tid; i < (MSQ_IQ2XXS_GRID_N + 128) * 16; i += nt) {
-      const int e = i >> 4;
-      dst[i] = e < 128 ? sign[e] : grid[e - 128];
-    }
+    for (int i = tid; i < 128 * SIGNS; i += nt) dst[i] = sign[i / SIGNS];
+    dst += 128 * SIGNS;
+    for (int i = tid; i < MSQ_IQ2XXS_GRID_N * 16; i += nt) dst[i] = grid[i / 16];
   }
-  struct Raw { uint32_t w[4]; uint32_t d; };  // {a0, a1} of sub-block 2 q, then of 2 q + 1; fp16 bits of d
-  __device__ static Raw load(gptr_t blk, uint32_t q) {
+  struct Raw { uint32_t w[4]; uint32_t d; };  // {a0, a1} of sub-block 2 q, then of 2 q + 1; fp16 bits of d in the high half
+  // 17 dwords (BlkIQ1S says why through LDS). Rows 8-15 hold pieces 0-3 in the order 1, 0, 3, 2: a 16-byte read serves eight
+  // rows of chunk q and the other eight of chunk q ^ 1 together
+  static constexpr int PIECES = 5;
+  __device__ static uint32_t piece_at(uint32_t row, uint32_t p) { return p < 4u ? p ^ (row >> 3) : 4u; }
+  // LDS addresses, from the slot's start, of what the lane reads of its row
+  struct At { uint32_t x, tail, d; };
+  __device__ static At at_of(uint32_t row, uint32_t q) {
+    const uint32_t b = row * (16u * PIECES);
+    return {b + 16u * piece_at(row, q), b + 16u * piece_at(row, q + 1u), b + 16u * piece_at(row, 0u)};
+  }
+  __device__ static Raw load(const At& at, uint32_t slot, uint32_t sel) {
+    const u32x4 x = lds_at<u32x4>(at.x, slot);
+    const uint32_t tail = lds_at<uint32_t>(at.tail, slot), d = lds_at<uint32_t>(at.d, slot);
     Raw r;
-    ld_dwords_2aligned<4>(blk + 2 + 16 * q, r.w);
-    r.d = ld16(blk);
+#pragma unroll
+    for (int i = 0; i < 4; i++) r.w[i] = halves_of(x[i], i < 3 ? x[i + 1] : tail, sel);
+    r.d = halves_of(d, d, sel);
     return r;
   }
-  struct Look { uint4 g, s; };
-  // byte offsets in the replicated tables: entry << 8 | column << 4
-  __device__ static Look lookup(const Raw& r, int j, const uint32_t* tbl, uint32_t col) {
-    const uint32_t a0 = r.w[2 * (j >> 2)], a1 = r.w[2 * (j >> 2) + 1];
-    const int l = j & 3;
-    const uint32_t cg = col << 4;
-    const uint32_t g8 = l == 0 ? a0 << 8 : l == 1 ? a0 : a0 >> (8 * l - 8);    // grid index byte at bits 8..15
-    const uint32_t s8 = 7 * l < 8 ? a1 << (8 - 7 * l) : a1 >> (7 * l - 8);     // sign index at bits 8..14
-    const uint8_t* t8 = (const uint8_t*)tbl;
-    return {*(const uint4*)(t8 + GRID_AT + ((g8 & 0xFF00u) | cg)), *(const uint4*)(t8 + ((s8 & 0x7F00u) | cg))};
+  struct Look { u32x4 g, s; };
+  // low bytes of a lane's lookup addresses: its columns of the two tables' rows of copies
+  struct Low { uint32_t g, s; };
+  __device__ static Low lane_low(uint32_t col) {
+    Low l;
+    l.g = opaque(col << 4);
+    l.s = SIGNS == 16 ? l.g : opaque((col % SIGNS) << 4);
+    return l;
+  }
+  template <int J>
+  __device__ static Look lookup(const Raw& r, Low low) {
+    constexpr int l = J & 3, at = SIGNS == 16 ? 8 : 6;  // the sign index goes to bits at .. at + 6
+    const uint32_t a0 = r.w[2 * (J >> 2)], a1 = r.w[2 * (J >> 2) + 1];
+    const uint32_t s7 = 7 * l < at ? a1 << (7 * l < at ? at - 7 * l : 0) : a1 >> (7 * l < at ? 0 : 7 * l - at);
+    return {lds_at<u32x4>(byte_over<l>(a0, low.g), GRID_AT), lds_at<u32x4>(bits_from(127u << at, s7, low.s), 0u)};
   }
   // weight = fp16(fp16(d (2 s + 1) / 8) * (+-grid)): the whole scale rides in the payload, rounded to fp16 before the
   // multiply (the reference's tile rounds the fp32 product once, src/kernels/quant_moe_prefill.metal:153-167)
-  __device__ static void finish(const Raw& r, int j, const Look& k, uint32_t (&h)[4]) {
-    const uint32_t a1 = r.w[2 * (j >> 2) + 1];
-    const float m = (half_bits_to_float(r.d) * 0.125f) * (float)(((a1 >> 27) & 0x1Eu) | 1u);
-    const uint32_t m2 = pack_h2(m, m);
-    h[0] = pk_mul_f16(k.g.x ^ k.s.x, m2); h[1] = pk_mul_f16(k.g.y ^ k.s.y, m2);
-    h[2] = pk_mul_f16(k.g.z ^ k.s.z, m2); h[3] = pk_mul_f16(k.g.w ^ k.s.w, m2);
+  __device__ static uint32_t scale(const Raw& r, int sub) {
+    const uint32_t a1 = r.w[2 * sub + 1];
+    const float m = (half_bits_to_float(r.d >> 16) * 0.125f) * (float)(((a1 >> 27) & 0x1Eu) | 1u);
+    return pack_h2(m, m);
+  }
+  __device__ static void finish(uint32_t m2, const Look& k, uint32_t (&h)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) h[i] = pk_mul_f16(k.g[i] ^ k.s[i], m2);
   }
 };
 
@@ -400,30 +426,53 @@ __device__ __forceinline__ uint32_t fp8_pair_to_h2(uint32_t w) {
 }
 
 struct BlkIQ1S {
-  static constexpr int LDS_WORDS = 4 * MSQ_IQ1S_GRID_N, BLOCK_BYTES = 50;
-  __device__ static void fill_lds(uint32_t* lds, int tid, int nt) { copy_words16(lds, &g_tbl_iq1s8.w[0][0][0], LDS_WORDS, tid, nt); }
-  struct Raw { uint32_t qs[2]; uint32_t qh; uint32_t d; };  // qs bytes 8 q .. 8 q + 7; qh[2 q] | qh[2 q + 1] << 16
-  // the lane's bytes: read from LDS, where a row's 50 lie somewhere in PIECES aligned pieces. Fetched from memory in fragment
-  // order neighbouring lanes touch different rows: 290 vector cache lookups per 16 rows and block (58 a load), one in every
-  // cycle of a launch with few tokens per expert; by pieces 18 a load, one in five cycles
-  static constexpr int PIECES = 5;  // 50 + 14 bytes of misalignment fit four; an odd number spreads the rows over the banks
-  __device__ static Raw load(LdsRow b, uint32_t q) {
-    return {{ld32(b + (2u + 8u * q)), ld32(b + (6u + 8u * q))}, ld32(b + (34u + 4u * q)), ld16(b)};
+  // Entry (b = qs byte, h = 3 bits of qh, sign of delta) lives at LDS byte b << 8 | (copy << 7) | sign << 6 | h << 3: two
+  // copies, since one entry set of 256-byte pitch would sit in half of the banks
+  static constexpr int LDS_WORDS = 8 * MSQ_IQ1S_GRID_N, BLOCK_BYTES = 50;
+  __device__ static void fill_lds(uint32_t* lds, int tid, int nt) {
+    for (int i = tid; i < 2 * MSQ_IQ1S_GRID_N; i += nt) {  // item i: sign, then entry h << 8 | b
+      const uint2 v = ((const uint2*)&g_tbl_iq1s8.w[0][0][0])[i];
+      uint2* dst = (uint2*)((uint8_t*)lds + ((i & 255) << 8) + ((i >> 11) << 6) + (((i >> 8) & 7) << 3));
+      dst[0] = v;
+      dst[16] = v;
+    }
   }
-  struct Look { uint2 g; };
-  __device__ static Look lookup(const Raw& r, int j, const uint32_t* tbl, uint32_t) {
-    const uint32_t qs = r.qs[j >> 2], qh = (j >> 2) ? r.qh >> 16 : r.qh & 0xFFFFu;
-    const int l = j & 3;
-    return {((const uint2*)tbl)[((qh >> 15) * MSQ_IQ1S_GRID_N + (((qh >> (3 * l)) & 7u) << 8)) + ((qs >> (8 * l)) & 0xFFu)]};
+  struct Raw { uint32_t qs[2]; uint32_t qh; uint32_t d; };  // qs bytes 8 q .. 8 q + 7; qh[2 q] | qh[2 q + 1] << 16; d in the high half
+  // The lane's bytes come through LDS. Fetched from memory in fragment order neighbouring lanes touch different rows: 290
+  // vector cache lookups per 16 rows and block (58 a load), one in every cycle of a launch with few tokens per expert; by
+  // pieces about 18 a load. 13 dwords of a row fit four pieces: one load per 16 rows. Piece p sits at place p ^ (row / 4) % 4.
+  static constexpr int PIECES = 4;
+  __device__ static uint32_t piece_at(uint32_t row, uint32_t p) { return p ^ ((row >> 2) & 3u); }
+  struct At { uint32_t x, tail, h0, h1, d; };
+  __device__ static At at_of(uint32_t row, uint32_t q) {
+    auto dw = [&](uint32_t i) { return row * (16u * PIECES) + 16u * piece_at(row, i >> 2) + 4u * (i & 3u); };
+    return {dw(2u * q), dw(2u * q + 2u), dw(8u + q), dw(9u + q), dw(0u)};
+  }
+  __device__ static Raw load(const At& at, uint32_t slot, uint32_t sel) {
+    const u32x2 x = lds_at<u32x2>(at.x, slot);
+    const uint32_t tail = lds_at<uint32_t>(at.tail, slot), h0 = lds_at<uint32_t>(at.h0, slot), h1 = lds_at<uint32_t>(at.h1, slot), d = lds_at<uint32_t>(at.d, slot);
+    return {{halves_of(x[0], x[1], sel), halves_of(x[1], tail, sel)}, halves_of(h0, h1, sel), halves_of(d, d, sel)};
+  }
+  struct Look { u32x2 g; };
+  using Low = uint32_t;
+  __device__ static uint32_t lane_low(uint32_t col) { return opaque((col & 1u) << 7); }
+  template <int J>
+  __device__ static Look lookup(const Raw& r, uint32_t low) {
+    constexpr int l = J & 3, sh = 3 * l + 16 * (J >> 2);  // the entry's three bits of qh start at bit sh
+    const uint32_t sgn = bits_from(0x40u, r.qh >> (J < 4 ? 9 : 25), low);
+    const uint32_t h8 = sh < 3 ? r.qh << (sh < 3 ? 3 - sh : 0) : r.qh >> (sh < 3 ? 0 : sh - 3);
+    return {lds_at<u32x2>(byte_over<l>(r.qs[J >> 2], bits_from(0x38u, h8, sgn)), 0u)};
   }
   // weight = fp16(s2 * (grid + delta)) with s2 = fp16(d (2 s + 1)): scale and product are rounded once each (the reference's
   // tile rounds the fp32 product once, src/kernels/quant_moe_prefill.metal:137-147)
-  __device__ static void finish(const Raw& r, int j, const Look& k, uint32_t (&h)[4]) {
-    const uint32_t qh = (j >> 2) ? r.qh >> 16 : r.qh & 0xFFFFu;
-    const float m = half_bits_to_float(r.d) * (float)(((qh >> 11) & 0xEu) | 1u);
-    const uint32_t m2 = pack_h2(m, m);
-    h[0] = pk_mul_f16(fp8_pair_to_h2<false>(k.g.x), m2); h[1] = pk_mul_f16(fp8_pair_to_h2<true>(k.g.x), m2);
-    h[2] = pk_mul_f16(fp8_pair_to_h2<false>(k.g.y), m2); h[3] = pk_mul_f16(fp8_pair_to_h2<true>(k.g.y), m2);
+  __device__ static uint32_t scale(const Raw& r, int sub) {
+    const uint32_t qh = sub ? r.qh >> 16 : r.qh & 0xFFFFu;
+    const float m = half_bits_to_float(r.d >> 16) * (float)(((qh >> 11) & 0xEu) | 1u);
+    return pack_h2(m, m);
+  }
+  __device__ static void finish(uint32_t m2, const Look& k, uint32_t (&h)[4]) {
+    h[0] = pk_mul_f16(fp8_pair_to_h2<false>(k.g[0]), m2); h[1] = pk_mul_f16(fp8_pair_to_h2<true>(k.g[0]), m2);
+    h[2] = pk_mul_f16(fp8_pair_to_h2<false>(k.g[1]), m2); h[3] = pk_mul_f16(fp8_pair_to_h2<true>(k.g[1]), m2);
   }
 };
 

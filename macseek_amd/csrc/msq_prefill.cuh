@@ -10,7 +10,9 @@
 // The routed experts and a shared expert of a codebook type go through the block GEMM below, a K-quant / Q8_0 shared
 // expert through the dense tile kernel of msq_prefill_tile.cuh.
 #pragma once
+#include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "msq_mfma.cuh"
 
@@ -18,12 +20,17 @@ namespace msq {
 
 // ------------------------------------------------------------------------------------------------ block GEMM
 // Grouped GEMM for the 256-weight codebook formats (block fragments, see msq_mfma.cuh). A work item is one expert's
-// block of up to 48 entries (T <= 3 token tiles) times a chunk of weight rows; the item's waves own different
-// weight-row tiles and walk K block by block (256 columns): the activation block [48][256] fp16 is staged in LDS for
+// block of entries (T token tiles of 16) times a chunk of weight rows; the item's waves own different
+// weight-row tiles and walk K block by block (256 columns): the activation block is staged in LDS for
 // all waves, every wave decodes the fragments of its own rows once per block and reuses each of them for all T token
-// tiles, accumulates the block in the matrix cores and applies the fp32 block scale once. Weights are decoded exactly
+// tiles, and accumulates in the matrix cores; the scale rides in the fragments. Weights are decoded exactly
 // once per (item, row), no lane loads a weight byte twice, and the next block's bytes are in flight during a block.
-// Table lookups run one fragment pair ahead of the pair being multiplied.
+// What bounds it. Small items (T <= 3): vector issue (14 instructions per eight weights of a lane, 61 % of the cycles), LDS (51 %)
+// and the texture addresser (53 %) beside each other, four waves per SIMD; 12 % (gate/up) to 30 % (down) is a workgroup's first
+// trip to memory and its end. Larger blocks: see pf_big_body. Against a variant that fetched IQ2_XXS rows lane by lane (three loads
+// a row, 50 vector cache lookups each), staged activations through registers and tested the tile count in every step
+// (27 instructions per eight weights): 2048 tokens, 384 IQ2_XXS experts of 7168x2048: gate/up 644 -> 554 us (T > 3) and 1080
+// -> 1050, down 348 -> 312 and 569 -> 555; IQ1_S 5120x2304, 37 tokens: the call 543 -> 477, 4096 tokens: 3534 -> 3268.
 struct PfBlkArgs {
   const uint16_t* A;        // fp16 activations [entries][K]
   const uint64_t* ptrs;     // per expert: gate, up, down addresses
@@ -39,266 +46,82 @@ struct PfBlkArgs {
   uint32_t row_groups;      // workgroups per item: row_chunks / chunks_per_wg, rounded up
 };
 
-constexpr int kPfBlkTokens = 48, kPfBigTokens = 112, kPfBigTiles = kPfBigTokens / 16, kPfBlkPitch = 256 * 2 + 16;
+constexpr int kPfBigTokens = 112, kPfBigTiles = kPfBigTokens / 16;
 // waves per workgroup by token tiles per item: four per SIMD for up to three tiles, three for more (registers)
 constexpr int pf_blk_waves(int T) { return T > 3 ? 12 : 16; }
 // weight-row tiles per wave: two fragments per K step (gate + up of one tile, or two tiles of the down matrix) keep the
 // register count low enough for three or four waves per SIMD, which is what overlaps decode, matrix and LDS work
 constexpr int pf_blk_rt(bool gu, int) { return gu ? 1 : 2; }
 constexpr int pf_blk_rows(bool gu, int T) { return pf_blk_waves(T) * pf_blk_rt(gu, T) * 16; }  // weight rows per work item
-// activation staging: double-buffered for up to three token tiles, a single buffer (two barriers per block) for seven
-constexpr size_t pf_blk_act_lds(int T) { return (T > 3 ? 1 : 2) * (size_t)(T > 3 ? kPfBigTokens : kPfBlkTokens) * kPfBlkPitch; }
-// A decoder with PIECES takes its bytes from LDS: a wave's block bytes of 16 rows (its R fragments: twice that) as
-// consecutive aligned 16-byte pieces, PIECES a row, by loads that write LDS themselves
+// Weight bytes come through LDS: a wave's block bytes of 16 rows (its two fragments: twice that), PIECES 16-byte pieces a
+// row, by loads that write LDS themselves
 template <class B>
-constexpr size_t pf_blk_raw_slot() { if constexpr (requires { B::PIECES; }) return 16 * 16 * B::PIECES; else return 0; }
+constexpr size_t pf_blk_raw_lds(int T) { return pf_blk_waves(T) * 2 * (16 * 16 * B::PIECES); }
+// Activations are staged by halves of a block: the columns of steps 0-3 and those of steps 4-7, in two planes each (chunks 0
+// and 2, chunks 1 and 3) of 128-byte rows. Unit 4 (q / 2) + j % 4 of a row sits at place unit ^ (row / 2) % 8. A 16-byte LDS
+// read serves the lanes in four groups of sixteen -- {0-7, 24-31}, {8-15, 16-23}, {32-39, 56-63}, {40-47, 48-55}, measured
+// -- so a group holds tokens 0-7 of one chunk and tokens 8-15 of its neighbour (lane = 16 q + token): sixteen different
+// bank groups. Two whole blocks (one barrier a block) where they fit, else one block, whose halves are refilled in turn.
+constexpr int pf_half_bytes(int T) { return 16 * T * 256; }
+constexpr size_t kPfLds = 160 * 1024;
 template <class B>
-constexpr size_t pf_blk_lds(int T) { return (size_t)B::LDS_WORDS * 4 + pf_blk_act_lds(T) + pf_blk_waves(T) * 2 * pf_blk_raw_slot<B>(); }
+constexpr bool pf_two_blocks(int T) { return T <= 3 && (size_t)B::LDS_WORDS * 4 + pf_blk_raw_lds<B>(T) + 4 * pf_half_bytes(T) <= kPfLds; }
+template <class B>
+constexpr size_t pf_act_lds(int T) { return (pf_two_blocks<B>(T) ? 4 : 2) * (size_t)pf_half_bytes(T); }
+// ... of a launch: T = 3 holds items of one to three tiles, T = 7 of four to seven
+template <class B>
+constexpr size_t pf_act_lds_of_launch(int T) { return T > 3 ? pf_act_lds<B>(T) : std::max({pf_act_lds<B>(1), pf_act_lds<B>(2), pf_act_lds<B>(3)}); }
+template <class B>
+constexpr size_t pf_blk_lds(int T) { return (size_t)B::LDS_WORDS * 4 + pf_act_lds_of_launch<B>(T) + pf_blk_raw_lds<B>(T); }
 
-// Where the 16 bytes of step j of chunk q (columns blk_col_of(q, j) .. + 7 of a block) sit in a token's staged row: the
-// chunks in the order 0, 2, 1, 3. A 16-byte LDS read serves the lanes in four groups of sixteen -- {0-7, 24-31},
-// {8-15, 16-23}, {32-39, 56-63}, {40-47, 48-55}, measured -- so a group holds tokens 0-7 of one chunk and tokens 8-15 of
-// its neighbour (lane = 16 q + token); rows are 33 sixteen-byte units apart, token n starts in bank group n mod 16, and the
-// two halves of a group only miss each other when the neighbouring chunks are a multiple of 256 bytes apart (in column
-// order they are 128 apart and every read took two passes).
-__device__ __forceinline__ uint32_t pf_lds_at(uint32_t q, uint32_t j) { return 16u * (16u * (q & 1u) + 8u * (q >> 1) + j); }
+template <int N, class F>
+__device__ __forceinline__ void static_for(F f) {
+  [&]<int... I>(std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }(std::make_integer_sequence<int, N>{});
+}
 
-template <class B, bool GU, int T>
-__device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
-  constexpr int WAVES = pf_blk_waves(T), NT = 64 * WAVES;
-  constexpr int NM = GU ? 2 : 1, RT = pf_blk_rt(GU, T), R = RT * NM, PITCH = kPfBlkPitch;
-  constexpr bool DB = T <= 3;  // two activation buffers
-  constexpr int ABUF = (DB ? kPfBlkTokens : kPfBigTokens) * PITCH;
-  constexpr int PPS = R / 2, NP = 8 * PPS;  // fragment pairs per K step, per block
-  static_assert(R == 2 || R == 4, "fragments are processed in pairs");
-  static_assert(T <= 3 || T == kPfBigTiles, "the single-buffer variant is sized for kPfBigTokens");
-  extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
-  uint32_t* tbl = smem;
-  uint8_t* abuf = (uint8_t*)(smem + B::LDS_WORDS);  // [2][T * 16 tokens][PITCH]
-  const uint32_t tid = threadIdx.x, lane = tid & 63u;
-  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-  const uint32_t n16 = lane & 15u, q = lane >> 4;
-
-  // consecutive workgroups land on different XCDs: the row chunks of one item stay on one XCD (shared L2 for its
-  // activations), and items are dealt round-robin over the XCDs
-  const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
-  const uint32_t item = (slot / a.row_groups) * 8u + xcd, rc0 = (slot % a.row_groups) * a.chunks_per_wg;
-  if (item >= a.nitems) return;
-  const uint32_t e = a.items[3 * item], t0 = a.items[3 * item + 1], cnt = a.items[3 * item + 2];
-  const uint32_t base = a.offs[e] + t0;
-  // A workgroup takes chunks_per_wg consecutive row chunks of its item, one after the other: the first trip to memory
-  // (about 4.5 us before the first block can be multiplied, 17 % of a down-projection workgroup's life) is paid once, and
-  // the next chunk's first block is requested during the last block of the one before, where a single chunk would
-  // fetch its last block again
-  // (built into the down projection of the small items only: the other variants have no registers to spare for it)
-  constexpr bool MULTI = !GU && T <= 3;
-  const uint32_t nch = MULTI ? min(a.chunks_per_wg, a.row_chunks - rc0) : 1u;
-
-  // a weight row = the expert's matrix (a scalar address) + the lane's row offset (32 bits: a matrix is far below 4 GiB)
-  gptr_t wbase[NM];
-  uint32_t woff[RT], row_of[RT];
-#pragma unroll
-  for (int m = 0; m < NM; m++) wbase[m] = as_global((const void*)a.ptrs[3 * e + (GU ? m : 2)]);
-#pragma unroll
-  for (int jt = 0; jt < RT; jt++) {
-    row_of[jt] = ((rc0 * WAVES + wave) * RT + jt) * 16u + n16;
-    woff[jt] = min(row_of[jt], a.N - 1) * a.row_bytes;
+// An expert's matrix: a descriptor over the whole aligned 16-byte pieces that hold it, and where in the first it starts.
+// (A matrix is far below 4 GiB; a weight row is then a 32-bit offset per lane and the block's a scalar one.)
+struct PfMatrix {
+  rsrc_t rs;
+  uint32_t mis, bytes;
+  __device__ __forceinline__ static PfMatrix of(const PfBlkArgs& a, uint64_t at) {
+    // (uniform, which an inline assembly operand has to be shown)
+    const uintptr_t base = ((uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32)) << 32) |
+                           (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
+    const uint32_t mis = (uint32_t)base & 15u, bytes = (mis + a.N * a.row_bytes + 15u) & ~15u;
+    return {make_rsrc((const void*)(base - mis), bytes), mis, bytes};
   }
-  auto wrow = [&](int r, uint32_t off) { return wbase[r % NM] + (size_t)(woff[r / NM] + off); };
-  // ... or, staged: bytes off .. of the 16 rows of fragment r into the wave's slot r; lane l of piece group k fetches piece
-  // 64 k + l. Rows past the matrix's end: no traffic.
-  constexpr bool STAGED = requires { B::PIECES; };
-  uint8_t* const raw_lds = abuf + pf_blk_act_lds(T) + wave * (uint32_t)(R * pf_blk_raw_slot<B>());
-  auto request = [&](int r, uint32_t off) {
-    if constexpr (STAGED) {
-      const uint64_t b64 = (uint64_t)(uintptr_t)wbase[r % NM];  // (uniform, which an inline assembly operand has to be shown)
-      const uintptr_t base = ((uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b64 >> 32)) << 32) |
-                             (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b64);
-      const uint32_t mis = (uint32_t)base & 15u, end = mis + a.N * a.row_bytes, bytes = (end + 15u) & ~15u;  // whole aligned pieces
-      const rsrc_t rs = make_rsrc((const void*)(base - mis), bytes);
-      const uint32_t tile = ((rc0 * WAVES + wave) * RT + r / NM) * 16u;
+};
+// The weight bytes of a wave's fragments: the block at scalar byte `at` of 16 rows, into an LDS slot of the wave's own. Lane l
+// of load k fetches the piece at place 64 k + l. (Dwords past the matrix's end lie past its descriptor's: zeros, no traffic.)
+template <class B>
+struct PfRows {
+  static constexpr int LOADS = (16 * B::PIECES + 63) / 64;
+  static constexpr uint32_t SLOT = 16 * 16 * B::PIECES;
+  uint32_t from[LOADS];  // where the lane's piece lies behind the first row's block
+  uint32_t sel;          // the lane's row: which half of a dword a block starts in when the first row's starts in the low one
+  __device__ __forceinline__ void init(uint32_t row_bytes, uint32_t lane) {
 #pragma unroll
-      for (uint32_t p0 = 0; p0 < 16u * B::PIECES; p0 += 64u) {
-        const uint32_t p = p0 + lane, v = mis + (tile + p / B::PIECES) * a.row_bytes + off;
-        if (p < 16u * B::PIECES) lds_dma16(rs, raw_lds + r * pf_blk_raw_slot<B>() + 16u * p0, v < end ? (v & ~15u) + 16u * (p % B::PIECES) : bytes, 0u);
-      }
+    for (int k = 0; k < LOADS; k++) {
+      const uint32_t l = 64u * k + lane, row = min(l / B::PIECES, 15u), place = l % B::PIECES;
+      from[k] = row * row_bytes + 16u * B::piece_at(row, place);  // (piece_at is its own inverse)
     }
-  };
-  auto fetched = [&](int r, uint32_t off) {  // (the lane's row; what the slot holds of rows past the end is never stored)
-    if constexpr (STAGED)
-      return B::load(LdsRow::of(raw_lds + r * pf_blk_raw_slot<B>() + n16 * (16u * B::PIECES),
-                                ((uint32_t)(uintptr_t)wbase[r % NM] + (((rc0 * WAVES + wave) * RT + r / NM) * 16u + n16) * a.row_bytes + off) & 15u), q);
-  };
-
-  // activation chunk loader: T * 512 granules of 16 bytes (token g / 32, column g % 32) over the workgroup's threads
-  constexpr int AG = (T * 512 + NT - 1) / NT;
-  u32x4 pa[AG];  // (a plain vector type: the HIP struct type keeps the array in scratch memory)
-  auto a_issue = [&](uint32_t kc) {
-#pragma unroll
-    for (int i = 0; i < AG; i++) {
-      // rows past the block's last entry repeat it (their products are never stored): no branch around the load, so
-      // the number of loads in flight stays known to every wait that follows
-      const uint32_t g = min(tid + i * NT, T * 512u - 1u);
-      const uint32_t tok = min(g >> 5, cnt - 1);
-      pa[i] = *(const u32x4*)(a.A + (size_t)(base + tok) * a.K + kc * 256u + (g & 31u) * 8u);
-    }
-  };
-  auto a_store = [&](uint32_t buf) {
-#pragma unroll
-    for (int i = 0; i < AG; i++) {
-      const uint32_t g = tid + i * NT;
-      if (g < T * 512u) *(u32x4*)(abuf + buf * ABUF + (g >> 5) * PITCH + pf_lds_at((g >> 3) & 3u, g & 7u)) = pa[i];
-    }
-  };
-
-  typename B::Raw cur[R], nxt[R];
-#pragma unroll
-  for (int r = 0; r < R; r++)
-    if constexpr (STAGED) request(r, 0u); else cur[r] = B::load(wrow(r, 0u), q);
-  a_issue(0);
-  B::fill_lds(tbl, (int)tid, NT);
-  a_store(0);
-  if constexpr (STAGED) {
-    wait_vm<0>();
-#pragma unroll
-    for (int r = 0; r < R; r++) cur[r] = fetched(r, 0u);
+    sel = ((lane & 15u) * row_bytes) & 2u ? SEL_LOW ^ SEL_FLIP : SEL_LOW;
   }
-  __syncthreads();
-
-  uint32_t kb = 0;  // blocks done so far (double buffering: block kb sits in buffer kb % 2)
-  for (uint32_t c = 0; c < nch; c++) {
-  const bool more = c + 1 < nch;
-  f4_t acc[T][R];
+  __device__ __forceinline__ void request(const PfMatrix& w, uint8_t* slot, uint32_t at, uint32_t lane) const {
 #pragma unroll
-  for (int t = 0; t < T; t++)
-#pragma unroll
-    for (int r = 0; r < R; r++) acc[t][r] = f4_t{0.f, 0.f, 0.f, 0.f};
-
-  for (uint32_t kc = 0; kc < a.nblocks; kc++, kb++) {
-    // the block requested during this one: the chunk's next, or the first of the workgroup's next chunk, or (nothing left)
-    // this one again: no branch around the loads
-    const bool lastb = kc + 1 == a.nblocks;
-    const uint32_t kn = !lastb ? kc + 1 : more ? 0u : kc;
-    // (the host lets a workgroup take several chunks only when all chunks are whole: the next chunk's rows are then the
-    // same number of bytes further for every lane)
-    const uint32_t wn = kn * (uint32_t)B::BLOCK_BYTES + (c + (lastb && more ? 1u : 0u)) * ((uint32_t)(WAVES * RT * 16) * a.row_bytes);
-    const uint8_t* arow = abuf + (DB ? (kb & 1u) * ABUF : 0u) + n16 * PITCH;
-    if constexpr (T > 3) {
-      // many token tiles: a step's fragments are all decoded first, then every tile's activation fragment (read from
-      // LDS two tiles ahead of its use) feeds one matrix instruction per fragment
-      uint32_t af[3][4];
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        // the next block's bytes are requested a few at a time between the steps: requested all at once by all waves
-        // right after the barrier, they queue up in the texture addresser and hold the waves at issue
-        if (j == 1) {
-          __builtin_amdgcn_sched_barrier(0);  // keep the requests here: the scheduler would sink them to their first use
-          a_issue(kn);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (j >= 2 && j - 2 < R) {
-          __builtin_amdgcn_sched_barrier(0);
-          if constexpr (STAGED) {
-            if (j == 2) wait_lgkm0();  // the slots are read: refill them
-            request(j - 2, wn);
-          } else {
-            nxt[j - 2] = B::load(wrow(j - 2, wn), q);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        typename B::Look lk[R];
-#pragma unroll
-        for (int r = 0; r < R; r++) lk[r] = B::lookup(cur[r], j, tbl, n16);
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-          const uint4 av = *(const uint4*)(arow + u * 16 * PITCH + pf_lds_at(q, j));
-          af[u][0] = av.x; af[u][1] = av.y; af[u][2] = av.z; af[u][3] = av.w;
-        }
-        uint32_t h[R][4];
-#pragma unroll
-        for (int r = 0; r < R; r++) B::finish(cur[r], j, lk[r], h[r]);
-#pragma unroll
-        for (int t = 0; t < T; t++) {
-          const uint32_t(&x)[4] = af[t % 3];
-          if (t + 2 < T) {
-            const uint4 av = *(const uint4*)(arow + (t + 2) * 16 * PITCH + pf_lds_at(q, j));
-            uint32_t(&y)[4] = af[(t + 2) % 3];
-            y[0] = av.x; y[1] = av.y; y[2] = av.z; y[3] = av.w;
-          }
-          if (16u * t < cnt) {  // (uniform) a block of fewer entries leaves its last tiles out
-#pragma unroll
-            for (int r = 0; r < R; r++) acc[t][r] = mfma_f16(x, h[r], acc[t][r]);
-          }
-        }
-      }
-    } else {
-    // table reads run one fragment pair ahead where registers allow (pair p = 2 j + half uses lk[p & 1]: fragments
-    // 2 half, 2 half + 1 of step j): the one-tile variant has four waves per SIMD to hide them behind instead, the
-    // three-tile variant six matrix instructions per pair
-    constexpr bool AHEAD = T == 2;
-    typename B::Look lk[2][2];
-    if (AHEAD) {
-      lk[0][0] = B::lookup(cur[0], 0, tbl, n16);
-      lk[0][1] = B::lookup(cur[1], 0, tbl, n16);
-    }
-    uint32_t af[T][4];
-#pragma unroll
-    for (int p = 0; p < NP; p++) {
-      const int j = p / PPS, r0 = 2 * (p % PPS);
-      // the next block's bytes are requested a few at a time between the fragment pairs: requested all at once by
-      // all waves right after the barrier, they queue up in the texture addresser and hold the waves at issue
-      if (p == 1) {
-        __builtin_amdgcn_sched_barrier(0);  // keep the requests here: the scheduler would sink them to their first use
-        a_issue(kn);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (p % 2 == 0 && p >= 2 && p / 2 - 1 < R) {
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (STAGED) {
-          if (p == 2) wait_lgkm0();
-          request(p / 2 - 1, wn);
-        } else {
-          nxt[p / 2 - 1] = B::load(wrow(p / 2 - 1, wn), q);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (p % PPS == 0) {  // activations of step j, read with the fragments' column mapping
-#pragma unroll
-        for (int t = 0; t < T; t++) {
-          const uint4 av = *(const uint4*)(arow + t * 16 * PITCH + pf_lds_at(q, j));
-          af[t][0] = av.x; af[t][1] = av.y; af[t][2] = av.z; af[t][3] = av.w;
-        }
-      }
-      if (!AHEAD) {
-        lk[p & 1][0] = B::lookup(cur[r0], j, tbl, n16);
-        lk[p & 1][1] = B::lookup(cur[r0 + 1], j, tbl, n16);
-      } else if (p + 1 < NP) {  // table reads of the next pair
-        const int jn = (p + 1) / PPS, rn = 2 * ((p + 1) % PPS);
-        lk[(p + 1) & 1][0] = B::lookup(cur[rn], jn, tbl, n16);
-        lk[(p + 1) & 1][1] = B::lookup(cur[rn + 1], jn, tbl, n16);
-      }
-      uint32_t h[2][4];
-      B::finish(cur[r0], j, lk[p & 1][0], h[0]);
-      B::finish(cur[r0 + 1], j, lk[p & 1][1], h[1]);
-#pragma unroll
-      for (int t = 0; t < T; t++) {
-        const uint32_t(&x)[4] = af[t];
-        acc[t][r0] = mfma_f16(x, h[0], acc[t][r0]);
-        acc[t][r0 + 1] = mfma_f16(x, h[1], acc[t][r0 + 1]);
-      }
-    }
-    }
-    // the other activation buffer was last read one block ago, before the previous barrier: free to refill (with a
-    // single buffer every wave has to be done with the block first)
-    if (!DB) __syncthreads();
-    a_store(DB ? (kb & 1u) ^ 1u : 0u);
-    if constexpr (STAGED) wait_vm<0>();
-#pragma unroll
-    for (int r = 0; r < R; r++)
-      if constexpr (STAGED) cur[r] = fetched(r, wn); else cur[r] = nxt[r];
-    __syncthreads();
+    for (int k = 0; k < LOADS; k++)
+      if (64 * (k + 1) <= 16 * B::PIECES || 64u * k + lane < 16u * B::PIECES) lds_dma16(w.rs, slot + 1024 * k, (from[k] + at) & ~3u, 0u);
   }
+  __device__ __forceinline__ typename B::Raw fetched(const typename B::At& lane_at, const uint8_t* slot, uint32_t at) const {
+    return B::load(lane_at, (uint32_t)(uintptr_t)(lds_cptr_t)slot, sel ^ (at & 2u ? SEL_FLIP : 0u));
+  }
+};
 
+// Results of an item's rows: SwiGLU and routing weight to H, or the plain sums to Z
+template <bool GU, int T, int RT>
+__device__ __forceinline__ void pf_epilogue(const PfBlkArgs& a, const f4_t (&acc)[T][GU ? 2 * RT : RT], uint32_t base, uint32_t cnt, uint32_t q,
+                                            const uint32_t (&row_of)[RT]) {
   float wts[T][4];  // routing weights of the lane's entries, fetched together ahead of the epilogue's math
 #pragma unroll
   for (int t = 0; t < T; t++)
@@ -328,10 +151,322 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
       }
     }
   }
+}
+
+template <class B, bool GU, int T>
+__device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
+  constexpr int WAVES = pf_blk_waves(T), NT = 64 * WAVES;
+  constexpr int NM = GU ? 2 : 1, RT = pf_blk_rt(GU, T), R = RT * NM;
+  constexpr int HALF = pf_half_bytes(T), PLANE = HALF / 2;
+  constexpr bool TWO = pf_two_blocks<B>(T);
+  static_assert(R == 2 && T <= 3, "fragments are processed in pairs; more token tiles: pf_big_body");
+  extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
+  uint8_t* abuf = (uint8_t*)(smem + B::LDS_WORDS);  // [TWO: 2][2 halves][2 planes][T * 16 tokens][128 bytes]
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t n16 = lane & 15u, q = lane >> 4;
+  const typename B::Low low = B::lane_low(n16);
+
+  // consecutive workgroups land on different XCDs: the row chunks of one item stay on one XCD (shared L2 for its
+  // activations), and items are dealt round-robin over the XCDs
+  const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+  const uint32_t item = (slot / a.row_groups) * 8u + xcd, rc0 = (slot % a.row_groups) * a.chunks_per_wg;
+  const uint32_t e = a.items[3 * item], t0 = a.items[3 * item + 1], cnt = a.items[3 * item + 2];
+  const uint32_t base = a.offs[e] + t0;
+  // A workgroup takes chunks_per_wg consecutive row chunks of its item, one after the other: the first trip to memory
+  // (about 4.5 us before the first block can be multiplied, 17 % of a down-projection workgroup's life) is paid once, and
+  // the next chunk's first block is requested during the last block of the one before, where a single chunk would
+  // fetch its last block again
+  // (built into the down projection of the small items only: the other variants have no registers to spare for it)
+  constexpr bool MULTI = !GU;
+  const uint32_t nch = MULTI ? min(a.chunks_per_wg, a.row_chunks - rc0) : 1u;
+
+  PfMatrix wm[NM];
+  uint32_t row_of[RT];
+#pragma unroll
+  for (int m = 0; m < NM; m++) wm[m] = PfMatrix::of(a, a.ptrs[3 * e + (GU ? m : 2)]);
+#pragma unroll
+  for (int jt = 0; jt < RT; jt++) row_of[jt] = ((rc0 * WAVES + wave) * RT + jt) * 16u + n16;
+  PfRows<B> rows;
+  rows.init(a.row_bytes, lane);
+  auto block_at = [&](int r, uint32_t off) { return wm[r % NM].mis + ((rc0 * WAVES + wave) * RT + r / NM) * 16u * a.row_bytes + off; };
+  const typename B::At at_row = B::at_of(n16, q);
+  uint8_t* const raw_lds = abuf + pf_act_lds_of_launch<B>(3) + wave * (R * PfRows<B>::SLOT);
+  auto request = [&](int r, uint32_t off) { rows.request(wm[r % NM], raw_lds + r * PfRows<B>::SLOT, block_at(r, off), lane); };
+  auto fetched = [&](int r, uint32_t off) { return rows.fetched(at_row, raw_lds + r * PfRows<B>::SLOT, block_at(r, off)); };
+
+  // activation loader. Piece g of a block (TWO) or of half h: row g / 32 (g / 16), then (half,) plane and unit.
+  constexpr int PB = TWO ? 5 : 4, AG = ((T << (4 + PB)) + NT - 1) / NT;
+  static_assert(TWO || AG == 1);
+  const rsrc_t ars = make_rsrc(a.A + (size_t)base * a.K, cnt * a.K * 2u);
+  uint32_t aoff[AG];
+  uint8_t* adst[AG];
+#pragma unroll
+  for (int i = 0; i < AG; i++) {
+    // rows past the block's last entry repeat it (their products are never stored): no branch around the load, so
+    // the number of loads in flight stays known to every wait that follows
+    const uint32_t g = min(tid + i * NT, (16u * T << PB) - 1u), row = g >> PB, h = TWO ? (g >> 4) & 1u : 0u, plane = (g >> 3) & 1u, unit = g & 7u;
+    aoff[i] = min(row, cnt - 1u) * (a.K * 2u) + (64u * (2u * (unit >> 2) + plane) + 32u * h + 8u * (unit & 3u)) * 2u;
+    adst[i] = abuf + h * HALF + plane * PLANE + row * 128u + 16u * (unit ^ ((row >> 1) & 7u));
+  }
+  u32x4 pa[TWO ? 1 : 2][AG];  // (a plain vector type: the HIP struct type keeps the array in scratch memory)
+  auto a_issue = [&](int h, uint32_t kc) {
+#pragma unroll
+    for (int i = 0; i < AG; i++) pa[h][i] = buf_ld128v(ars, aoff[i], kc * 512u + 64u * h);
+  };
+  auto a_store = [&](int h, uint32_t at) {
+#pragma unroll
+    for (int i = 0; i < AG; i++)
+      if (tid + i * NT < (16u * T << PB)) *(u32x4*)(adst[i] + at) = pa[h][i];
+  };
+  const uint32_t afrag = (uint32_t)(uintptr_t)(lds_cptr_t)abuf + (q & 1u) * PLANE + n16 * 128u + 16u * ((4u * (q >> 1)) ^ (n16 >> 1));
+  auto next_k = [&](uint32_t kc) { return kc + 1u < a.nblocks ? kc + 1u : 0u; };  // (past a workgroup's last block: the first again)
+
+  typename B::Raw cur[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) request(r, 0u);
+  a_issue(0, 0);
+  if constexpr (!TWO) a_issue(1, 0);
+  B::fill_lds(smem, (int)tid, NT);
+  a_store(0, 0);
+  if constexpr (!TWO) a_issue(0, next_k(0));
+  wait_vm<0>();
+#pragma unroll
+  for (int r = 0; r < R; r++) cur[r] = fetched(r, 0u);
+  __syncthreads();
+
+  constexpr bool A2 = T < 3, LA = GU || T < 3;  // activations, table entries read a step ahead (three tiles: registers)
+  typename B::Look lk[2][2];
+  if constexpr (LA) {
+    lk[0][0] = B::template lookup<0>(cur[0], low);
+    lk[0][1] = B::template lookup<0>(cur[1], low);
+  }
+  u32x4 af[A2 ? 2 : 1][T];
+  uint32_t sc[R];
+  uint32_t kb = 0;  // blocks done so far (double buffering: block kb sits in buffer kb % 2)
+  for (uint32_t c = 0; c < nch; c++) {
+  const bool more = c + 1 < nch;
+  f4_t acc[T][R];
+#pragma unroll
+  for (int t = 0; t < T; t++)
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[t][r] = f4_t{0.f, 0.f, 0.f, 0.f};
+
+  for (uint32_t kc = 0; kc < a.nblocks; kc++, kb++) {
+    // the block requested during this one: the chunk's next, or the first of the workgroup's next chunk, or (nothing left)
+    // this one again: no branch around the loads
+    const bool lastb = kc + 1 == a.nblocks;
+    const uint32_t kn = !lastb ? kc + 1 : more ? 0u : kc;
+    // (the host lets a workgroup take several chunks only when all chunks are whole: the next chunk's rows are then the
+    // same number of bytes further for every lane)
+    const uint32_t wn = kn * (uint32_t)B::BLOCK_BYTES + (c + (lastb && more ? 1u : 0u)) * ((uint32_t)(WAVES * RT * 16) * a.row_bytes);
+    const uint32_t at = afrag + (TWO ? (kb & 1u) * (2u * HALF) : 0u), ka = next_k(kc);
+    static_for<8>([&](auto j_) __attribute__((always_inline)) {
+      constexpr int j = j_;
+      constexpr bool fresh = !A2 || j == 0 || (!TWO && j == 4);  // behind a barrier: nothing could be read ahead of it
+      auto a_read = [&](int i) {  // activations of step i, read with the fragments' column mapping
+#pragma unroll
+        for (int t = 0; t < T; t++) af[A2 ? i & 1 : 0][t] = lds_at<u32x4>(at ^ (16u * (i & 3)), (i >> 2) * HALF + t * 2048);
+      };
+      // The reads of step j + 1 are issued ahead of the arithmetic of step j (the scheduler would sink them to their use, and
+      // the waves of a workgroup, in step behind every barrier, then take the LDS and the vector unit in turns)
+      __builtin_amdgcn_sched_barrier(0);
+      // the next block's bytes are requested a few at a time between the steps: requested all at once by
+      // all waves right after the barrier, they queue up in the texture addresser and hold the waves at issue
+      if constexpr (j < 2) request(j, wn);  // (the slots are read: the barrier has waited for that)
+      if constexpr (TWO && j == 3) a_issue(0, ka);
+      if constexpr (!TWO && j == 4) {
+        // one block staged: its second half arrives, into the buffer that the block before has left
+        a_store(1, HALF);
+        __syncthreads();
+        a_issue(1, ka);
+      }
+      if constexpr (fresh) a_read(j);
+      if constexpr (!LA || j < 7) {
+        constexpr int jl = LA ? j + 1 : j;
+        lk[jl & 1][0] = B::template lookup<jl & 7>(cur[0], low);
+        lk[jl & 1][1] = B::template lookup<jl & 7>(cur[1], low);
+      }
+      if constexpr (A2 && j < 7 && (TWO || j != 3)) a_read(j + 1);
+      if constexpr (j == 7) {  // the block's own bytes are used up
+        wait_vm<0>();
+#pragma unroll
+        for (int r = 0; r < R; r++) cur[r] = fetched(r, wn);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (j % 4 == 0) {
+#pragma unroll
+        for (int r = 0; r < R; r++) sc[r] = B::scale(cur[r], j / 4);
+      }
+      uint32_t h[2][4];
+      B::finish(sc[0], lk[j & 1][0], h[0]);
+      B::finish(sc[1], lk[j & 1][1], h[1]);
+#pragma unroll
+      for (int t = 0; t < T; t++) {
+        const u32x4 v = af[A2 ? j & 1 : 0][t];
+        const uint32_t x[4] = {v[0], v[1], v[2], v[3]};
+        acc[t][0] = mfma_f16(x, h[0], acc[t][0]);
+        acc[t][1] = mfma_f16(x, h[1], acc[t][1]);
+      }
+    });
+    __builtin_amdgcn_sched_barrier(0);
+    // the other buffer was last read one block ago (or, one block staged, ahead of the barrier between the halves)
+    a_store(0, TWO ? ((kb & 1u) ^ 1u) * (2u * HALF) : 0u);
+    if constexpr (LA) {
+      lk[0][0] = B::template lookup<0>(cur[0], low);
+      lk[0][1] = B::template lookup<0>(cur[1], low);
+    }
+    __syncthreads();
+    if constexpr (!TWO) a_issue(0, next_k(ka));
+  }
+
+  pf_epilogue<GU, T, RT>(a, acc, base, cnt, q, row_of);
   // the next chunk: its first block is in `cur` and in LDS already
 #pragma unroll
   for (int jt = 0; jt < RT; jt++) row_of[jt] += WAVES * RT * 16;
   }
+}
+
+// The blocks of 49 to 112 entries (T = 4 .. 7 token tiles, each with a body of its own: a test per tile and step splits
+// the loop into blocks that nothing is scheduled across). The matrix cores' T instructions per fragment should hide the
+// fourteen vector instructions of decoding; what keeps them at about half of that is three waves per SIMD in step:
+//   * the activations are staged by halves of a block (the columns of steps 0-3 and 4-7), one buffer each: while a half is
+//     multiplied the other one's buffer is refilled by loads that write LDS themselves, so the two barriers of a block stand
+//     between steps and not around a copy;
+//   * the fragments of step j + 1 are looked up at the start of step j and finished between its matrix instructions.
+template <class B, bool GU, int T>
+__device__ __forceinline__ void pf_big_body(const PfBlkArgs& a) {
+  constexpr int WAVES = pf_blk_waves(kPfBigTiles), NT = 64 * WAVES;
+  constexpr int NM = GU ? 2 : 1, RT = pf_blk_rt(GU, T), R = RT * NM;
+  constexpr int HALF = pf_half_bytes(T), PLANE = HALF / 2;
+  static_assert(R == 2 && T > 3 && T <= kPfBigTiles);
+  extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
+  uint8_t* abuf = (uint8_t*)(smem + B::LDS_WORDS);  // [2 halves][2 planes][112 tokens][128 bytes]
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t n16 = lane & 15u, q = lane >> 4;
+  const typename B::Low low = B::lane_low(n16);
+
+  // the row chunks of one item stay on one XCD (shared L2 for its activations), items are dealt round-robin over the XCDs
+  const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
+  const uint32_t item = (slot / a.row_groups) * 8u + xcd, rc = slot % a.row_groups;
+  const uint32_t e = a.items[3 * item], t0 = a.items[3 * item + 1], cnt = a.items[3 * item + 2];
+  const uint32_t base = a.offs[e] + t0;
+
+  PfMatrix wm[NM];
+  uint32_t row_of[RT];
+#pragma unroll
+  for (int m = 0; m < NM; m++) wm[m] = PfMatrix::of(a, a.ptrs[3 * e + (GU ? m : 2)]);
+#pragma unroll
+  for (int jt = 0; jt < RT; jt++) row_of[jt] = ((rc * WAVES + wave) * RT + jt) * 16u + n16;
+  PfRows<B> rows;
+  rows.init(a.row_bytes, lane);
+  auto block_at = [&](int r, uint32_t off) { return wm[r % NM].mis + ((rc * WAVES + wave) * RT + r / NM) * 16u * a.row_bytes + off; };
+  const typename B::At at_row = B::at_of(n16, q);
+  typename B::Raw cur[R];
+  uint8_t* const raw_lds = abuf + pf_act_lds_of_launch<B>(kPfBigTiles) + wave * (R * PfRows<B>::SLOT);
+  auto request = [&](int r, uint32_t off) { rows.request(wm[r % NM], raw_lds + r * PfRows<B>::SLOT, block_at(r, off), lane); };
+  auto fetched = [&](int r, uint32_t off) { return rows.fetched(at_row, raw_lds + r * PfRows<B>::SLOT, block_at(r, off)); };
+
+  // activation loader: a half of a block is 4 T kilobytes, a load (eight rows of a plane) each; wave w's are w, w + 12, ...
+  constexpr int AL = 4 * T, AMIN = AL / WAVES, AMAX = (AL + WAVES - 1) / WAVES;
+  const rsrc_t ars = make_rsrc(a.A + (size_t)base * a.K, cnt * a.K * 2u);
+  uint32_t aoff[AMAX];
+#pragma unroll
+  for (int i = 0; i < AMAX; i++) {  // rows past the block's last entry repeat it (their products are never stored)
+    const uint32_t l = wave + i * WAVES, plane = l >= 2u * T ? 1u : 0u, row = 8u * (l - plane * 2u * T) + (lane >> 3), unit = (lane & 7u) ^ ((row >> 1) & 7u);
+    aoff[i] = min(row, cnt - 1u) * (a.K * 2u) + (64u * (2u * (unit >> 2) + plane) + 8u * (unit & 3u)) * 2u;
+  }
+  const bool amore = wave + AMIN * WAVES < AL;  // (uniform) one load more than the waves that have the fewest
+  auto a_request = [&](int h, uint32_t kc) {
+#pragma unroll
+    for (int i = 0; i < AMAX; i++)
+      if (i < AMIN || amore) lds_dma16(ars, abuf + h * HALF + (wave + i * WAVES) * 1024u, aoff[i], kc * 512u + 64u * h);
+  };
+  constexpr int WLOADS = R * PfRows<B>::LOADS;
+  // where the lane's fragments of step 0 start (tile t: 2048 bytes further; step j: the place's low bits the other way)
+  uint32_t afrag = (uint32_t)(uintptr_t)(lds_cptr_t)abuf + (q & 1u) * PLANE + n16 * 128u + 16u * ((4u * (q >> 1)) ^ (n16 >> 1));
+
+#pragma unroll
+  for (int r = 0; r < R; r++) request(r, 0u);
+  a_request(0, 0);
+  B::fill_lds(smem, (int)tid, NT);
+  wait_vm<0>();
+#pragma unroll
+  for (int r = 0; r < R; r++) cur[r] = fetched(r, 0u);
+  __syncthreads();
+
+  f4_t acc[T][R];
+#pragma unroll
+  for (int t = 0; t < T; t++)
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[t][r] = f4_t{0.f, 0.f, 0.f, 0.f};
+  uint32_t h[2][R][4], sc[R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    sc[r] = B::scale(cur[r], 0);
+    B::finish(sc[r], B::template lookup<0>(cur[r], low), h[0][r]);
+  }
+  // activation fragments are read AHEAD tiles before their use, across the ends of steps
+  constexpr int AHEAD = 3, RING = 4;
+  uint32_t af[RING][4];
+  auto a_read = [&](int i) {  // i: step T + tile of the block
+    const int j = i / T & 7, t = i % T;
+    const u32x4 av = lds_at<u32x4>(afrag ^ (16u * (j & 3)), (j >> 2) * HALF + t * 2048);
+#pragma unroll
+    for (int k = 0; k < 4; k++) af[i % RING][k] = av[k];
+  };
+  // (8 T is a multiple of the ring's four places: a block's first tile is always in the same one)
+#pragma unroll
+  for (int i = 0; i < AHEAD; i++) a_read(i);
+
+  for (uint32_t kc = 0; kc < a.nblocks; kc++) {
+    const uint32_t kn = min(kc + 1u, a.nblocks - 1u), wn = kn * (uint32_t)B::BLOCK_BYTES;  // (the last block is fetched again)
+    typename B::Look lk;
+    afrag = opaque(afrag);  // (one register: the steps' places are not worth keeping)
+    static_for<8 * T>([&](auto i_) __attribute__((always_inline)) {
+      constexpr int i = i_, j = i / T, t = i % T, jn = (j + 1) & 7;
+      // The order below is the order of issue (the scheduler would sink every read to its use)
+      __builtin_amdgcn_sched_barrier(0);
+      // Loads complete in order, and nothing but these is in flight, so a wait names the loads behind what it waits for.
+      // Half 1 of this block, into the buffer that the block before has left; the next block's weight bytes (the slots are
+      // read: the barrier has waited for that), a few at a time: all at once they queue up in the texture addresser.
+      if constexpr (i == 0) a_request(1, kc);
+      if constexpr (i == 1 || i == 3) request(i / 2, wn);
+      // the last reads of a half are issued: what follows comes from the other buffer
+      if constexpr (j == 3 && t == T - AHEAD) {
+        wait_vm<WLOADS>();
+        __syncthreads();
+        a_request(0, kn);
+      }
+      if constexpr (j == 7 && t == 0) {  // the block's own bytes are used up
+        if (amore) wait_vm<AMIN + 1>(); else wait_vm<AMIN>();
+#pragma unroll
+        for (int r = 0; r < R; r++) cur[r] = fetched(r, wn);
+      }
+      if constexpr (j == 7 && t == T - AHEAD) {
+        wait_vm<0>();
+        __syncthreads();
+      }
+      a_read(i + AHEAD);
+      // the next step's fragments, one after the other
+      if constexpr (t == 0) lk = B::template lookup<jn>(cur[0], low);
+      if constexpr (t == T / 2) {
+        if constexpr ((jn & 3) == 0) sc[0] = B::scale(cur[0], jn / 4);
+        B::finish(sc[0], lk, h[jn & 1][0]);
+        lk = B::template lookup<jn>(cur[1], low);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < R; r++) acc[t][r] = mfma_f16(af[i % RING], h[j & 1][r], acc[t][r]);
+      if constexpr (t == T - 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr ((jn & 3) == 0) sc[1] = B::scale(cur[1], jn / 4);
+        B::finish(sc[1], lk, h[jn & 1][1]);
+      }
+    });
+  }
+  pf_epilogue<GU, T, RT>(a, acc, base, cnt, q, row_of);
 }
 
 // Kernel variants: T = 3 takes the items of up to three token tiles in one launch, largest first (each runs the body
@@ -339,12 +474,15 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
 // popular experts are cut into (their weights are then decoded once per 112 entries; 12 waves, one activation buffer).
 template <class B, bool GU, int T>
 __global__ __launch_bounds__(64 * pf_blk_waves(T)) void moe_pf_block_kernel(const PfBlkArgs a) {
+  const uint32_t item = ((blockIdx.x >> 3) / a.row_groups) * 8u + (blockIdx.x & 7u);
+  if (item >= a.nitems) return;
+  const uint32_t cnt = a.items[3 * item + 2];
   if constexpr (T > 3) {
-    pf_block_body<B, GU, T>(a);
+    if (cnt > 96) pf_big_body<B, GU, 7>(a);
+    else if (cnt > 80) pf_big_body<B, GU, 6>(a);
+    else if (cnt > 64) pf_big_body<B, GU, 5>(a);
+    else pf_big_body<B, GU, 4>(a);
   } else {
-    const uint32_t item = ((blockIdx.x >> 3) / a.row_groups) * 8u + (blockIdx.x & 7u);
-    if (item >= a.nitems) return;
-    const uint32_t cnt = a.items[3 * item + 2];
     if (cnt > 32) pf_block_body<B, GU, 3>(a);
     else if (cnt > 16) pf_block_body<B, GU, 2>(a);
     else pf_block_body<B, GU, 1>(a);

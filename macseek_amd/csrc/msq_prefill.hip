@@ -113,13 +113,13 @@ SideStream* side_stream(hipStream_t st) {
 // items are sorted by size, largest first: n6 blocks of more than 48 entries, n3 items of three token tiles, n2 of two,
 // then the one-tile items: the blocks in one launch, everything up to three tiles in another (one tail of half-idle CUs
 // instead of two); skip: profiling mask (see msq_moe_prefill)
-template <class B, bool GU>
+template <class BIG, class B, bool GU>
 int launch_block_t(hipStream_t st, PfBlkArgs a, uint32_t n6, uint32_t n3, uint32_t n2, int skip) {
   const uint32_t* items = a.items;
   const uint32_t n = a.nitems;
   int rc;
   a.items = items; a.nitems = n6;
-  if (!(skip & 256) && (rc = launch_block_tt<B, GU, kPfBigTiles>(st, a))) return rc;
+  if (!(skip & 256) && (rc = launch_block_tt<BIG, GU, kPfBigTiles>(st, a))) return rc;
   const uint32_t lo = (skip & 128) ? n6 + n3 + n2 : n6, hi = (skip & 64) ? n6 + n3 + n2 : n;
   a.items = items + 3 * (size_t)lo; a.nitems = hi > lo ? hi - lo : 0u;
   return launch_block_tt<B, GU, 3>(st, a);
@@ -127,8 +127,8 @@ int launch_block_t(hipStream_t st, PfBlkArgs a, uint32_t n6, uint32_t n3, uint32
 bool block_path(int t) { return t == MSQ_IQ1_S || t == MSQ_IQ2_XXS; }
 template <bool GU>
 int launch_block(int t, hipStream_t st, const PfBlkArgs& a, uint32_t n6, uint32_t n3, uint32_t n2, int skip) {
-  return t == MSQ_IQ1_S ? launch_block_t<BlkIQ1S, GU>(st, a, n6, n3, n2, skip)
-                        : launch_block_t<BlkIQ2XXS, GU>(st, a, n6, n3, n2, skip);
+  return t == MSQ_IQ1_S ? launch_block_t<BlkIQ1S, BlkIQ1S, GU>(st, a, n6, n3, n2, skip)
+                        : launch_block_t<BlkIQ2XXS<4>, BlkIQ2XXS<16>, GU>(st, a, n6, n3, n2, skip);
 }
 
 }  // namespace

@@ -1,0 +1,21 @@
+"""The block GEMM of msq_moe_prefill with every number of token tiles an item can have, each full, one short of full and
+with one entry in its last tile; one block of K (nothing to fetch ahead) and several, an odd and an even number."""
+import pytest
+
+import oracle as O
+import test_moe_prefill_gpu as P
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [113, 112, 111, 97, 96, 81, 80, 65, 64, 49, 48, 47, 33, 32, 17, 16, 1]
+
+
+@pytest.mark.parametrize("t", [O.IQ1_S, O.IQ2_XXS], ids=["IQ1_S", "IQ2_XXS"])
+@pytest.mark.parametrize("dim,inter", [(256, 512), (768, 256), (1024, 768)])
+def test_every_number_of_token_tiles(dev, monkeypatch, t, dim, inter):
+    n, k = max(SIZES), len(SIZES)
+    monkeypatch.setattr(P, "make_routing", lambda *_: [[e for e in range(k) if i < SIZES[e]] for i in range(n)])
+    c = P.build(t, t, O.Q6_K, n, k, k, False, "", dim, inter)
+    y, same = P.run_gpu(c)
+    err_h, err_f, _ = P.check(c, y, 0)
+    assert same and err_h <= 1e-3 and err_f <= 5e-3  # the bounds of test_moe_prefill_gpu.py (the reference's)
