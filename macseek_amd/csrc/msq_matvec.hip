@@ -260,11 +260,13 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   // one / in pairs: Q6_K 129280x5120 113.2 / 99.8 us, 1536x7168 6.41 / 6.10, 2304x5120 6.61 / 6.29, Q8_0 2304x5120
   // 6.67 / 6.52; the codebook formats, bound by their lookups, lose 1 % and keep the one-row form. MSQ_MV_PAIR = 0 / 2:
   // never / every format.
+  // Under a fused norm likewise, but for Q8_0 below 20 MB (4096x2560 6.19 / 6.40).
+  const double bytes = (double)a.rows * a.row_bytes;
   bool pair = false;
   {
     static const int env_pair = env_knob_early("MSQ_MV_PAIR", -1);
     const int u = (int)(a.cols / D::UNIT), k1 = (u + 63) / 64, k2 = (2 * u + 63) / 64;
-    pair = s.iters == 1 && s.free_shape && (D::LDS_WORDS == 0 || env_pair == 2) && !a.norm_w && env_pair != 0 && a.rows % 2 == 0 && a.rows_per_group >= a.rows && u % 16 == 0 &&
+    pair = s.iters == 1 && s.free_shape && (D::LDS_WORDS == 0 || env_pair == 2) && !(a.norm_w && std::is_same_v<D, DecQ8_0> && bytes < 20e6) && env_pair != 0 && a.rows % 2 == 0 && a.rows_per_group >= a.rows && u % 16 == 0 &&
            k2 < 2 * k1 && k2 <= 8;
     if (pair) {
       a.rows /= 2;
@@ -288,7 +290,10 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
     // one workgroup per CU: all of its LDS (decoders that stage only in the four-token kernel read directly when a round does not fit)
     if (!place_x_row(a, lds, tok_round<D, T>(), kMaxLds - kStaticLds<D>, D::STAGE_X)) return MSQ_ERR_UNSUPPORTED;
   }
-  const bool sw = tok_stages_w<D, 1, T>() && s.iters == 1 && s.stage_w && !a.norm_w;
+  // Under a fused norm weight rows go through LDS from 17 MB on (Q6_K 4096x4608 8.5 / 9.2 us, 4096x7168 11.2 / 10.8, 16384x5120
+  // 23.7 / 19.0, 129280x5120 138 / 101), but for Q6_K rows of whole waves of 200 MB and more (129280x2048 38.5 / 40.1).
+  const bool norm_sw = bytes >= 17e6 && (std::is_same_v<D, DecQ8_0> || bytes < 200e6 || (a.cols / D::UNIT) % 64 != 0);
+  const bool sw = tok_stages_w<D, 1, T>() && s.iters == 1 && s.stage_w && (!a.norm_w || norm_sw);
   if (sw) {  // the waves' weight-row buffers
     lds = (lds + 15) / 16 * 16;
     a.w_off = (uint32_t)(lds / 4);
@@ -298,22 +303,31 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
     allow_large_lds(kernel, lds);
     hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a.W, a.rows, a.row_bytes, a.units, a.ks, a.rpw, a.ntiles, a.rows_per_group, a.x, a.cols, ta);
   };
+  // persistent workgroups, one per CU over all token groups (two for a large matrix: MvShape::per_cu)
+  // A fused norm's prologue of one trip leaves Q5_K, Q6_K rows in registers (144) and two units of F32 no room for a second one:
+  // they would run one by one (Q5_K 16384x7168 0.89 of the speed, F32 768x5120 0.79; IQ4_NL, Q8_0 and the fp16 types gain 3 to 25 %).
+  const bool one_trip = a.norm_w && norm_one_trip<D>(true, a.cols, bytes, device_info().cus, threads);
+  constexpr bool wide = std::is_same_v<D, DecQ5KQ> || std::is_same_v<D, DecQ6KQ>;
+  const bool alone = one_trip && ((wide && !sw) || (std::is_same_v<D, DecDense<MSQ_F32>> && s.iters > 1));
+  const int per_cu = (T == 1 && !alone && (lds + kStaticLds<D>) * s.per_cu <= (size_t)kMaxLds) ? s.per_cu : 1;
+  const int gx = (int)std::min<long>(a.ntiles, std::max(1, per_cu * device_info().cus / gy));
+  const dim3 grid((unsigned)gx, (unsigned)gy);
   if (a.norm_w) {  // fused input norm (single token)
     if constexpr (T != 1 || requires { D::STAGES; }) return MSQ_ERR_UNSUPPORTED;
     else {
-      const dim3 gxn((unsigned)std::min<long>(a.ntiles, std::max(1, device_info().cus)));
-      const bool one = norm_one_trip<D>(true, a.cols, (double)a.rows * a.row_bytes, (int)gxn.x, threads);
-      if (s.iters == 1) one ? launch(mv_tok_kernel<D, 1, 1, kNormOneTrip>, gxn) : launch(mv_tok_kernel<D, 1, 1, kNormTwoTrips>, gxn);
-      else if constexpr (D::UNIT == 8) one ? launch(mv_tok_kernel<D, 2, 1, kNormOneTrip>, gxn) : launch(mv_tok_kernel<D, 2, 1, kNormTwoTrips>, gxn);
+      auto by_norm = [&]<int ITERS, bool SW, bool PAIR>() {
+        one_trip ? launch(mv_tok_kernel<D, ITERS, 1, kNormOneTrip, SW, PAIR>, grid) : launch(mv_tok_kernel<D, ITERS, 1, kNormTwoTrips, SW, PAIR>, grid);
+      };
+      if (sw) {
+        if constexpr (tok_stages_w<D, 1, 1>()) pair ? by_norm.template operator()<1, true, true>() : by_norm.template operator()<1, true, false>();
+      } else if (s.iters == 1) {
+        pair ? by_norm.template operator()<1, false, true>() : by_norm.template operator()<1, false, false>();
+      } else if constexpr (D::UNIT == 8) by_norm.template operator()<2, false, false>();
       else return MSQ_ERR_UNSUPPORTED;
       MSQ_HIP(hipGetLastError());
       return MSQ_OK;
     }
   }
-  // persistent workgroups, one per CU over all token groups (two for a large matrix: MvShape::per_cu)
-  const int per_cu = (T == 1 && !a.norm_w && (lds + kStaticLds<D>) * s.per_cu <= (size_t)kMaxLds) ? s.per_cu : 1;
-  const int gx = (int)std::min<long>(a.ntiles, std::max(1, per_cu * device_info().cus / gy));
-  const dim3 grid((unsigned)gx, (unsigned)gy);
   if (sw) {
     if constexpr (tok_stages_w<D, 1, T>()) {
       if (pair) launch(mv_tok_kernel<D, 1, T, kNormNone, true, true>, grid);

@@ -131,3 +131,18 @@ LINES = [
 @pytest.mark.parametrize("t,rows,cols", LINES, ids=lambda v: None)
 def test_both_prologues_of_the_fused_norm(dev, t, rows, cols):
     test_fused_equals_norm_then_matvec_and_oracle(dev, t, rows, cols)
+
+
+# weight rows through LDS, two rows as one, a second workgroup per CU under a fused norm, on either side of each line: Q6_K at
+# 17 MB (rows in pairs; an odd number of rows; whole waves) and 200 MB (whole waves), Q8_0 at 20 MB (pairs) and 40 MB, two
+# workgroups from 48 MB (Q5_K with either prologue) and 8 MB (dense; F32 of one and two units a lane)
+LARGE = [
+    (O.Q6_K, 4000, 5120), (O.Q6_K, 4096, 5120), (O.Q6_K, 4097, 5120), (O.Q6_K, 10300, 2048), (O.Q6_K, 16390, 3584), (O.Q6_K, 119500, 2048),
+    (O.Q8_0, 7300, 2560), (O.Q8_0, 7400, 2560), (O.Q8_0, 14800, 2560), (O.Q8_0, 9200, 4096), (O.Q5_K, 16400, 4608), (O.Q5_K, 34200, 2048),
+    (O.IQ4_NL, 16800, 5120), (O.F32, 600, 4096), (O.F32, 600, 5120), (O.BF16, 4100, 1280),
+]
+
+
+@pytest.mark.parametrize("t,rows,cols", LARGE, ids=lambda v: None)
+def test_fused_norm_of_large_matrices(dev, t, rows, cols):
+    test_fused_equals_norm_then_matvec_and_oracle(dev, t, rows, cols)
