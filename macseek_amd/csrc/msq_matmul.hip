@@ -87,10 +87,8 @@ int launch_f32_to_f16(hipStream_t st, const float* X, uint16_t* X16, size_t coun
 }
 
 int launch_deq_f16(hipStream_t st, int t, const uint8_t* W, uint16_t* out, int64_t n_elems) {
-  const int64_t nchunks = n_elems / 8;
-  const dim3 grid((unsigned)((nchunks + 255) / 256)), block(256);
   switch (t) {
-#define MSQ_DEQH(T) case T: hipLaunchKernelGGL((dequant_kernel<T, uint16_t>), grid, block, 0, st, W, out, nchunks); break;
+#define MSQ_DEQH(T) case T: launch_dequant<T>(st, W, out, n_elems); break;
     MSQ_DEQH(MSQ_F32) MSQ_DEQH(MSQ_BF16) MSQ_DEQH(MSQ_Q8_0) MSQ_DEQH(MSQ_IQ4_NL) MSQ_DEQH(MSQ_IQ1_S) MSQ_DEQH(MSQ_IQ2_XXS)
     MSQ_DEQH(MSQ_Q6_K) MSQ_DEQH(MSQ_Q5_K)
 #undef MSQ_DEQH

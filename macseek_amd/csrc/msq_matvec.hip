@@ -568,11 +568,9 @@ int msq_dequant(void* stream, int t, const MsqBuffer* W, int64_t n, const MsqBuf
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: dequant: buffer missing or too small");
   const uint8_t* src = bptr(W);
   float* dst = (float*)bptr_mut(out);
-  const int64_t nchunks = n / 8;
-  const dim3 grid((unsigned)((nchunks + 255) / 256)), block(256);
   hipStream_t st = (hipStream_t)stream;
   switch (t) {
-#define MSQ_DEQ(T) case T: hipLaunchKernelGGL((dequant_kernel<T>), grid, block, 0, st, src, dst, nchunks); break;
+#define MSQ_DEQ(T) case T: launch_dequant<T>(st, src, dst, n); break;
     MSQ_DEQ(MSQ_F32) MSQ_DEQ(MSQ_F16) MSQ_DEQ(MSQ_BF16) MSQ_DEQ(MSQ_Q8_0) MSQ_DEQ(MSQ_IQ4_NL) MSQ_DEQ(MSQ_IQ1_S)
     MSQ_DEQ(MSQ_IQ2_XXS) MSQ_DEQ(MSQ_Q6_K) MSQ_DEQ(MSQ_Q5_K)
 #undef MSQ_DEQ
