@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restric
 // expert row and leaving the expert's logit, score and key in scratch; the workgroup that finishes last (device-scope
 // counter, one increment per workgroup: n_exp / 4 of them contend, not n_exp) selects from the keys, then re-arms the
 // counter. W is F32 (QT = MSQ_F32) or BF16. No bit of the result depends on which workgroup is last.
-template <int QT>
+template <int QT, uint32_t U>
 __global__ __launch_bounds__(256) void router_fused_kernel(const float* __restrict__ x, const void* __restrict__ W, uint32_t dim,
                                                            uint32_t n_exp, const float* __restrict__ bias, float* logits,
                                                            RouterRec* recs, uint32_t* counter, int* __restrict__ ids,
@@ -120,8 +120,7 @@ __global__ __launch_bounds__(256) void router_fused_kernel(const float* __restri
   __shared__ uint32_t last;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, e = blockIdx.x * 4u + wave;
   // the row's weights are requested U vectors per lane at a time before any is used: with one wave per row the loop is
-  // otherwise a chain of memory latencies
-  constexpr uint32_t U = 8;
+  // otherwise a chain of memory latencies (the launcher picks U)
   float acc = 0.f;
   if constexpr (QT == MSQ_F32) {
     const float4* wr = (const float4*)((const float*)W + (size_t)e * dim);
@@ -389,14 +388,20 @@ int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffe
   uint32_t* counter = (uint32_t*)(bptr_mut(scratch) + msq_router_scratch_bytes(n_exp) - 256);
   const dim3 grid((unsigned)(n_exp / 4)), block(256);
   hipStream_t st = (hipStream_t)stream;
-  if (wtype == MSQ_F32)
-    hipLaunchKernelGGL((router_fused_kernel<MSQ_F32>), grid, block, 0, st, (const float*)bptr(x), (const void*)bptr(W),
-                       (uint32_t)dim, (uint32_t)n_exp, (const float*)bptr(bias), logits, recs, counter, (int*)bptr_mut(ids),
-                       (float*)bptr_mut(w), route_scale);
-  else
-    hipLaunchKernelGGL((router_fused_kernel<MSQ_BF16>), grid, block, 0, st, (const float*)bptr(x), (const void*)bptr(W),
-                       (uint32_t)dim, (uint32_t)n_exp, (const float*)bptr(bias), logits, recs, counter, (int*)bptr_mut(ids),
-                       (float*)bptr_mut(w), route_scale);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, (const float*)bptr(x), (const void*)bptr(W), (uint32_t)dim, (uint32_t)n_exp,
+                       (const float*)bptr(bias), logits, recs, counter, (int*)bptr_mut(ids), (float*)bptr_mut(w), route_scale);
+  };
+  // One trip to memory for a row of nine to twelve vectors a lane (4097 to 6144 columns of BF16, half of F32) instead of two: 384
+  // BF16 experts x 5120 10.6 -> 10.0 us. Thirteen and more gain nothing (7168 columns 11.3 / 11.0, in the layer the same).
+  const int per_lane = (dim / (wtype == MSQ_F32 ? 4 : 8) + 63) / 64;
+  auto by_u = [&]<int QT>() {
+    if (per_lane == 9 || per_lane == 10) launch(router_fused_kernel<QT, 10>);
+    else if (per_lane == 11 || per_lane == 12) launch(router_fused_kernel<QT, 12>);
+    else launch(router_fused_kernel<QT, 8>);
+  };
+  if (wtype == MSQ_F32) by_u.template operator()<MSQ_F32>();
+  else by_u.template operator()<MSQ_BF16>();
   MSQ_HIP(hipGetLastError());
   return MSQ_OK;
 }

@@ -244,3 +244,10 @@ def test_route_lists_over_waves_and_rounds(dev, n, n_exp):
     slot = np.full(6 * n, -5)
     slot[order] = np.arange(m)
     assert np.array_equal(L.t_slot_of.cpu().numpy()[: 6 * n], slot)
+
+
+# rows of as many vectors a lane as one trip to memory takes, one vector more, and the kernels of ten and twelve
+@pytest.mark.parametrize("dim", [4096, 4104, 5120, 5128, 6144, 6152])
+@pytest.mark.parametrize("wtype", [q.QType.BF16, q.QType.F32])
+def test_router_fused_row_lengths(dev, wtype, dim):
+    test_router_fused_vs_oracle(dev, wtype, dim if wtype == q.QType.BF16 else dim // 2)
