@@ -247,7 +247,6 @@ def test_route_lists_over_waves_and_rounds(dev, n, n_exp):
 
 
 # rows of as many vectors a lane as one trip to memory takes, one vector more, and the kernels of ten and twelve
-@pytest.mark.parametrize("dim", [4096, 4104, 5120, 5128, 6144, 6152])
-@pytest.mark.parametrize("wtype", [q.QType.BF16, q.QType.F32])
+@pytest.mark.parametrize("wtype,dim", [(q.QType.BF16, d) for d in (4096, 4104, 5120, 5128, 6144, 6152)] + [(q.QType.F32, d) for d in (2048, 2056, 2560, 2568, 3072, 3080)])
 def test_router_fused_row_lengths(dev, wtype, dim):
-    test_router_fused_vs_oracle(dev, wtype, dim if wtype == q.QType.BF16 else dim // 2)
+    test_router_fused_vs_oracle(dev, wtype, dim)
