@@ -43,7 +43,33 @@ struct PfBlkArgs {
   uint32_t K, N, row_bytes, nblocks;
   uint32_t row_chunks;      // chunks of pf_blk_rows() weight rows
   uint32_t chunks_per_wg;   // consecutive row chunks one workgroup takes, one after the other
-  uint32_t row_groups;      // workgroups per item: row_chunks / chunks_per_wg, rounded up
+  uint32_t row_groups;      // units of work per item: row_chunks / chunks_per_wg, rounded up
+  uint32_t per_xcd;         // units of an XCD (see PfUnit)
+  uint32_t* queue;          // eight counters, one per XCD: units taken beyond those that the workgroups start with; or null
+};
+
+// A unit of work is one item's row chunks of one workgroup. Unit 8 s + x belongs to XCD x: the units of one item stay on one
+// XCD (shared L2 for its activations), and items are dealt round-robin over the XCDs; consecutive workgroups land on
+// different XCDs. There is a workgroup for every unit, or (QUEUE) as many as the chip holds: a workgroup then takes units of
+// its XCD until they are used up, the first by its number, the others from the XCD's counter. The tables are in LDS once, and a
+// unit does not wait for the workgroup before it to be taken down and its own to be set up (4096 tokens of IQ1_S: blocks of
+// the first product 942 -> 859 us, calls 3349 -> 3160; 2048 of IQ2_XXS 2500 -> 2470). The rule is at the launch.
+// (The tables are read as constants, which they are while the kernel runs: scalar loads, and an expert's offset and addresses
+// in one trip.)
+struct PfUnit {
+  uint32_t cnt, base;  // the item's entries (none: the last items of eight may be missing), the first one
+  uint32_t group;
+  uint64_t w[2];       // the expert's matrices: gate and up, or down
+  template <bool GU>
+  __device__ __forceinline__ static PfUnit of(const PfBlkArgs& a, uint32_t s) {
+    const uint32_t item = (s / a.row_groups) * 8u + (blockIdx.x & 7u);
+    if (item >= a.nitems) return PfUnit{};
+    const auto items = (const __attribute__((address_space(4))) uint32_t*)(uintptr_t)(a.items + 3 * (size_t)item);
+    const uint32_t e = items[0];
+    const auto ptrs = (const __attribute__((address_space(4))) uint64_t*)(uintptr_t)(a.ptrs + 3 * (size_t)e);
+    const uint32_t first = *(const __attribute__((address_space(4))) uint32_t*)(uintptr_t)(a.offs + e);
+    return {items[2], first + items[1], s % a.row_groups, {ptrs[GU ? 0 : 2], ptrs[GU ? 1 : 2]}};
+  }
 };
 
 constexpr int kPfBigTokens = 112, kPfBigTiles = kPfBigTokens / 16;
@@ -154,7 +180,7 @@ __device__ __forceinline__ void pf_epilogue(const PfBlkArgs& a, const f4_t (&acc
 }
 
 template <class B, bool GU, int T>
-__device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
+__device__ __forceinline__ void pf_block_body(const PfBlkArgs& a, PfUnit unit, bool first) {
   constexpr int WAVES = pf_blk_waves(T), NT = 64 * WAVES;
   constexpr int NM = GU ? 2 : 1, RT = pf_blk_rt(GU, T), R = RT * NM;
   constexpr int HALF = pf_half_bytes(T), PLANE = HALF / 2;
@@ -162,17 +188,14 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
   static_assert(R == 2 && T <= 3, "fragments are processed in pairs; more token tiles: pf_big_body");
   extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
   uint8_t* abuf = (uint8_t*)(smem + B::LDS_WORDS);  // [TWO: 2][2 halves][2 planes][T * 16 tokens][128 bytes]
-  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  uint32_t tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (kept from one unit to the next, what follows from it would cost registers)
+  const uint32_t lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t n16 = lane & 15u, q = lane >> 4;
   const typename B::Low low = B::lane_low(n16);
 
-  // consecutive workgroups land on different XCDs: the row chunks of one item stay on one XCD (shared L2 for its
-  // activations), and items are dealt round-robin over the XCDs
-  const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
-  const uint32_t item = (slot / a.row_groups) * 8u + xcd, rc0 = (slot % a.row_groups) * a.chunks_per_wg;
-  const uint32_t e = a.items[3 * item], t0 = a.items[3 * item + 1], cnt = a.items[3 * item + 2];
-  const uint32_t base = a.offs[e] + t0;
+  const uint32_t cnt = unit.cnt, base = unit.base, rc0 = unit.group * a.chunks_per_wg;
   // A workgroup takes chunks_per_wg consecutive row chunks of its item, one after the other: the first trip to memory
   // (about 4.5 us before the first block can be multiplied, 17 % of a down-projection workgroup's life) is paid once, and
   // the next chunk's first block is requested during the last block of the one before, where a single chunk would
@@ -184,7 +207,7 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
   PfMatrix wm[NM];
   uint32_t row_of[RT];
 #pragma unroll
-  for (int m = 0; m < NM; m++) wm[m] = PfMatrix::of(a, a.ptrs[3 * e + (GU ? m : 2)]);
+  for (int m = 0; m < NM; m++) wm[m] = PfMatrix::of(a, unit.w[m]);
 #pragma unroll
   for (int jt = 0; jt < RT; jt++) row_of[jt] = ((rc0 * WAVES + wave) * RT + jt) * 16u + n16;
   PfRows<B> rows;
@@ -227,7 +250,7 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
   for (int r = 0; r < R; r++) request(r, 0u);
   a_issue(0, 0);
   if constexpr (!TWO) a_issue(1, 0);
-  B::fill_lds(smem, (int)tid, NT);
+  if (first) B::fill_lds(smem, (int)tid, NT);
   a_store(0, 0);
   if constexpr (!TWO) a_issue(0, next_k(0));
   wait_vm<0>();
@@ -335,28 +358,26 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a) {
 //     between steps and not around a copy;
 //   * the fragments of step j + 1 are looked up at the start of step j and finished between its matrix instructions.
 template <class B, bool GU, int T>
-__device__ __forceinline__ void pf_big_body(const PfBlkArgs& a) {
+__device__ __forceinline__ void pf_big_body(const PfBlkArgs& a, PfUnit unit, bool first) {
   constexpr int WAVES = pf_blk_waves(kPfBigTiles), NT = 64 * WAVES;
   constexpr int NM = GU ? 2 : 1, RT = pf_blk_rt(GU, T), R = RT * NM;
   constexpr int HALF = pf_half_bytes(T), PLANE = HALF / 2;
   static_assert(R == 2 && T > 3 && T <= kPfBigTiles);
   extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
   uint8_t* abuf = (uint8_t*)(smem + B::LDS_WORDS);  // [2 halves][2 planes][112 tokens][128 bytes]
-  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  uint32_t tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // (as in pf_block_body)
+  const uint32_t lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t n16 = lane & 15u, q = lane >> 4;
   const typename B::Low low = B::lane_low(n16);
 
-  // the row chunks of one item stay on one XCD (shared L2 for its activations), items are dealt round-robin over the XCDs
-  const uint32_t xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
-  const uint32_t item = (slot / a.row_groups) * 8u + xcd, rc = slot % a.row_groups;
-  const uint32_t e = a.items[3 * item], t0 = a.items[3 * item + 1], cnt = a.items[3 * item + 2];
-  const uint32_t base = a.offs[e] + t0;
+  const uint32_t cnt = unit.cnt, base = unit.base, rc = unit.group;
 
   PfMatrix wm[NM];
   uint32_t row_of[RT];
 #pragma unroll
-  for (int m = 0; m < NM; m++) wm[m] = PfMatrix::of(a, a.ptrs[3 * e + (GU ? m : 2)]);
+  for (int m = 0; m < NM; m++) wm[m] = PfMatrix::of(a, unit.w[m]);
 #pragma unroll
   for (int jt = 0; jt < RT; jt++) row_of[jt] = ((rc * WAVES + wave) * RT + jt) * 16u + n16;
   PfRows<B> rows;
@@ -390,7 +411,7 @@ __device__ __forceinline__ void pf_big_body(const PfBlkArgs& a) {
 #pragma unroll
   for (int r = 0; r < R; r++) request(r, 0u);
   a_request(0, 0);
-  B::fill_lds(smem, (int)tid, NT);
+  if (first) B::fill_lds(smem, (int)tid, NT);
   wait_vm<0>();
 #pragma unroll
   for (int r = 0; r < R; r++) cur[r] = fetched(r, 0u);
@@ -473,19 +494,44 @@ __device__ __forceinline__ void pf_big_body(const PfBlkArgs& a) {
 // built for its tile count; one launch has one tail of half-idle CUs); T = 7 the blocks of 49 to 112 entries that the
 // popular experts are cut into (their weights are then decoded once per 112 entries; 12 waves, one activation buffer).
 template <class B, bool GU, int T>
-__global__ __launch_bounds__(64 * pf_blk_waves(T)) void moe_pf_block_kernel(const PfBlkArgs a) {
-  const uint32_t item = ((blockIdx.x >> 3) / a.row_groups) * 8u + (blockIdx.x & 7u);
-  if (item >= a.nitems) return;
-  const uint32_t cnt = a.items[3 * item + 2];
+__device__ __forceinline__ void pf_unit(const PfBlkArgs& a, const PfUnit& unit, bool first) {
+  const uint32_t cnt = unit.cnt;
   if constexpr (T > 3) {
-    if (cnt > 96) pf_big_body<B, GU, 7>(a);
-    else if (cnt > 80) pf_big_body<B, GU, 6>(a);
-    else if (cnt > 64) pf_big_body<B, GU, 5>(a);
-    else pf_big_body<B, GU, 4>(a);
+    if (cnt > 96) pf_big_body<B, GU, 7>(a, unit, first);
+    else if (cnt > 80) pf_big_body<B, GU, 6>(a, unit, first);
+    else if (cnt > 64) pf_big_body<B, GU, 5>(a, unit, first);
+    else pf_big_body<B, GU, 4>(a, unit, first);
   } else {
-    if (cnt > 32) pf_block_body<B, GU, 3>(a);
-    else if (cnt > 16) pf_block_body<B, GU, 2>(a);
-    else pf_block_body<B, GU, 1>(a);
+    if (cnt > 32) pf_block_body<B, GU, 3>(a, unit, first);
+    else if (cnt > 16) pf_block_body<B, GU, 2>(a, unit, first);
+    else pf_block_body<B, GU, 1>(a, unit, first);
+  }
+}
+template <class B, bool GU, int T, bool QUEUE>
+__global__ __launch_bounds__(64 * pf_blk_waves(T)) void moe_pf_block_kernel(const PfBlkArgs a) {
+  uint32_t s = blockIdx.x >> 3;
+  if constexpr (!QUEUE) {
+    const PfUnit unit = PfUnit::of<GU>(a, s);
+    if (unit.cnt) pf_unit<B, GU, T>(a, unit, true);
+  } else {
+    extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
+    uint32_t* const next_unit = smem + B::LDS_WORDS;  // (in the activation buffers, between two units)
+    for (bool first = true; s < a.per_xcd;) {
+      uint32_t next = 0;  // (asked for beside the item's words; a lane register held over the unit would be one too many)
+      if (threadIdx.x == 0) next = atomicAdd(a.queue + (blockIdx.x & 7u), 1u);
+      const PfUnit unit = PfUnit::of<GU>(a, s);
+      next = (gridDim.x >> 3) + (uint32_t)__builtin_amdgcn_readfirstlane((int)next);
+      if (unit.cnt) {
+        pf_unit<B, GU, T>(a, unit, first);
+        first = false;
+      }
+      wait_vm<0>();  // (requests past the unit's last block still write the buffers)
+      __syncthreads();
+      if (threadIdx.x == 0) *next_unit = next;
+      __syncthreads();
+      s = (uint32_t)__builtin_amdgcn_readfirstlane((int)*next_unit);
+      __syncthreads();
+    }
   }
 }
 
@@ -501,6 +547,7 @@ __global__ __launch_bounds__(64 * pf_blk_waves(T)) void moe_pf_block_kernel(cons
 // fills, seven-tile blocks first, one-tile blocks last, inside a group in expert order (a counting sort over seven
 // buckets: nothing in it depends on timing, so the table is the same on every run).
 constexpr int kHdrChunkWords = 960, kHdrRawHead = 8, kHdrThreads = 1024;
+constexpr uint32_t kPfCounters = 32;  // four launches of the routed experts' block GEMM (two projections, two sizes of items)
 struct HdrChunk { uint32_t w[kHdrChunkWords]; };
 struct HdrBuild {
   uint32_t* raw;        // the image, behind the header
@@ -595,13 +642,15 @@ __global__ __launch_bounds__(kHdrThreads) void moe_pf_header_kernel(const HdrBui
 }
 
 // Xg[i] = fp16(X[src(i)]): i < total gathers token tok[i]; rows total .. total + n - 1 are the tokens themselves. One
-// workgroup per row, eight elements (one 16-byte store) per thread and pass.
+// workgroup per row, eight elements (one 16-byte store) per thread and pass. The first workgroup also clears the block GEMM's
+// counters (null: it has none).
 template <bool X_BF16>
 __global__ __launch_bounds__(256) void moe_pf_gather_kernel(const void* __restrict__ X, uint16_t* __restrict__ Xg,
                                                             const int* __restrict__ tok, uint32_t total, uint32_t nrows,
-                                                            uint32_t dim) {
+                                                            uint32_t dim, uint32_t* __restrict__ counters) {
   const uint32_t i = blockIdx.x;
   if (i >= nrows) return;
+  if (counters && i == 0 && threadIdx.x < kPfCounters) counters[threadIdx.x] = 0u;
   const uint32_t src = i < total ? (uint32_t)tok[i] : i - total;
   auto f = [](uint32_t w) { return __builtin_bit_cast(float, w); };
   for (uint32_t c8 = threadIdx.x; c8 < dim / 8; c8 += blockDim.x) {

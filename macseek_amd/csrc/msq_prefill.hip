@@ -47,16 +47,22 @@ template <bool GU>
 int launch_tile(int t, hipStream_t st, const PfTileArgs& a) {
   return t == MSQ_Q6_K ? launch_tile_t<TileQ6K, GU>(st, a) : launch_tile_t<TileQ8_0, GU>(st, a);
 }
+template <class B, bool GU, int T, bool QUEUE>
+int launch_block_q(hipStream_t st, uint32_t grid, const PfBlkArgs& a) {
+  static bool attr_set = false;  // per instantiation: allow more than 64 KiB of dynamic LDS
+  if (!attr_set) {
+    MSQ_HIP(hipFuncSetAttribute((const void*)moe_pf_block_kernel<B, GU, T, QUEUE>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL((moe_pf_block_kernel<B, GU, T, QUEUE>), dim3(grid), dim3(64 * pf_blk_waves(T)), pf_blk_lds<B>(T), st, a);
+  MSQ_HIP(hipGetLastError());
+  return MSQ_OK;
+}
 template <class B, bool GU, int T>
 int launch_block_tt(hipStream_t st, PfBlkArgs a) {
   if (!a.nitems) return MSQ_OK;
   const uint32_t rows_per_item = pf_blk_rows(GU, T);
   a.row_chunks = (a.N + rows_per_item - 1) / rows_per_item;
-  static bool attr_set = false;  // per instantiation: allow more than 64 KiB of dynamic LDS
-  if (!attr_set) {
-    MSQ_HIP(hipFuncSetAttribute((const void*)moe_pf_block_kernel<B, GU, T>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-    attr_set = true;
-  }
   // two row chunks per workgroup while that leaves three workgroups and more per CU (MSQ_MOEP_CHUNKS imposes a count)
   static const int env_ch = [] { const char* e = getenv("MSQ_MOEP_CHUNKS"); return e && *e ? atoi(e) : 0; }();
   const uint32_t items8 = ((a.nitems + 7) / 8) * 8;
@@ -65,10 +71,10 @@ int launch_block_tt(hipStream_t st, PfBlkArgs a) {
   if (a.N % rows_per_item || GU || T > 3) ch = 1;  // (a ragged last chunk clamps its rows: the chunks are then not a fixed stride apart)
   a.chunks_per_wg = ch;
   a.row_groups = (a.row_chunks + ch - 1) / ch;
-  const uint32_t grid = items8 * a.row_groups;
-  hipLaunchKernelGGL((moe_pf_block_kernel<B, GU, T>), dim3(grid), dim3(64 * pf_blk_waves(T)), pf_blk_lds<B>(T), st, a);
-  MSQ_HIP(hipGetLastError());
-  return MSQ_OK;
+  a.per_xcd = items8 / 8 * a.row_groups;
+  // workgroups that stay (see PfUnit) once there are more units than the chip holds workgroups
+  const uint32_t held = (uint32_t)device_info().cus / 8 * (160 * 1024 / (uint32_t)pf_blk_lds<B>(T));
+  return a.queue && a.per_xcd > held ? launch_block_q<B, GU, T, true>(st, 8 * held, a) : launch_block_q<B, GU, T, false>(st, 8 * a.per_xcd, a);
 }
 // A second stream of the library's own, per device, and the two events that fork work onto it and join it back: the
 // shared expert's two products run beside the routed experts', which they only meet in the reduction. With few tokens
@@ -118,12 +124,19 @@ int launch_block_t(hipStream_t st, PfBlkArgs a, uint32_t n6, uint32_t n3, uint32
   const uint32_t* items = a.items;
   const uint32_t n = a.nitems;
   int rc;
+  uint32_t* const queue = a.queue;
   a.items = items; a.nitems = n6;
   if (!(skip & 256) && (rc = launch_block_tt<BIG, GU, kPfBigTiles>(st, a))) return rc;
   const uint32_t lo = (skip & 128) ? n6 + n3 + n2 : n6, hi = (skip & 64) ? n6 + n3 + n2 : n;
   a.items = items + 3 * (size_t)lo; a.nitems = hi > lo ? hi - lo : 0u;
+  a.queue = queue ? queue + 8 : nullptr;
   return launch_block_tt<B, GU, 3>(st, a);
 }
+// With the shared expert's products on the side stream, workgroups that stay pay from this many tokens on. They leave no room
+// for the shared expert's second product until the routed experts' first has ended, and with few tokens the shared expert's chain
+// is as long as theirs. Over 180 random calls, against a workgroup per unit: one stream 0.98 to 1.10 (mean 1.02) at any number of
+// tokens; two streams 0.90 to 1.08 (0.99) from 7 to 178 tokens, 1.00 to 1.09 (1.05) from 223 on.
+constexpr int kPfQueueTokens = 2 * kPfBigTokens;
 bool block_path(int t) { return t == MSQ_IQ1_S || t == MSQ_IQ2_XXS; }
 template <bool GU>
 int launch_block(int t, hipStream_t st, const PfBlkArgs& a, uint32_t n6, uint32_t n3, uint32_t n2, int skip) {
@@ -210,6 +223,8 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   for (int j = 0; j < ne; j++) count(p->offs[j + 1] - p->offs[j], ni_routed, nc_routed);
   if (p->has_shared) count(n, ni_shared, nc_shared);
   uint8_t* sc = bptr_mut(&p->scratch);
+  // the block GEMM's counters take the place of the raw image, which is used up by then (a header of one or two experts may be too short)
+  uint32_t* const counters = hl.bytes - hl.raw >= 4 * kPfCounters ? (uint32_t*)(sc + hl.raw) : nullptr;
   {
     const int nptr = 3 * (ne + (p->has_shared ? 1 : 0));
     std::vector<uint64_t> ptrs((size_t)nptr);
@@ -265,19 +280,21 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   if (grows > 0 && !(skip & 1)) {
     const dim3 grid(grows), block(256);
     const int* tok = total > 0 ? (const int*)bptr(&p->tok) : nullptr;
-    if (p->x_is_bf16) hipLaunchKernelGGL((moe_pf_gather_kernel<true>), grid, block, 0, st, (const void*)bptr(&p->X), Xg, tok, (uint32_t)total, grows, (uint32_t)dim);
-    else hipLaunchKernelGGL((moe_pf_gather_kernel<false>), grid, block, 0, st, (const void*)bptr(&p->X), Xg, tok, (uint32_t)total, grows, (uint32_t)dim);
+    if (p->x_is_bf16) hipLaunchKernelGGL((moe_pf_gather_kernel<true>), grid, block, 0, st, (const void*)bptr(&p->X), Xg, tok, (uint32_t)total, grows, (uint32_t)dim, counters);
+    else hipLaunchKernelGGL((moe_pf_gather_kernel<false>), grid, block, 0, st, (const void*)bptr(&p->X), Xg, tok, (uint32_t)total, grows, (uint32_t)dim, counters);
     MSQ_HIP(hipGetLastError());
   }
   PfBlkArgs b{};
   b.H = H; b.Z = Z; b.wt = total > 0 ? (const float*)bptr(&p->wt) : nullptr;
   b.ptrs = d_ptrs; b.offs = d_offs; b.total = (uint32_t)total;
   // one product over the routed experts' items
+  bool forked = false;
   auto routed = [&](auto gu_tag, hipStream_t gs) -> int {
     constexpr bool GU = decltype(gu_tag)::value;
     b.A = GU ? Xg : H; b.K = (uint32_t)(GU ? dim : inter); b.N = (uint32_t)(GU ? inter : dim);
     b.nblocks = b.K / 256; b.row_bytes = (uint32_t)(GU ? rb_gu : rb_d);
     b.items = d_items; b.nitems = ni_routed;
+    b.queue = counters && (!forked || n >= kPfQueueTokens) ? counters + (GU ? 0 : 16) : nullptr;
     return launch_block<GU>(GU ? p->t_gate_up : p->t_down, gs, b, nc_routed[0], nc_routed[1], nc_routed[2], skip);
   };
   // ... and one over all tokens with the shared expert's weights
@@ -286,7 +303,7 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
     const uint32_t K = (uint32_t)(GU ? dim : inter), N = (uint32_t)(GU ? inter : dim), rb = (uint32_t)(GU ? rb_sgu : rb_sd);
     if (block_path(p->t_shared)) {
       b.A = GU ? Xg : H; b.K = K; b.N = N; b.nblocks = K / 256; b.row_bytes = rb;
-      b.items = d_items + 3 * (size_t)ni_routed; b.nitems = ni_shared;
+      b.items = d_items + 3 * (size_t)ni_routed; b.nitems = ni_shared; b.queue = nullptr;
       return launch_block<GU>(p->t_shared, gs, b, nc_shared[0], nc_shared[1], nc_shared[2], skip);
     }
     PfTileArgs t{};
@@ -301,7 +318,6 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   const bool routed_gu = any_routed && !(skip & 2), routed_dn = any_routed && !(skip & 8);
   const bool shared_gu = p->has_shared && !(skip & 4), shared_dn = p->has_shared && !(skip & 16);
   // The shared expert and the routed experts only meet in the reduction: two pipelines on two streams (see SideStream)
-  bool forked = false;
   if (p->has_shared && any_routed) {
     std::lock_guard<std::mutex> lock(g_side_mu);
     SideStream* s = side_stream(st);

@@ -19,3 +19,22 @@ def test_every_number_of_token_tiles(dev, monkeypatch, t, dim, inter):
     y, same = P.run_gpu(c)
     err_h, err_f, _ = P.check(c, y, 0)
     assert same and err_h <= 1e-3 and err_f <= 5e-3  # the bounds of test_moe_prefill_gpu.py (the reference's)
+
+
+@pytest.mark.parametrize("t", [O.IQ1_S, O.IQ2_XXS], ids=["IQ1_S", "IQ2_XXS"])
+@pytest.mark.parametrize("dim,inter,small", [(256, 4096, 14), (8192, 256, 87)])
+def test_more_units_than_workgroups(dev, monkeypatch, t, dim, inter, small):
+    """Workgroups that take unit after unit, of every number of token tiles: both sizes of items have more units than the
+    chip holds workgroups, in the first product (4096 rows; a shared expert beside it) and in the second (8192: row chunks in
+    pairs)."""
+    sizes = SIZES + [15, 1] * (small // 2) + [2] * (small % 2)
+    n, k = 224, 8
+    routes = [[] for _ in range(n)]
+    for e, m in enumerate(sizes):
+        for i in sorted(range(n), key=lambda i: (len(routes[i]), (i + 37 * e) % n))[:m]:
+            routes[i].append(e)
+    monkeypatch.setattr(P, "make_routing", lambda *_: routes)
+    c = P.build(t, t, O.Q6_K, n, k, len(sizes), dim == 256, "", dim, inter)
+    y, same = P.run_gpu(c)
+    err_h, err_f, _ = P.check(c, y, 0)
+    assert same and err_h <= 1e-3 and err_f <= 5e-3  # the bounds of test_moe_prefill_gpu.py (the reference's)
