@@ -2,7 +2,7 @@
 // src/kernels/quant.mm:433-612; reference kernels q_moe_gather / q_moe_rgu / q_moe_rdown / q_moe_reduce,
 // src/kernels/quant_moe_prefill.metal:22-29,190-239,275-303,330-344).
 //
-//   gather : Xg[i] = fp16(X[tok[i]]) for the expert-sorted entries, then Xg[total + t] = fp16(X[t]) (shared expert)
+//   convert: Xg[total + t] = fp16(X[t]); an entry's row is its token's (or gather: Xg[i] = fp16(X[tok[i]]), see the host)
 //   gate/up: H[i][r] = fp16(silu(min(Xg_e[i].Wg[r], 10)) * clamp(Xg_e[i].Wu[r], -10, 10) * wt[i])
 //   down   : Z[i][c] = H_e[i] . Wd[c]   (fp32, one row per entry)
 //   reduce : Y[t] += Z[total + t] + sum_k Z[slot_of[t][k]]   in that fixed order
@@ -32,10 +32,11 @@ namespace msq {
 // (27 instructions per eight weights): 2048 tokens, 384 IQ2_XXS experts of 7168x2048: gate/up 644 -> 554 us (T > 3) and 1080
 // -> 1050, down 348 -> 312 and 569 -> 555; IQ1_S 5120x2304, 37 tokens: the call 543 -> 477, 4096 tokens: 3534 -> 3268.
 struct PfBlkArgs {
-  const uint16_t* A;        // fp16 activations [entries][K]
+  const uint16_t* A;        // fp16 activations [entries][K], or (tok) [tokens][K]
+  const int* tok;           // per entry: its row of A; null: the entry itself
+  uint32_t a_bytes;         // (tok) bytes of A
   const uint64_t* ptrs;     // per expert: gate, up, down addresses
-  const uint32_t* offs;     // per expert: first entry
-  const uint32_t* items;    // per item: expert, first entry of the block inside the expert, entries in the block
+  const uint32_t* items;    // per item: expert, first entry of the block, entries in the block
   const float* wt;          // per routed entry: routing weight
   uint16_t* H;              // gate/up output [entries][N] fp16
   float* Z;                 // down output [entries][N] fp32
@@ -54,8 +55,7 @@ struct PfBlkArgs {
 // its XCD until they are used up, the first by its number, the others from the XCD's counter. The tables are in LDS once, and a
 // unit does not wait for the workgroup before it to be taken down and its own to be set up (4096 tokens of IQ1_S: blocks of
 // the first product 942 -> 859 us, calls 3349 -> 3160; 2048 of IQ2_XXS 2500 -> 2470). The rule is at the launch.
-// (The tables are read as constants, which they are while the kernel runs: scalar loads, and an expert's offset and addresses
-// in one trip.)
+// (The tables are read as constants, which they are while the kernel runs: scalar loads.)
 struct PfUnit {
   uint32_t cnt, base;  // the item's entries (none: the last items of eight may be missing), the first one
   uint32_t group;
@@ -65,10 +65,9 @@ struct PfUnit {
     const uint32_t item = (s / a.row_groups) * 8u + (blockIdx.x & 7u);
     if (item >= a.nitems) return PfUnit{};
     const auto items = (const __attribute__((address_space(4))) uint32_t*)(uintptr_t)(a.items + 3 * (size_t)item);
-    const uint32_t e = items[0];
+    const uint32_t e = items[0], base = items[1];
     const auto ptrs = (const __attribute__((address_space(4))) uint64_t*)(uintptr_t)(a.ptrs + 3 * (size_t)e);
-    const uint32_t first = *(const __attribute__((address_space(4))) uint32_t*)(uintptr_t)(a.offs + e);
-    return {items[2], first + items[1], s % a.row_groups, {ptrs[GU ? 0 : 2], ptrs[GU ? 1 : 2]}};
+    return {items[2], base, s % a.row_groups, {ptrs[GU ? 0 : 2], ptrs[GU ? 1 : 2]}};
   }
 };
 
@@ -179,6 +178,19 @@ __device__ __forceinline__ void pf_epilogue(const PfBlkArgs& a, const f4_t (&acc
   }
 }
 
+// The activations of an item's entries: consecutive rows of A, or (the first product) the rows that the entries' tokens name.
+// A gathered copy costs a write and a read of every entry's row; the list costs one word a lane, beside the item's addresses
+// in the same trip (4096 tokens, 36864 rows of 7168: copy 123 us, conversion of the tokens' own rows 22).
+template <bool GU>
+__device__ __forceinline__ rsrc_t pf_act_rows(const PfBlkArgs& a, const PfUnit& unit) {
+  if (GU && a.tok) return make_rsrc(a.A, a.a_bytes);
+  return make_rsrc(a.A + (size_t)unit.base * a.K, unit.cnt * a.K * 2u);
+}
+template <bool GU>
+__device__ __forceinline__ uint32_t pf_act_row(const PfBlkArgs& a, uint32_t base, uint32_t row) {
+  return GU && a.tok ? (uint32_t)a.tok[base + row] : row;
+}
+
 template <class B, bool GU, int T>
 __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a, PfUnit unit, bool first) {
   constexpr int WAVES = pf_blk_waves(T), NT = 64 * WAVES;
@@ -221,7 +233,7 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a, PfUnit unit, b
   // activation loader. Piece g of a block (TWO) or of half h: row g / 32 (g / 16), then (half,) plane and unit.
   constexpr int PB = TWO ? 5 : 4, AG = ((T << (4 + PB)) + NT - 1) / NT;
   static_assert(TWO || AG == 1);
-  const rsrc_t ars = make_rsrc(a.A + (size_t)base * a.K, cnt * a.K * 2u);
+  const rsrc_t ars = pf_act_rows<GU>(a, unit);
   uint32_t aoff[AG];
   uint8_t* adst[AG];
 #pragma unroll
@@ -229,9 +241,12 @@ __device__ __forceinline__ void pf_block_body(const PfBlkArgs& a, PfUnit unit, b
     // rows past the block's last entry repeat it (their products are never stored): no branch around the load, so
     // the number of loads in flight stays known to every wait that follows
     const uint32_t g = min(tid + i * NT, (16u * T << PB) - 1u), row = g >> PB, h = TWO ? (g >> 4) & 1u : 0u, plane = (g >> 3) & 1u, unit = g & 7u;
-    aoff[i] = min(row, cnt - 1u) * (a.K * 2u) + (64u * (2u * (unit >> 2) + plane) + 32u * h + 8u * (unit & 3u)) * 2u;
+    aoff[i] = pf_act_row<GU>(a, base, min(row, cnt - 1u)) * (a.K * 2u) + (64u * (2u * (unit >> 2) + plane) + 32u * h + 8u * (unit & 3u)) * 2u;
     adst[i] = abuf + h * HALF + plane * PLANE + row * 128u + 16u * (unit ^ ((row >> 1) & 7u));
   }
+  if constexpr (GU)
+#pragma unroll
+    for (int i = 0; i < AG; i++) asm volatile("" : "+v"(aoff[i]));  // (waited for here, not behind the weights that are asked for next)
   u32x4 pa[TWO ? 1 : 2][AG];  // (a plain vector type: the HIP struct type keeps the array in scratch memory)
   auto a_issue = [&](int h, uint32_t kc) {
 #pragma unroll
@@ -391,13 +406,16 @@ __device__ __forceinline__ void pf_big_body(const PfBlkArgs& a, PfUnit unit, boo
 
   // activation loader: a half of a block is 4 T kilobytes, a load (eight rows of a plane) each; wave w's are w, w + 12, ...
   constexpr int AL = 4 * T, AMIN = AL / WAVES, AMAX = (AL + WAVES - 1) / WAVES;
-  const rsrc_t ars = make_rsrc(a.A + (size_t)base * a.K, cnt * a.K * 2u);
+  const rsrc_t ars = pf_act_rows<GU>(a, unit);
   uint32_t aoff[AMAX];
 #pragma unroll
   for (int i = 0; i < AMAX; i++) {  // rows past the block's last entry repeat it (their products are never stored)
     const uint32_t l = wave + i * WAVES, plane = l >= 2u * T ? 1u : 0u, row = 8u * (l - plane * 2u * T) + (lane >> 3), unit = (lane & 7u) ^ ((row >> 1) & 7u);
-    aoff[i] = min(row, cnt - 1u) * (a.K * 2u) + (64u * (2u * (unit >> 2) + plane) + 8u * (unit & 3u)) * 2u;
+    aoff[i] = pf_act_row<GU>(a, base, min(row, cnt - 1u)) * (a.K * 2u) + (64u * (2u * (unit >> 2) + plane) + 8u * (unit & 3u)) * 2u;
   }
+  if constexpr (GU)
+#pragma unroll
+    for (int i = 0; i < AMAX; i++) asm volatile("" : "+v"(aoff[i]));  // (as in pf_block_body)
   const bool amore = wave + AMIN * WAVES < AL;  // (uniform) one load more than the waves that have the fewest
   auto a_request = [&](int h, uint32_t kc) {
 #pragma unroll
@@ -536,13 +554,14 @@ __global__ __launch_bounds__(64 * pf_blk_waves(T)) void moe_pf_block_kernel(cons
 }
 
 // ------------------------------------------------------------------------------------------------ scratch header
-// The header of the prefill scratch (expert addresses, entry offsets, the work items of the block GEMM) is built on the device. What only the host knows travels in kernel arguments: a raw image
+// The header of the prefill scratch (expert addresses, the work items of the block GEMM) is built on the device. What only the
+// host knows travels in kernel arguments: a raw image
 //   word 0 n_exp | 1 has_shared | 2 n_tokens | 3 total | 4, 5 base address | 6 address mode | 7 unused
 //   words 8 .. 8 + n_exp: entry offsets offs[0 .. n_exp]
 //   then 3 addresses per expert (gate, up, down; the shared expert last): mode 0 one word each, (address - base) / 4;
 //   mode 1 two words each
 // cut into pieces of kHdrChunkWords (the argument block holds 4 KB). Every launch stores its piece behind the header;
-// the last one then expands the image: addresses and offsets as the GEMM kernels read them, and the work items --
+// the last one then expands the image: addresses as the GEMM kernels read them, and the work items --
 // an expert of m entries gives m / 112 blocks of 112 entries and one of m % 112 -- grouped by the token tiles a block
 // fills, seven-tile blocks first, one-tile blocks last, inside a group in expert order (a counting sort over seven
 // buckets: nothing in it depends on timing, so the table is the same on every run).
@@ -552,7 +571,6 @@ struct HdrChunk { uint32_t w[kHdrChunkWords]; };
 struct HdrBuild {
   uint32_t* raw;        // the image, behind the header
   uint64_t* ptrs;       // (n_exp + 1) x {gate, up, down}
-  uint32_t* offs;       // n_exp + 2
   uint32_t* items;      // routed items, then the shared expert's
   uint32_t build;       // 1: this launch holds the image's last piece and expands it
 };
@@ -594,8 +612,6 @@ __global__ __launch_bounds__(kHdrThreads) void moe_pf_header_kernel(const HdrBui
   const uint32_t* rp = roffs + ne + 1;
   for (uint32_t i = tid; i < 3u * (ne + has_shared); i += kHdrThreads)
     b.ptrs[i] = mode ? ((uint64_t)rp[2 * i] | ((uint64_t)rp[2 * i + 1] << 32)) : base + 4ull * rp[i];
-  for (uint32_t i = tid; i <= ne; i += kHdrThreads) b.offs[i] = roffs[i];
-  if (tid == 0) b.offs[ne + 1] = total + n;
   // routed items: this thread's experts [j0, j1)
   const uint32_t per = (ne + kHdrThreads - 1) / kHdrThreads, j0 = min(ne, tid * per), j1 = min(ne, j0 + per);
   uint32_t cnt[7] = {0, 0, 0, 0, 0, 0, 0};
@@ -619,7 +635,7 @@ __global__ __launch_bounds__(kHdrThreads) void moe_pf_header_kernel(const HdrBui
     const uint32_t m = roffs[j + 1] - roffs[j], q = m / 112u, r = m % 112u;
     for (uint32_t k = 0; k < q; k++) {
       uint32_t* it = b.items + 3 * (size_t)at[0]++;
-      it[0] = j; it[1] = 112u * k; it[2] = 112u;
+      it[0] = j; it[1] = roffs[j] + 112u * k; it[2] = 112u;
     }
     if (r) {
       const uint32_t bk = pf_item_bucket(r);
@@ -628,7 +644,7 @@ __global__ __launch_bounds__(kHdrThreads) void moe_pf_header_kernel(const HdrBui
       for (int k = 0; k < 7; k++)
         if (bk == (uint32_t)k) pos = at[k]++;
       uint32_t* it = b.items + 3 * (size_t)pos;
-      it[0] = j; it[1] = 112u * q; it[2] = r;
+      it[0] = j; it[1] = roffs[j] + 112u * q; it[2] = r;
     }
   }
   // the shared expert's items follow: blocks of 112 tokens, then the rest
@@ -636,7 +652,7 @@ __global__ __launch_bounds__(kHdrThreads) void moe_pf_header_kernel(const HdrBui
     const uint32_t q = n / 112u, r = n % 112u;
     for (uint32_t k = tid; k < q + (r ? 1u : 0u); k += kHdrThreads) {
       uint32_t* it = b.items + 3 * (size_t)(first + k);
-      it[0] = ne; it[1] = 112u * k; it[2] = k < q ? 112u : r;
+      it[0] = ne; it[1] = total + 112u * k; it[2] = k < q ? 112u : r;
     }
   }
 }

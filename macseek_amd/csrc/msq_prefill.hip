@@ -15,15 +15,14 @@ namespace msq {
 namespace {
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
-// header: addresses | offsets | work items | raw image (see moe_pf_header_kernel)
-struct HdrLayout { size_t ptrs, offs, items, raw, bytes; };
+// header: addresses | n_exp + 2 words that nothing uses (callers keep the scratch size) | work items | raw image (see moe_pf_header_kernel)
+struct HdrLayout { size_t ptrs, items, raw, bytes; };
 HdrLayout header_layout(int total, int n, int n_exp) {
   HdrLayout h;
   const size_t items = 2 * ((size_t)n_exp + 1) + (size_t)total / kPfBigTokens + (size_t)n / kPfBigTokens;  // m / 112 blocks + a rest per expert
   const size_t raw_words = kHdrRawHead + ((size_t)n_exp + 1) + 6 * ((size_t)n_exp + 1);
   h.ptrs = 0;
-  h.offs = 24 * (size_t)(n_exp + 1);
-  h.items = h.offs + 4 * (size_t)(n_exp + 2);
+  h.items = 24 * (size_t)(n_exp + 1) + 4 * (size_t)(n_exp + 2);
   h.raw = h.items + 12 * items;
   h.bytes = align256(h.raw + 4 * raw_words);
   return h;
@@ -254,7 +253,7 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
       else { raw.push_back((uint32_t)v); raw.push_back((uint32_t)(v >> 32)); }
     }
     HdrBuild hb{};
-    hb.raw = (uint32_t*)(sc + hl.raw); hb.ptrs = (uint64_t*)(sc + hl.ptrs); hb.offs = (uint32_t*)(sc + hl.offs);
+    hb.raw = (uint32_t*)(sc + hl.raw); hb.ptrs = (uint64_t*)(sc + hl.ptrs);
     hb.items = (uint32_t*)(sc + hl.items);
     for (size_t w0 = 0; w0 < raw.size(); w0 += kHdrChunkWords) {
       HdrChunk c;
@@ -271,27 +270,32 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   uint16_t* H = (uint16_t*)((uint8_t*)Xg + align256(rows * dim * 2));
   float* Z = (float*)((uint8_t*)H + align256(rows * inter * 2));
   const uint64_t* d_ptrs = (const uint64_t*)(sc + hl.ptrs);
-  const uint32_t* d_offs = (const uint32_t*)(sc + hl.offs);
   const uint32_t* d_items = (const uint32_t*)(sc + hl.items);
   const bool any_routed = total > 0;
 
   // 1) gather + convert
-  const uint32_t grows = (uint32_t)(total + (p->has_shared ? n : 0));
+  // The block GEMM finds an entry's row by its token, and only the tokens' own rows are converted, where these are wanted anyway
+  // (shared expert) or no more than the entries, and within what one descriptor reaches; else the entries' rows are gathered.
+  const bool by_token = any_routed && (p->has_shared || n <= total) && (size_t)n * dim * 2 < 0xFFFFFFF0ull;
+  const uint32_t gathered = by_token ? 0u : (uint32_t)total, grows = gathered + (uint32_t)(p->has_shared || by_token ? n : 0);
+  uint16_t* const Xt = Xg + (size_t)total * dim;  // the tokens' own rows
+  const int* tok = any_routed ? (const int*)bptr(&p->tok) : nullptr;
   if (grows > 0 && !(skip & 1)) {
     const dim3 grid(grows), block(256);
-    const int* tok = total > 0 ? (const int*)bptr(&p->tok) : nullptr;
-    if (p->x_is_bf16) hipLaunchKernelGGL((moe_pf_gather_kernel<true>), grid, block, 0, st, (const void*)bptr(&p->X), Xg, tok, (uint32_t)total, grows, (uint32_t)dim, counters);
-    else hipLaunchKernelGGL((moe_pf_gather_kernel<false>), grid, block, 0, st, (const void*)bptr(&p->X), Xg, tok, (uint32_t)total, grows, (uint32_t)dim, counters);
+    uint16_t* to = gathered ? Xg : Xt;
+    if (p->x_is_bf16) hipLaunchKernelGGL((moe_pf_gather_kernel<true>), grid, block, 0, st, (const void*)bptr(&p->X), to, tok, gathered, grows, (uint32_t)dim, counters);
+    else hipLaunchKernelGGL((moe_pf_gather_kernel<false>), grid, block, 0, st, (const void*)bptr(&p->X), to, tok, gathered, grows, (uint32_t)dim, counters);
     MSQ_HIP(hipGetLastError());
   }
   PfBlkArgs b{};
   b.H = H; b.Z = Z; b.wt = total > 0 ? (const float*)bptr(&p->wt) : nullptr;
-  b.ptrs = d_ptrs; b.offs = d_offs; b.total = (uint32_t)total;
+  b.ptrs = d_ptrs; b.total = (uint32_t)total;
   // one product over the routed experts' items
   bool forked = false;
   auto routed = [&](auto gu_tag, hipStream_t gs) -> int {
     constexpr bool GU = decltype(gu_tag)::value;
-    b.A = GU ? Xg : H; b.K = (uint32_t)(GU ? dim : inter); b.N = (uint32_t)(GU ? inter : dim);
+    b.A = !GU ? H : by_token ? Xt : Xg; b.tok = GU && by_token ? tok : nullptr; b.a_bytes = (uint32_t)((size_t)n * dim * 2);
+    b.K = (uint32_t)(GU ? dim : inter); b.N = (uint32_t)(GU ? inter : dim);
     b.nblocks = b.K / 256; b.row_bytes = (uint32_t)(GU ? rb_gu : rb_d);
     b.items = d_items; b.nitems = ni_routed;
     b.queue = counters && (!forked || n >= kPfQueueTokens) ? counters + (GU ? 0 : 16) : nullptr;
@@ -302,7 +306,7 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
     constexpr bool GU = decltype(gu_tag)::value;
     const uint32_t K = (uint32_t)(GU ? dim : inter), N = (uint32_t)(GU ? inter : dim), rb = (uint32_t)(GU ? rb_sgu : rb_sd);
     if (block_path(p->t_shared)) {
-      b.A = GU ? Xg : H; b.K = K; b.N = N; b.nblocks = K / 256; b.row_bytes = rb;
+      b.A = GU ? Xg : H; b.tok = nullptr; b.K = K; b.N = N; b.nblocks = K / 256; b.row_bytes = rb;
       b.items = d_items + 3 * (size_t)ni_routed; b.nitems = ni_shared; b.queue = nullptr;
       return launch_block<GU>(p->t_shared, gs, b, nc_shared[0], nc_shared[1], nc_shared[2], skip);
     }

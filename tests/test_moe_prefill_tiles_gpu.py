@@ -38,3 +38,14 @@ def test_more_units_than_workgroups(dev, monkeypatch, t, dim, inter, small):
     y, same = P.run_gpu(c)
     err_h, err_f, _ = P.check(c, y, 0)
     assert same and err_h <= 1e-3 and err_f <= 5e-3  # the bounds of test_moe_prefill_gpu.py (the reference's)
+
+
+@pytest.mark.parametrize("entries", [1, 39, 40, 41])
+def test_rows_by_entry_and_by_token(dev, monkeypatch, entries):
+    """Fewer entries than the 40 tokens: their rows are gathered; as many and more: found by the token."""
+    n, k = 40, 2
+    monkeypatch.setattr(P, "make_routing", lambda *_: [[0] * (i < entries) + [1] * (n + i < entries) for i in range(n - 1, -1, -1)])
+    c = P.build(O.IQ2_XXS, O.IQ1_S, O.Q6_K, n, k, 2, False, "", 512, 256)
+    y, same = P.run_gpu(c)
+    err_h, err_f, _ = P.check(c, y, 0)
+    assert same and err_h <= 1e-3 and err_f <= 5e-3  # the bounds of test_moe_prefill_gpu.py (the reference's)
