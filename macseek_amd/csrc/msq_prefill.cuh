@@ -576,36 +576,50 @@ struct HdrBuild {
 };
 __host__ __device__ constexpr uint32_t pf_item_bucket(uint32_t cnt) { return 7u - (cnt + 15u) / 16u; }  // cnt in 1..112
 
-// exclusive prefix of v over the workgroup's threads; total = sum over all; wsum: 17 words of LDS
-__device__ __forceinline__ uint32_t hdr_scan(uint32_t v, uint32_t* wsum, uint32_t tid, uint32_t& total) {
+// Where a thread's items of each of the seven buckets start: the buckets one behind the other, in each the threads' in order.
+// All seven go through the two steps (inside a wave, over the waves) together: the kernel is one workgroup's chain of
+// latencies, and a bucket at a time, three barriers and 16 serial additions each, took it 8.9 us (now 7.2; the 37 tokens of the performance cases).
+struct HdrScan { uint32_t wave[kHdrThreads / 64][8], all[8]; };
+__device__ __forceinline__ uint32_t hdr_scan(uint32_t (&v)[7], HdrScan& m, uint32_t tid) {
   const uint32_t lane = tid & 63u, wave = tid >> 6;
-  uint32_t inc = v;
+  uint32_t inc[7];
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t t = (uint32_t)__shfl_up((int)inc, d, 64);
-    if (lane >= (uint32_t)d) inc += t;
+  for (int k = 0; k < 7; k++) {
+    inc[k] = v[k];
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t t = (uint32_t)__shfl_up((int)inc[k], d, 64);
+      if (lane >= (uint32_t)d) inc[k] += t;
+    }
+    if (lane == 63u) m.wave[wave][k] = inc[k];
   }
-  if (lane == 63u) wsum[wave] = inc;
   __syncthreads();
-  if (tid == 0) {
+  if (tid < 8u) {
     uint32_t run = 0;
-    for (uint32_t w = 0; w < kHdrThreads / 64; w++) { const uint32_t t = wsum[w]; wsum[w] = run; run += t; }
-    wsum[kHdrThreads / 64] = run;
+#pragma unroll
+    for (int w = 0; w < kHdrThreads / 64; w++) { const uint32_t t = tid < 7u ? m.wave[w][tid] : 0u; m.wave[w][tid] = run; run += t; }
+    m.all[tid] = run;
   }
   __syncthreads();
-  total = wsum[kHdrThreads / 64];
-  const uint32_t r = wsum[wave] + inc - v;
-  __syncthreads();
-  return r;
+  uint32_t first = 0;
+#pragma unroll
+  for (int k = 0; k < 7; k++) {
+    v[k] = first + m.wave[wave][k] + inc[k] - v[k];
+    first += m.all[k];
+  }
+  return first;  // all items
 }
 
 __global__ __launch_bounds__(kHdrThreads) void moe_pf_header_kernel(const HdrBuild b, const HdrChunk c, uint32_t word0, uint32_t nwords) {
-  __shared__ uint32_t wsum[kHdrThreads / 64 + 1];
+  __shared__ HdrScan scan;
+  __shared__ uint32_t whole[kHdrChunkWords];
   const uint32_t tid = threadIdx.x;
-  for (uint32_t i = tid; i < nwords; i += kHdrThreads) b.raw[word0 + i] = c.w[i];
+  // (an image of one piece stays in LDS: no trip to memory and back)
+  uint32_t* const image = b.build && word0 == 0 ? whole : b.raw;
+  for (uint32_t i = tid; i < nwords; i += kHdrThreads) image[word0 + i] = c.w[i];
   if (!b.build) return;
   __syncthreads();  // the image's earlier pieces were stored by earlier launches, the last one just now
-  const uint32_t* raw = b.raw;
+  const uint32_t* raw = image;
   const uint32_t ne = raw[0], has_shared = raw[1], n = raw[2], total = raw[3], mode = raw[6];
   const uint64_t base = (uint64_t)raw[4] | ((uint64_t)raw[5] << 32);
   const uint32_t* roffs = raw + kHdrRawHead;
@@ -614,23 +628,17 @@ __global__ __launch_bounds__(kHdrThreads) void moe_pf_header_kernel(const HdrBui
     b.ptrs[i] = mode ? ((uint64_t)rp[2 * i] | ((uint64_t)rp[2 * i + 1] << 32)) : base + 4ull * rp[i];
   // routed items: this thread's experts [j0, j1)
   const uint32_t per = (ne + kHdrThreads - 1) / kHdrThreads, j0 = min(ne, tid * per), j1 = min(ne, j0 + per);
-  uint32_t cnt[7] = {0, 0, 0, 0, 0, 0, 0};
+  uint32_t at[7] = {0, 0, 0, 0, 0, 0, 0};  // items of each bucket, then where they start
   for (uint32_t j = j0; j < j1; j++) {
     const uint32_t m = roffs[j + 1] - roffs[j], r = m % 112u;
-    cnt[0] += m / 112u;
+    at[0] += m / 112u;
     if (r) {
       const uint32_t bk = pf_item_bucket(r);
 #pragma unroll
-      for (int k = 0; k < 7; k++) cnt[k] += bk == (uint32_t)k;
+      for (int k = 0; k < 7; k++) at[k] += bk == (uint32_t)k;
     }
   }
-  uint32_t at[7], first = 0;  // where this thread's items of each bucket start
-#pragma unroll
-  for (int k = 0; k < 7; k++) {
-    uint32_t tot;
-    at[k] = first + hdr_scan(cnt[k], wsum, tid, tot);
-    first += tot;
-  }
+  const uint32_t first = hdr_scan(at, scan, tid);
   for (uint32_t j = j0; j < j1; j++) {
     const uint32_t m = roffs[j + 1] - roffs[j], q = m / 112u, r = m % 112u;
     for (uint32_t k = 0; k < q; k++) {
