@@ -280,8 +280,8 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   const uint32_t gathered = by_token ? 0u : (uint32_t)total, grows = gathered + (uint32_t)(p->has_shared || by_token ? n : 0);
   uint16_t* const Xt = Xg + (size_t)total * dim;  // the tokens' own rows
   const int* tok = any_routed ? (const int*)bptr(&p->tok) : nullptr;
-  if (grows > 0 && !(skip & 1)) {
-    const dim3 grid(grows), block(256);
+  if (grows > 0) {
+    const dim3 grid(skip & 1 ? 1u : grows), block(256);  // (skipped: one row is left, with the counters)
     uint16_t* to = gathered ? Xg : Xt;
     if (p->x_is_bf16) hipLaunchKernelGGL((moe_pf_gather_kernel<true>), grid, block, 0, st, (const void*)bptr(&p->X), to, tok, gathered, grows, (uint32_t)dim, counters);
     else hipLaunchKernelGGL((moe_pf_gather_kernel<false>), grid, block, 0, st, (const void*)bptr(&p->X), to, tok, gathered, grows, (uint32_t)dim, counters);
