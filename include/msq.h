@@ -263,12 +263,12 @@ typedef struct MsqMoePrefillArgs {
 } MsqMoePrefillArgs;
 
 /* reference: ms::q::moe_prefill_scratch_bytes (quant.hpp:117, quant.mm:427-431). Layout (caller-owned device memory):
- * header (expert pointer table, offsets, work items) | Xg fp16[(total+n) x dim] | H fp16[(total+n) x inter] |
+ * header (expert pointer table, work items, counters) | Xg fp16[(total+n) x dim] | H fp16[(total+n) x inter] |
  * Z f32[(total+n) x dim]. The header is written by small kernels that carry it in their arguments, so unlike the
  * reference the scratch may still be in use by earlier work on the same stream. */
 size_t msq_moe_prefill_scratch_bytes(int total_entries, int n_tokens, int n_exp, int dim, int inter);
 
-/* reference: ms::q::encode_moe_prefill (quant.hpp:118, quant.mm:433-612). Enqueues gather, grouped gate/up GEMM +
+/* reference: ms::q::encode_moe_prefill (quant.hpp:118, quant.mm:433-612). Enqueues conversion, grouped gate/up GEMM +
  * SwiGLU, grouped down GEMM and the ordered reduction into Y. Activations and H are staged as fp16 and weights enter
  * the matrix instructions as fp16 like the reference's tiles (IQ1_S / IQ2_XXS: the sub-block scale is rounded to fp16 and
  * its product with the grid value is rounded again, where the reference rounds the fp32 product once; a Q6_K / Q8_0 shared

@@ -25,12 +25,13 @@ namespace msq {
 // all waves, every wave decodes the fragments of its own rows once per block and reuses each of them for all T token
 // tiles, and accumulates in the matrix cores; the scale rides in the fragments. Weights are decoded exactly
 // once per (item, row), no lane loads a weight byte twice, and the next block's bytes are in flight during a block.
-// What bounds it. Small items (T <= 3): vector issue (14 instructions per eight weights of a lane, 61 % of the cycles), LDS (51 %)
-// and the texture addresser (53 %) beside each other, four waves per SIMD; 12 % (gate/up) to 30 % (down) is a workgroup's first
-// trip to memory and its end. Larger blocks: see pf_big_body. Against a variant that fetched IQ2_XXS rows lane by lane (three loads
+// What bounds it. Small items (T <= 3): vector issue (14 instructions per eight weights of a lane, 62 % of the cycles), LDS (51 %)
+// and the texture addresser (53 %) beside each other, four waves per SIMD; a unit's first trip to memory and its end are 10 %
+// (gate/up) to 25 % (down). Larger blocks: see pf_big_body. Against a variant that fetched IQ2_XXS rows lane by lane (three loads
 // a row, 50 vector cache lookups each), staged activations through registers and tested the tile count in every step
-// (27 instructions per eight weights): 2048 tokens, 384 IQ2_XXS experts of 7168x2048: gate/up 644 -> 554 us (T > 3) and 1080
-// -> 1050, down 348 -> 312 and 569 -> 555; IQ1_S 5120x2304, 37 tokens: the call 543 -> 477, 4096 tokens: 3534 -> 3268.
+// (27 instructions per eight weights), launched a workgroup per unit and gathered a copy of the entries' rows: 2048 tokens,
+// 384 IQ2_XXS experts of 7168x2048: gate/up 644 -> 537 us (T > 3) and 1080 -> 1009, down 348 -> 308 and 569 -> 565, the call
+// 2735 -> 2501; IQ1_S 5120x2304: 37 tokens 515 -> 451, 4096 tokens 3693 -> 3141.
 struct PfBlkArgs {
   const uint16_t* A;        // fp16 activations [entries][K], or (tok) [tokens][K]
   const int* tok;           // per entry: its row of A; null: the entry itself
