@@ -549,8 +549,8 @@ __global__ __launch_bounds__(MAXT) void moe_down_kernel(const uint64_t* table, c
     // everything else (no registers are held for them, and they return -- loads return in order -- ahead of the first
     // weight rows' trip to HBM instead of behind it); what does not fill a group of 64 items goes through one register.
     constexpr bool DMA = RING_R && RING_S && HALF && MAXT <= 768;  // (the 1024-thread instantiations have no registers to spare)
-    [[maybe_unused]] u32x4 rest[4];
-    [[maybe_unused]] uint32_t rest_at[4] = {0u, 0u, 0u, 0u};  // LDS word offset + 1 of the thread's leftover item, 0: none
+    [[maybe_unused]] u32x4 rest[5];
+    [[maybe_unused]] uint32_t rest_at[5] = {0u, 0u, 0u, 0u, 0u};  // LDS word offset + 1 of the thread's leftover item, 0: none
     if constexpr (DMA) {
       if (first && a.stage_x) {
         const uint32_t lo = NE ? 0u : a.n_routed * a.inter;
@@ -564,8 +564,8 @@ __global__ __launch_bounds__(MAXT) void moe_down_kernel(const uint64_t* table, c
           if (jobs[j].n16 == 0) continue;
           const uint32_t done = j == 4 ? lds_dma_groups(tbl + jobs[j].dst, jobs[j].src, jobs[j].n16, wave, nwaves, lane, xhalf_rot_src)
                                        : lds_dma_groups(tbl + jobs[j].dst, jobs[j].src, jobs[j].n16, wave, nwaves, lane, same);
-          if (j < 4 && done + tid < jobs[j].n16) {  // (the h rows are whole groups: inter is a multiple of 256)
-            rest[j] = *(const u32x4*)(jobs[j].src + done + tid);
+          if (done + tid < jobs[j].n16) {  // (h rows: half a group where the rows are odd in number and in 256s)
+            rest[j] = *(const u32x4*)(jobs[j].src + (j == 4 ? xhalf_rot_src(done + tid) : done + tid));
             rest_at[j] = jobs[j].dst + 4u * (done + tid) + 1u;
           }
         }
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(MAXT) void moe_down_kernel(const uint64_t* table, c
     if (DMA && first && a.stage_x) {
       wait_vm<NR * DR::FETCH_LOADS + 1>();  // everything older than the routed ring and y: the copy
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+      for (int j = 0; j < 5; j++)
         if (rest_at[j]) *(u32x4*)(tbl + rest_at[j] - 1u) = rest[j];
       const uint32_t lo = NE ? 0u : a.n_routed * a.inter;
       const uint32_t* hs = smem + a.xs_off;
