@@ -293,11 +293,13 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   // Under a fused norm weight rows go through LDS from 17 MB on (Q6_K 4096x4608 8.5 / 9.2 us, 4096x7168 11.2 / 10.8, 16384x5120
   // 23.7 / 19.0, 129280x5120 138 / 101), but for Q6_K rows of whole waves of 200 MB and more (129280x2048 38.5 / 40.1).
   const bool norm_sw = bytes >= 17e6 && (std::is_same_v<D, DecQ8_0> || bytes < 200e6 || (a.cols / D::UNIT) % 64 != 0);
-  const bool sw = tok_stages_w<D, 1, T>() && s.iters == 1 && s.stage_w && (!a.norm_w || norm_sw);
-  if (sw) {  // the waves' weight-row buffers
-    lds = (lds + 15) / 16 * 16;
-    a.w_off = (uint32_t)(lds / 4);
-    lds += (size_t)(threads / 64) * 4 * wspan_loads<D>() * 1024;  // four slots per wave
+  // ... and where the waves' buffers, four slots each, find room behind the staged activations (Q8_0 rows of more than 14336
+  // columns, eight waves of three pieces a slot, leave none)
+  const size_t w_at = (lds + 15) / 16 * 16, w_end = w_at + (size_t)(threads / 64) * 4 * wspan_loads<D>() * 1024;
+  const bool sw = tok_stages_w<D, 1, T>() && s.iters == 1 && s.stage_w && (!a.norm_w || norm_sw) && w_end + kStaticLds<D> <= (size_t)kMaxLds;
+  if (sw) {
+    a.w_off = (uint32_t)(w_at / 4);
+    lds = w_end;
   }
   auto launch = [&](auto kernel, dim3 grid) {
     allow_large_lds(kernel, lds);

@@ -146,3 +146,10 @@ LARGE = [
 @pytest.mark.parametrize("t,rows,cols", LARGE, ids=lambda v: None)
 def test_fused_norm_of_large_matrices(dev, t, rows, cols):
     test_fused_equals_norm_then_matvec_and_oracle(dev, t, rows, cols)
+
+
+# Q8_0 rows of 40 MB matrices, which go through LDS where a workgroup's buffers find room beside its activations: the longest
+# row that leaves it, one block more, and the longest that a workgroup takes (with the norm and, to compare, without)
+@pytest.mark.parametrize("rows,cols", [(2700, 14336), (2720, 14368), (2400, 16384)], ids=lambda v: None)
+def test_large_matrices_of_long_rows(dev, rows, cols):
+    test_fused_equals_norm_then_matvec_and_oracle(dev, O.Q8_0, rows, cols)
