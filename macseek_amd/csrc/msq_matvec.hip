@@ -290,12 +290,18 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
     // one workgroup per CU: all of its LDS (decoders that stage only in the four-token kernel read directly when a round does not fit)
     if (!place_x_row(a, lds, tok_round<D, T>(), kMaxLds - kStaticLds<D>, D::STAGE_X)) return MSQ_ERR_UNSUPPORTED;
   }
-  // Under a fused norm weight rows go through LDS from 17 MB on (Q6_K 4096x4608 8.5 / 9.2 us, 4096x7168 11.2 / 10.8, 16384x5120
-  // 23.7 / 19.0, 129280x5120 138 / 101), but for Q6_K rows of whole waves of 200 MB and more (129280x2048 38.5 / 40.1).
-  const bool norm_sw = bytes >= 17e6 && (std::is_same_v<D, DecQ8_0> || bytes < 200e6 || (a.cols / D::UNIT) % 64 != 0);
-  // ... and where the waves' buffers, four slots each, find room behind the staged activations (Q8_0 rows of more than 14336
-  // columns, eight waves of three pieces a slot, leave none)
+  // Weight rows through LDS: where the waves' buffers, four slots each, find room behind the staged activations (Q8_0 rows of more
+  // than 14336 columns, eight waves of three pieces a slot, leave none), ...
   const size_t w_at = (lds + 15) / 16 * 16, w_end = w_at + (size_t)(threads / 64) * 4 * wspan_loads<D>() * 1024;
+  const int w_per_cu = (w_end + kStaticLds<D>) * s.per_cu <= (size_t)kMaxLds ? s.per_cu : 1;
+  // ... and under a fused norm, for Q6_K, where a CU then holds six waves and more and the matrix has 17 MB, or 26 where the rows
+  // take the norm in one trip. Time without / with them, matrices and rows rotated beyond the caches:
+  //   2048 to 4352 columns (six to eight waves) 17.5 MB 1.00 to 1.06, 26 MB 1.03 to 1.08;
+  //   5632, 6144, 7168, 8192, 12288 columns (six to eight waves) 17.5 MB 0.98 to 1.00, 23 MB 0.99 to 1.00, 26 MB 1.01, 47 MB 1.02 to 1.05;
+  //   4608, 5120, 9216, 10240 columns (five waves) 17.5 MB 0.95 to 0.97, 30 MB 0.98 to 1.00, 47 MB 1.00 to 1.01; the first two with a
+  //   second workgroup (from 48 MB) 1.15 to 1.19, the other two, which have no room for it, 0.97 to 0.99;
+  //   2048, 4096, 6144, 8192 columns 210 MB 1.12 to 1.21 (one such matrix alone, which stays in the 256 MB cache, 0.91 to 1.00).
+  const bool norm_sw = std::is_same_v<D, DecQ8_0> || (threads / 64 * w_per_cu >= 6 && bytes >= (a.cols < 4608 ? 17e6 : 26e6));
   const bool sw = tok_stages_w<D, 1, T>() && s.iters == 1 && s.stage_w && (!a.norm_w || norm_sw) && w_end + kStaticLds<D> <= (size_t)kMaxLds;
   if (sw) {
     a.w_off = (uint32_t)(w_at / 4);

@@ -153,3 +153,11 @@ def test_fused_norm_of_large_matrices(dev, t, rows, cols):
 @pytest.mark.parametrize("rows,cols", [(2700, 14336), (2720, 14368), (2400, 16384)], ids=lambda v: None)
 def test_large_matrices_of_long_rows(dev, rows, cols):
     test_fused_equals_norm_then_matvec_and_oracle(dev, O.Q8_0, rows, cols)
+
+
+# Q6_K rows through LDS under a fused norm, on either side of each line: six waves a CU and 17 MB (short rows: 2048 columns) or 26
+# MB (6144); five waves a CU (4608, 10240 columns), and ten once a second workgroup fits (4608 columns, 48 MB)
+@pytest.mark.parametrize("rows,cols", [(10100, 2048), (10140, 2048), (5150, 6144), (5170, 6144), (7200, 4608), (12690, 4608), (12710, 4608), (3572, 10240), (5730, 10240)],
+                         ids=lambda v: None)
+def test_rows_through_lds_by_waves(dev, rows, cols):
+    test_fused_equals_norm_then_matvec_and_oracle(dev, O.Q6_K, rows, cols)
