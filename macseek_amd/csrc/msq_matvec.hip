@@ -260,7 +260,8 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   // one / in pairs: Q6_K 129280x5120 113.2 / 99.8 us, 1536x7168 6.41 / 6.10, 2304x5120 6.61 / 6.29, Q8_0 2304x5120
   // 6.67 / 6.52; the codebook formats, bound by their lookups, lose 1 % and keep the one-row form. MSQ_MV_PAIR = 0 / 2:
   // never / every format.
-  // Under a fused norm likewise, but for Q8_0 below 20 MB (4096x2560 6.19 / 6.40).
+  // Under a fused norm likewise, but for Q8_0 below 20 MB (2560, 4608, 5120 and 7168 columns, one by one over in pairs: 6 to 18 MB
+  // 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04).
   const double bytes = (double)a.rows * a.row_bytes;
   bool pair = false;
   {

@@ -132,9 +132,12 @@ int launch_block_t(hipStream_t st, PfBlkArgs a, uint32_t n6, uint32_t n3, uint32
   return launch_block_tt<B, GU, 3>(st, a);
 }
 // With the shared expert's products on the side stream, workgroups that stay pay from this many tokens on. They leave no room
-// for the shared expert's second product until the routed experts' first has ended, and with few tokens the shared expert's chain
-// is as long as theirs. Over 180 random calls, against a workgroup per unit: one stream 0.98 to 1.10 (mean 1.02) at any number of
-// tokens; two streams 0.90 to 1.08 (0.99) from 7 to 178 tokens, 1.00 to 1.09 (1.05) from 223 on.
+// for the shared expert's second product until the routed experts' first has ended, which costs while the shared expert's chain
+// is as long as theirs. Time of a workgroup per unit over workgroups that stay, one stream:
+// 0.98 to 1.10 (mean 1.02) at any number of tokens. Two streams, 104 calls of all types, 128 and 384 experts, back to back
+// (in brackets each alone): 7 to 60 tokens 0.88 to 1.05 (0.90 to 1.17), 100 and 140 0.96 to 1.10 (1.01 to 1.13), 178 to 212 0.99 to
+// 1.11 (1.01 to 1.11), 224 to 420 0.98 to 1.10 (1.01 to 1.10). Where the loss ends lies between 100 and 178 tokens and differs from
+// layer to layer; the line is drawn above all of it.
 constexpr int kPfQueueTokens = 2 * kPfBigTokens;
 bool block_path(int t) { return t == MSQ_IQ1_S || t == MSQ_IQ2_XXS; }
 template <bool GU>

@@ -392,8 +392,10 @@ int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffe
     hipLaunchKernelGGL(kernel, grid, block, 0, st, (const float*)bptr(x), (const void*)bptr(W), (uint32_t)dim, (uint32_t)n_exp,
                        (const float*)bptr(bias), logits, recs, counter, (int*)bptr_mut(ids), (float*)bptr_mut(w), route_scale);
   };
-  // One trip to memory for a row of nine to twelve vectors a lane (4097 to 6144 columns of BF16, half of F32) instead of two: 384
-  // BF16 experts x 5120 10.6 -> 10.0 us. Thirteen and more gain nothing (7168 columns 11.3 / 11.0, in the layer the same).
+  // One trip to memory for a row of nine to twelve vectors a lane (4097 to 6144 columns of BF16, half of F32) instead of two. Time
+  // of two trips over one, 64 to 384 experts, rows rotated beyond the caches: BF16 4104 to 5120 columns 1.06 to 1.10 (384x5120
+  // 10.6 -> 9.8 us), 5632 and 6144 1.03 to 1.06; F32 2056 to 3072 columns 1.05 to 1.08 (384x2560 9.8 -> 9.1). Thirteen vectors and
+  // more gain nothing (7168 columns 11.3 / 11.0, in the layer the same).
   const int per_lane = (dim / (wtype == MSQ_F32 ? 4 : 8) + 63) / 64;
   auto by_u = [&]<int QT>() {
     if (per_lane == 9 || per_lane == 10) launch(router_fused_kernel<QT, 10>);
