@@ -30,22 +30,33 @@ METRIC = "MoE decode matvec GB/s (% of HBM peak) + prefill MoE GEMM TFLOP/s (% M
 HBM_PEAK_GBPS = 8000.0
 
 
-def profile_traffic(name, line_start):
-    """HBM bytes that profiles/<name> records for the line that starts with `line_start`: the summaries of the
-    FETCH_SIZE / WRITE_SIZE counter runs give such a line's total as "= <MB> MB per launch" or ": <MB> MB per step" (KiB per
-    dispatch scaled by what the same counters read for a 1 GiB copy; the file says how). None when the file or the
-    line is missing, so a stale constant can never stand in for a measurement."""
+# Kernels that the lines below name, as the library holds them; those of TRAFFIC have their HBM bytes counted under profiles/
+DECODE_GATE_UP, DECODE_DOWN = "moe_gu_kernel<DecIQ1SQ, DecIQ2XXSQ>", "moe_down_kernel<DecIQ1S, DecIQ2XXS, 768>"
+PREFILL_GATE_UP = ("moe_pf_block_kernel<BlkIQ2XXS<4>, true, 7, true>", "moe_pf_block_kernel<BlkIQ2XXS<16>, true, 3, true>")
+PREFILL_DOWN = ("moe_pf_block_kernel<BlkIQ2XXS<4>, false, 7, true>", "moe_pf_block_kernel<BlkIQ2XXS<16>, false, 3, true>")
+MATVEC_N, ROUTER = "mm_rows_kernel<FragQ6KG, 2, 2, 8, 1, false, false>", "router_fused_kernel<30, 8u>"
+MATMUL_CONVERT = ("f32_to_f16_kernel", "dequant_kq_kernel<14, unsigned short>")
+TRAFFIC = {"moe_hbm_traffic_fetch_write.txt": (DECODE_GATE_UP,), "moe_prefill_hbm_traffic_fetch_write.txt": PREFILL_GATE_UP}
+
+
+def profile_traffic(name):
+    """HBM bytes that profiles/<name> records for the kernels TRAFFIC[name], all of them together: the summaries of the
+    FETCH_SIZE / WRITE_SIZE counter runs end a kernel's line with "= <MB> MB per launch" (KiB per dispatch scaled by what the
+    same counters read for a 1 GiB copy; the file says how). None when the file or the line of one of them, under its
+    full name, is missing, so that figures of an earlier kernel can never stand in for a measurement."""
     import re
+    found = {}
     try:
         with open(os.path.join(ROOT, "profiles", name)) as f:
             for l in f:
-                if l.startswith(line_start):
-                    m = re.search(r"[=:]\s*([0-9.]+) MB per (?:launch|step)", l)
-                    if m:
-                        return int(round(float(m.group(1)) * 1e6))
+                m = re.match(r"(\S.*?): .*= *([0-9.]+) MB per launch", l)
+                if m:
+                    found[m.group(1)] = float(m.group(2))
     except OSError:
         pass
-    return None
+    if any(k not in found for k in TRAFFIC[name]):
+        return None
+    return int(round(sum(found[k] for k in TRAFFIC[name]) * 1e6))
 
 
 def cores():
@@ -272,11 +283,11 @@ def bench_moe_decode(torch, args):
                                "top-6 of a seeded softmax router + 1 shared IQ2_XXS expert, SwiGLU; fresh top-6 per step",
                    "bytes_per_step": step_bytes, "experts": NE, "top_k": TOPK, "dim": DIM, "inter": INTER},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBPS,
-                     "traffic": profile_traffic("moe_hbm_traffic_fetch_write.txt", "moe_gu_kernel<"), "traffic_source": "profiles/moe_hbm_traffic_fetch_write.txt", "kernel": "moe_gu_kernel<DecIQ1SQ,DecIQ2XXSQ>", "bytes_per_launch": gu_bytes,
+                     "traffic": profile_traffic("moe_hbm_traffic_fetch_write.txt"), "traffic_source": "profiles/moe_hbm_traffic_fetch_write.txt", "kernel": DECODE_GATE_UP, "bytes_per_launch": gu_bytes,
                      "avg_launch_us": gu_graph * 1e3,
                      "timing": "HIP event pair around one graph replay of %d back-to-back launches of this kernel" % n_ev,
                      "eager_event_pair_us": {"mean": gu_mean * 1e3, "median": gu_med * 1e3, "min": gu_min * 1e3},
-                     "second_kernel": {"kernel": "moe_down_kernel<DecIQ1S,DecIQ2XXS>", "bytes_per_launch": dn_bytes,
+                     "second_kernel": {"kernel": DECODE_DOWN, "bytes_per_launch": dn_bytes,
                                        "avg_launch_us": dn_graph * 1e3, "achieved": dn_bytes / (dn_graph * 1e-3) / 1e9,
                                        "eager_event_pair_us": {"mean": dn_mean * 1e3, "median": dn_med * 1e3, "min": dn_min * 1e3}}},
         "cpu_baseline": {"value": cpu_value, "unit": "GB/s", "cores": nth, "kind": "port",
@@ -449,13 +460,13 @@ def bench_moe_prefill(torch, steps, warmup, with_cpu=True):
                    "tokens_per_expert_median": float(np.median(counts[used])), "flops_per_step": flops,
                    "weight_bytes_touched": int(len(used)) * per_exp},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / MFMA_PEAK_TFLOPS,
-                     "traffic": profile_traffic("moe_prefill_hbm_traffic_fetch_write.txt", "gate/up ("), "traffic_source": "profiles/moe_prefill_hbm_traffic_fetch_write.txt",
-                     "kernel": "moe_pf_block_kernel<BlkIQ2XXS, gate/up> (two launches: blocks of 49..112 entries of the popular experts; items of one to three token tiles)",
+                     "traffic": profile_traffic("moe_prefill_hbm_traffic_fetch_write.txt"), "traffic_source": "profiles/moe_prefill_hbm_traffic_fetch_write.txt",
+                     "kernel": "%s (blocks of 49..112 entries of the popular experts) and %s (items of one to three token tiles)" % PREFILL_GATE_UP,
                      "gate_up_time_split": split,
                      "flops_per_launch": gu_flops,
                      "avg_launch_us": gu_mean * 1e3, "min_launch_us": gu_min * 1e3,
                      "weight_GBps": int(len(used)) * 2 * gu_b / (gu_mean * 1e-3) / 1e9,
-                     "second_kernel": {"kernel": "moe_pf_block_kernel<BlkIQ2XXS, down> (two launches)", "avg_launch_us": dn_mean * 1e3,
+                     "second_kernel": {"kernel": "%s and %s" % PREFILL_DOWN, "avg_launch_us": dn_mean * 1e3,
                                        "achieved": 2.0 * DIM * INTER * total / (dn_mean * 1e-3) / 1e12}},
         "pct_of_mfma_peak": 100 * value / MFMA_PEAK_TFLOPS,
     }
@@ -739,7 +750,7 @@ def bench_matvec_n(torch, args):
             "config": {"workload": "BASELINE configs[4]: small-N matvec (speculative verify), attention projections, N in {1,2,4,8,16}; "
                                    "one step = one msq_matvec_n launch of Q6_K 1536x7168 at N=8", "cases": cases},
             "roofline": {"bound": "hbm", "achieved": head["GBps"], "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": head["GBps"] / HBM_PEAK_GBPS,
-                         "traffic": None, "kernel": "mv_tok_kernel<DecQ6K, 1, 8>", "bytes_per_launch": head["bytes"],
+                         "traffic": None, "kernel": MATVEC_N, "bytes_per_launch": head["bytes"],
                          "avg_launch_us": head["us_per_launch"], "timing": "HIP event pair around one graph replay of 200 back-to-back launches"},
             "cpu_baseline": cpu, "pct_of_hbm_peak": 100 * head["GBps"] / HBM_PEAK_GBPS}
 
@@ -869,7 +880,7 @@ def bench_router(torch, args):
                        "fused_bytes_per_launch": fused_bytes, "fused_us": fused_ms * 1e3, "topk_2048_tokens_us": topk_ms * 1e3,
                        "route_lists_2048_tokens_us": lists_ms * 1e3},
             "roofline": {"bound": "hbm", "achieved": gbps, "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": gbps / HBM_PEAK_GBPS, "traffic": None,
-                         "kernel": "router_fused_kernel<BF16>", "bytes_per_launch": fused_bytes, "avg_launch_us": fused_ms * 1e3},
+                         "kernel": ROUTER, "bytes_per_launch": fused_bytes, "avg_launch_us": fused_ms * 1e3},
             "cpu_baseline": cpu, "pct_of_hbm_peak": 100 * gbps / HBM_PEAK_GBPS}
 
 
@@ -929,7 +940,7 @@ def bench_matmul(torch, args):
     return {"value": head["TFLOPs"], "ms_per_step": head["us_per_call"] * 1e-3, "dtype": "f16 x f16 MFMA (weights and activations rounded to fp16), f32 accumulate",
             "config": {"workload": "prefill matmul, 2048 tokens, BASELINE configs[4] shapes; one step = one msq_matmul call of the Q6_K 1536x7168 case", "cases": rows_out},
             "roofline": {"bound": "mfma", "achieved": head["TFLOPs"], "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": head["TFLOPs"] / MFMA_PEAK_TFLOPS,
-                         "traffic": None, "kernel": "f32_to_f16_kernel + dequant_kernel<Q6_K, fp16> + rocBLAS fp16 GEMM (whole call; few tokens: mm_fused_kernel, see cases)", "flops_per_launch": 2.0 * n * 1536 * 7168,
+                         "traffic": None, "kernel": "%s + %s (Q6_K to fp16) + rocBLAS fp16 GEMM (whole call; few tokens: mm_fused_kernel, see cases)" % MATMUL_CONVERT, "flops_per_launch": 2.0 * n * 1536 * 7168,
                          "avg_launch_us": head["us_per_call"]},
             "cpu_baseline": cpu}
 
