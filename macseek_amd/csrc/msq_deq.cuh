@@ -74,9 +74,9 @@ __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict_
   put8(dst + 8 * c, y);
 }
 
-// Q6_K, Q5_K: a thread takes eight low bytes and so 16 weights, eight from either nibble (64 and 32 elements apart; eight threads
-// store 128 consecutive bytes of fp16), and works on words of four. Bound by memory as far as the launch is long: one nibble and
-// a byte at a time (16 vector instructions a weight) took Q6_K 32768x1280 29.5 us, 1024x4096 7.7.
+// Q6_K, Q5_K: a thread takes eight low bytes and so 16 weights, eight from either nibble (64 and 32 elements apart: of fp16 eight
+// threads store 128 consecutive bytes of Q6_K, four threads 64 of Q5_K), and works on words of four. Bound by memory as far as the
+// launch is long: one nibble and a byte at a time (16 vector instructions a weight) took Q6_K 32768x1280 29.5 us, 1024x4096 7.7.
 template <int QT, class OUT>
 __global__ __launch_bounds__(256) void dequant_kq_kernel(const uint8_t* __restrict__ src, OUT* __restrict__ dst, int64_t nchunks) {
 #pragma clang fp contract(off)

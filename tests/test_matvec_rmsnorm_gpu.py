@@ -133,8 +133,8 @@ def test_both_prologues_of_the_fused_norm(dev, t, rows, cols):
     test_fused_equals_norm_then_matvec_and_oracle(dev, t, rows, cols)
 
 
-# weight rows through LDS, two rows as one, a second workgroup per CU under a fused norm, on either side of each line: Q6_K at
-# 17 MB (rows in pairs; an odd number of rows; whole waves) and 200 MB (whole waves), Q8_0 at 20 MB (pairs) and 40 MB, two
+# weight rows through LDS, two rows as one, a second workgroup per CU under a fused norm: Q6_K of 17 MB (rows in pairs; an odd
+# number of rows; whole waves), 48 and 200 MB (its lines: test_rows_through_lds_by_waves), Q8_0 on either side of 20 MB (pairs) and 40 MB, two
 # workgroups from 48 MB (Q5_K with either prologue) and 8 MB (dense; F32 of one and two units a lane)
 LARGE = [
     (O.Q6_K, 4000, 5120), (O.Q6_K, 4096, 5120), (O.Q6_K, 4097, 5120), (O.Q6_K, 10300, 2048), (O.Q6_K, 16390, 3584), (O.Q6_K, 119500, 2048),
@@ -156,8 +156,8 @@ def test_large_matrices_of_long_rows(dev, rows, cols):
 
 
 # Q6_K rows through LDS under a fused norm, on either side of each line: six waves a CU and 17 MB (short rows: 2048 columns) or 26
-# MB (6144); five waves a CU (4608, 10240 columns), and ten once a second workgroup fits (4608 columns, 48 MB)
-@pytest.mark.parametrize("rows,cols", [(10100, 2048), (10140, 2048), (5150, 6144), (5170, 6144), (7200, 4608), (12690, 4608), (12710, 4608), (3572, 10240), (5730, 10240)],
+# MB (6144); five waves a CU (4608, 10240 columns), and ten once a second workgroup fits (4608 columns, 48 MB); an odd number of rows
+@pytest.mark.parametrize("rows,cols", [(10100, 2048), (10140, 2048), (5150, 6144), (5170, 6144), (7200, 4608), (12690, 4608), (12710, 4608), (11701, 5120), (3572, 10240), (5730, 10240)],
                          ids=lambda v: None)
 def test_rows_through_lds_by_waves(dev, rows, cols):
     test_fused_equals_norm_then_matvec_and_oracle(dev, O.Q6_K, rows, cols)
