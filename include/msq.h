@@ -295,10 +295,10 @@ int msq_router_topk(void* stream, const MsqBuffer* logits, const MsqBuffer* bias
 /* reference: ms::arch::encode_router_fused (arch.hpp:79-83; kernel arch_router_fused, arch_router.metal:86-121):
  * logits = W[n_exp][dim] . x[dim] and the selection in one launch; W is F32 (the reference's ffn_gate_inp) or BF16.
  * scratch (>= msq_router_scratch_bytes(n_exp), the reference's Scratch::router_logits + counter) receives the logits in
- * its first n_exp floats; the caller zeroes it once before the first call and the call leaves its counter re-armed.
+ * its first n_exp floats; the caller zeroes it once before the first call, and the calls count themselves in it.
  * A scratch belongs to one stream at a time: calls sharing it must not overlap. A launch that fails (MSQ_ERR_HIP) or is
- * torn down part-way may leave the counter between zero and the workgroup count, after which calls would select
- * nothing: zero the scratch again before it is reused. */
+ * torn down part-way may leave results of a call that is not counted, which the next call would take for its own:
+ * zero the scratch again before it is reused. */
 size_t msq_router_scratch_bytes(int n_exp);
 int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffer* W, const MsqBuffer* bias,
                      const MsqBuffer* scratch, const MsqBuffer* ids, const MsqBuffer* w, int dim, int n_exp,

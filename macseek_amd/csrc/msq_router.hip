@@ -39,8 +39,6 @@ __device__ __forceinline__ int wave_min_i(int v) {
   return __builtin_amdgcn_readlane(v, 63);
 }
 
-struct alignas(16) RouterRec { double score; float key; float logit; };
-
 // score and key of one expert, rounded where the reference's CPU twin rounds (tests/ref/arch_ref.cpp:100-105)
 __device__ __forceinline__ void score_key(float logit, float bias, double& sc, float& key) {
   const double x = (double)logit;
@@ -108,160 +106,138 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restric
   select6(key, sc, epl, route_scale, lane, ids + (size_t)t * kTopK, wts + (size_t)t * kTopK);
 }
 
-// Decode: logits = W[n_exp][dim] . x[dim] and the selection in one launch. A workgroup is four waves, each taking one
-// expert row and leaving the expert's logit, score and key in scratch; the workgroup that finishes last (device-scope
-// counter, one increment per workgroup: n_exp / 4 of them contend, not n_exp) selects from the keys, then re-arms the
-// counter. W is F32 (QT = MSQ_F32) or BF16. No bit of the result depends on which workgroup is last.
+// Decode: logits = W[n_exp][dim] . x[dim] and the selection in one launch. A workgroup is eight waves, four to an expert's row,
+// so that a row of up to 8192 columns is one trip to memory; the launch's last workgroup has no rows and selects.
+//
+// What bounds it is a chain of latencies: launch, one trip to memory, the hand-over of the logits between workgroups, the
+// scores' double-precision arithmetic, the selection. The hand-over is a record per expert: the logit and the number of the
+// call in one 64-bit device-scope store, and the selecting workgroup, one expert a thread, reads its record until it holds
+// this call's number. Against workgroups that waited for their stores, counted themselves in and left the selection to the last
+// one, with a wave a row (14 vectors a lane in two trips) and two reductions per choice: 384x7168 of BF16 10.9 -> 7.7 us,
+// 384x5120 10.1 -> 7.2, 64x2048 8.3 -> 5.4, F32 384x7168 12.4 -> 8.6 (calls back to back, weights from HBM).
+// The call's number stands behind the records; the selecting workgroup counts it up at its end, when every other workgroup
+// has read it (it has their records). Every wait ends: the other workgroups wait for nothing, and the selecting one, the last
+// of the launch, gives up after kRouterPolls reads (seconds; the experts without a record then count as NaN).
+constexpr uint32_t kRouterPolls = 1u << 22;
 template <int QT, uint32_t U>
-__global__ __launch_bounds__(256) void router_fused_kernel(const float* __restrict__ x, const void* __restrict__ W, uint32_t dim,
+__global__ __launch_bounds__(512) void router_fused_kernel(const float* __restrict__ x, const void* __restrict__ W, uint32_t dim,
                                                            uint32_t n_exp, const float* __restrict__ bias, float* logits,
-                                                           RouterRec* recs, uint32_t* counter, int* __restrict__ ids,
+                                                           uint64_t* recs, uint32_t* call, int* __restrict__ ids,
                                                            float* __restrict__ wts, float route_scale) {
-  __shared__ uint32_t last;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, e = blockIdx.x * 4u + wave;
-  // the row's weights are requested U vectors per lane at a time before any is used: with one wave per row the loop is
-  // otherwise a chain of memory latencies (the launcher picks U)
-  float acc = 0.f;
-  if constexpr (QT == MSQ_F32) {
-    const float4* wr = (const float4*)((const float*)W + (size_t)e * dim);
-    const float4* xv = (const float4*)x;
-    const uint32_t nv = dim / 4u;
-    for (uint32_t c0 = 0; c0 < nv; c0 += 64u * U) {
-      float4 a[U], b[U];
+  constexpr uint32_t WAVES = 8, SPLIT = 4;
+  __shared__ float part[WAVES];
+  __shared__ float c_key[WAVES * kTopK];
+  __shared__ int c_id[WAVES * kTopK];
+  __shared__ double c_sc[WAVES * kTopK];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t number = *call + 1u;
+  if (blockIdx.x + 1u < gridDim.x) {
+    const uint32_t e = blockIdx.x * (WAVES / SPLIT) + wave / SPLIT, first = 64u * (wave % SPLIT) + lane;
+    constexpr uint32_t STEP = 64u * SPLIT;
+    float acc = 0.f;
+    if constexpr (QT == MSQ_F32) {
+      const float4* wr = (const float4*)((const float*)W + (size_t)e * dim);
+      const float4* xv = (const float4*)x;
+      const uint32_t nv = dim / 4u;
+      for (uint32_t c0 = first; c0 < nv; c0 += STEP * U) {
+        float4 a[U], b[U];
 #pragma unroll
-      for (uint32_t u = 0; u < U; u++) { const uint32_t c = min(c0 + 64u * u + lane, nv - 1u); a[u] = wr[c]; b[u] = xv[c]; }
+        for (uint32_t u = 0; u < U; u++) { const uint32_t c = min(c0 + STEP * u, nv - 1u); a[u] = wr[c]; b[u] = xv[c]; }
 #pragma unroll
-      for (uint32_t u = 0; u < U; u++)
-        if (c0 + 64u * u + lane < nv) acc += a[u].x * b[u].x + a[u].y * b[u].y + a[u].z * b[u].z + a[u].w * b[u].w;
-    }
-  } else {
-    const uint4* wr = (const uint4*)((const uint16_t*)W + (size_t)e * dim);
-    const float4* xv = (const float4*)x;
-    const uint32_t nv = dim / 8u;
-    for (uint32_t c0 = 0; c0 < nv; c0 += 64u * U) {
-      uint4 a[U];
-      float4 b0[U], b1[U];
-#pragma unroll
-      for (uint32_t u = 0; u < U; u++) {
-        const uint32_t c = min(c0 + 64u * u + lane, nv - 1u);
-        a[u] = wr[c]; b0[u] = xv[2 * c]; b1[u] = xv[2 * c + 1];
+        for (uint32_t u = 0; u < U; u++)
+          if (c0 + STEP * u < nv) acc += a[u].x * b[u].x + a[u].y * b[u].y + a[u].z * b[u].z + a[u].w * b[u].w;
       }
+    } else {
+      const uint4* wr = (const uint4*)((const uint16_t*)W + (size_t)e * dim);
+      const float4* xv = (const float4*)x;
+      const uint32_t nv = dim / 8u;
+      for (uint32_t c0 = first; c0 < nv; c0 += STEP * U) {
+        uint4 a[U];
+        float4 b0[U], b1[U];
 #pragma unroll
-      for (uint32_t u = 0; u < U; u++)
-        if (c0 + 64u * u + lane < nv)
-          acc += __builtin_bit_cast(float, a[u].x << 16) * b0[u].x + __builtin_bit_cast(float, a[u].x & 0xFFFF0000u) * b0[u].y +
-                 __builtin_bit_cast(float, a[u].y << 16) * b0[u].z + __builtin_bit_cast(float, a[u].y & 0xFFFF0000u) * b0[u].w +
-                 __builtin_bit_cast(float, a[u].z << 16) * b1[u].x + __builtin_bit_cast(float, a[u].z & 0xFFFF0000u) * b1[u].y +
-                 __builtin_bit_cast(float, a[u].w << 16) * b1[u].z + __builtin_bit_cast(float, a[u].w & 0xFFFF0000u) * b1[u].w;
-    }
-  }
-  const float v = wave_sum(acc);
-  if (lane == 0) {
-    double sc;
-    float key;
-    score_key(v, bias[e], sc, key);
-    // Hand-over to the selecting workgroup. Writer side: the three results are device-scope atomic stores (they are
-    // written through to the level of the memory system that all XCDs share, never parked in this XCD's L2), the
-    // wave waits until the memory system has acknowledged them (vmcnt(0)), and only then, after the workgroup
-    // barrier, is the counter incremented: a store that is acknowledged is visible to every device-scope load, so no
-    // record can be observed older than the count that announces it. This is the effect of a release fence without its
-    // price: a device-scope release writes back the whole L2 of this workgroup's XCD (measured: the launch takes
-    // 19 us with plain stores and a fence, 15 us with atomic stores and a fence, less without the fence). Reader side:
-    // the workgroup that draws the last count passes an acquire fence (cheap: it drops cached lines, writes nothing)
-    // and reads the records with device-scope atomic loads.
-    uint64_t* r = (uint64_t*)(recs + e);
-    __hip_atomic_store(logits + e, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(r, __builtin_bit_cast(uint64_t, sc), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(r + 1, (uint64_t)__builtin_bit_cast(uint32_t, key) | ((uint64_t)__builtin_bit_cast(uint32_t, v) << 32),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
-  __syncthreads();
-  if (tid == 0) {
-    const uint32_t prev = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last = prev == gridDim.x - 1u ? 1u : 0u;
-  }
-  __syncthreads();
-  if (!last) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  // Selection in two levels. Six rounds of "wave-wide best, then remove it" by one wave over all experts is a chain of
-  // twelve DPP reductions plus a six-way local maximum per round, run by a wave that has its SIMD to itself: 3 us.
-  // Here each of the four waves picks the six best of its quarter of the experts (two per lane at most: the local
-  // maximum is one comparison), leaves them in LDS, and wave 0 picks the six best of those 24 (one per lane). The six
-  // best overall are among the six best of their quarters, and "greater key, then lower expert id" is a total order, so
-  // the result is the one-level selection's.
-  __shared__ float c_key[4 * kTopK];
-  __shared__ int c_id[4 * kTopK];
-  __shared__ double c_sc[4 * kTopK];
-  const uint32_t quarter = n_exp >> 2;  // experts of this wave: quarter * wave + {lane, lane + 64}
-  {
-    float key[2];
-    double sc[2];
+        for (uint32_t u = 0; u < U; u++) {
+          const uint32_t c = min(c0 + STEP * u, nv - 1u);
+          a[u] = wr[c]; b0[u] = xv[2 * c]; b1[u] = xv[2 * c + 1];
+        }
 #pragma unroll
-    for (uint32_t i = 0; i < 2; i++) {
-      key[i] = -INFINITY;
-      sc[i] = 0.0;
-      if (lane + 64u * i < quarter) {  // device-scope loads: the records were written by other CUs during this launch
-        const uint64_t* r = (const uint64_t*)(recs + quarter * wave + lane + 64u * i);
-        const uint64_t s64 = __hip_atomic_load(r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint64_t k64 = __hip_atomic_load(r + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sc[i] = __builtin_bit_cast(double, s64);
-        key[i] = __builtin_bit_cast(float, (uint32_t)k64);
+        for (uint32_t u = 0; u < U; u++)
+          if (c0 + STEP * u < nv)
+            acc += __builtin_bit_cast(float, a[u].x << 16) * b0[u].x + __builtin_bit_cast(float, a[u].x & 0xFFFF0000u) * b0[u].y +
+                   __builtin_bit_cast(float, a[u].y << 16) * b0[u].z + __builtin_bit_cast(float, a[u].y & 0xFFFF0000u) * b0[u].w +
+                   __builtin_bit_cast(float, a[u].z << 16) * b1[u].x + __builtin_bit_cast(float, a[u].z & 0xFFFF0000u) * b1[u].y +
+                   __builtin_bit_cast(float, a[u].w << 16) * b1[u].z + __builtin_bit_cast(float, a[u].w & 0xFFFF0000u) * b1[u].w;
       }
     }
+    const float v = wave_sum(acc);
+    if (lane == 0) part[wave] = v;
+    __syncthreads();
+    if (wave % SPLIT == 0 && lane == 0) {
+      const float logit = (part[wave] + part[wave + 1]) + (part[wave + 2] + part[wave + 3]);
+      __hip_atomic_store(recs + e, (uint64_t)__builtin_bit_cast(uint32_t, logit) | ((uint64_t)number << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      logits[e] = logit;
+    }
+    return;
+  }
+  // Selection in two levels: each wave picks the six best of its 64 experts, one a lane, and leaves them in LDS; wave 0 picks
+  // the six best of those 48. The six best overall are among the six best of their waves, and "greater key, then lower expert
+  // id" is a total order: experts, and the candidates that a wave leaves, stand in the lanes in the order of their ids where keys
+  // are equal, so the first lane with the greatest key is the choice. NaN and -inf are never chosen.
+  float key = -INFINITY;
+  double sc = 0.0;
+  if (tid < n_exp) {
+    const float b = bias[tid];
+    uint64_t r = 0;
+    for (uint32_t k = 0; k < kRouterPolls; k++) {
+      r = __hip_atomic_load(recs + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if ((uint32_t)(r >> 32) == number) break;
+    }
+    const float logit = (uint32_t)(r >> 32) == number ? __builtin_bit_cast(float, (uint32_t)r) : __builtin_nanf("");
+    score_key(logit, b, sc, key);
+    if (!(key > -INFINITY)) key = -INFINITY;
+  }
 #pragma unroll
-    for (int k = 0; k < kTopK; k++) {
-      // the lane's best: strict comparisons from -inf up, so NaN and -inf keys are never candidates and the lower id
-      // wins among equals
-      float bk = -INFINITY;
-      bool second = false, any = false;
-      if (key[0] > bk) { bk = key[0]; any = true; }
-      if (key[1] > bk) { bk = key[1]; second = true; any = true; }
-      const int be = any ? (int)(quarter * wave + lane + (second ? 64u : 0u)) : 0x7fffffff;
-      const float m = wave_max_f(bk);
-      const int win = wave_min_i(bk == m ? be : 0x7fffffff);
-      if (win != 0x7fffffff && be == win) {  // one lane
-        c_key[wave * kTopK + k] = bk;
-        c_id[wave * kTopK + k] = win;
-        c_sc[wave * kTopK + k] = second ? sc[1] : sc[0];
-        if (second) key[1] = -INFINITY; else key[0] = -INFINITY;
-      }
-      if (win == 0x7fffffff && lane == 0) { c_key[wave * kTopK + k] = -INFINITY; c_id[wave * kTopK + k] = 0x7fffffff; c_sc[wave * kTopK + k] = 0.0; }
+  for (int k = 0; k < kTopK; k++) {
+    const float m = wave_max_f(key);
+    const uint64_t best = __builtin_amdgcn_ballot_w64(key == m && m > -INFINITY);
+    const bool won = best ? (uint32_t)__builtin_ctzll(best) == lane : lane == 0;
+    if (won) {
+      c_key[wave * kTopK + k] = m;
+      c_id[wave * kTopK + k] = (int)tid;
+      c_sc[wave * kTopK + k] = sc;
+      key = -INFINITY;
     }
   }
   __syncthreads();
-  if (wave == 0) {
-    float ck = lane < 4u * kTopK ? c_key[lane] : -INFINITY;
-    const int ce = lane < 4u * kTopK ? c_id[lane] : 0x7fffffff;
-    const double cs = lane < 4u * kTopK ? c_sc[lane] : 0.0;
-    int sel_e[kTopK];
-    double sel_s[kTopK];
-    double sum = 0.0;  // the six scores are added in selection order, as the reference adds them
+  if (wave != 0) return;
+  if (lane == 0) __hip_atomic_store(call, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  float ck = lane < WAVES * kTopK ? c_key[lane] : -INFINITY;
+  const int ce = lane < WAVES * kTopK ? c_id[lane] : 0;
+  const uint64_t cs = lane < WAVES * kTopK ? __builtin_bit_cast(uint64_t, c_sc[lane]) : 0;
+  int sel_e[kTopK];
+  double sel_s[kTopK];
+  double sum = 0.0;  // the six scores are added in selection order, as the reference adds them
 #pragma unroll
-    for (int k = 0; k < kTopK; k++) {
-      const float m = wave_max_f(ck);
-      const int win = wave_min_i((ck == m && ce != 0x7fffffff) ? ce : 0x7fffffff);
-      if (win == 0x7fffffff) {  // fewer than six comparable keys (NaN logits): expert 0 with weight 0
-        sel_e[k] = 0;
-        sel_s[k] = 0.0;
-        continue;
-      }
-      const uint64_t holder = __builtin_amdgcn_ballot_w64(ce == win);
-      const int src = (int)__builtin_ctzll(holder);
-      if (ce == win) ck = -INFINITY;
-      const uint64_t bits = __builtin_bit_cast(uint64_t, cs);
-      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, src);
-      const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), src);
-      sel_e[k] = win;
-      sel_s[k] = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-      sum += sel_s[k];
+  for (int k = 0; k < kTopK; k++) {
+    const float m = wave_max_f(ck);
+    const uint64_t best = __builtin_amdgcn_ballot_w64(ck == m && m > -INFINITY);
+    if (!best) {  // fewer than six comparable keys (NaN logits): expert 0 with weight 0
+      sel_e[k] = 0;
+      sel_s[k] = 0.0;
+      continue;
     }
-    if (lane < (uint32_t)kTopK) {
+    const int src = (int)__builtin_ctzll(best);
+    if (lane == (uint32_t)src) ck = -INFINITY;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cs, src);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cs >> 32), src);
+    sel_e[k] = __builtin_amdgcn_readlane(ce, src);
+    sel_s[k] = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+    sum += sel_s[k];
+  }
+  if (lane < (uint32_t)kTopK) {
 #pragma unroll
-      for (int k = 0; k < kTopK; k++)
-        if (lane == (uint32_t)k) { ids[k] = sel_e[k]; wts[k] = (float)(sel_s[k] / (sum + 1e-20) * (double)route_scale); }
-    }
-    if (lane == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = 0; k < kTopK; k++)
+      if (lane == (uint32_t)k) { ids[k] = sel_e[k]; wts[k] = (float)(sel_s[k] / (sum + 1e-20) * (double)route_scale); }
   }
 }
 
@@ -369,8 +345,8 @@ int msq_router_topk(void* stream, const MsqBuffer* logits, const MsqBuffer* bias
   return MSQ_OK;
 }
 
-// scratch: logits f32 [n_exp] (padded to 256 bytes), {score f64, key f32, logit f32} [n_exp], then the counter in a
-// 256-byte line of its own
+// scratch: logits f32 [n_exp] (padded to 256 bytes), records {logit f32, number of the call u32} [n_exp] in the first half of 16
+// bytes an expert (callers keep the scratch size), then the number of the last call in a 256-byte line of its own
 size_t msq_router_scratch_bytes(int n_exp) { return ((size_t)n_exp * 4 + 255) / 256 * 256 + (size_t)n_exp * 16 + 256; }
 
 int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffer* W, const MsqBuffer* bias,
@@ -384,23 +360,22 @@ int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffe
     return fail(MSQ_ERR_SCRATCH, "macseek quant: router_fused scratch too small unsupported (type %s rows %d cols %d)",
                 msq_type_name_of(wtype), n_exp, dim);
   float* logits = (float*)bptr_mut(scratch);
-  RouterRec* recs = (RouterRec*)(bptr_mut(scratch) + ((size_t)n_exp * 4 + 255) / 256 * 256);
-  uint32_t* counter = (uint32_t*)(bptr_mut(scratch) + msq_router_scratch_bytes(n_exp) - 256);
-  const dim3 grid((unsigned)(n_exp / 4)), block(256);
+  uint64_t* recs = (uint64_t*)(bptr_mut(scratch) + ((size_t)n_exp * 4 + 255) / 256 * 256);
+  uint32_t* call = (uint32_t*)(bptr_mut(scratch) + msq_router_scratch_bytes(n_exp) - 256);
+  const dim3 grid((unsigned)(n_exp / 2 + 1)), block(512);  // two rows a workgroup, and the selecting one
   hipStream_t st = (hipStream_t)stream;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, st, (const float*)bptr(x), (const void*)bptr(W), (uint32_t)dim, (uint32_t)n_exp,
-                       (const float*)bptr(bias), logits, recs, counter, (int*)bptr_mut(ids), (float*)bptr_mut(w), route_scale);
+                       (const float*)bptr(bias), logits, recs, call, (int*)bptr_mut(ids), (float*)bptr_mut(w), route_scale);
   };
-  // One trip to memory for a row of nine to twelve vectors a lane (4097 to 6144 columns of BF16, half of F32) instead of two. Time
-  // of two trips over one, 64 to 384 experts, rows rotated beyond the caches: BF16 4104 to 5120 columns 1.06 to 1.10 (384x5120
-  // 10.6 -> 9.8 us), 5632 and 6144 1.03 to 1.06; F32 2056 to 3072 columns 1.05 to 1.08 (384x2560 9.8 -> 9.1). Thirteen vectors and
-  // more gain nothing (7168 columns 11.3 / 11.0, in the layer the same).
-  const int per_lane = (dim / (wtype == MSQ_F32 ? 4 : 8) + 63) / 64;
+  // vectors a lane of the four waves that share a row: one trip to memory up to 8192 columns
+  const int per_lane = (dim / (wtype == MSQ_F32 ? 4 : 8) + 255) / 256;
   auto by_u = [&]<int QT>() {
-    if (per_lane == 9 || per_lane == 10) launch(router_fused_kernel<QT, 10>);
-    else if (per_lane == 11 || per_lane == 12) launch(router_fused_kernel<QT, 12>);
-    else launch(router_fused_kernel<QT, 8>);
+    if (per_lane <= 2) return launch(router_fused_kernel<QT, 2>);
+    if constexpr (QT == MSQ_F32) {
+      if (per_lane > 4) return launch(router_fused_kernel<QT, 8>);
+    }
+    launch(router_fused_kernel<QT, 4>);
   };
   if (wtype == MSQ_F32) by_u.template operator()<MSQ_F32>();
   else by_u.template operator()<MSQ_BF16>();

@@ -250,3 +250,9 @@ def test_route_lists_over_waves_and_rounds(dev, n, n_exp):
 @pytest.mark.parametrize("wtype,dim", [(q.QType.BF16, d) for d in (4096, 4104, 5120, 5128, 6144, 6152)] + [(q.QType.F32, d) for d in (2048, 2056, 2560, 2568, 3072, 3080)])
 def test_router_fused_row_lengths(dev, wtype, dim):
     test_router_fused_vs_oracle(dev, wtype, dim)
+
+
+# four waves share a row: vectors a lane of one, two, four and (F32) eight requested at once, a row's last vector, a second trip
+@pytest.mark.parametrize("wtype,dim", [(q.QType.BF16, d) for d in (8, 2048, 2056, 8192, 8200)] + [(q.QType.F32, d) for d in (8, 1024, 1032, 4096, 4104, 8192, 8200)])
+def test_router_fused_shared_rows(dev, wtype, dim):
+    test_router_fused_vs_oracle(dev, wtype, dim)
