@@ -32,6 +32,7 @@ struct RowsArgs {
   uint32_t n, rows, cols, x_stride, row_bytes, accumulate;
   uint32_t rows_per_group, x_group_stride;  // block-diagonal: rows per group (whole tiles), elements between the groups' inputs
   uint32_t nws;             // weight stages of a row
+  uint32_t w_bytes;         // bytes from W to the matrix's end
   uint32_t tiles_per_wg;    // consecutive row tiles of a workgroup (of one group)
   uint32_t ntiles;
 };
@@ -42,6 +43,8 @@ template <class F> constexpr int rows_pieces() { return ((F::WS_BYTES + 14 + 15)
 template <class F> constexpr int rows_slot() { return 16 * rows_pieces<F>() * 16; }            // bytes of a stage of 16 rows
 // slots requested ahead of the activations, which pass through the rest of the ring
 template <class F> constexpr int rows_early(int S) { return rows_slot<F>() < 2048 ? 1 : S - 1; }
+// words of the waves' partial tiles
+__host__ __device__ constexpr uint32_t rows_red_words(uint32_t waves, int UT, int TT) { return (TT == 1 ? 2u : TT) * waves * 256u * UT; }
 template <class F> constexpr int rows_ring(int S) {
   const int x = rows_early<F>(S) * rows_slot<F>() + kRowsXBytes;
   return S * rows_slot<F>() > x ? S * rows_slot<F>() : x;
@@ -83,8 +86,11 @@ __device__ __forceinline__ f4_t fma4(float s, f4_t p, f4_t c) {
 }
 
 // ROUND: the arithmetic of msq_matmul -- scale times payload rounded to fp16, summed in the matrix cores -- over any number
-// of tokens, sixteen per workgroup (blockIdx.y). XH: activations in memory are fp16.
-template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false>
+// of tokens, 16 TT per workgroup (blockIdx.y). XH: activations in memory are fp16. Decoding bounds the larger of these products
+// (about 37 vector instructions a fragment, which one matrix instruction uses), hence TT = 2: 8192x4096 at 64 tokens against
+// the routes of msq_matmul that slice K over workgroups: IQ4_NL 38.2 -> 22.0 us, Q6_K 30.8 -> 22.5, IQ2_XXS 38.1 -> 21.3; 1536x4096 of
+// IQ1_S at 200 32.1 -> 17.2. Three tiles' activations do not fit the registers of four waves a SIMD.
+template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false, int TT = 1>
 __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   constexpr int P = rows_pieces<F>(), PIECES = 16 * P, NPI = (PIECES + 63) / 64, SLOT = rows_slot<F>();
   constexpr bool GROUPS = requires { F::GROUPS; };
@@ -95,16 +101,16 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   const uint32_t n16 = lane & 15u, q = lane >> 4;
   uint32_t* tbl = smem;
   float* red = (float*)(smem + F::LDS_WORDS);                    // [2][wave][tile][token][16]
-  uint8_t* mine = (uint8_t*)(red + 2u * nwaves * (256u * UT)) + wave * (uint32_t)rows_ring<F>(S);
+  uint8_t* mine = (uint8_t*)(red + rows_red_words(nwaves, UT, TT)) + wave * (uint32_t)rows_ring<F>(S);
 
-  const uint32_t m0 = ROUND ? blockIdx.y * 16u : 0u, ntok = ROUND ? min(a.n - m0, 16u) : a.n;
+  const uint32_t m0 = ROUND ? blockIdx.y * (16u * TT) : 0u, ntok = ROUND ? min(a.n - m0, 16u * TT) : a.n;
   const uint32_t tile0 = blockIdx.x * a.tiles_per_wg, ntile = min(a.tiles_per_wg, a.ntiles - tile0);  // (grid: tile0 < ntiles)
   const uint32_t group = (tile0 * 16u) / a.rows_per_group;
   const uint32_t ws0 = wave * BPW;
 
   const uintptr_t wa = (uintptr_t)a.W;
   const uint32_t wmis = (uint32_t)wa & 15u;
-  const uint32_t wbytes = (wmis + a.rows * a.row_bytes + 15u) & ~15u;  // whole aligned pieces: no piece straddles the end
+  const uint32_t wbytes = (wmis + a.w_bytes + 15u) & ~15u;  // whole aligned pieces: no piece straddles the end
   const rsrc_t wrs = make_rsrc((const void*)(wa - wmis), wbytes);
   // stage i of the wave's walk: tile i / BPW, weight stage ws0 + i % BPW
   uint32_t rowoff[NPI], pc[NPI];  // per piece: row inside the tile (in bytes), 16-byte piece of the row
@@ -113,7 +119,7 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
     const uint32_t p = (uint32_t)k * 64u + lane;
     rowoff[k] = (p / P) * a.row_bytes; pc[k] = 16u * (p % P);
   }
-  const uint32_t end = wmis + a.rows * a.row_bytes;
+  const uint32_t end = wmis + a.w_bytes;
   auto request = [&](uint32_t tile, int b, uint32_t slot) {
     const uint32_t at = wmis + (tile * 16u) * a.row_bytes + min(ws0 + b, a.nws - 1u) * (uint32_t)F::WS_BYTES;  // (a stage past the row's end: bytes nobody reads)
 #pragma unroll
@@ -131,26 +137,27 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   F::fill_lds(tbl, (int)tid, (int)nthreads);
   // ---- activations of the wave's columns, through LDS: rows are read along the columns (lane by lane in fragment order
   // every load would touch sixteen rows), rounded to fp16, and read back as fragments
-  uint32_t xr[BPW * 8][4];
+  uint32_t xr[TT][BPW * 8][4];
   {
     uint8_t* xs = mine + rows_early<F>(S) * SLOT;
     using XT = std::conditional_t<XH, uint16_t, float>;
     using XV = std::conditional_t<XH, uint2, f4_t>;  // four activations
     const XT* xg = (const XT*)a.X + (size_t)group * a.x_group_stride + (size_t)m0 * a.x_stride;
     // (all of them requested at once where the registers hold them)
-    constexpr int NK = NT / 2, NB = 2 * BPW, AHEAD = NB * NK <= 16 ? NB : 2;
+    constexpr int NK = NT / 2, NH = 2 * BPW, NB = TT * NH, AHEAD = NB * NK <= 16 ? NB : 2;
     XV raw[AHEAD][NK];
-    auto fetch = [&](int hb, XV (&r)[NK]) {  // half stage hb: 128 columns; lanes 0-31 even tokens, 32-63 odd ones
-      const uint32_t col = min((ws0 * 2u + hb) * 128u, a.cols - 128u) + 4u * (lane & 31u);
+    auto fetch = [&](int i, XV (&r)[NK]) {  // half stage i % NH (128 columns) of token tile i / NH; lanes 0-31 even tokens, 32-63 odd ones
+      const uint32_t col = min((ws0 * 2u + i % NH) * 128u, a.cols - 128u) + 4u * (lane & 31u);
 #pragma unroll
-      for (int k = 0; k < NK; k++) r[k] = *(const XV*)(xg + (size_t)min(2u * k + (lane >> 5), ntok - 1u) * a.x_stride + col);  // tokens past n repeat the last
+      for (int k = 0; k < NK; k++) r[k] = *(const XV*)(xg + (size_t)min(16u * (i / NH) + 2u * k + (lane >> 5), ntok - 1u) * a.x_stride + col);  // tokens past n repeat the last
     };
 #pragma unroll
-    for (int hb = 0; hb < AHEAD; hb++) fetch(hb, raw[hb]);
+    for (int i = 0; i < AHEAD; i++) fetch(i, raw[i]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int hb = 0; hb < NB; hb++) {
-      XV(&r)[NK] = raw[hb % AHEAD];
+    for (int i = 0; i < NB; i++) {
+      const int hb = i % NH;
+      XV(&r)[NK] = raw[i % AHEAD];
 #pragma unroll
       for (int k = 0; k < NK; k++) {
         uint2 v;
@@ -159,11 +166,11 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
         *(uint2*)(xs + (2u * k + (lane >> 5)) * kRowsXPitch + 8u * (lane & 31u)) = v;
       }
       asm volatile("" ::: "memory");  // (written and read through different types)
-      if (hb + AHEAD < NB) fetch(hb + AHEAD, raw[hb % AHEAD]);
+      if (i + AHEAD < NB) fetch(i + AHEAD, raw[i % AHEAD]);
 #pragma unroll
       for (int js = 0; js < 4; js++) {
         const uint8_t* p = xs + (n16 & (NT - 1u)) * kRowsXPitch + 64u * js;
-        uint32_t(&x)[4] = xr[hb * 4 + js];
+        uint32_t(&x)[4] = xr[i / NH][hb * 4 + js];
         if constexpr (PAIR || GROUPS) {
           const uint2 lo = *(const uint2*)(p + 8u * q), hi = *(const uint2*)(p + 32u + 8u * q);
           if constexpr (PAIR) {
@@ -192,10 +199,11 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   const uint32_t ones[4] = {0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
   uint32_t i = 0, slot = 0;
   for (uint32_t tl = 0; tl < ntile; tl += UT) {
-    f4_t acc[UT];
+    f4_t acc[UT][TT];
 #pragma unroll
     for (int u = 0; u < UT; u++) {
-      acc[u] = zero;
+#pragma unroll
+      for (int t = 0; t < TT; t++) acc[u][t] = zero;
       if (tl + u >= ntile) continue;
       const uint32_t row = min((tile0 + tl + u) * 16u + n16, a.rows - 1u);
 #pragma unroll
@@ -207,11 +215,12 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
         if (ws0 + b < a.nws) {
 #pragma unroll
           for (int js = 0; js < 8; js++) {
-            const uint32_t(&x)[4] = xr[b * 8 + js];
+            const uint32_t(&x)[4] = xr[0][b * 8 + js];
+            f4_t& sum = acc[u][0];
             if constexpr (GROUPS) {
               const auto f = F::get(lrow, js, q, tbl);
-              acc[u] = fma4(f.sa, mfma_f16_k16(x[0], x[1], f.h[0], f.h[1], zero), acc[u]);
-              acc[u] = fma4(f.sb, mfma_f16_k16(x[2], x[3], f.h[2], f.h[3], zero), acc[u]);
+              sum = fma4(f.sa, mfma_f16_k16(x[0], x[1], f.h[0], f.h[1], zero), sum);
+              sum = fma4(f.sb, mfma_f16_k16(x[2], x[3], f.h[2], f.h[3], zero), sum);
             } else {
               const FragOut f = F::finish(F::load_raw(lrow, (uint32_t)js, q), (uint32_t)js, q, tbl);
               // (formats of 32-weight blocks: past a row that ends with half a stage the bytes are no blocks)
@@ -220,10 +229,11 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
                 uint32_t h[4];
 #pragma unroll
                 for (int p = 0; p < 4; p++) h[p] = scale_round_h2(f.h[p], sc, F::HAS_ADD ? f.add : 0.f);
-                acc[u] = mfma_f16(x, h, acc[u]);
+#pragma unroll
+                for (int t = 0; t < TT; t++) acc[u][t] = mfma_f16(xr[t][b * 8 + js], h, acc[u][t]);
               } else {
-                acc[u] = fma4(sc, mfma_f16(x, f.h, zero), acc[u]);
-                if constexpr (F::HAS_ADD) acc[u] = fma4(f.add, mfma_f16(x, ones, zero), acc[u]);
+                sum = fma4(sc, mfma_f16(x, f.h, zero), sum);
+                if constexpr (F::HAS_ADD) sum = fma4(f.add, mfma_f16(x, ones, zero), sum);
               }
             }
           }
@@ -233,11 +243,16 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
         slot = slot + 1 == S ? 0u : slot + 1;
       }
     }
-    float* rb = red + ((tl / UT) & 1u) * (nwaves * (256u * UT));
+    // [wave][row tile][token tile][token][row]; two buffers, so that one barrier separates the meetings, or (TT > 1: LDS) one
+    // that everyone has read when the next partial tiles come
+    float* rb = red + (TT == 1 ? (tl / UT) & 1u : 0u) * (nwaves * (256u * UT));
+    if (TT > 1 && tl > 0) __syncthreads();
 #pragma unroll
     for (int u = 0; u < UT; u++)
 #pragma unroll
-      for (int k = 0; k < 4; k++) rb[((wave * UT + u) * 16u + 4u * q + k) * 16u + n16] = acc[u][k];
+      for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) rb[(((wave * UT + u) * TT + t) * 16u + 4u * q + k) * 16u + n16] = acc[u][t][k];
     __syncthreads();  // (everyone read this buffer's last contents before the barrier between)
     for (uint32_t idx = tid; idx < 16u * UT * ntok; idx += nthreads) {
       const uint32_t t = idx / (16u * UT), r = idx % (16u * UT), u = r >> 4, orow = (tile0 + tl) * 16u + r;
@@ -246,7 +261,7 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
       for (uint32_t w0 = 0; w0 < nwaves; w0 += 8u) {  // eight partials requested before the first is added
         float v[8];
 #pragma unroll
-        for (uint32_t k = 0; k < 8u; k++) v[k] = rb[((min(w0 + k, nwaves - 1u) * UT + u) * 16u + t) * 16u + (r & 15u)];
+        for (uint32_t k = 0; k < 8u; k++) v[k] = rb[((min(w0 + k, nwaves - 1u) * UT + u) * (16u * TT) + t) * 16u + (r & 15u)];
 #pragma unroll
         for (uint32_t k = 0; k < 8u; k++) s += w0 + k < nwaves ? v[k] : 0.f;
       }

@@ -8,23 +8,30 @@ namespace msq {
 namespace {
 
 // workgroups: as many as are resident (four waves per SIMD, LDS), each a run of consecutive row tiles
-template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false>
+template <class F>
+size_t rows_lds(uint32_t waves, int S, int UT, int TT) {
+  return (size_t)F::LDS_WORDS * 4 + (size_t)rows_red_words(waves, UT, TT) * 4 + (size_t)waves * rows_ring<F>(S);
+}
+uint32_t rows_tiles_per_wg(uint32_t ntiles, uint32_t waves, size_t lds, uint32_t blocks) {
+  const uint32_t per_cu = std::max<uint32_t>(1, std::min<uint32_t>(16 / waves, (uint32_t)(kMaxLds / lds)));
+  const uint32_t slots = std::max<uint32_t>(1, (uint32_t)device_info().cus * per_cu / blocks);
+  return (ntiles + slots - 1) / slots;
+}
+template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false, int TT = 1>
 int launch_nt(hipStream_t st, RowsArgs a, uint32_t waves) {
-  const size_t lds = (size_t)F::LDS_WORDS * 4 + (size_t)waves * (2 * UT * 16 * 16 * 4 + rows_ring<F>(S));
+  const size_t lds = rows_lds<F>(waves, S, UT, TT);
   if (lds > (size_t)kMaxLds) return MSQ_ERR_UNSUPPORTED;
-  const int rc = allow_large_lds(mm_rows_kernel<F, BPW, S, NT, UT, ROUND, XH>, lds);
+  const int rc = allow_large_lds(mm_rows_kernel<F, BPW, S, NT, UT, ROUND, XH, TT>, lds);
   if (rc != MSQ_OK) return rc;
   a.ntiles = (a.rows + 15) / 16;
-  const uint32_t per_cu = std::max<uint32_t>(1, std::min<uint32_t>(16 / waves, (uint32_t)(kMaxLds / lds)));
-  const uint32_t blocks = ROUND ? (a.n + 15) / 16 : 1;
-  const uint32_t slots = std::max<uint32_t>(1, (uint32_t)device_info().cus * per_cu / blocks);
-  a.tiles_per_wg = (a.ntiles + slots - 1) / slots;
+  const uint32_t blocks = ROUND ? (a.n + 16 * TT - 1) / (16 * TT) : 1;
+  a.tiles_per_wg = rows_tiles_per_wg(a.ntiles, waves, lds, blocks);
   if (a.rows_per_group != a.rows) {  // a workgroup's tiles belong to one group
     const uint32_t tg = a.rows_per_group / 16;
     while (tg % a.tiles_per_wg) a.tiles_per_wg--;
   }
   const uint32_t grid = (a.ntiles + a.tiles_per_wg - 1) / a.tiles_per_wg;
-  hipLaunchKernelGGL((mm_rows_kernel<F, BPW, S, NT, UT, ROUND, XH>), dim3(grid, blocks), dim3(64 * waves), lds, st, a);
+  hipLaunchKernelGGL((mm_rows_kernel<F, BPW, S, NT, UT, ROUND, XH, TT>), dim3(grid, blocks), dim3(64 * waves), lds, st, a);
   MSQ_HIP(hipGetLastError());
   return MSQ_OK;
 }
@@ -84,10 +91,24 @@ bool serves(int t, int rows, uint32_t nws, int cols, int n, int groups) {
   return kq && nws <= 5 && cols % 512 && rows >= 20480;
 }
 
+// Blocks of sixteen or of 32 tokens (TT = 2: a decoded fragment feeds two matrix instructions, activations and partial tiles
+// take twice the registers and LDS)? Row tiles per workgroup either way, t1 and t2, decide, since a launch takes about 5.7 +
+// 2.9 t1 or 7.5 + 3.5 t2 us (IQ4_NL, 4096 columns). Measured over 20000 random calls that came here before, time with sixteen
+// over time with 32, median (lowest of 100): up to 2048 columns, t1 over t2: 3 / 2 1.12 (0.98), 4 / 2 1.24, 5 / 3 1.14, 7 / 4 1.27; 4 / 3
+// 0.98 (0.89), 2 / 2 0.90, 2 / 1 1.01 (0.89); beyond 2 / 1 1.10 (1.00), 3 / 2 1.08, 4 / 2 1.26, 5 / 3 1.20. Up to 512 rows, whose few
+// tiles make t1 and t2 coarse, 0.8 to 1.2: sixteen. The sums are the same either way.
 template <class F, bool XH>
 int launch_mm(hipStream_t st, const RowsArgs& a) {
   constexpr int S = rows_slot<F>() <= 2048 ? 4 : 2;
-  if (a.nws <= 8) return launch_nt<F, 1, S, 16, 2, true, XH>(st, a, a.nws);
+  const uint32_t nt = (a.rows + 15) / 16, b1 = (a.n + 15) / 16, b2 = (a.n + 31) / 32;
+  auto tiles = [&](int UT, int TT) { return rows_tiles_per_wg(nt, a.nws, rows_lds<F>(a.nws, S, UT, TT), TT == 1 ? b1 : b2); };
+  if (a.nws <= 8) {
+    const uint32_t t1 = tiles(2, 1), t2 = tiles(2, 2);
+    if (a.rows > 512 && t1 >= 3 && 2 * t1 >= 3 * t2) return launch_nt<F, 1, S, 16, 2, true, XH, 2>(st, a, a.nws);
+    return launch_nt<F, 1, S, 16, 2, true, XH>(st, a, a.nws);
+  }
+  const uint32_t t1 = tiles(1, 1), t2 = tiles(1, 2);
+  if (a.rows > 512 && 5 * t1 >= 6 * t2 + 3) return launch_nt<F, 1, S, 16, 1, true, XH, 2>(st, a, a.nws);
   return launch_nt<F, 1, S, 16, 1, true, XH>(st, a, a.nws);
 }
 template <bool XH>
@@ -117,17 +138,40 @@ int launch_mm(hipStream_t st, int t, const RowsArgs& a) {
 //  * more than 4096 rows of five stages and more: up to 32 tokens (Q5_K 8192x1280 at 48 0.89, IQ1_S 8192x2048 at 48 0.93);
 //    never more than 8192 (IQ1_S 16384x1536 at 17 0.86);
 //  * two workgroups a token block at least, or a part of the device has none (IQ1_S 202x1536 at 2387, 150 blocks, 0.75).
+//
+// ... and in blocks of 32 tokens more work, up to 256 tokens (serves_32), `work` of it per wave of the device in units of 16 rows x
+// 256 columns x 32 tokens. Measured over 7000 random calls against the route that each took before, median (lowest of 100):
+//  * up to 64 tokens (not 33 to 39, whose second block is nearly empty) at 1280 to 4096 columns, work of at most five: IQ4_NL 1.59
+//    (1.24), IQ2_XXS 1.55 (1.24), Q6_K 1.40 (1.11), IQ1_S 1.41 (1.10) but for more than 16384 rows (32768x1280 at 32 0.95) and 40 to 47
+//    tokens (0.94 to 1.0), Q5_K 1.27 likewise (16427x1536 at 54 0.90, 10437x3840 at 42 0.96);
+//  * in two launches of half the columns, 6144 to 8192: from 5120 rows on for the codebook formats and IQ4_NL (1.1 to 1.9; 3500 rows
+//    0.87 to 1.2; IQ1_S from 40 tokens on and of fp32 activations, 0.9 with fp16), from 6144 rows on for the K-quants up to 32 tokens
+//    (1.05 to 1.5; 5120 rows 0.86, more tokens 0.7 to 1.2);
+//  * 65 to 128 tokens: IQ4_NL from 1536 columns on, work of at most seven (1.36, lowest 1.0; 20587x1536 at 102, 7.5, 0.94); Q6_K
+//    from 3584 on, Q5_K 4096, at most eight (1.33; Q5_K 4500x3584 at 114 0.91); the codebook formats have the tile kernel;
+//  * 129 to 256 tokens: 1152 to 2048 rows of 1536 columns and more, at most four (1.2 to 1.7).
+bool serves_32(int t, int rows, size_t nws, int n) {
+  const bool iq4 = t == MSQ_IQ4_NL, iq1 = t == MSQ_IQ1_S, q5 = t == MSQ_Q5_K, kq = q5 || t == MSQ_Q6_K;
+  const size_t work = ((size_t)rows + 15) / 16 * nws * (((size_t)n + 31) / 32), waves = 16 * (size_t)device_info().cus;
+  if (n <= 16 || nws > 32 || (n > 32 && n < 40)) return false;
+  if (nws > 16) return n <= 64 && nws >= 24 && work <= 5 * waves && (kq ? n <= 32 && rows >= 6144 : rows >= 5120 && !(iq1 && n <= 32));
+  if (n <= 32) return nws >= 5 && work <= 5 * waves && !(iq1 && rows > 16384);
+  if (n <= 64) return nws >= 5 && work <= 5 * waves && !((iq1 || q5) && (rows > 16384 || n < 48));
+  if (n <= 128) return iq4 ? nws >= 6 && work <= 7 * waves : kq && nws >= (q5 ? 16u : 14u) && work <= 8 * waves;
+  return n <= 256 && nws >= 6 && rows >= 1152 && rows <= 2048 && work <= 4 * waves;
+}
 bool matmul_rows_serves(int t, int rows, int cols, int n, const void* X, bool x_half, size_t x_stride) {
   switch (t) {
     case MSQ_Q6_K: case MSQ_Q5_K: case MSQ_IQ4_NL: case MSQ_IQ1_S: case MSQ_IQ2_XXS: break;
     default: return false;
   }
   const size_t nws = ((size_t)cols + 255) / 256, waves = 16 * (size_t)device_info().cus;
+  if (cols % 128 || ((uintptr_t)X & (x_half ? 7 : 15)) || x_stride % 4 || x_stride > 0xFFFFFFFFull) return false;
+  if (!(x_half && t == MSQ_IQ1_S && nws > 16) && serves_32(t, rows, nws, n)) return true;
   const size_t stages = ((size_t)rows + 15) / 16 * nws * (((size_t)n + 15) / 16);
-  if (n <= 16 || cols % 128 || nws < 2 || nws > 16 || rows > 8192 || 2 * (((size_t)n + 15) / 16) > (size_t)device_info().cus) return false;
+  if (n <= 16 || nws < 2 || nws > 16 || rows > 8192 || 2 * (((size_t)n + 15) / 16) > (size_t)device_info().cus) return false;
   if ((nws == 2 && rows > 4096) || (nws > 4 && rows > 4096 && n > 32)) return false;
-  if (stages > waves * (nws == 2 ? 2 : n <= 256 && rows <= 2048 ? 4 : 3)) return false;
-  return !((uintptr_t)X & (x_half ? 7 : 15)) && x_stride % 4 == 0 && x_stride <= 0xFFFFFFFFull;
+  return stages <= waves * (nws == 2 ? 2 : n <= 256 && rows <= 2048 ? 4 : 3);
 }
 int matmul_rows(hipStream_t st, int t, const uint8_t* W, int rows, int cols, const void* X, bool x_half, size_t x_stride, float* Y, int n,
                 int accumulate) {
@@ -136,7 +180,19 @@ int matmul_rows(hipStream_t st, int t, const uint8_t* W, int rows, int cols, con
   a.n = (uint32_t)n; a.rows = (uint32_t)rows; a.cols = (uint32_t)cols; a.x_stride = (uint32_t)x_stride;
   a.row_bytes = (uint32_t)msq_type_row_bytes(t, cols); a.accumulate = accumulate ? 1u : 0u;
   a.rows_per_group = (uint32_t)rows; a.x_group_stride = 0; a.nws = ((uint32_t)cols + 255) / 256;
-  return x_half ? launch_mm<true>(st, t, a) : launch_mm<false>(st, t, a);
+  // rows of more than sixteen weight stages in pieces of equal length, each a launch of its own that adds to the one before
+  const uint32_t pieces = (a.nws + 15) / 16, per = (a.nws + pieces - 1) / pieces, ws = (uint32_t)msq_type_row_bytes(t, 256);
+  for (uint32_t s0 = 0; s0 < a.nws; s0 += per) {
+    RowsArgs b = a;
+    b.W = a.W + (size_t)s0 * ws;
+    b.X = (const uint8_t*)X + (size_t)s0 * 256 * (x_half ? 2 : 4);
+    b.nws = std::min(per, a.nws - s0); b.cols = std::min(per * 256, a.cols - s0 * 256);
+    b.w_bytes = a.rows * a.row_bytes - s0 * ws;
+    if (s0) b.accumulate = 1u;
+    const int rc = x_half ? launch_mm<true>(st, t, b) : launch_mm<false>(st, t, b);
+    if (rc != MSQ_OK) return rc;
+  }
+  return MSQ_OK;
 }
 
 bool matvec_rows_serves(int t, int rows, int cols, int n, int groups, const void* X) {
@@ -154,6 +210,7 @@ int matvec_rows(hipStream_t st, int t, const uint8_t* W, int rows, int cols, con
   a.n = (uint32_t)n; a.rows = (uint32_t)rows; a.cols = (uint32_t)cols; a.x_stride = (uint32_t)cols * (uint32_t)groups;
   a.row_bytes = (uint32_t)msq_type_row_bytes(t, cols); a.accumulate = accumulate ? 1u : 0u;
   a.rows_per_group = (uint32_t)(rows / groups); a.x_group_stride = (uint32_t)cols; a.nws = ((uint32_t)cols + 255) / 256;
+  a.w_bytes = a.rows * a.row_bytes;
   switch (t) {
     case MSQ_Q6_K: return launch_f<FragQ6KG>(st, a);
     case MSQ_Q5_K: return launch_f<FragQ5K>(st, a);
