@@ -117,28 +117,33 @@ bool place_x_row(MvArgs& a, size_t& lds, int tokens = 1, size_t limit = 64 * 102
 // norm's weights wait behind the first weight rows: two trips are ahead where a row is short, one trip where it is long or
 // the matrix large. Measured with an input row of its own for every launch, as layers have (a row that stays in the caches
 // makes two trips look better by 5 to 10 %); in brackets two trips' time over one trip's.
-//  * F32 always (0.98 to 1.3), but for the crowded case below.
 //  * mv_tok_kernel, block formats: from 4608 columns on (Q5_K 4096x4096 0.96, x4608 1.04, IQ4_NL 1100x5120 1.09), and 40 MB and
 //    more of more than 2048 columns (Q6_K 16384x3072 1.04; IQ4_NL 32768x2048 0.98); Q8_0, whose activations stay fp32, from 3072
 //    (2048x2560 0.98, x3072 1.00, 4096x4096 1.03), from 16 MB of more than 2048 (8192x2304 1.05) and from 30 MB (16384x2048 1.04,
-//    8192x2048 0.98); fp16 types up to 1024 columns (2048x1024 1.06), beyond 2048 (1100x2560 1.06, 4096x2304 0.98, x3072 1.05) and
-//    from 32 MB (8192x2048 1.02, 1100x2048 0.96).
-//  * mv_kernel, block formats: from 2560 columns on (Q6_K 512x2304 0.96, x2560 0.98, Q5_K 768x2560 1.04), with more than one
-//    workgroup per CU, whose overlap the registers cut, beyond 4096 (IQ4_NL 1536x4096 0.97), Q8_0 there from 3072 (1.02 to 1.04); fp16
-//    types beyond 2048 (BF16 768x2048 0.96, 512x2304 1.08).
-//  * Dense rows over more than twelve waves and more than one workgroup per CU keep two: of 80 registers a CU holds 24 waves,
-//    so such workgroups would run one by one (F32 512x7168 0.87, 256x7168 1.17).
+//    8192x2048 0.98); F32 always (0.98 to 1.3); fp16 types up to 1024 columns (2048x1024 1.06), beyond 2048 (1100x2560 1.06, 4096x2304
+//    0.98, x3072 1.05) and from 32 MB (8192x2048 1.02, 1100x2048 0.96).
+//  * mv_kernel, sums from registers, lowest, median and highest of 8000 random matrices: block formats from 2304 columns on, Q8_0 from
+//    2560 (up to 4096 0.99, 1.05, 1.2, beyond 0.99, 1.3, 1.45; 2048 columns 0.92, 0.97, 1.0); dense types from 2304 on where they are
+//    alone on a CU (1.07, 1.24, 1.35), else, since the registers cut the overlap of workgroups, up to 4096 (0.99, 1.03, 1.18; beyond
+//    0.88, 1.00, 1.04).
+//  * mv_kernel, sums from LDS: dense types of more than 4096 columns with more than one workgroup per CU (two trips 0.79 to 0.92 of its
+//    speed at 4352 to 10240), but rows over more than twelve waves: of 80 registers a CU holds 24 waves, so these would run one by one
+//    (F32 512x7168 0.87); F32 of less than 3072 columns (sums from registers 0.96 to 1.03 of its speed at 2304, 0.93 to 1.05 at 1280).
 template <class D>
-bool norm_one_trip(bool tok, uint32_t cols, double bytes, int grid, int threads) {
-  const bool crowded = grid > device_info().cus;
+Norm norm_of_tok(uint32_t cols, double bytes) {
+  if constexpr (D::UNIT == 8) return std::is_same_v<D, DecDense<MSQ_F32>> || cols > 2048 || cols <= 1024 || bytes >= 32e6 ? kNormOneTrip : kNormTwoTrips;
+  else if constexpr (std::is_same_v<D, DecQ8_0>) return cols >= 3072 || bytes >= (cols > 2048 ? 16e6 : 30e6) ? kNormOneTrip : kNormTwoTrips;
+  else return cols >= 4608 || (cols > 2048 && bytes >= 40e6) ? kNormOneTrip : kNormTwoTrips;
+}
+template <class D>
+Norm norm_of_mv(uint32_t cols, int grid, int threads) {
   if constexpr (D::UNIT == 8) {
-    if (!tok && threads > 768 && crowded) return false;
-    return std::is_same_v<D, DecDense<MSQ_F32>> || cols > 2048 || (tok && (cols <= 1024 || bytes >= 32e6));
+    constexpr bool f32 = std::is_same_v<D, DecDense<MSQ_F32>>;
+    const bool crowded = grid > device_info().cus;
+    if (cols >= (f32 ? 3072 : 2304)) return !crowded || cols <= 4096 ? kNormOneTripRegs : threads <= 768 ? kNormOneTrip : kNormTwoTrips;
+    return f32 ? kNormOneTrip : kNormTwoTrips;
   } else {
-    constexpr bool q8 = std::is_same_v<D, DecQ8_0>;
-    if (!tok) return cols > 4096 || (crowded ? q8 && cols >= 3072 : cols >= 2560);
-    if (q8) return cols >= 3072 || bytes >= (cols > 2048 ? 16e6 : 30e6);
-    return cols >= 4608 || (cols > 2048 && bytes >= 40e6);
+    return cols >= (std::is_same_v<D, DecQ8_0> ? 2560u : 2304u) ? kNormOneTripRegs : kNormTwoTrips;
   }
 }
 
@@ -159,11 +164,16 @@ int launch_mv(hipStream_t st, const MvShape& s, MvArgs& a) {
     if constexpr (requires { D::STAGES; }) return MSQ_ERR_UNSUPPORTED;  // codebook formats: as in the reference (quant.mm:110)
     else {
       auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, st, a); };
-      const bool one = norm_one_trip<D>(false, a.cols, (double)a.rows * a.row_bytes, grid, threads);
+      const Norm norm = norm_of_mv<D>(a.cols, grid, threads);
+      auto by_norm = [&]<int ITERS>() {
+        if (norm == kNormTwoTrips) return launch(mv_kernel<D, ITERS, kNormTwoTrips>);
+        if constexpr (D::UNIT == 8) { if (norm == kNormOneTrip) return launch(mv_kernel<D, ITERS, kNormOneTrip>); }
+        launch(mv_kernel<D, ITERS, kNormOneTripRegs>);
+      };
       switch (s.iters) {
-        case 1: one ? launch(mv_kernel<D, 1, kNormOneTrip>) : launch(mv_kernel<D, 1, kNormTwoTrips>); break;
-        case 2: one ? launch(mv_kernel<D, 2, kNormOneTrip>) : launch(mv_kernel<D, 2, kNormTwoTrips>); break;
-        default: one ? launch(mv_kernel<D, 4, kNormOneTrip>) : launch(mv_kernel<D, 4, kNormTwoTrips>); break;
+        case 1: by_norm.template operator()<1>(); break;
+        case 2: by_norm.template operator()<2>(); break;
+        default: by_norm.template operator()<4>(); break;
       }
       MSQ_HIP(hipGetLastError());
       return MSQ_OK;
@@ -315,7 +325,7 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   // persistent workgroups, one per CU over all token groups (two for a large matrix: MvShape::per_cu)
   // A fused norm's prologue of one trip leaves Q5_K, Q6_K rows in registers (144) and two units of F32 no room for a second one:
   // they would run one by one (Q5_K 16384x7168 0.89 of the speed, F32 768x5120 0.79; IQ4_NL, Q8_0 and the fp16 types gain 3 to 25 %).
-  const bool one_trip = a.norm_w && norm_one_trip<D>(true, a.cols, bytes, device_info().cus, threads);
+  const bool one_trip = a.norm_w && norm_of_tok<D>(a.cols, bytes) == kNormOneTrip;
   constexpr bool wide = std::is_same_v<D, DecQ5KQ> || std::is_same_v<D, DecQ6KQ>;
   const bool alone = one_trip && ((wide && !sw) || (std::is_same_v<D, DecDense<MSQ_F32>> && s.iters > 1));
   const int per_cu = (T == 1 && !alone && (lds + kStaticLds<D>) * s.per_cu <= (size_t)kMaxLds) ? s.per_cu : 1;

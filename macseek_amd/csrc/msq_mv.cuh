@@ -142,8 +142,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* x, const floa
 
 // Prologues of the NORM matvec kernels: the normalized activations of the (single) input row go to LDS as fp32 (padded
 // layout of XLds), from where load_x() converts them exactly as it would from device memory. Both are chains of latencies
-// and add in the same order; the launch chooses (norm_one_trip in msq_matvec.hip, where both sides stand).
-enum Norm { kNormNone, kNormTwoTrips, kNormOneTrip };
+// and add in the same order; the launch chooses (norm_of_tok, norm_of_mv in msq_matvec.hip, where both sides stand).
+enum Norm { kNormNone, kNormTwoTrips, kNormOneTrip, kNormOneTripRegs };
 
 // Two trips: four waves fetch the row in pieces of 2048 elements and add, then all waves fetch it again with the weights.
 // Few registers and little code: ahead for short rows, whose second trip hits the caches.
@@ -174,18 +174,35 @@ __device__ __forceinline__ void stage_normed_x_two_trips(const MvArgs& a, uint32
   __syncthreads();
 }
 
-// One trip: all threads request the row and the norm's weights (kept in registers up to 16 elements a thread) and the
-// kernel's first weight rows with them (`with()`, called between the two); the reduction then reads the row from LDS in its
-// own order. Rows are 4-byte aligned. Against two trips: Q5_K 512x7168 6.6 -> 5.7 us, IQ4_NL 512x5120 5.7 -> 4.8.
-template <class With>
+// One trip: all threads request the row and the norm's weights in pieces of four elements (kept in registers up to 16 a
+// thread) and the kernel's first weight rows with them (`with()`, called between the two). Rows are 4-byte aligned. The sums:
+//  * from the row in LDS, in their own order;
+//  * REGS: the four waves that add request the elements of their virtual lanes as well, ahead of everything, up to 32 a lane:
+//    one barrier and one pass through LDS less (Q5_K 512x7168 two trips 6.6, one 5.4, this 4.8 us; 5.0 with a bound checked in code for every element). mv_tok_kernel does without: the
+//    registers would cost a large matrix its second workgroup a CU (output head 99 -> 120 us), and one of a workgroup a CU gains nothing.
+template <bool REGS, class With>
 __device__ __forceinline__ void stage_normed_x_one_trip(const MvArgs& a, uint32_t* smem, float* xs, uint32_t tid, uint32_t lane,
                                                         uint32_t wave, uint32_t nwaves, With with) {
   typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
   constexpr int K = 4;
+  constexpr uint32_t S = 32;
   float* red = (float*)(smem + a.norm_off);
   const uint32_t nt = nwaves * 64u, n4 = a.cols >> 2;  // (cols is a multiple of 32)
   const f4u *xg = (const f4u*)a.x, *wg = (const f4u*)a.norm_w;
   auto at = [&](uint32_t i4) { return (f4_t*)(xs + 4u * i4 + (i4 >> 3) * 4u); };
+  // (the sums' elements come through a descriptor over the row: past its end zeros, which change no sum, and no code to tell;
+  // a launch of a few microseconds waits for its instructions as well)
+  [[maybe_unused]] const rsrc_t xrs = make_rsrc(a.x, a.cols * 4u);
+  [[maybe_unused]] float t[S];
+  auto batch = [&](uint32_t k0, float (&e)[8]) {
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; k++) e[k] = __builtin_bit_cast(float, buf_ld32(xrs, 4u * tid, 1024u * (k0 + k)));
+  };
+  if (REGS && wave < 4u) {
+#pragma unroll
+    for (uint32_t k0 = 0; k0 < S; k0 += 8u)
+      if (256u * k0 < a.cols) batch(k0, *(float(*)[8])(t + k0));
+  }
   f4_t xv[K], wv[K];
 #pragma unroll
   for (int k = 0; k < K; k++) xv[k] = xg[min(tid + k * nt, n4 - 1u)];
@@ -194,23 +211,47 @@ __device__ __forceinline__ void stage_normed_x_one_trip(const MvArgs& a, uint32_
 #pragma unroll
   for (int k = 0; k < K; k++) wv[k] = wg[min(tid + k * nt, n4 - 1u)];
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (REGS) {
+    if (wave < 4u) {
+      float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < K; k++)
-    if (tid + k * nt < n4) *at(tid + k * nt) = xv[k];
-  for (uint32_t i = tid + K * nt; i < n4; i += nt) *at(i) = xg[i];
-  __syncthreads();
-  for (uint32_t v = wave; v < 4u; v += nwaves) {
-    float ss = 0.f;
-    for (uint32_t i0 = v * 64u + lane; i0 < a.cols; i0 += 8u * 256u) {
-      float t[8];
+      for (uint32_t k0 = 0; k0 < S; k0 += 8u)
+        if (256u * k0 < a.cols) {
 #pragma unroll
-      for (int k = 0; k < 8; k++) { const uint32_t i = min(i0 + 256u * k, a.cols - 1u); t[k] = xs[i + (i >> 5) * 4u]; }
+          for (uint32_t k = k0; k < k0 + 8u; k++) ss = __builtin_fmaf(t[k], t[k], ss);
+        }
+      for (uint32_t k0 = S; 256u * k0 < a.cols; k0 += 8u) {  // the rest of a longer row
+        float e[8];
+        batch(k0, e);
 #pragma unroll
-      for (int k = 0; k < 8; k++)
-        if (i0 + 256u * k < a.cols) ss = __builtin_fmaf(t[k], t[k], ss);
+        for (uint32_t k = 0; k < 8u; k++) ss = __builtin_fmaf(e[k], e[k], ss);
+      }
+      ss = wave_sum(ss);
+      if (lane == 0) red[wave] = ss;
     }
-    ss = wave_sum(ss);
-    if (lane == 0) red[v] = ss;
+    for (uint32_t v = wave + nwaves; v < 4u; v += nwaves) {  // (workgroups of fewer waves)
+      const float ss = rms_virtual_wave(a.x, a.cols, v, lane);
+      if (lane == 0) red[v] = ss;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < K; k++)
+      if (tid + k * nt < n4) *at(tid + k * nt) = xv[k];
+    for (uint32_t i = tid + K * nt; i < n4; i += nt) *at(i) = xg[i];
+    __syncthreads();
+    for (uint32_t v = wave; v < 4u; v += nwaves) {
+      float ss = 0.f;
+      for (uint32_t i0 = v * 64u + lane; i0 < a.cols; i0 += 8u * 256u) {
+        float e[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) { const uint32_t i = min(i0 + 256u * k, a.cols - 1u); e[k] = xs[i + (i >> 5) * 4u]; }
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+          if (i0 + 256u * k < a.cols) ss = __builtin_fmaf(e[k], e[k], ss);
+      }
+      ss = wave_sum(ss);
+      if (lane == 0) red[v] = ss;
+    }
   }
   __syncthreads();
   const float r = rms_of_sums(red, a.cols, a.eps);
@@ -221,7 +262,7 @@ __device__ __forceinline__ void stage_normed_x_one_trip(const MvArgs& a, uint32_
 #pragma unroll
   for (int k = 0; k < K; k++)
     if (tid + k * nt < n4) *at(tid + k * nt) = normed(xv[k], wv[k]);
-  for (uint32_t i = tid + K * nt; i < n4; i += nt) *at(i) = normed(*at(i), wg[i]);
+  for (uint32_t i = tid + K * nt; i < n4; i += nt) *at(i) = normed(REGS ? (f4_t)xg[i] : *at(i), wg[i]);
   __syncthreads();
 }
 
@@ -250,11 +291,11 @@ __global__ __launch_bounds__(1024) void mv_kernel(const MvArgs a) {
   typename D::X xr[ITERS];
   uint32_t cur_group = 0xFFFFFFFFu;
   float* xs = (float*)(smem + a.xs_off);
-  constexpr bool FIRST = NORM == kNormOneTrip && ITERS == 1;  // the wave's first row is requested with the activations
+  constexpr bool ONE = NORM == kNormOneTrip || NORM == kNormOneTripRegs, FIRST = ONE && ITERS == 1;  // the wave's first row is requested with the activations
   [[maybe_unused]] typename D::Raw raw0;
-  if constexpr (NORM == kNormOneTrip) {
+  if constexpr (ONE) {
     const uint8_t* wr = a.W + (size_t)min(blockIdx.x * tile_rows + rw * a.rpw, a.rows - 1) * a.row_bytes;
-    stage_normed_x_one_trip(a, smem, xs, tid, lane, wave, nwaves, [&] {  // synchronises (one group only)
+    stage_normed_x_one_trip<NORM == kNormOneTripRegs>(a, smem, xs, tid, lane, wave, nwaves, [&] {  // synchronises (one group only)
       if constexpr (FIRST) raw0 = D::load(wr, unit[0]);
     });
   } else if constexpr (NORM == kNormTwoTrips) {
@@ -621,7 +662,7 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
         else fetch(ring[s], s);
       }
     };
-    if (NORM == kNormOneTrip && cur_group == 0xFFFFFFFFu) stage_normed_x_one_trip(a, smem, xs, tid, lane, wave, nwaves, ahead);  // synchronises (one token, one group)
+    if (NORM == kNormOneTrip && cur_group == 0xFFFFFFFFu) stage_normed_x_one_trip<false>(a, smem, xs, tid, lane, wave, nwaves, ahead);  // synchronises (one token, one group)
     else ahead();
     if (group != cur_group) {
       // tokens past the last repeat it; their results are never stored
