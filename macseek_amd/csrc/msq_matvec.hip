@@ -264,38 +264,55 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   MvTokArgs ta = ta_;  // (the launch may reshape rows into pairs: the caller's arguments stay as they are)
   MvArgs& a = ta.m;
   MvShape s = s_;
-  // One token, rows whose units fill a whole number of waves and at most half of another (5120 or 7168 columns of a
-  // block format: 2.5 and 3.5 waves): two rows are launched as one of twice the units, which leaves no lane idle
-  // (mv_tok_kernel, PAIR). One group, an even number of rows, a row's units a multiple of 16. Measured, rows one by
-  // one / in pairs: Q6_K 129280x5120 113.2 / 99.8 us, 1536x7168 6.41 / 6.10, 2304x5120 6.61 / 6.29, Q8_0 2304x5120
-  // 6.67 / 6.52; the codebook formats, bound by their lookups, lose 1 % and keep the one-row form. MSQ_MV_PAIR = 0 / 2:
-  // never / every format.
+  // Rows whose units do not fill whole waves: two, four or eight rows are launched as one (mv_tok_kernel, PACK), as few as leave
+  // the fewest waves per row. One group, a number of rows that divides, a row's units a multiple of 8 (several tokens: two rows, 16).
+  // Measured, rows one by one (512 and 5120 columns, and all of 7168: in pairs at most) / packed: Q6_K 32768 rows of 256 columns 2.0 times
+  // the speed, 512 7.57 / 6.05 us, 768 10.84 / 7.39, 1280 11.64 / 10.57, 1536 12.13 / 10.87, 129280x5120 113.2 / 99.8, 1536x7168 6.41 / 6.10;
+  // Q8_0 32768x512 7.01 / 5.93, 2304x5120 6.67 / 6.52; over 8000 random matrices of the K-quants, Q8_0, BF16 and F32 0.97 to 2.1. More than two
+  // rows for an eighth fewer waves or less gain nothing (3328 columns 0.96 to 1.06), nor do five waves a workgroup where there are
+  // not four packed rows for each (2304x2304 0.95), nor rows of 2304 columns below 6 MB (0.94 to 0.97); the codebook formats, bound by their lookups, lose 1 % and keep the one-row
+  // form. MSQ_MV_PAIR = 0 / 2: never / every format.
   // Under a fused norm likewise, but for Q8_0 below 20 MB (2560, 4608, 5120 and 7168 columns, one by one over in pairs: 6 to 18 MB
-  // 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04).
+  // 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04). (Sums of 16 lanes are added in one order whether rows are packed or not; with
+  // sums of 8, which are not, the norm's calls and the plain ones have to agree, so Q8_0 has these from 20 MB on.)
   const double bytes = (double)a.rows * a.row_bytes;
-  bool pair = false;
+  int pack = 1;
   {
     static const int env_pair = env_knob_early("MSQ_MV_PAIR", -1);
-    const int u = (int)(a.cols / D::UNIT), k1 = (u + 63) / 64, k2 = (2 * u + 63) / 64;
-    pair = s.iters == 1 && s.free_shape && (D::LDS_WORDS == 0 || env_pair == 2) && !(a.norm_w && std::is_same_v<D, DecQ8_0> && bytes < 20e6) && env_pair != 0 && a.rows % 2 == 0 && a.rows_per_group >= a.rows && u % 16 == 0 &&
-           k2 < 2 * k1 && k2 <= 8;
-    if (pair) {
-      a.rows /= 2;
+    const int u = (int)(a.cols / D::UNIT), cus = device_info().cus;
+    constexpr bool q8 = std::is_same_v<D, DecQ8_0>;
+    auto waves = [&](int p) { return (p * u + 63) / 64; };
+    if (s.iters == 1 && s.free_shape && (D::LDS_WORDS == 0 || env_pair == 2) && env_pair != 0 && a.rows_per_group >= a.rows &&
+        !(a.norm_w && q8 && bytes < 20e6) && u % (T == 1 && D::LDS_WORDS == 0 ? 8 : 16) == 0)
+      for (int p = 2; p <= (T == 1 ? 8 : 2); p *= 2)
+        if (a.rows % p == 0 && waves(p) <= 8 && (u % 16 == 0 || bytes >= (q8 ? 20e6 : u < 64 ? 0. : 6e6)) && waves(p) * pack < waves(pack) * p &&
+            (p == 2 || (8 * waves(p) < 7 * p * waves(1) && (waves(p) != 5 || (long)a.rows >= 4L * p * cus))))
+          pack = p;
+    // Five waves a workgroup leave the SIMDs unequal work: K-quants take two of them per CU from 16 MB on (2560 and 5120 columns, one / two:
+    // 12 MB 0.95 to 1.03, 16 MB 1.02 to 1.06, 26 MB 1.10 to 1.17, 44 MB 1.17 to 1.24), under a norm of two trips from 26 MB on (1.03 to
+    // 1.12; Q6_K 20 MB 0.93); Q8_0 does not (0.69 to 0.92 up to 34 MB).
+    constexpr bool kq = std::is_same_v<D, DecQ6KQ> || std::is_same_v<D, DecQ5KQ>;
+    if (kq && pack > 1 && waves(pack) == 5 && bytes >= (a.norm_w ? 26e6 : 16e6) && !(a.norm_w && norm_of_tok<D>(a.cols, bytes) == kNormOneTrip)) s.per_cu = 2;
+    if (pack > 1) {
+      a.pack = pack;
+      a.pack_units = u;
+      a.rows /= pack;
       a.rows_per_group = a.rows;
-      a.row_bytes *= 2;
-      s.ks = k2;
-      s.rw = std::max(1, 8 / k2);
+      a.row_bytes *= pack;
+      s.ks = (pack * u + 63) / 64;
+      s.rw = std::max(1, 8 / s.ks);
       const long wgs = std::max<long>(1, s.per_cu * device_info().cus / (((long)ta.n + T - 1) / T));
       s.rpw = (int)std::min<long>(32, std::max<long>(1, (a.rows + wgs * s.rw - 1) / (wgs * s.rw)));
     }
   }
+  const bool sums8 = pack > 1 && a.pack_units % 16;
   const int threads = 64 * s.rw * s.ks;
   const int tile_rows = s.rw * s.rpw;
-  a.units = (pair ? 2 : 1) * (a.cols / D::UNIT);
+  a.units = pack * (a.cols / D::UNIT);
   a.ks = s.ks;
   a.rpw = s.rpw;
   a.ntiles = (a.rows + tile_rows - 1) / tile_rows;
-  size_t lds = (size_t)tile_rows * s.ks * 4 * T * 4;  // dynamic LDS: partial sums, staged activations (the table is static)
+  size_t lds = (size_t)tile_rows * s.ks * (sums8 ? 8 : 4) * T * 4;  // dynamic LDS: partial sums, staged activations (the table is static)
   const int gy = ((int)ta.n + T - 1) / T;
   if (tok_stages_x<D, T>() || a.norm_w) {
     // one workgroup per CU: all of its LDS (decoders that stage only in the four-token kernel read directly when a round does not fit)
@@ -334,27 +351,31 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   if (a.norm_w) {  // fused input norm (single token)
     if constexpr (T != 1 || requires { D::STAGES; }) return MSQ_ERR_UNSUPPORTED;
     else {
-      auto by_norm = [&]<int ITERS, bool SW, bool PAIR>() {
-        one_trip ? launch(mv_tok_kernel<D, ITERS, 1, kNormOneTrip, SW, PAIR>, grid) : launch(mv_tok_kernel<D, ITERS, 1, kNormTwoTrips, SW, PAIR>, grid);
+      auto by_norm = [&]<int ITERS, bool SW, int PACK>() {
+        one_trip ? launch(mv_tok_kernel<D, ITERS, 1, kNormOneTrip, SW, PACK>, grid) : launch(mv_tok_kernel<D, ITERS, 1, kNormTwoTrips, SW, PACK>, grid);
+      };
+      auto by_pack = [&]<int ITERS, bool SW>() {
+        pack == 1 ? by_norm.template operator()<ITERS, SW, 0>() : sums8 ? by_norm.template operator()<ITERS, SW, 8>() : by_norm.template operator()<ITERS, SW, 16>();
       };
       if (sw) {
-        if constexpr (tok_stages_w<D, 1, 1>()) pair ? by_norm.template operator()<1, true, true>() : by_norm.template operator()<1, true, false>();
+        if constexpr (tok_stages_w<D, 1, 1>()) by_pack.template operator()<1, true>();
       } else if (s.iters == 1) {
-        pair ? by_norm.template operator()<1, false, true>() : by_norm.template operator()<1, false, false>();
-      } else if constexpr (D::UNIT == 8) by_norm.template operator()<2, false, false>();
+        by_pack.template operator()<1, false>();
+      } else if constexpr (D::UNIT == 8) by_norm.template operator()<2, false, 0>();
       else return MSQ_ERR_UNSUPPORTED;
       MSQ_HIP(hipGetLastError());
       return MSQ_OK;
     }
   }
+  auto by_pack = [&]<bool SW>() {
+    if (pack == 1) return launch(mv_tok_kernel<D, 1, T, kNormNone, SW>, grid);
+    if constexpr (T == 1 && D::LDS_WORDS == 0) { if (sums8) return launch(mv_tok_kernel<D, 1, T, kNormNone, SW, 8>, grid); }
+    launch(mv_tok_kernel<D, 1, T, kNormNone, SW, 16>, grid);
+  };
   if (sw) {
-    if constexpr (tok_stages_w<D, 1, T>()) {
-      if (pair) launch(mv_tok_kernel<D, 1, T, kNormNone, true, true>, grid);
-      else launch(mv_tok_kernel<D, 1, T, kNormNone, true>, grid);
-    }
+    if constexpr (tok_stages_w<D, 1, T>()) by_pack.template operator()<true>();
   } else if (s.iters == 1) {
-    if (pair) launch(mv_tok_kernel<D, 1, T, kNormNone, false, true>, grid);
-    else launch(mv_tok_kernel<D, 1, T>, grid);
+    by_pack.template operator()<false>();
   } else if constexpr (D::UNIT == 8) launch(mv_tok_kernel<D, 2, T>, grid);
   else return MSQ_ERR_UNSUPPORTED;  // two block-format units per lane and T activation slices do not fit the registers
   MSQ_HIP(hipGetLastError());

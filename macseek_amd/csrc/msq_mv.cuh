@@ -32,6 +32,7 @@ struct MvArgs {
   // (xlds_words(cols) words), and whether the plain kernels stage at all (rows too long for LDS are read directly)
   uint32_t xs_off;
   uint32_t stage_x;
+  uint32_t pack, pack_units;  // token kernel, PACK: rows of the matrix in a launched row, units of each
   uint32_t w_off;     // word offset in dynamic LDS of the waves' weight-row buffers (token kernel, one token of a block format)
 };
 
@@ -524,12 +525,12 @@ __device__ __forceinline__ void wait_rows_n(int n) {
 
 // Decoders with STAGE_X take the activations through LDS (contiguous loads, tok_round() tokens per round); with the
 // others every lane reads its slices from device memory, all T tokens' loads in flight at once.
-// PAIR (with SW): the launch treats two consecutive rows as one row of twice the units -- rows are contiguous in memory,
-// so a wave's slice of 64 units may run from the end of one row into the next -- which leaves no lane idle when a row's
-// units fill a whole number of waves and a half (5120 columns: five waves per row pair instead of twice three). rows_,
-// row_bytes_, units_, ks_ and the tile shape then describe the pairs; the two rows' 16-lane sums are told apart when
-// the partial sums are added (a row's units must be a multiple of 16 for that).
-template <class D, int ITERS, int T, int NORM = kNormNone, bool SW = false, bool PAIR = false>
+// PACK: the launch treats two, four or eight consecutive rows as one row of as many times the units -- rows are contiguous in
+// memory, so a wave's slice of 64 units may run from the end of one row into the next -- which leaves no or fewer lanes idle when a
+// row's units do not fill whole waves (5120 columns: five waves per two rows instead of twice three; 1280: five per eight rows
+// instead of eight). rows_, row_bytes_, units_, ks_ and the tile shape then describe the packed rows; the rows' sums of PACK lanes, 16
+// or 8 (a row's units must be a multiple of that), are told apart when the partial sums are added.
+template <class D, int ITERS, int T, int NORM = kNormNone, bool SW = false, int PACK = 0>
 __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t rows_, uint32_t row_bytes_, uint32_t units_, uint32_t ks_,
                                                      uint32_t rpw_, uint32_t ntiles_, uint32_t rows_per_group_, const float* x_,
                                                      uint32_t cols_, const MvTokArgs ta) {
@@ -544,7 +545,8 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
   // the codebook table is a static array: its LDS address is a compile-time constant, which saves the addition of a base
   // in every lookup address; partial sums (and staged activations) follow in dynamic LDS
   __shared__ __attribute__((aligned(16))) uint32_t tbl[D::LDS_WORDS > 0 ? D::LDS_WORDS : 4];
-  float* part = (float*)smem;  // [row of tile][ks][16-lane row of the wave][T]
+  constexpr uint32_t SUMS = PACK == 8 ? 8 : 4;  // of a wave: 8 or 16 lanes each
+  float* part = (float*)smem;  // [row of tile][ks][SUMS][T]
 
   const uint32_t tid = threadIdx.x, lane = tid & 63u, nwaves = blockDim.x >> 6;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -578,9 +580,9 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
     valid[i] = u < units_;
     unit[i] = valid[i] ? u : units_ - 1;  // idle lanes shadow the last unit; their result is dropped
   }
-  uint32_t xu[ITERS];  // the unit of the activations that goes with unit[i] (second row of a pair: the same columns again)
+  uint32_t xu[ITERS];  // the unit of the activations that goes with unit[i] (every row of a packed one: the same columns again)
 #pragma unroll
-  for (int i = 0; i < ITERS; i++) xu[i] = PAIR && unit[i] >= (units_ >> 1) ? unit[i] - (units_ >> 1) : unit[i];
+  for (int i = 0; i < ITERS; i++) xu[i] = PACK ? unit[i] - a.pack_units * small_div(unit[i], a.pack_units) : unit[i];
   typename D::X xr[T][ITERS];
   uint32_t cur_group = 0xFFFFFFFFu;
   float* xs = (float*)(smem + a.xs_off);
@@ -759,21 +761,22 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
             if constexpr (REFILL) fetch(ring[s], j0 + s + NR);
           }
         }
-        row16_fold<RF * T>(acc, lane);
+        if constexpr (PACK == 8) group8_fold<RF * T>(acc, lane);
+        else row16_fold<RF * T>(acc, lane);
         const uint32_t k = group8_sel<RF * T>(lane), j = j0 + f + k / T;
-        if (!(lane & 8u) && j < rpw_) part[(((rw * rpw_ + j) * KS + ks) * 4 + (lane >> 4)) * T + k % T] = acc[0];
+        if ((PACK == 8 || !(lane & 8u)) && j < rpw_) part[(((rw * rpw_ + j) * KS + ks) * SUMS + lane / (64 / SUMS)) * T + k % T] = acc[0];
       }
     };
     uint32_t j0 = 0;
     for (; j0 + NR < rpw_; j0 += NR) round.template operator()<true>(j0);
     round.template operator()<false>(j0);
     __syncthreads();
-    if constexpr (PAIR) {  // pair r / 2, its first or second units / 32 sixteen-lane sums
-      const uint32_t G = units_ >> 5;
-      for (uint32_t idx = tid; idx < 2u * tile_rows * T; idx += blockDim.x) {
-        const uint32_t r = idx % (2u * tile_rows), t = idx / (2u * tile_rows), row = 2u * tile_row0 + r;
-        if (row < 2u * rows_ && t0 + t < ta.n) {
-          const float s = sum_in_order(part + ((r >> 1) * 4 * KS + (r & 1u) * G) * T + t, G, T);
+    if constexpr (PACK) {  // packed row r / pack, its sums pack_units / PACK of each row
+      const uint32_t G = a.pack_units / PACK, sh = (uint32_t)__builtin_ctz(a.pack), n = tile_rows << sh;
+      for (uint32_t idx = tid; idx < n * T; idx += blockDim.x) {
+        const uint32_t r = T == 1 ? idx : idx % n, t = T == 1 ? 0u : idx / n, row = (tile_row0 << sh) + r;
+        if (row < rows_ << sh && t0 + t < ta.n) {
+          const float s = sum_in_order(part + ((r >> sh) * SUMS * KS + (r & (a.pack - 1u)) * G) * T + t, G, T);
           float* y = a.y + (size_t)(t0 + t) * ta.y_stride + row;
           *y = a.accumulate ? *y + s : s;
         }
