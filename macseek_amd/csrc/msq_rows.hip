@@ -39,12 +39,17 @@ template <class F, int BPW, int S, int UT>
 int launch(hipStream_t st, const RowsArgs& a, uint32_t waves) {
   return a.n <= 8 ? launch_nt<F, BPW, S, 8, UT>(st, a, waves) : launch_nt<F, BPW, S, 16, UT>(st, a, waves);
 }
-// one stage per wave up to 4096 columns (with LDS to spare up to 2048: two tiles per meeting), two stages up to 8192; rings
-// of two stages, four of the small codebook blocks
+// one stage per wave up to 4096 columns, two stages up to 8192; rings of two stages, four of the small codebook blocks. Up to 2048
+// columns, where there is LDS to spare, two tiles per meeting, but for workgroups of a single tile, which would carry an empty one
+// through it (against two, 4000 random calls: up to eight tokens 1.00 to 1.10, more 1.01 to 1.15; IQ4_NL up to eight tokens 0.95 to 1.02;
+// with two tiles and more 0.86 to 1.1), and of a single wave (1.01 to 1.28).
 template <class F>
 int launch_f(hipStream_t st, const RowsArgs& a) {
   constexpr int S = rows_slot<F>() <= 2048 ? 4 : 2;
-  if (a.nws <= 8) return launch<F, 1, S, 2>(st, a, a.nws);
+  if (a.nws <= 8) {
+    const bool one = rows_tiles_per_wg((a.rows + 15) / 16, a.nws, rows_lds<F>(a.nws, S, 2, 1), 1) == 1 && !(std::is_same_v<F, FragIQ4NL> && a.n <= 8);
+    return one || a.nws == 1 ? launch<F, 1, S, 1>(st, a, a.nws) : launch<F, 1, S, 2>(st, a, a.nws);
+  }
   if (a.nws <= 16) return launch<F, 1, S, 1>(st, a, a.nws);
   if (a.nws <= 32) return launch<F, 2, S, 1>(st, a, (a.nws + 1) / 2);
   return MSQ_ERR_UNSUPPORTED;
@@ -105,7 +110,7 @@ int launch_mm(hipStream_t st, const RowsArgs& a) {
   if (a.nws <= 8) {
     const uint32_t t1 = tiles(2, 1), t2 = tiles(2, 2);
     if (a.rows > 512 && t1 >= 3 && 2 * t1 >= 3 * t2) return launch_nt<F, 1, S, 16, 2, true, XH, 2>(st, a, a.nws);
-    return launch_nt<F, 1, S, 16, 2, true, XH>(st, a, a.nws);
+    return t1 == 1 ? launch_nt<F, 1, S, 16, 1, true, XH>(st, a, a.nws) : launch_nt<F, 1, S, 16, 2, true, XH>(st, a, a.nws);
   }
   const uint32_t t1 = tiles(1, 1), t2 = tiles(1, 2);
   if (a.rows > 512 && 5 * t1 >= 6 * t2 + 3) return launch_nt<F, 1, S, 16, 1, true, XH, 2>(st, a, a.nws);
