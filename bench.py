@@ -34,7 +34,7 @@ HBM_PEAK_GBPS = 8000.0
 DECODE_GATE_UP, DECODE_DOWN = "moe_gu_kernel<DecIQ1SQ, DecIQ2XXSQ>", "moe_down_kernel<DecIQ1S, DecIQ2XXS, 768>"
 PREFILL_GATE_UP = ("moe_pf_block_kernel<BlkIQ2XXS<4>, true, 7, true>", "moe_pf_block_kernel<BlkIQ2XXS<16>, true, 3, true>")
 PREFILL_DOWN = ("moe_pf_block_kernel<BlkIQ2XXS<4>, false, 7, true>", "moe_pf_block_kernel<BlkIQ2XXS<16>, false, 3, true>")
-MATVEC_N, ROUTER = "mm_rows_kernel<FragQ6KG, 2, 2, 8, 1, false, false, 1>", "router_fused_kernel<30, 4u>"
+MATVEC_N, ROUTER = "mm_rows_kernel<FragQ6KG, 2, 2, 8, 1, false, false, 1, false>", "router_fused_kernel<30, 4u>"
 MATMUL_CONVERT = ("f32_to_f16_kernel", "dequant_kq_kernel<14, unsigned short>")
 TRAFFIC = {"moe_hbm_traffic_fetch_write.txt": (DECODE_GATE_UP,), "moe_prefill_hbm_traffic_fetch_write.txt": PREFILL_GATE_UP}
 

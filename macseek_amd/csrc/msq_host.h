@@ -58,6 +58,9 @@ void prefill_side_stream_setup();  // msq_prefill.hip: creates the current devic
 int matvec_tok(hipStream_t st, int t, const uint8_t* W, int rows, int cols, const float* X, float* Y, int n, int accumulate,
                int groups, const MsqMvCfg* cfg = nullptr, const float* norm_w = nullptr, float eps = 0.f);
 
+// shared expert over few tokens (msq_rows.hip), where its waves fit a workgroup: gate and up with SwiGLU into H, or (up null) the down product into Z
+bool shared_rows_serves(int t, int dim, int inter);
+int shared_rows(hipStream_t st, int t, const uint8_t* W, const uint8_t* up, int rows, int cols, const uint16_t* X, uint16_t* H, float* Z, int n);
 // few-token product over block formats on the matrix cores (msq_rows.hip), for the calls that the rule gives it
 bool matvec_rows_serves(int t, int rows, int cols, int n, int groups, const void* X);
 int matvec_rows(hipStream_t st, int t, const uint8_t* W, int rows, int cols, const float* X, float* Y, int n, int accumulate, int groups);

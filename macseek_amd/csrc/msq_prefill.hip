@@ -304,7 +304,12 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
     b.queue = counters && (!forked || n >= kPfQueueTokens) ? counters + (GU ? 0 : 16) : nullptr;
     return launch_block<GU>(GU ? p->t_gate_up : p->t_down, gs, b, nc_routed[0], nc_routed[1], nc_routed[2], skip);
   };
-  // ... and one over all tokens with the shared expert's weights
+  // ... and one over all tokens with the shared expert's weights. A K-quant / Q8_0 expert over few tokens takes the few-token kernel, on the
+  // caller's stream: the tile kernel's 128 x 128 tiles are a chain of 150 us however few the tokens, and the fork to a second stream
+  // costs 14 us by itself. Time before / after, 384 IQ1_S experts (Q6_K and Q8_0 alike): 5120x2304 at 2 tokens 186 / 119, 16 307 / 280, 37
+  // 517 / 502, 64 650 / 606, 100 761 / 761, 150 (the tile kernel ahead) 992 / 978; 7168x2048 at 64 703 / 694, 100 918 / 889, 150 1171 / 1190;
+  // 2560x1024 at 100 252 / 229, 150 347 / 338.
+  const bool few = p->has_shared && n <= 112 && shared_rows_serves(p->t_shared, dim, inter);
   auto shared = [&](auto gu_tag, hipStream_t gs) -> int {
     constexpr bool GU = decltype(gu_tag)::value;
     const uint32_t K = (uint32_t)(GU ? dim : inter), N = (uint32_t)(GU ? inter : dim), rb = (uint32_t)(GU ? rb_sgu : rb_sd);
@@ -313,6 +318,9 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
       b.items = d_items + 3 * (size_t)ni_routed; b.nitems = ni_shared; b.queue = nullptr;
       return launch_block<GU>(p->t_shared, gs, b, nc_shared[0], nc_shared[1], nc_shared[2], skip);
     }
+    if (few)
+      return GU ? shared_rows(gs, p->t_shared, bptr(&p->shared.gate), bptr(&p->shared.up), inter, dim, Xt, H + (size_t)total * inter, nullptr, n)
+                : shared_rows(gs, p->t_shared, bptr(&p->shared.down), nullptr, dim, inter, H + (size_t)total * inter, nullptr, Z + (size_t)total * dim, n);
     PfTileArgs t{};
     t.A = (GU ? Xg : H) + (size_t)total * K;
     t.H = H + (size_t)total * inter; t.Z = Z + (size_t)total * dim;
@@ -325,7 +333,7 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   const bool routed_gu = any_routed && !(skip & 2), routed_dn = any_routed && !(skip & 8);
   const bool shared_gu = p->has_shared && !(skip & 4), shared_dn = p->has_shared && !(skip & 16);
   // The shared expert and the routed experts only meet in the reduction: two pipelines on two streams (see SideStream)
-  if (p->has_shared && any_routed) {
+  if (p->has_shared && any_routed && !few) {
     std::lock_guard<std::mutex> lock(g_side_mu);
     SideStream* s = side_stream(st);
     if (s && hipEventRecord(s->fork, st) == hipSuccess && hipStreamWaitEvent(s->stream, s->fork, 0) == hipSuccess) {

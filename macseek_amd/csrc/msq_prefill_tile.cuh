@@ -1,4 +1,4 @@
-// Prefill MoE, shared expert of a K-quant / Q8_0 type: dense gate/up and down products over all tokens of the call
+// Prefill MoE, shared expert of a K-quant / Q8_0 type (few tokens: msq_rows.cuh): dense gate/up and down products over all tokens of the call
 // (reference: the shared expert's part of ms::q::encode_moe_prefill, src/kernels/quant.mm:433-612).
 //
 // A workgroup of eight waves owns 128 weight rows x 128 tokens and walks K in stages of 64 columns, both operands in LDS

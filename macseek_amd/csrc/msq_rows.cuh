@@ -35,6 +35,8 @@ struct RowsArgs {
   uint32_t w_bytes;         // bytes from W to the matrix's end
   uint32_t tiles_per_wg;    // consecutive row tiles of a workgroup (of one group)
   uint32_t ntiles;
+  const uint8_t* W1;        // GU: the up matrix (W: gate), of the same shape
+  uint16_t* H;              // GU: output [n][rows]
 };
 
 constexpr int kRowsXPitch = 128 * 2 + 16;           // activations pass through LDS 128 columns at a time, fp16
@@ -44,7 +46,7 @@ template <class F> constexpr int rows_slot() { return 16 * rows_pieces<F>() * 16
 // slots requested ahead of the activations, which pass through the rest of the ring
 template <class F> constexpr int rows_early(int S) { return rows_slot<F>() < 2048 ? 1 : S - 1; }
 // words of the waves' partial tiles
-__host__ __device__ constexpr uint32_t rows_red_words(uint32_t waves, int UT, int TT) { return (TT == 1 ? 2u : TT) * waves * 256u * UT; }
+__host__ __device__ constexpr uint32_t rows_red_words(uint32_t waves, int UT, int TT, bool gu = false) { return (TT == 1 && !gu ? 2u : TT) * waves * 256u * UT; }
 template <class F> constexpr int rows_ring(int S) {
   const int x = rows_early<F>(S) * rows_slot<F>() + kRowsXBytes;
   return S * rows_slot<F>() > x ? S * rows_slot<F>() : x;
@@ -90,7 +92,9 @@ __device__ __forceinline__ f4_t fma4(float s, f4_t p, f4_t c) {
 // (about 37 vector instructions a fragment, which one matrix instruction uses), hence TT = 2: 8192x4096 at 64 tokens against
 // the routes of msq_matmul that slice K over workgroups: IQ4_NL 38.2 -> 22.0 us, Q6_K 30.8 -> 22.5, IQ2_XXS 38.1 -> 21.3; 1536x4096 of
 // IQ1_S at 200 32.1 -> 17.2. Three tiles' activations do not fit the registers of four waves a SIMD.
-template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false, int TT = 1>
+// GU (the prefill MoE layer's shared expert, few tokens): row tiles 2 k and 2 k + 1 are tile k of the gate and of the up matrix, which
+// meet together and leave silu(min(gate, 10)) * clamp(up, -10, 10) in fp16.
+template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false, int TT = 1, bool GU = false>
 __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   constexpr int P = rows_pieces<F>(), PIECES = 16 * P, NPI = (PIECES + 63) / 64, SLOT = rows_slot<F>();
   constexpr bool GROUPS = requires { F::GROUPS; };
@@ -101,17 +105,24 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
   const uint32_t n16 = lane & 15u, q = lane >> 4;
   uint32_t* tbl = smem;
   float* red = (float*)(smem + F::LDS_WORDS);                    // [2][wave][tile][token][16]
-  uint8_t* mine = (uint8_t*)(red + rows_red_words(nwaves, UT, TT)) + wave * (uint32_t)rows_ring<F>(S);
+  static_assert(!GU || (UT == 2 && TT == 1));
+  uint8_t* mine = (uint8_t*)(red + rows_red_words(nwaves, UT, TT, GU)) + wave * (uint32_t)rows_ring<F>(S);
 
-  const uint32_t m0 = ROUND ? blockIdx.y * (16u * TT) : 0u, ntok = ROUND ? min(a.n - m0, 16u * TT) : a.n;
+  constexpr bool BLOCKS = ROUND || XH;  // any number of tokens
+  const uint32_t m0 = BLOCKS ? blockIdx.y * (16u * TT) : 0u, ntok = BLOCKS ? min(a.n - m0, 16u * TT) : a.n;
   const uint32_t tile0 = blockIdx.x * a.tiles_per_wg, ntile = min(a.tiles_per_wg, a.ntiles - tile0);  // (grid: tile0 < ntiles)
   const uint32_t group = (tile0 * 16u) / a.rows_per_group;
   const uint32_t ws0 = wave * BPW;
 
-  const uintptr_t wa = (uintptr_t)a.W;
-  const uint32_t wmis = (uint32_t)wa & 15u;
-  const uint32_t wbytes = (wmis + a.w_bytes + 15u) & ~15u;  // whole aligned pieces: no piece straddles the end
-  const rsrc_t wrs = make_rsrc((const void*)(wa - wmis), wbytes);
+  struct Matrix { rsrc_t rs; uint32_t mis, bytes, end; };
+  auto matrix = [&](const uint8_t* w) {
+    const uintptr_t wa = (uintptr_t)w;
+    const uint32_t mis = (uint32_t)wa & 15u, bytes = (mis + a.w_bytes + 15u) & ~15u;  // whole aligned pieces: no piece straddles the end
+    return Matrix{make_rsrc((const void*)(wa - mis), bytes), mis, bytes, mis + a.w_bytes};
+  };
+  const Matrix w0 = matrix(a.W), w1 = GU ? matrix(a.W1) : w0;
+  auto of_tile = [&](uint32_t tile) -> const Matrix& { return GU && (tile & 1u) ? w1 : w0; };
+  auto row_tile = [&](uint32_t tile) { return GU ? tile >> 1 : tile; };
   // stage i of the wave's walk: tile i / BPW, weight stage ws0 + i % BPW
   uint32_t rowoff[NPI], pc[NPI];  // per piece: row inside the tile (in bytes), 16-byte piece of the row
 #pragma unroll
@@ -119,14 +130,14 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
     const uint32_t p = (uint32_t)k * 64u + lane;
     rowoff[k] = (p / P) * a.row_bytes; pc[k] = 16u * (p % P);
   }
-  const uint32_t end = wmis + a.w_bytes;
   auto request = [&](uint32_t tile, int b, uint32_t slot) {
-    const uint32_t at = wmis + (tile * 16u) * a.row_bytes + min(ws0 + b, a.nws - 1u) * (uint32_t)F::WS_BYTES;  // (a stage past the row's end: bytes nobody reads)
+    const Matrix& w = of_tile(tile);
+    const uint32_t at = w.mis + (row_tile(tile) * 16u) * a.row_bytes + min(ws0 + b, a.nws - 1u) * (uint32_t)F::WS_BYTES;  // (a stage past the row's end: bytes nobody reads)
 #pragma unroll
     for (int k = 0; k < NPI; k++) {
       const uint32_t v = at + rowoff[k];
       if (PIECES % 64 == 0 || k + 1 < NPI || (uint32_t)k * 64u + lane < (uint32_t)PIECES)
-        lds_dma16(wrs, mine + slot * SLOT + k * 1024, v < end ? (v & ~15u) + pc[k] : wbytes, 0u);  // rows past the end: no traffic
+        lds_dma16(w.rs, mine + slot * SLOT + k * 1024, v < w.end ? (v & ~15u) + pc[k] : w.bytes, 0u);  // rows past the end: no traffic
     }
   };
 
@@ -205,7 +216,7 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
 #pragma unroll
       for (int t = 0; t < TT; t++) acc[u][t] = zero;
       if (tl + u >= ntile) continue;
-      const uint32_t row = min((tile0 + tl + u) * 16u + n16, a.rows - 1u);
+      const uint32_t row = min(row_tile(tile0 + tl + u) * 16u + n16, a.rows - 1u), wmis = of_tile(tile0 + tl + u).mis;
 #pragma unroll
       for (int b = 0; b < BPW; b++, i++) {
         if (i + S <= total) wait_vm<NPI*(S - 1)>();  // S - 1 younger stages may stay in flight
@@ -243,10 +254,10 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
         slot = slot + 1 == S ? 0u : slot + 1;
       }
     }
-    // [wave][row tile][token tile][token][row]; two buffers, so that one barrier separates the meetings, or (TT > 1: LDS) one
+    // [wave][row tile][token tile][token][row]; two buffers, so that one barrier separates the meetings, or (TT > 1, GU: LDS) one
     // that everyone has read when the next partial tiles come
-    float* rb = red + (TT == 1 ? (tl / UT) & 1u : 0u) * (nwaves * (256u * UT));
-    if (TT > 1 && tl > 0) __syncthreads();
+    float* rb = red + (TT == 1 && !GU ? (tl / UT) & 1u : 0u) * (nwaves * (256u * UT));
+    if ((TT > 1 || GU) && tl > 0) __syncthreads();
 #pragma unroll
     for (int u = 0; u < UT; u++)
 #pragma unroll
@@ -254,17 +265,29 @@ __global__ __launch_bounds__(1024) void mm_rows_kernel(const RowsArgs a) {
 #pragma unroll
         for (int k = 0; k < 4; k++) rb[(((wave * UT + u) * TT + t) * 16u + 4u * q + k) * 16u + n16] = acc[u][t][k];
     __syncthreads();  // (everyone read this buffer's last contents before the barrier between)
-    for (uint32_t idx = tid; idx < 16u * UT * ntok; idx += nthreads) {
-      const uint32_t t = idx / (16u * UT), r = idx % (16u * UT), u = r >> 4, orow = (tile0 + tl) * 16u + r;
-      if (tl + u >= ntile || orow >= a.rows) continue;
+    auto sum = [&](uint32_t t, uint32_t u, uint32_t r) {
       float s = 0.f;
       for (uint32_t w0 = 0; w0 < nwaves; w0 += 8u) {  // eight partials requested before the first is added
         float v[8];
 #pragma unroll
-        for (uint32_t k = 0; k < 8u; k++) v[k] = rb[((min(w0 + k, nwaves - 1u) * UT + u) * (16u * TT) + t) * 16u + (r & 15u)];
+        for (uint32_t k = 0; k < 8u; k++) v[k] = rb[((min(w0 + k, nwaves - 1u) * UT + u) * (16u * TT) + t) * 16u + r];
 #pragma unroll
         for (uint32_t k = 0; k < 8u; k++) s += w0 + k < nwaves ? v[k] : 0.f;
       }
+      return s;
+    };
+    if constexpr (GU) {
+      for (uint32_t idx = tid; idx < 16u * ntok; idx += nthreads) {
+        const uint32_t t = idx >> 4, orow = row_tile(tile0 + tl) * 16u + (idx & 15u);
+        if (orow >= a.rows) continue;
+        const float g = fminf(sum(t, 0u, idx & 15u), 10.f), u = fminf(fmaxf(sum(t, 1u, idx & 15u), -10.f), 10.f);
+        a.H[(size_t)(m0 + t) * a.rows + orow] = __builtin_bit_cast(uint16_t, (_Float16)(g / (1.f + expf(-g)) * u));
+      }
+    } else
+    for (uint32_t idx = tid; idx < 16u * UT * ntok; idx += nthreads) {
+      const uint32_t t = idx / (16u * UT), r = idx % (16u * UT), u = r >> 4, orow = (tile0 + tl) * 16u + r;
+      if (tl + u >= ntile || orow >= a.rows) continue;
+      const float s = sum(t, u, r & 15u);
       float* y = a.Y + (size_t)(m0 + t) * a.rows + orow;
       *y = a.accumulate ? *y + s : s;
     }

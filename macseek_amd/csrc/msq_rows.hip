@@ -9,29 +9,30 @@ namespace {
 
 // workgroups: as many as are resident (four waves per SIMD, LDS), each a run of consecutive row tiles
 template <class F>
-size_t rows_lds(uint32_t waves, int S, int UT, int TT) {
-  return (size_t)F::LDS_WORDS * 4 + (size_t)rows_red_words(waves, UT, TT) * 4 + (size_t)waves * rows_ring<F>(S);
+size_t rows_lds(uint32_t waves, int S, int UT, int TT, bool gu = false) {
+  return (size_t)F::LDS_WORDS * 4 + (size_t)rows_red_words(waves, UT, TT, gu) * 4 + (size_t)waves * rows_ring<F>(S);
 }
 uint32_t rows_tiles_per_wg(uint32_t ntiles, uint32_t waves, size_t lds, uint32_t blocks) {
   const uint32_t per_cu = std::max<uint32_t>(1, std::min<uint32_t>(16 / waves, (uint32_t)(kMaxLds / lds)));
   const uint32_t slots = std::max<uint32_t>(1, (uint32_t)device_info().cus * per_cu / blocks);
   return (ntiles + slots - 1) / slots;
 }
-template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false, int TT = 1>
+template <class F, int BPW, int S, int NT, int UT, bool ROUND = false, bool XH = false, int TT = 1, bool GU = false>
 int launch_nt(hipStream_t st, RowsArgs a, uint32_t waves) {
-  const size_t lds = rows_lds<F>(waves, S, UT, TT);
+  const size_t lds = rows_lds<F>(waves, S, UT, TT, GU);
   if (lds > (size_t)kMaxLds) return MSQ_ERR_UNSUPPORTED;
-  const int rc = allow_large_lds(mm_rows_kernel<F, BPW, S, NT, UT, ROUND, XH, TT>, lds);
+  const int rc = allow_large_lds(mm_rows_kernel<F, BPW, S, NT, UT, ROUND, XH, TT, GU>, lds);
   if (rc != MSQ_OK) return rc;
   a.ntiles = (a.rows + 15) / 16;
-  const uint32_t blocks = ROUND ? (a.n + 16 * TT - 1) / (16 * TT) : 1;
+  const uint32_t blocks = ROUND || XH ? (a.n + 16 * TT - 1) / (16 * TT) : 1;
   a.tiles_per_wg = rows_tiles_per_wg(a.ntiles, waves, lds, blocks);
+  if (GU) { a.ntiles *= 2; a.tiles_per_wg *= 2; }
   if (a.rows_per_group != a.rows) {  // a workgroup's tiles belong to one group
     const uint32_t tg = a.rows_per_group / 16;
     while (tg % a.tiles_per_wg) a.tiles_per_wg--;
   }
   const uint32_t grid = (a.ntiles + a.tiles_per_wg - 1) / a.tiles_per_wg;
-  hipLaunchKernelGGL((mm_rows_kernel<F, BPW, S, NT, UT, ROUND, XH, TT>), dim3(grid, blocks), dim3(64 * waves), lds, st, a);
+  hipLaunchKernelGGL((mm_rows_kernel<F, BPW, S, NT, UT, ROUND, XH, TT, GU>), dim3(grid, blocks), dim3(64 * waves), lds, st, a);
   MSQ_HIP(hipGetLastError());
   return MSQ_OK;
 }
@@ -198,6 +199,33 @@ int matmul_rows(hipStream_t st, int t, const uint8_t* W, int rows, int cols, con
     if (rc != MSQ_OK) return rc;
   }
   return MSQ_OK;
+}
+
+// A shared expert of a K-quant / Q8_0 type over few tokens (fp16 activations, fp32 scales as in the small-N product): gate, up and
+// SwiGLU in one launch, or the down product.
+namespace {
+template <class F>
+bool shared_fits(uint32_t nws_gu, uint32_t nws_dn) {  // a workgroup's waves and their LDS
+  const uint32_t gu = (nws_gu + 1) / 2, dn = nws_dn <= 16 ? nws_dn : (nws_dn + 1) / 2;
+  return gu <= 16 && dn <= 16 && rows_lds<F>(gu, 2, 2, 1, true) <= (size_t)kMaxLds && rows_lds<F>(dn, 2, 1, 1) <= (size_t)kMaxLds;
+}
+template <class F>
+int launch_shared(hipStream_t st, const RowsArgs& a, bool gu) {
+  if (gu) return launch_nt<F, 2, 2, 16, 2, false, true, 1, true>(st, a, (a.nws + 1) / 2);
+  return a.nws <= 16 ? launch_nt<F, 1, 2, 16, 1, false, true>(st, a, a.nws) : launch_nt<F, 2, 2, 16, 1, false, true>(st, a, (a.nws + 1) / 2);
+}
+}  // namespace
+bool shared_rows_serves(int t, int dim, int inter) {
+  const uint32_t g = (uint32_t)dim / 256, d = (uint32_t)inter / 256;
+  return t == MSQ_Q6_K ? shared_fits<FragQ6KG>(g, d) : t == MSQ_Q8_0 && shared_fits<FragQ8_0>(g, d);
+}
+int shared_rows(hipStream_t st, int t, const uint8_t* W, const uint8_t* up, int rows, int cols, const uint16_t* X, uint16_t* H, float* Z, int n) {
+  RowsArgs a{};
+  a.W = W; a.W1 = up; a.X = X; a.Y = Z; a.H = H;
+  a.n = (uint32_t)n; a.rows = (uint32_t)rows; a.cols = (uint32_t)cols; a.x_stride = (uint32_t)cols;
+  a.row_bytes = (uint32_t)msq_type_row_bytes(t, cols); a.rows_per_group = (uint32_t)rows; a.nws = (uint32_t)cols / 256;
+  a.w_bytes = a.rows * a.row_bytes;
+  return t == MSQ_Q6_K ? launch_shared<FragQ6KG>(st, a, up != nullptr) : launch_shared<FragQ8_0>(st, a, up != nullptr);
 }
 
 bool matvec_rows_serves(int t, int rows, int cols, int n, int groups, const void* X) {
