@@ -87,6 +87,66 @@ __device__ __forceinline__ void select6(float (&key)[kMaxEpl], const double (&sc
   }
 }
 
+// A workgroup of up to eight waves selects the top six of one token, one expert a thread (key -inf: none, or not comparable) and writes ids
+// and weights; after(): by one thread, behind the barrier.
+// Selection in two levels: each wave picks the six best of its 64 experts, one a lane, and leaves them in LDS; wave 0 picks
+// the six best of those 48. The six best overall are among the six best of their waves, and "greater key, then lower expert
+// id" is a total order: experts, and the candidates that a wave leaves, stand in the lanes in the order of their ids where keys
+// are equal, so the first lane with the greatest key is the choice. NaN and -inf are never chosen.
+template <class After>
+__device__ __forceinline__ void select6_of_block(float key, double sc, uint32_t tid, float route_scale, int* __restrict__ ids, float* __restrict__ wts,
+                                               After after) {
+  constexpr uint32_t WAVES = 8;
+  __shared__ float c_key[WAVES * kTopK];
+  __shared__ int c_id[WAVES * kTopK];
+  __shared__ double c_sc[WAVES * kTopK];
+  const uint32_t lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+#pragma unroll
+  for (int k = 0; k < kTopK; k++) {
+    const float m = wave_max_f(key);
+    const uint64_t best = __builtin_amdgcn_ballot_w64(key == m && m > -INFINITY);
+    const bool won = best ? (uint32_t)__builtin_ctzll(best) == lane : lane == 0;
+    if (won) {
+      c_key[wave * kTopK + k] = m;
+      c_id[wave * kTopK + k] = (int)tid;
+      c_sc[wave * kTopK + k] = sc;
+      key = -INFINITY;
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  if (lane == 0) after();
+  const uint32_t candidates = (blockDim.x >> 6) * kTopK;
+  float ck = lane < candidates ? c_key[lane] : -INFINITY;
+  const int ce = lane < candidates ? c_id[lane] : 0;
+  const uint64_t cs = lane < candidates ? __builtin_bit_cast(uint64_t, c_sc[lane]) : 0;
+  int sel_e[kTopK];
+  double sel_s[kTopK];
+  double sum = 0.0;  // the six scores are added in selection order, as the reference adds them
+#pragma unroll
+  for (int k = 0; k < kTopK; k++) {
+    const float m = wave_max_f(ck);
+    const uint64_t best = __builtin_amdgcn_ballot_w64(ck == m && m > -INFINITY);
+    if (!best) {  // fewer than six comparable keys (NaN logits): expert 0 with weight 0
+      sel_e[k] = 0;
+      sel_s[k] = 0.0;
+      continue;
+    }
+    const int src = (int)__builtin_ctzll(best);
+    if (lane == (uint32_t)src) ck = -INFINITY;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cs, src);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cs >> 32), src);
+    sel_e[k] = __builtin_amdgcn_readlane(ce, src);
+    sel_s[k] = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+    sum += sel_s[k];
+  }
+  if (lane < (uint32_t)kTopK) {
+#pragma unroll
+    for (int k = 0; k < kTopK; k++)
+      if (lane == (uint32_t)k) { ids[k] = sel_e[k]; wts[k] = (float)(sel_s[k] / (sum + 1e-20) * (double)route_scale); }
+  }
+}
+
 // logits [n][n_exp] -> ids [n][6], weights [n][6]; one wave per token, four per workgroup.
 __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
                                                           int* __restrict__ ids, float* __restrict__ wts, uint32_t n_tokens,
@@ -104,6 +164,19 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restric
     if (i < epl) score_key(row[lane + 64u * i], bias[lane + 64u * i], sc[i], key[i]);
   }
   select6(key, sc, epl, route_scale, lane, ids + (size_t)t * kTopK, wts + (size_t)t * kTopK);
+}
+
+// The same, a workgroup per token and an expert a thread: the double-precision chain of one expert instead of up to eight.
+__global__ __launch_bounds__(512) void router_topk_wide_kernel(const float* __restrict__ logits, const float* __restrict__ bias, int* __restrict__ ids,
+                                                               float* __restrict__ wts, uint32_t n_exp, float route_scale) {
+  const uint32_t tid = threadIdx.x, t = blockIdx.x;
+  float key = -INFINITY;
+  double sc = 0.0;
+  if (tid < n_exp) {
+    score_key(logits[(size_t)t * n_exp + tid], bias[tid], sc, key);
+    if (!(key > -INFINITY)) key = -INFINITY;
+  }
+  select6_of_block(key, sc, tid, route_scale, ids + (size_t)t * kTopK, wts + (size_t)t * kTopK, [] {});
 }
 
 // Decode: logits = W[n_exp][dim] . x[dim] and the selection in one launch. A workgroup is eight waves, four to an expert's row,
@@ -126,9 +199,6 @@ __global__ __launch_bounds__(512) void router_fused_kernel(const float* __restri
                                                            float* __restrict__ wts, float route_scale) {
   constexpr uint32_t WAVES = 8, SPLIT = 4;
   __shared__ float part[WAVES];
-  __shared__ float c_key[WAVES * kTopK];
-  __shared__ int c_id[WAVES * kTopK];
-  __shared__ double c_sc[WAVES * kTopK];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t number = *call + 1u;
@@ -179,10 +249,6 @@ __global__ __launch_bounds__(512) void router_fused_kernel(const float* __restri
     }
     return;
   }
-  // Selection in two levels: each wave picks the six best of its 64 experts, one a lane, and leaves them in LDS; wave 0 picks
-  // the six best of those 48. The six best overall are among the six best of their waves, and "greater key, then lower expert
-  // id" is a total order: experts, and the candidates that a wave leaves, stand in the lanes in the order of their ids where keys
-  // are equal, so the first lane with the greatest key is the choice. NaN and -inf are never chosen.
   float key = -INFINITY;
   double sc = 0.0;
   if (tid < n_exp) {
@@ -196,49 +262,7 @@ __global__ __launch_bounds__(512) void router_fused_kernel(const float* __restri
     score_key(logit, b, sc, key);
     if (!(key > -INFINITY)) key = -INFINITY;
   }
-#pragma unroll
-  for (int k = 0; k < kTopK; k++) {
-    const float m = wave_max_f(key);
-    const uint64_t best = __builtin_amdgcn_ballot_w64(key == m && m > -INFINITY);
-    const bool won = best ? (uint32_t)__builtin_ctzll(best) == lane : lane == 0;
-    if (won) {
-      c_key[wave * kTopK + k] = m;
-      c_id[wave * kTopK + k] = (int)tid;
-      c_sc[wave * kTopK + k] = sc;
-      key = -INFINITY;
-    }
-  }
-  __syncthreads();
-  if (wave != 0) return;
-  if (lane == 0) __hip_atomic_store(call, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  float ck = lane < WAVES * kTopK ? c_key[lane] : -INFINITY;
-  const int ce = lane < WAVES * kTopK ? c_id[lane] : 0;
-  const uint64_t cs = lane < WAVES * kTopK ? __builtin_bit_cast(uint64_t, c_sc[lane]) : 0;
-  int sel_e[kTopK];
-  double sel_s[kTopK];
-  double sum = 0.0;  // the six scores are added in selection order, as the reference adds them
-#pragma unroll
-  for (int k = 0; k < kTopK; k++) {
-    const float m = wave_max_f(ck);
-    const uint64_t best = __builtin_amdgcn_ballot_w64(ck == m && m > -INFINITY);
-    if (!best) {  // fewer than six comparable keys (NaN logits): expert 0 with weight 0
-      sel_e[k] = 0;
-      sel_s[k] = 0.0;
-      continue;
-    }
-    const int src = (int)__builtin_ctzll(best);
-    if (lane == (uint32_t)src) ck = -INFINITY;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cs, src);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cs >> 32), src);
-    sel_e[k] = __builtin_amdgcn_readlane(ce, src);
-    sel_s[k] = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-    sum += sel_s[k];
-  }
-  if (lane < (uint32_t)kTopK) {
-#pragma unroll
-    for (int k = 0; k < kTopK; k++)
-      if (lane == (uint32_t)k) { ids[k] = sel_e[k]; wts[k] = (float)(sel_s[k] / (sum + 1e-20) * (double)route_scale); }
-  }
+  select6_of_block(key, sc, tid, route_scale, ids, wts, [&] { __hip_atomic_store(call, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
 }
 
 // Routing lists: one workgroup per expert e, its waves on consecutive slices of the entries. A first pass over the ids
@@ -338,7 +362,13 @@ int msq_router_topk(void* stream, const MsqBuffer* logits, const MsqBuffer* bias
   if (!buf_ok(logits, (size_t)n_tokens * n_exp * 4) || !buf_ok(bias, (size_t)n_exp * 4) ||
       !buf_ok(ids, (size_t)n_tokens * kTopK * 4) || !buf_ok(w, (size_t)n_tokens * kTopK * 4))
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: router_topk: buffer missing or too small (tokens %d experts %d)", n_tokens, n_exp);
-  hipLaunchKernelGGL(router_topk_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+  // Up to 1024 tokens the chain of a wave bounds the launch: an expert a thread. Beyond, the double-precision arithmetic of all of
+  // them, and a wave per token has fewer reductions; with up to 128 experts there is nothing in it. A wave per token / an expert a
+  // thread, us: 384 experts, 2 tokens 8.0 / 4.4, 37 8.6 / 4.6, 512 8.9 / 6.1, 1024 9.2 / 7.8, 2048 11.5 / 13.0; 128, 37 tokens 5.8 / 4.3, 4096 10.2 / 9.8.
+  if (n_tokens <= 1024 || n_exp <= 128)
+    hipLaunchKernelGGL(router_topk_wide_kernel, dim3((unsigned)n_tokens), dim3((unsigned)n_exp), 0, (hipStream_t)stream, (const float*)bptr(logits),
+                       (const float*)bptr(bias), (int*)bptr_mut(ids), (float*)bptr_mut(w), (uint32_t)n_exp, route_scale);
+  else hipLaunchKernelGGL(router_topk_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
                      (const float*)bptr(logits), (const float*)bptr(bias), (int*)bptr_mut(ids), (float*)bptr_mut(w),
                      (uint32_t)n_tokens, (uint32_t)n_exp, route_scale);
   MSQ_HIP(hipGetLastError());
