@@ -421,21 +421,31 @@ __global__ __launch_bounds__(64 * WV) void mm_tile_kernel(const void* X_, const 
   }
 }
 
-// Y (+)= partials[0] + partials[1] + ... in that order, element by element
+// Y (+)= partials[0] + partials[1] + ... in that order, element by element. Bound by the trip to memory, so up to 32 slices are
+// requested before the first is added (twenty slices of 1280x16: in three trips of eight 4.5 us, so 3.0, under the profiler).
 __global__ __launch_bounds__(256) void mm_reduce_kernel(const float* __restrict__ partials, float* __restrict__ Y, size_t count,
                                                         uint32_t slices, uint32_t accumulate) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= count) return;
+  const float y = accumulate ? Y[i] : 0.f;
   float s = 0.f;
-  for (uint32_t z0 = 0; z0 < slices; z0 += 8u) {  // eight slices requested before the first is added
-    float t[8];
+  for (uint32_t z0 = 0; z0 < slices; z0 += 32u) {
+    float t[32];
 #pragma unroll
-    for (uint32_t k = 0; k < 8u; k++) t[k] = partials[(size_t)min(z0 + k, slices - 1u) * count + i];
+    for (uint32_t b = 0; b < 32u; b += 8u)
+      if (z0 + b < slices) {
 #pragma unroll
-    for (uint32_t k = 0; k < 8u; k++)
-      if (z0 + k < slices) s += t[k];
+        for (uint32_t k = b; k < b + 8u; k++) t[k] = partials[(size_t)min(z0 + k, slices - 1u) * count + i];
+      }
+#pragma unroll
+    for (uint32_t b = 0; b < 32u; b += 8u)
+      if (z0 + b < slices) {
+#pragma unroll
+        for (uint32_t k = b; k < b + 8u; k++)
+          if (z0 + k < slices) s += t[k];
+      }
   }
-  Y[i] = accumulate ? Y[i] + s : s;
+  Y[i] = accumulate ? y + s : s;
 }
 
 }  // namespace msq
