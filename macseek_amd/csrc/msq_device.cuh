@@ -334,6 +334,21 @@ __device__ __forceinline__ float sum_in_order(const float* p, uint32_t n, uint32
   return s;
 }
 
+// Sum of n sums of eight lanes each in the order that sums of sixteen lanes (row16_fold) take: (p[0] + p[1]) + (p[2] + p[3]) + ...; behind
+// an odd last one the sixteen lanes' other half is idle and adds zero.
+__device__ __forceinline__ float sum_pairs_in_order(const float* p, uint32_t n) {
+  float s = 0.f;
+  for (uint32_t k0 = 0; k0 < n; k0 += 8u) {
+    float t[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) t[j] = p[min(k0 + j, n - 1u)];
+#pragma unroll
+    for (int j = 0; j < 8; j += 2)
+      if (k0 + j < n) s += k0 + j + 1u < n ? t[j] + t[j + 1] : t[j];
+  }
+  return s;
+}
+
 // ------------------------------------------------------------------------------------------------ LDS table copies
 __device__ __forceinline__ void copy_words16(uint32_t* dst, const uint32_t* src, int nwords, int tid, int nthreads) {
   const uint4* s = (const uint4*)src;

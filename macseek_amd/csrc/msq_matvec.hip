@@ -273,8 +273,7 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   // not four packed rows for each (2304x2304 0.95), nor rows of 2304 columns below 6 MB (0.94 to 0.97); the codebook formats, bound by their lookups, lose 1 % and keep the one-row
   // form. MSQ_MV_PAIR = 0 / 2: never / every format.
   // Under a fused norm likewise, but for Q8_0 below 20 MB (2560, 4608, 5120 and 7168 columns, one by one over in pairs: 6 to 18 MB
-  // 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04). (Sums of 16 lanes are added in one order whether rows are packed or not; with
-  // sums of 8, which are not, the norm's calls and the plain ones have to agree, so Q8_0 has these from 20 MB on.)
+  // 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04). A row's bits are the same packed or not, so the rule is free to differ.
   const double bytes = (double)a.rows * a.row_bytes;
   int pack = 1;
   {

@@ -529,7 +529,8 @@ __device__ __forceinline__ void wait_rows_n(int n) {
 // memory, so a wave's slice of 64 units may run from the end of one row into the next -- which leaves no or fewer lanes idle when a
 // row's units do not fill whole waves (5120 columns: five waves per two rows instead of twice three; 1280: five per eight rows
 // instead of eight). rows_, row_bytes_, units_, ks_ and the tile shape then describe the packed rows; the rows' sums of PACK lanes, 16
-// or 8 (a row's units must be a multiple of that), are told apart when the partial sums are added.
+// or 8 (a row's units must be a multiple of that), are told apart when the partial sums are added -- in the one order that rows
+// launched singly take as well, so that a row's bits do not depend on how the matrix around it is launched.
 template <class D, int ITERS, int T, int NORM = kNormNone, bool SW = false, int PACK = 0>
 __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t rows_, uint32_t row_bytes_, uint32_t units_, uint32_t ks_,
                                                      uint32_t rpw_, uint32_t ntiles_, uint32_t rows_per_group_, const float* x_,
@@ -776,7 +777,8 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
       for (uint32_t idx = tid; idx < n * T; idx += blockDim.x) {
         const uint32_t r = T == 1 ? idx : idx % n, t = T == 1 ? 0u : idx / n, row = (tile_row0 << sh) + r;
         if (row < rows_ << sh && t0 + t < ta.n) {
-          const float s = sum_in_order(part + ((r >> sh) * SUMS * KS + (r & (a.pack - 1u)) * G) * T + t, G, T);
+          const float* sums = part + ((r >> sh) * SUMS * KS + (r & (a.pack - 1u)) * G) * T + t;
+          const float s = PACK == 8 ? sum_pairs_in_order(sums, G) : sum_in_order(sums, G, T);  // (eight lanes: one token)
           float* y = a.y + (size_t)(t0 + t) * ta.y_stride + row;
           *y = a.accumulate ? *y + s : s;
         }

@@ -44,3 +44,20 @@ def test_packed_rows_vs_oracle(dev, t, rows, cols, acc):
                                          (O.Q8_0, 16392, 1280), (O.Q6_K, 12004, 2560), (O.Q5_K, 8008, 2304)], ids=lambda v: None)
 def test_packed_rows_with_norm(dev, t, rows, cols):
     with_norm(dev, t, rows, cols)
+
+
+@pytest.mark.parametrize("t,rows,cols", [(O.Q6_K, 32768, 1280), (O.Q5_K, 8196, 512), (O.Q6_K, 9000, 768), (O.Q5_K, 8008, 2304), (O.Q8_0, 20000, 1280),
+                                         (O.Q6_K, 32776, 256), (O.Q6_K, 4100, 1536), (O.Q8_0, 32772, 768)], ids=lambda v: None)
+def test_packed_rows_have_the_bits_of_chunks(dev, t, rows, cols):
+    # chunks launched with matvec_cfg's shape go row by row, the whole matrix packed: sums of 16 and of 8 lanes
+    Wd, xd = up(O.random_blocks(t, rows * cols, 11 + cols)), up(O.randn(cols, 12))
+    W, rb, cfg = q.Buffer.of(Wd), q.row_bytes(t, cols), q.matvec_cfg(t, rows, cols)
+    full, parts = torch.empty(rows, device=dev), torch.empty(rows, device=dev)
+    e = q.Enc()
+    q.encode_matvec(e, t, W, rows, cols, q.Buffer.of(xd), q.Buffer.of(full))
+    chunk = cfg.nr * cfg.rsg * 37
+    for r0 in range(0, rows, chunk):
+        n = min(chunk, rows - r0)
+        q.encode_matvec(e, t, W.sub(r0 * rb, n * rb), n, cols, q.Buffer.of(xd), q.Buffer.of(parts).sub(r0 * 4, n * 4), False, 1, cfg)
+    e.wait()
+    assert torch.equal(full, parts)
