@@ -298,7 +298,9 @@ int msq_router_topk(void* stream, const MsqBuffer* logits, const MsqBuffer* bias
  * its first n_exp floats; the caller zeroes it once before the first call, and the calls count themselves in it.
  * A scratch belongs to one stream at a time: calls sharing it must not overlap. A launch that fails (MSQ_ERR_HIP) or is
  * torn down part-way may leave results of a call that is not counted, which the next call would take for its own:
- * zero the scratch again before it is reused. */
+ * zero the scratch again before it is reused. A call whose logits do not all arrive within seconds (calls overlapping on
+ * one scratch, a device that stalls) ends all the same: its six weights are NaN (its ids are in range), and so are
+ * those of every later call on this scratch until the caller zeroes it again. */
 size_t msq_router_scratch_bytes(int n_exp);
 int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffer* W, const MsqBuffer* bias,
                      const MsqBuffer* scratch, const MsqBuffer* ids, const MsqBuffer* w, int dim, int n_exp,

@@ -88,18 +88,19 @@ __device__ __forceinline__ void select6(float (&key)[kMaxEpl], const double (&sc
 }
 
 // A workgroup of up to eight waves selects the top six of one token, one expert a thread (key -inf: none, or not comparable) and writes ids
-// and weights; after(): by one thread, behind the barrier.
+// and weights; after(any): by one thread, behind the barrier; any (WAITS): a thread came with `missing`, which makes all six weights NaN.
 // Selection in two levels: each wave picks the six best of its 64 experts, one a lane, and leaves them in LDS; wave 0 picks
 // the six best of those 48. The six best overall are among the six best of their waves, and "greater key, then lower expert
 // id" is a total order: experts, and the candidates that a wave leaves, stand in the lanes in the order of their ids where keys
 // are equal, so the first lane with the greatest key is the choice. NaN and -inf are never chosen.
-template <class After>
-__device__ __forceinline__ void select6_of_block(float key, double sc, uint32_t tid, float route_scale, int* __restrict__ ids, float* __restrict__ wts,
-                                               After after) {
+template <bool WAITS, class After>
+__device__ __forceinline__ void select6_of_block(float key, double sc, bool missing, uint32_t tid, float route_scale, int* __restrict__ ids,
+                                               float* __restrict__ wts, After after) {
   constexpr uint32_t WAVES = 8;
   __shared__ float c_key[WAVES * kTopK];
   __shared__ int c_id[WAVES * kTopK];
   __shared__ double c_sc[WAVES * kTopK];
+  [[maybe_unused]] __shared__ uint32_t c_missing[WAVES];
   const uint32_t lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
 #pragma unroll
   for (int k = 0; k < kTopK; k++) {
@@ -113,16 +114,22 @@ __device__ __forceinline__ void select6_of_block(float key, double sc, uint32_t 
       key = -INFINITY;
     }
   }
+  if constexpr (WAITS) {
+    const uint64_t lacks = __builtin_amdgcn_ballot_w64(missing);
+    if (lane == 0) c_missing[wave] = lacks != 0;
+  }
   __syncthreads();
   if (wave != 0) return;
-  if (lane == 0) after();
+  bool any = false;
+  if constexpr (WAITS) any = __builtin_amdgcn_ballot_w64(lane < (blockDim.x >> 6) && c_missing[lane & (WAVES - 1u)] != 0) != 0;
+  if (lane == 0) after(any);
   const uint32_t candidates = (blockDim.x >> 6) * kTopK;
   float ck = lane < candidates ? c_key[lane] : -INFINITY;
   const int ce = lane < candidates ? c_id[lane] : 0;
   const uint64_t cs = lane < candidates ? __builtin_bit_cast(uint64_t, c_sc[lane]) : 0;
   int sel_e[kTopK];
   double sel_s[kTopK];
-  double sum = 0.0;  // the six scores are added in selection order, as the reference adds them
+  double sum = any ? __builtin_nan("") : 0.0;  // the six scores are added in selection order, as the reference adds them
 #pragma unroll
   for (int k = 0; k < kTopK; k++) {
     const float m = wave_max_f(ck);
@@ -176,7 +183,7 @@ __global__ __launch_bounds__(512) void router_topk_wide_kernel(const float* __re
     score_key(logits[(size_t)t * n_exp + tid], bias[tid], sc, key);
     if (!(key > -INFINITY)) key = -INFINITY;
   }
-  select6_of_block(key, sc, tid, route_scale, ids + (size_t)t * kTopK, wts + (size_t)t * kTopK, [] {});
+  select6_of_block<false>(key, sc, false, tid, route_scale, ids + (size_t)t * kTopK, wts + (size_t)t * kTopK, [](bool) {});
 }
 
 // Decode: logits = W[n_exp][dim] . x[dim] and the selection in one launch. A workgroup is eight waves, four to an expert's row,
@@ -190,18 +197,22 @@ __global__ __launch_bounds__(512) void router_topk_wide_kernel(const float* __re
 // 384x5120 10.1 -> 7.2, 64x2048 8.3 -> 5.4, F32 384x7168 12.4 -> 8.6 (calls back to back, weights from HBM).
 // The call's number stands behind the records; the selecting workgroup counts it up at its end, when every other workgroup
 // has read it (it has their records). Every wait ends: the other workgroups wait for nothing, and the selecting one, the last
-// of the launch, gives up after kRouterPolls reads (seconds; the experts without a record then count as NaN).
+// of the launch, gives up after `polls` reads (kRouterPolls: seconds). Then a workgroup may still be to come that reads the number
+// only after it has been counted up, and its record would pass for one of the next call. So a call that gave up leaves
+// kRouterGaveUp in place of its number: records written under it name no call (0), and this call and all that follow return six NaN
+// weights, until the scratch is zeroed.
 constexpr uint32_t kRouterPolls = 1u << 22;
+constexpr uint32_t kRouterGaveUp = 0xFFFFFFFFu;  // (as a number, the last before counting starts again at 1: never left by a call that ended well)
 template <int QT, uint32_t U>
 __global__ __launch_bounds__(512) void router_fused_kernel(const float* __restrict__ x, const void* __restrict__ W, uint32_t dim,
                                                            uint32_t n_exp, const float* __restrict__ bias, float* logits,
                                                            uint64_t* recs, uint32_t* call, int* __restrict__ ids,
-                                                           float* __restrict__ wts, float route_scale) {
+                                                           float* __restrict__ wts, float route_scale, uint32_t polls) {
   constexpr uint32_t WAVES = 8, SPLIT = 4;
   __shared__ float part[WAVES];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-  const uint32_t number = *call + 1u;
+  const uint32_t number = *call + 1u;  // 0: an earlier call gave up
   if (blockIdx.x + 1u < gridDim.x) {
     const uint32_t e = blockIdx.x * (WAVES / SPLIT) + wave / SPLIT, first = 64u * (wave % SPLIT) + lane;
     constexpr uint32_t STEP = 64u * SPLIT;
@@ -251,18 +262,23 @@ __global__ __launch_bounds__(512) void router_fused_kernel(const float* __restri
   }
   float key = -INFINITY;
   double sc = 0.0;
+  bool missing = false;
   if (tid < n_exp) {
     const float b = bias[tid];
     uint64_t r = 0;
-    for (uint32_t k = 0; k < kRouterPolls; k++) {
+    for (uint32_t k = 0; k < polls; k++) {
       r = __hip_atomic_load(recs + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if ((uint32_t)(r >> 32) == number) break;
     }
-    const float logit = (uint32_t)(r >> 32) == number ? __builtin_bit_cast(float, (uint32_t)r) : __builtin_nanf("");
+    missing = (uint32_t)(r >> 32) != number || number == 0u;
+    const float logit = missing ? __builtin_nanf("") : __builtin_bit_cast(float, (uint32_t)r);
     score_key(logit, b, sc, key);
     if (!(key > -INFINITY)) key = -INFINITY;
   }
-  select6_of_block(key, sc, tid, route_scale, ids, wts, [&] { __hip_atomic_store(call, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); });
+  select6_of_block<true>(key, sc, missing, tid, route_scale, ids, wts, [&](bool any) {
+    const uint32_t left = any ? kRouterGaveUp : number == kRouterGaveUp ? 0u : number;
+    __hip_atomic_store(call, left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  });
 }
 
 // Routing lists: one workgroup per expert e, its waves on consecutive slices of the entries. A first pass over the ids
@@ -379,8 +395,8 @@ int msq_router_topk(void* stream, const MsqBuffer* logits, const MsqBuffer* bias
 // bytes an expert (callers keep the scratch size), then the number of the last call in a 256-byte line of its own
 size_t msq_router_scratch_bytes(int n_exp) { return ((size_t)n_exp * 4 + 255) / 256 * 256 + (size_t)n_exp * 16 + 256; }
 
-int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffer* W, const MsqBuffer* bias,
-                     const MsqBuffer* scratch, const MsqBuffer* ids, const MsqBuffer* w, int dim, int n_exp, float route_scale) {
+static int router_fused_impl(void* stream, int wtype, const MsqBuffer* x, const MsqBuffer* W, const MsqBuffer* bias, const MsqBuffer* scratch,
+                             const MsqBuffer* ids, const MsqBuffer* w, int dim, int n_exp, float route_scale, uint32_t polls) {
   if (!exp_ok(n_exp) || dim < 8 || dim % 8 || (wtype != MSQ_F32 && wtype != MSQ_BF16)) return unsupported("router_fused", wtype, n_exp, dim);
   const size_t esz = wtype == MSQ_F32 ? 4 : 2;
   if (!buf_ok(x, (size_t)dim * 4) || !buf_ok(W, (size_t)n_exp * dim * esz) || !buf_ok(bias, (size_t)n_exp * 4) ||
@@ -396,7 +412,7 @@ int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffe
   hipStream_t st = (hipStream_t)stream;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, block, 0, st, (const float*)bptr(x), (const void*)bptr(W), (uint32_t)dim, (uint32_t)n_exp,
-                       (const float*)bptr(bias), logits, recs, call, (int*)bptr_mut(ids), (float*)bptr_mut(w), route_scale);
+                       (const float*)bptr(bias), logits, recs, call, (int*)bptr_mut(ids), (float*)bptr_mut(w), route_scale, polls);
   };
   // vectors a lane of the four waves that share a row: one trip to memory up to 8192 columns
   const int per_lane = (dim / (wtype == MSQ_F32 ? 4 : 8) + 255) / 256;
@@ -411,6 +427,16 @@ int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffe
   else by_u.template operator()<MSQ_BF16>();
   MSQ_HIP(hipGetLastError());
   return MSQ_OK;
+}
+
+int msq_router_fused(void* stream, int wtype, const MsqBuffer* x, const MsqBuffer* W, const MsqBuffer* bias, const MsqBuffer* scratch,
+                     const MsqBuffer* ids, const MsqBuffer* w, int dim, int n_exp, float route_scale) {
+  return router_fused_impl(stream, wtype, x, W, bias, scratch, ids, w, dim, n_exp, route_scale, kRouterPolls);
+}
+// the same with a limit of its own on the selecting workgroup's wait (for tests)
+int msq_test_router_fused_polls(void* stream, int wtype, const MsqBuffer* x, const MsqBuffer* W, const MsqBuffer* bias, const MsqBuffer* scratch,
+                                const MsqBuffer* ids, const MsqBuffer* w, int dim, int n_exp, float route_scale, uint32_t polls) {
+  return router_fused_impl(stream, wtype, x, W, bias, scratch, ids, w, dim, n_exp, route_scale, polls);
 }
 
 int msq_route_lists(void* stream, const MsqBuffer* ids, const MsqBuffer* w, int n_tokens, int n_exp, const MsqRouteLists* L) {

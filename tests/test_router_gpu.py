@@ -256,3 +256,40 @@ def test_router_fused_row_lengths(dev, wtype, dim):
 @pytest.mark.parametrize("wtype,dim", [(q.QType.BF16, d) for d in (8, 2048, 2056, 8192, 8200)] + [(q.QType.F32, d) for d in (8, 1024, 1032, 4096, 4104, 8192, 8200)])
 def test_router_fused_shared_rows(dev, wtype, dim):
     test_router_fused_vs_oracle(dev, wtype, dim)
+
+
+def test_router_fused_that_gave_up_shows_it(dev):
+    # a wait that ends at once (a limit of no reads): NaN weights then and on every later call, until the scratch is zeroed; the
+    # last number before counting starts again is an ordinary one
+    import ctypes as C
+    from macseek_amd import _lib
+    n_exp, dim = 384, 512
+    L = C.CDLL(_lib.SO)
+    f = L.msq_test_router_fused_polls
+    f.argtypes, f.restype = _lib.SIGNATURES["msq_router_fused"][1] + [C.c_uint32], C.c_int
+    Wd, bd, xd = up(O.randn(n_exp * dim, 1, 0.05)), up(O.randn(n_exp, 2, 0.1)), up(O.randn(dim, 3))
+    s, e = arch.Scratch.create(n_exp), q.Enc()
+    ids, w = torch.full((6,), -1, dtype=torch.int32, device=dev), torch.zeros(6, device=dev)
+    bufs = [q.Buffer.of(t).c() for t in (xd, Wd, bd, s.mem, ids, w)]
+
+    def call(polls=None):
+        if polls is None:
+            arch.encode_router_fused(e, q.Buffer.of(xd), q.Buffer.of(Wd), q.Buffer.of(bd), q.Buffer.of(ids), q.Buffer.of(w), s, dim)
+        else:
+            assert f(e.handle, int(q.QType.F32), *[C.byref(b) for b in bufs], dim, n_exp, 1.5, polls) == 0
+        e.wait()
+        return ids.tolist(), w.clone()
+
+    ids0, w0 = call()
+    assert len(set(ids0)) == 6 and bool((w0 > 0).all())
+    for polls in (0, None, None, 1 << 22):
+        i, v = call(polls)
+        assert bool(torch.isnan(v).all()) and all(0 <= k < n_exp for k in i)
+    s.mem.zero_()
+    number = s.mem.view(torch.int32)[(s.mem.numel() - 256) // 4:][:1]
+    for start in (0, -2):  # -2: the next call is number 0xFFFFFFFF, the one behind it number 1 again
+        number.fill_(start)
+        for _ in range(3):
+            i, v = call()
+            assert i == ids0 and torch.equal(v, w0)
+    assert int(number) == 2
