@@ -146,21 +146,40 @@ int launch_mm(hipStream_t st, int t, const RowsArgs& a) {
 //  * two workgroups a token block at least, or a part of the device has none (IQ1_S 202x1536 at 2387, 150 blocks, 0.75).
 //
 // ... and in blocks of 32 tokens more work, up to 256 tokens (serves_32), `work` of it per wave of the device in units of 16 rows x
-// 256 columns x 32 tokens. Measured over 7000 random calls against the route that each took before, median (lowest of 100):
+// 256 columns x 32 tokens. Measured over 28000 random calls against the route that each took before, median (lowest of 100):
 //  * up to 64 tokens (not 33 to 39, whose second block is nearly empty) at 1280 to 4096 columns, work of at most five: IQ4_NL 1.59
 //    (1.24), IQ2_XXS 1.55 (1.24), Q6_K 1.40 (1.11), IQ1_S 1.41 (1.10) but for more than 16384 rows (32768x1280 at 32 0.95) and 40 to 47
-//    tokens (0.94 to 1.0), Q5_K 1.27 likewise (16427x1536 at 54 0.90, 10437x3840 at 42 0.96);
+//    tokens (0.94 to 1.0), Q5_K 1.27 likewise (16427x1536 at 54 0.90, 10437x3840 at 42 0.96; fp16 activations, 48 to 55 tokens, 1.12
+//    but 0.92 to 0.98 in one call of twenty, 10620x3328, 15500x2304);
+//  * Q6_K of fp16 activations at 40 to 48 tokens over more than 16384 rows of 1280 or 1536 columns goes in steps, and so does the fused
+//    kernel: not in the first half of every 4096 rows (0.88 to 1.09, mean 0.97; the other half 0.97 to 1.17); 1792 columns 0.89 to 0.96
+//    at 14400 to 14900, 20800 to 21600 and 22700 rows, 1.03 to 1.3 between;
 //  * in two launches of half the columns, 6144 to 8192: from 5120 rows on for the codebook formats and IQ4_NL (1.1 to 1.9; 3500 rows
 //    0.87 to 1.2; IQ1_S from 40 tokens on and of fp32 activations, 0.9 with fp16), from 6144 rows on for the K-quants up to 32 tokens
-//    (1.05 to 1.5; 5120 rows 0.86, more tokens 0.7 to 1.2);
+//    (1.05 to 1.5; 5120 rows 0.86, more tokens 0.7 to 1.2); but not where the row tiles have just begun another round of the
+//    workgroups and the fused kernel's slices come out even (two_launches_lose(); 0.92 to 1.09, median 0.99; the rest from 0.976 on);
 //  * 65 to 128 tokens: IQ4_NL from 1536 columns on, work of at most seven (1.36, lowest 1.0; 20587x1536 at 102, 7.5, 0.94); Q6_K
 //    from 3584 on, Q5_K 4096, at most eight (1.33; Q5_K 4500x3584 at 114 0.91); the codebook formats have the tile kernel;
 //  * 129 to 256 tokens: 1152 to 2048 rows of 1536 columns and more, at most four (1.2 to 1.7).
-bool serves_32(int t, int rows, size_t nws, int n) {
+bool two_launches_lose(int t, int rows, int cols, int n, bool x_half) {
+  const bool narrow = cols > 6144 && cols <= 6656, iq2 = t == MSQ_IQ2_XXS, iq4 = t == MSQ_IQ4_NL;
+  if (t == MSQ_Q5_K) return narrow && !x_half && rows <= 6512;
+  if (n <= 32) return iq4 && cols >= 6400 && cols < 6656 && rows <= 5440;
+  if (iq2 && cols > 7168 && cols <= 7424) return rows <= 5440;
+  return narrow && (iq2 || iq4) && (rows <= 6144 ? n <= 48 && rows <= 5440 : rows <= 6512);
+}
+bool serves_32(int t, int rows, int cols, int n, bool x_half) {
+  const size_t nws = ((size_t)cols + 255) / 256;
   const bool iq4 = t == MSQ_IQ4_NL, iq1 = t == MSQ_IQ1_S, q5 = t == MSQ_Q5_K, kq = q5 || t == MSQ_Q6_K;
   const size_t work = ((size_t)rows + 15) / 16 * nws * (((size_t)n + 31) / 32), waves = 16 * (size_t)device_info().cus;
   if (n <= 16 || nws > 32 || (n > 32 && n < 40)) return false;
-  if (nws > 16) return n <= 64 && nws >= 24 && work <= 5 * waves && (kq ? n <= 32 && rows >= 6144 : rows >= 5120 && !(iq1 && n <= 32));
+  if (nws > 16)
+    return n <= 64 && nws >= 24 && work <= 5 * waves && (kq ? n <= 32 && rows >= 6144 : rows >= 5120 && !(iq1 && (n <= 32 || x_half))) &&
+           !two_launches_lose(t, rows, cols, n, x_half);
+  if (t == MSQ_Q6_K && x_half && n > 32 && n <= 48 && nws <= 6 && rows > 16384) {
+    const size_t cus = (size_t)device_info().cus;
+    if (2 * ((((size_t)rows + 15) / 16 - 1) % cus) < cus) return false;
+  }
   if (n <= 32) return nws >= 5 && work <= 5 * waves && !(iq1 && rows > 16384);
   if (n <= 64) return nws >= 5 && work <= 5 * waves && !((iq1 || q5) && (rows > 16384 || n < 48));
   if (n <= 128) return iq4 ? nws >= 6 && work <= 7 * waves : kq && nws >= (q5 ? 16u : 14u) && work <= 8 * waves;
@@ -173,7 +192,7 @@ bool matmul_rows_serves(int t, int rows, int cols, int n, const void* X, bool x_
   }
   const size_t nws = ((size_t)cols + 255) / 256, waves = 16 * (size_t)device_info().cus;
   if (cols % 128 || ((uintptr_t)X & (x_half ? 7 : 15)) || x_stride % 4 || x_stride > 0xFFFFFFFFull) return false;
-  if (!(x_half && t == MSQ_IQ1_S && nws > 16) && serves_32(t, rows, nws, n)) return true;
+  if (serves_32(t, rows, cols, n, x_half)) return true;
   const size_t stages = ((size_t)rows + 15) / 16 * nws * (((size_t)n + 15) / 16);
   if (n <= 16 || nws < 2 || nws > 16 || rows > 8192 || 2 * (((size_t)n + 15) / 16) > (size_t)device_info().cus) return false;
   if ((nws == 2 && rows > 4096) || (nws > 4 && rows > 4096 && n > 32)) return false;

@@ -31,9 +31,25 @@ ROUTES = [  # as in test_matmul_rows_gpu.py
     ((O.Q6_K, 16384, 1536, 40, 1, 1538), FUSED),
 ]
 
+LOSING = [  # the fused kernel is ahead: fp16 Q6_K in the first half of 4096 rows, two launches that have just begun another round of workgroups
+    ((O.Q6_K, 16384, 1280, 45, 1, 0), FEW), ((O.Q6_K, 16385, 1280, 45, 1, 0), FUSED), ((O.Q6_K, 18432, 1536, 40, 1, 0), FUSED),
+    ((O.Q6_K, 18433, 1536, 40, 1, 0), FEW), ((O.Q6_K, 20481, 1280, 48, 1, 0), FUSED), ((O.Q6_K, 20481, 1280, 49, 1, 0), FEW),
+    ((O.Q6_K, 20481, 1280, 48, 0, 0), FEW), ((O.Q6_K, 16385, 1792, 45, 1, 0), FEW), ((O.Q6_K, 18432, 1280, 32, 1, 0), FEW),
+    ((O.IQ2_XXS, 5440, 7424, 44, 1, 0), FUSED), ((O.IQ2_XXS, 5441, 7424, 44, 1, 0), FEW), ((O.IQ2_XXS, 5180, 7680, 44, 1, 0), FEW),
+    ((O.IQ2_XXS, 5180, 7424, 32, 1, 0), FEW), ((O.IQ2_XXS, 5180, 6656, 48, 0, 0), FUSED), ((O.IQ2_XXS, 5180, 6656, 49, 0, 0), FEW),
+    ((O.IQ2_XXS, 6144, 6400, 60, 0, 0), FEW), ((O.IQ2_XXS, 6145, 6400, 60, 0, 0), FUSED), ((O.IQ2_XXS, 6512, 6400, 60, 0, 0), FUSED),
+    ((O.IQ2_XXS, 6513, 6400, 60, 0, 0), FEW), ((O.IQ4_NL, 5200, 6528, 20, 0, 0), FUSED), ((O.IQ4_NL, 5441, 6528, 20, 0, 0), FEW),
+    ((O.IQ4_NL, 5200, 6656, 20, 0, 0), FEW), ((O.Q5_K, 6144, 6656, 20, 0, 0), FUSED), ((O.Q5_K, 6144, 6656, 20, 1, 0), FEW),
+    ((O.Q5_K, 6513, 6656, 20, 0, 0), FEW), ((O.Q6_K, 6144, 6656, 20, 0, 0), FEW),
+]
+
 
 def test_which_calls_it_serves():
     assert [(c, route(*c)) for c, _ in ROUTES] == ROUTES
+
+
+def test_which_calls_it_leaves_to_the_fused_kernel():
+    assert [(c, route(*c)) for c, _ in LOSING] == LOSING
 
 
 @pytest.mark.gpu
