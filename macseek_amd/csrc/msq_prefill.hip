@@ -139,6 +139,16 @@ int launch_block_t(hipStream_t st, PfBlkArgs a, uint32_t n6, uint32_t n3, uint32
 // 1.11 (1.01 to 1.11), 224 to 420 0.98 to 1.10 (1.01 to 1.10). Where the loss ends lies between 100 and 178 tokens and differs from
 // layer to layer; the line is drawn above all of it.
 constexpr int kPfQueueTokens = 2 * kPfBigTokens;
+// The shared expert of a K-quant / Q8_0 type through the few-token kernel (msq_rows.cuh), on the caller's stream? The tile kernel's 128 x 128
+// tiles are a chain of 150 us however few the tokens, and the fork to a second stream costs 14 us by itself; but they run beside the routed
+// experts, and the few-token kernel's 36 us (37 tokens) to 80 us (112) come behind them. Time before / after, Q6_K and Q8_0 alike, 384 IQ1_S
+// experts: 5120x2304 at 2 tokens 186 / 119, 16 307 / 280, 37 517 / 502, 64 650 / 606, 100 761 / 761, 150 (the tile kernel ahead) 992 / 978;
+// Q6_K 7168x2048 at 64 703 / 694, 100 918 / 889, 150 1171 / 1190 (Q8_0 of 7168 columns does not fit the LDS); 2560x1024 at 100 252 / 229, 150
+// 347 / 338. 94 to 242 experts in use 0.98 to 1.3 times the former speed at 37 to 112 tokens. Fewer of them leave compute units to the tile
+// kernel: 49 to 64 in use 1.02 to 1.5 at up to 48 tokens and, as long as no expert has more than 48 entries (the routed experts are one
+// launch then), 1.02 to 1.46 up to 112 (in a graph, where the fork is cheaper, 0.92 to 1.25); with such an expert, 9 to 64 in use, 0.86 to
+// 0.98 at 64 to 112 tokens of 5120x2304 and 4096x1536 (7168x2048 0.87 to 1.08, 2560x1024 0.98 to 1.08): the tile kernel has these.
+bool shared_few(int n, int used, bool crowded) { return n <= 112 && (!crowded || used >= 94); }
 bool block_path(int t) { return t == MSQ_IQ1_S || t == MSQ_IQ2_XXS; }
 template <bool GU>
 int launch_block(int t, hipStream_t st, const PfBlkArgs& a, uint32_t n6, uint32_t n3, uint32_t n2, int skip) {
@@ -166,6 +176,9 @@ size_t msq_moe_prefill_scratch_bytes(int total, int n, int n_exp, int dim, int i
   return header_bytes(std::max(total, 0), std::max(n, 0), std::max(n_exp, 0)) + align256(rows * dim * 2) +
          align256(rows * inter * 2) + align256(rows * dim * 4);
 }
+
+// whether a shared expert goes to the few-token kernel, without the LDS it needs (for tests)
+int msq_test_prefill_shared_few(int n, int used, int crowded) { return shared_few(n, used, crowded != 0) ? 1 : 0; }
 
 int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
   if (!p) return fail(MSQ_ERR_ARGUMENT, "macseek quant: moe_prefill: null arguments");
@@ -222,7 +235,11 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
     ni += q + (r ? 1u : 0u);
     nc[0] += q + (r > 48 ? 1u : 0u); nc[1] += r > 32 && r <= 48; nc[2] += r > 16 && r <= 32;
   };
-  for (int j = 0; j < ne; j++) count(p->offs[j + 1] - p->offs[j], ni_routed, nc_routed);
+  int used = 0;  // experts with entries
+  for (int j = 0; j < ne; j++) {
+    count(p->offs[j + 1] - p->offs[j], ni_routed, nc_routed);
+    used += p->offs[j + 1] > p->offs[j];
+  }
   if (p->has_shared) count(n, ni_shared, nc_shared);
   uint8_t* sc = bptr_mut(&p->scratch);
   // the block GEMM's counters take the place of the raw image, which is used up by then (a header of one or two experts may be too short)
@@ -304,12 +321,8 @@ int msq_moe_prefill(void* stream, const MsqMoePrefillArgs* p) {
     b.queue = counters && (!forked || n >= kPfQueueTokens) ? counters + (GU ? 0 : 16) : nullptr;
     return launch_block<GU>(GU ? p->t_gate_up : p->t_down, gs, b, nc_routed[0], nc_routed[1], nc_routed[2], skip);
   };
-  // ... and one over all tokens with the shared expert's weights. A K-quant / Q8_0 expert over few tokens takes the few-token kernel, on the
-  // caller's stream: the tile kernel's 128 x 128 tiles are a chain of 150 us however few the tokens, and the fork to a second stream
-  // costs 14 us by itself. Time before / after, 384 IQ1_S experts (Q6_K and Q8_0 alike): 5120x2304 at 2 tokens 186 / 119, 16 307 / 280, 37
-  // 517 / 502, 64 650 / 606, 100 761 / 761, 150 (the tile kernel ahead) 992 / 978; 7168x2048 at 64 703 / 694, 100 918 / 889, 150 1171 / 1190;
-  // 2560x1024 at 100 252 / 229, 150 347 / 338.
-  const bool few = p->has_shared && n <= 112 && shared_rows_serves(p->t_shared, dim, inter);
+  // ... and one over all tokens with the shared expert's weights
+  const bool few = p->has_shared && shared_few(n, used, nc_routed[0] > 0) && shared_rows_serves(p->t_shared, dim, inter);
   auto shared = [&](auto gu_tag, hipStream_t gs) -> int {
     constexpr bool GU = decltype(gu_tag)::value;
     const uint32_t K = (uint32_t)(GU ? dim : inter), N = (uint32_t)(GU ? inter : dim), rb = (uint32_t)(GU ? rb_sgu : rb_sd);

@@ -1,5 +1,5 @@
 """A Q6_K / Q8_0 shared expert over few tokens in msq_moe_prefill (the few-token kernel): one token, both sides of a block of sixteen
-and of the line to the tile kernel (112 tokens), one weight stage a row, an odd number of them over waves of two, the longest
+and of the lines to the tile kernel (112 tokens, few experts one of which has more than 48 entries), one weight stage a row, an odd number of them over waves of two, the longest
 rows, rows too long for the LDS (Q8_0: the tile kernel stays), a ragged number of row tiles per workgroup."""
 import pytest
 
@@ -21,3 +21,14 @@ def test_shared_expert_few_tokens(dev, sh, n, k, n_exp, dim, inter):
     y, same = run_gpu(c, n % 2 == 1)
     err_h, err_f, _ = check(c, y, 0, n % 2 == 1)
     assert same and err_h <= 1e-3 and err_f <= 5e-3  # the bounds of test_moe_prefill_gpu.py (the reference's)
+
+
+@pytest.mark.parametrize("sh,n,k,n_exp,kind", [(O.Q6_K, 112, 1, 4, "zipf:0"), (O.Q8_0, 112, 2, 6, "zipf:0"), (O.Q6_K, 48, 2, 3, "popular"),
+                                               (O.Q6_K, 49, 2, 3, "popular"), (O.Q8_0, 49, 2, 3, "popular")], ids=lambda v: None)
+def test_both_sides_of_a_crowded_expert(dev, sh, n, k, n_exp, kind):
+    c = build(O.IQ1_S, O.IQ2_XXS, sh, n, k, n_exp, True, kind, 1024, 768)
+    entries = [b - a for a, b in zip(c["offs"], c["offs"][1:])]
+    assert (max(entries) > 48) == (n == 49)
+    y, same = run_gpu(c)
+    err_h, err_f, _ = check(c, y, 0, False)
+    assert same and err_h <= 1e-3 and err_f <= 5e-3
