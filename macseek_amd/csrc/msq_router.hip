@@ -362,6 +362,12 @@ __global__ __launch_bounds__(1024) void route_lists_kernel(const int* __restrict
   }
 }
 
+// Up to 1024 tokens the chain of a wave bounds the launch: an expert a thread. Beyond, the double-precision arithmetic of all of
+// them, and a wave per token has fewer reductions, but 64 experts are one wave either way. A wave per token / an expert a thread,
+// us: 384 experts, 2 tokens 8.0 / 4.4, 37 8.6 / 4.6, 512 8.9 / 6.1, 1024 9.2 / 7.8, 2048 11.5 / 13.0; 128, 37 tokens 5.8 / 4.3, 4096 9.9 / 9.7,
+// 6000 13.0 / 13.7, 16384 27.5 / 29.5; 64, 4096 tokens 8.4 / 7.8, 262144 298 / 254. (A launch holds fewer than 2^32 threads: 64 a token of
+// either form here, where 128 would halve the tokens that a call can have.)
+bool topk_wide(int n_tokens, int n_exp) { return n_tokens <= 1024 || n_exp <= 64 || (n_exp <= 128 && n_tokens <= 4096); }
 bool exp_ok(int n_exp) { return n_exp >= 64 && n_exp <= 64 * kMaxEpl && n_exp % 64 == 0; }
 
 }  // namespace
@@ -371,6 +377,9 @@ using namespace msq;
 
 extern "C" {
 
+// which of its two forms msq_router_topk takes (for tests)
+int msq_test_router_topk_wide(int n_tokens, int n_exp) { return topk_wide(n_tokens, n_exp) ? 1 : 0; }
+
 int msq_router_topk(void* stream, const MsqBuffer* logits, const MsqBuffer* bias, const MsqBuffer* ids, const MsqBuffer* w,
                     int n_tokens, int n_exp, float route_scale) {
   if (!exp_ok(n_exp) || n_tokens < 0) return unsupported("router_topk", MSQ_F32, n_tokens, n_exp);
@@ -378,10 +387,7 @@ int msq_router_topk(void* stream, const MsqBuffer* logits, const MsqBuffer* bias
   if (!buf_ok(logits, (size_t)n_tokens * n_exp * 4) || !buf_ok(bias, (size_t)n_exp * 4) ||
       !buf_ok(ids, (size_t)n_tokens * kTopK * 4) || !buf_ok(w, (size_t)n_tokens * kTopK * 4))
     return fail(MSQ_ERR_ARGUMENT, "macseek quant: router_topk: buffer missing or too small (tokens %d experts %d)", n_tokens, n_exp);
-  // Up to 1024 tokens the chain of a wave bounds the launch: an expert a thread. Beyond, the double-precision arithmetic of all of
-  // them, and a wave per token has fewer reductions; with up to 128 experts there is nothing in it. A wave per token / an expert a
-  // thread, us: 384 experts, 2 tokens 8.0 / 4.4, 37 8.6 / 4.6, 512 8.9 / 6.1, 1024 9.2 / 7.8, 2048 11.5 / 13.0; 128, 37 tokens 5.8 / 4.3, 4096 10.2 / 9.8.
-  if (n_tokens <= 1024 || n_exp <= 128)
+  if (topk_wide(n_tokens, n_exp))
     hipLaunchKernelGGL(router_topk_wide_kernel, dim3((unsigned)n_tokens), dim3((unsigned)n_exp), 0, (hipStream_t)stream, (const float*)bptr(logits),
                        (const float*)bptr(bias), (int*)bptr_mut(ids), (float*)bptr_mut(w), (uint32_t)n_exp, route_scale);
   else hipLaunchKernelGGL(router_topk_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
