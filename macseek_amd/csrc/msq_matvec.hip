@@ -56,7 +56,9 @@ __global__ __launch_bounds__(1024) void bw_probe_kernel(const uint4* __restrict_
 namespace {
 
 // Launch shape of the decode matvec. units = cols / UNIT columns-slices per row; a wave covers 64 * iters of them.
-struct MvShape { int iters, ks, rw, rpw, unit; int per_cu = 1; bool stage_w = false, free_shape = false; };  // per_cu: persistent workgroups per CU, stage_w: weight rows through LDS (mv_tok_kernel), free_shape: no part of the shape was imposed by the caller
+// per_cu: persistent workgroups per CU (own_per_cu: not imposed by MSQ_MV_WGS), stage_w: weight rows through LDS (mv_tok_kernel), free_shape:
+// no part of the shape was imposed by the caller
+struct MvShape { int iters, ks, rw, rpw, unit; int per_cu = 1; bool stage_w = false, free_shape = false, own_per_cu = true; };
 
 int mv_unit(int t) { return msq_type_block_elems(t) == 1 ? 8 : 32; }
 
@@ -222,7 +224,7 @@ bool mv_tok_shape(int t, int rows, int cols, int groups, int n, int token_groups
   // per CU. Measured, one / two workgroups: Q6_K 129280x5120 165 / 132 us, Q6_K 25600x6144 43.6 / 29.9, F16 5120x5120
   // 13.7 / 11.2, BF16 4096x1280 6.75 / 5.2; the block formats between 5 and 35 MB lose up to 1.5 us with two.
   const bool table = t == MSQ_IQ1_S || t == MSQ_IQ2_XXS;
-  static const int env_wgs = env_knob_early("MSQ_MV_WGS", 0);
+  static const int env_wgs = env_knob_early("MSQ_MV_WGS", 0);  // imposes the number for every call of one token
   const bool free_shape = !(cfg && (cfg->nr > 0 || cfg->rsg > 0 || cfg->ks > 0));
   const double bytes = (double)msq_type_row_bytes(t, cols) * rows;
   const bool two = !table && (bytes >= 48e6 || (unit == 8 && bytes >= 8e6));
@@ -244,7 +246,7 @@ bool mv_tok_shape(int t, int rows, int cols, int groups, int n, int token_groups
   static const int env_sw = env_knob_early("MSQ_MV_STAGEW", -1);
   const bool stage_w = n == 1 && free_shape &&
                        (env_sw >= 0 ? env_sw > 0 : (t == MSQ_Q6_K && bytes >= 12e6) || (t == MSQ_Q8_0 && bytes >= 40e6));
-  *s = {iters, ks, rw, rpw, unit, per_cu, stage_w, free_shape};
+  *s = {iters, ks, rw, rpw, unit, per_cu, stage_w, free_shape, env_wgs <= 0};
   return true;
 }
 
@@ -259,50 +261,57 @@ bool tok_serves_single(int t, int rows, int cols, const MvShape& s, const MsqMvC
   return s.rpw >= 2 && (long)rows >= 2L * device_info().cus * s.rw;
 }
 
+// Rows whose units do not fill whole waves: two, four or eight rows are launched as one (mv_tok_kernel, PACK), as few as leave
+// the fewest waves per row. One group, a number of rows that divides, a row's units a multiple of 8 (several tokens: two rows, 16).
+// Measured, rows one by one (512 and 5120 columns, and all of 7168: in pairs at most) / packed: Q6_K 32768 rows of 256 columns 2.0 times
+// the speed, 512 7.57 / 6.05 us, 768 10.84 / 7.39, 1280 11.64 / 10.57, 1536 12.13 / 10.87, 129280x5120 113.2 / 99.8, 1536x7168 6.41 / 6.10;
+// Q8_0 32768x512 7.01 / 5.93, 2304x5120 6.67 / 6.52; over 8000 random matrices of the K-quants, Q8_0, BF16 and F32 0.97 to 2.1. More than two
+// rows for an eighth fewer waves or less gain nothing (3328 columns 0.96 to 1.06), nor do five waves a workgroup where there are
+// not four packed rows for each (2304x2304 0.95), nor rows of 2304 columns below 6 MB (0.94 to 0.97); the codebook formats, bound by their
+// lookups, lose 1 % and keep the one-row form. MSQ_MV_PAIR = 0 / 2: never / every format.
+// Under a fused norm likewise, but for Q8_0 below 20 MB (2560, 4608, 5120 and 7168 columns, one by one over in pairs: 6 to 18 MB
+// 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04). A row's bits are the same packed or not, so the rule is free to differ.
+//
+// Five waves a workgroup leave the SIMDs unequal work: K-quants take two of them per CU from 16 MB on (2560 and 5120 columns, one / two:
+// 12 MB 0.95 to 1.03, 16 MB 1.02 to 1.06, 26 MB 1.10 to 1.17, 44 MB 1.17 to 1.24), under a norm of two trips from 26 MB on (1.03 to
+// 1.12; Q6_K 20 MB 0.93); Q8_0 does not (0.69 to 0.92 up to 34 MB). Unless MSQ_MV_WGS names a number.
+template <class D, int T>
+int packed_rows(const MvArgs& a, MvShape& s) {
+  static const int env_pair = env_knob_early("MSQ_MV_PAIR", -1);
+  const double bytes = (double)a.rows * a.row_bytes;
+  const int u = (int)(a.cols / D::UNIT), cus = device_info().cus;
+  constexpr bool q8 = std::is_same_v<D, DecQ8_0>, kq = std::is_same_v<D, DecQ6KQ> || std::is_same_v<D, DecQ5KQ>;
+  auto waves = [&](int p) { return (p * u + 63) / 64; };
+  int pack = 1;
+  if (s.iters == 1 && s.free_shape && (D::LDS_WORDS == 0 || env_pair == 2) && env_pair != 0 && a.rows_per_group >= a.rows &&
+      !(a.norm_w && q8 && bytes < 20e6) && u % (T == 1 && D::LDS_WORDS == 0 ? 8 : 16) == 0)
+    for (int p = 2; p <= (T == 1 ? 8 : 2); p *= 2)
+      if (a.rows % p == 0 && waves(p) <= 8 && (u % 16 == 0 || bytes >= (q8 ? 20e6 : u < 64 ? 0. : 6e6)) && waves(p) * pack < waves(pack) * p &&
+          (p == 2 || (8 * waves(p) < 7 * p * waves(1) && (waves(p) != 5 || (long)a.rows >= 4L * p * cus))))
+        pack = p;
+  if (kq && s.own_per_cu && pack > 1 && waves(pack) == 5 && bytes >= (a.norm_w ? 26e6 : 16e6) &&
+      !(a.norm_w && norm_of_tok<D>(a.cols, bytes) == kNormOneTrip))
+    s.per_cu = 2;
+  return pack;
+}
+
 template <class D, int T>
 int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   MvTokArgs ta = ta_;  // (the launch may reshape rows into pairs: the caller's arguments stay as they are)
   MvArgs& a = ta.m;
   MvShape s = s_;
-  // Rows whose units do not fill whole waves: two, four or eight rows are launched as one (mv_tok_kernel, PACK), as few as leave
-  // the fewest waves per row. One group, a number of rows that divides, a row's units a multiple of 8 (several tokens: two rows, 16).
-  // Measured, rows one by one (512 and 5120 columns, and all of 7168: in pairs at most) / packed: Q6_K 32768 rows of 256 columns 2.0 times
-  // the speed, 512 7.57 / 6.05 us, 768 10.84 / 7.39, 1280 11.64 / 10.57, 1536 12.13 / 10.87, 129280x5120 113.2 / 99.8, 1536x7168 6.41 / 6.10;
-  // Q8_0 32768x512 7.01 / 5.93, 2304x5120 6.67 / 6.52; over 8000 random matrices of the K-quants, Q8_0, BF16 and F32 0.97 to 2.1. More than two
-  // rows for an eighth fewer waves or less gain nothing (3328 columns 0.96 to 1.06), nor do five waves a workgroup where there are
-  // not four packed rows for each (2304x2304 0.95), nor rows of 2304 columns below 6 MB (0.94 to 0.97); the codebook formats, bound by their lookups, lose 1 % and keep the one-row
-  // form. MSQ_MV_PAIR = 0 / 2: never / every format.
-  // Under a fused norm likewise, but for Q8_0 below 20 MB (2560, 4608, 5120 and 7168 columns, one by one over in pairs: 6 to 18 MB
-  // 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04). A row's bits are the same packed or not, so the rule is free to differ.
   const double bytes = (double)a.rows * a.row_bytes;
-  int pack = 1;
-  {
-    static const int env_pair = env_knob_early("MSQ_MV_PAIR", -1);
-    const int u = (int)(a.cols / D::UNIT), cus = device_info().cus;
-    constexpr bool q8 = std::is_same_v<D, DecQ8_0>;
-    auto waves = [&](int p) { return (p * u + 63) / 64; };
-    if (s.iters == 1 && s.free_shape && (D::LDS_WORDS == 0 || env_pair == 2) && env_pair != 0 && a.rows_per_group >= a.rows &&
-        !(a.norm_w && q8 && bytes < 20e6) && u % (T == 1 && D::LDS_WORDS == 0 ? 8 : 16) == 0)
-      for (int p = 2; p <= (T == 1 ? 8 : 2); p *= 2)
-        if (a.rows % p == 0 && waves(p) <= 8 && (u % 16 == 0 || bytes >= (q8 ? 20e6 : u < 64 ? 0. : 6e6)) && waves(p) * pack < waves(pack) * p &&
-            (p == 2 || (8 * waves(p) < 7 * p * waves(1) && (waves(p) != 5 || (long)a.rows >= 4L * p * cus))))
-          pack = p;
-    // Five waves a workgroup leave the SIMDs unequal work: K-quants take two of them per CU from 16 MB on (2560 and 5120 columns, one / two:
-    // 12 MB 0.95 to 1.03, 16 MB 1.02 to 1.06, 26 MB 1.10 to 1.17, 44 MB 1.17 to 1.24), under a norm of two trips from 26 MB on (1.03 to
-    // 1.12; Q6_K 20 MB 0.93); Q8_0 does not (0.69 to 0.92 up to 34 MB).
-    constexpr bool kq = std::is_same_v<D, DecQ6KQ> || std::is_same_v<D, DecQ5KQ>;
-    if (kq && pack > 1 && waves(pack) == 5 && bytes >= (a.norm_w ? 26e6 : 16e6) && !(a.norm_w && norm_of_tok<D>(a.cols, bytes) == kNormOneTrip)) s.per_cu = 2;
-    if (pack > 1) {
-      a.pack = pack;
-      a.pack_units = u;
-      a.rows /= pack;
-      a.rows_per_group = a.rows;
-      a.row_bytes *= pack;
-      s.ks = (pack * u + 63) / 64;
-      s.rw = std::max(1, 8 / s.ks);
-      const long wgs = std::max<long>(1, s.per_cu * device_info().cus / (((long)ta.n + T - 1) / T));
-      s.rpw = (int)std::min<long>(32, std::max<long>(1, (a.rows + wgs * s.rw - 1) / (wgs * s.rw)));
-    }
+  const int pack = packed_rows<D, T>(a, s), u = (int)(a.cols / D::UNIT);
+  if (pack > 1) {
+    a.pack = pack;
+    a.pack_units = u;
+    a.rows /= pack;
+    a.rows_per_group = a.rows;
+    a.row_bytes *= pack;
+    s.ks = (pack * u + 63) / 64;
+    s.rw = std::max(1, 8 / s.ks);
+    const long wgs = std::max<long>(1, s.per_cu * device_info().cus / (((long)ta.n + T - 1) / T));
+    s.rpw = (int)std::min<long>(32, std::max<long>(1, (a.rows + wgs * s.rw - 1) / (wgs * s.rw)));
   }
   const bool sums8 = pack > 1 && a.pack_units % 16;
   const int threads = 64 * s.rw * s.ks;
@@ -405,6 +414,20 @@ int launch_mv_tok_t(hipStream_t st, int t, const MvShape& s, MvTokArgs& ta) {
   return MSQ_ERR_UNSUPPORTED;
 }
 
+// rows launched as one and workgroups per CU of a one-token call (0: not through mv_tok_kernel)
+template <class D>
+int tok_launch_of(int t, int rows, int cols, bool norm, int* per_cu) {
+  MvShape s;
+  if (!mv_tok_shape(t, rows, cols, 1, 1, 1, nullptr, &s) || !tok_serves_single(t, rows, cols, s, nullptr)) return 0;
+  const float w = 0.f;
+  MvArgs a{};
+  a.rows = a.rows_per_group = (uint32_t)rows; a.cols = (uint32_t)cols; a.row_bytes = (uint32_t)msq_type_row_bytes(t, cols);
+  a.norm_w = norm ? &w : nullptr;
+  const int pack = packed_rows<D, 1>(a, s);
+  *per_cu = s.per_cu;
+  return pack;
+}
+
 bool mv_type_ok(int t) {
   switch (t) {
     case MSQ_F32: case MSQ_F16: case MSQ_BF16: case MSQ_Q8_0: case MSQ_Q5_K: case MSQ_Q6_K: case MSQ_IQ1_S:
@@ -499,6 +522,17 @@ int msq_matvec_cfg(int t, int rows, int cols, MsqMvCfg* out) {
   if (!tok && !mv_shape(t, rows, cols, 1, cfg, &s)) return unsupported("matvec_cfg", t, rows, cols);
   out->nr = s.rpw; out->rsg = s.rw; out->ks = s.ks;
   return MSQ_OK;
+}
+
+// for tests: what tok_launch_of says of the types whose rows are packed
+int msq_test_matvec_pack(int t, int rows, int cols, int norm, int* per_cu) {
+  switch (t) {
+    case MSQ_Q6_K: return tok_launch_of<DecQ6KQ>(t, rows, cols, norm != 0, per_cu);
+    case MSQ_Q5_K: return tok_launch_of<DecQ5KQ>(t, rows, cols, norm != 0, per_cu);
+    case MSQ_Q8_0: return tok_launch_of<DecQ8_0>(t, rows, cols, norm != 0, per_cu);
+    case MSQ_BF16: return tok_launch_of<DecDense<MSQ_BF16>>(t, rows, cols, norm != 0, per_cu);
+    default: return 0;
+  }
 }
 
 // msq_matvec and msq_matvec_rmsnorm (norm_w != nullptr: the activations are normalized on the way in; the kernel is the
