@@ -25,10 +25,10 @@ def sources():
 # Per-file additions. The one-token MoE kernels take the expert address table as their first argument and have it
 # delivered in scalar registers with the wave (kernel-argument preload): the table can be read while the rest of the
 # arguments is still on its way from memory.
-# The token matvec kernel takes what its first loads need (activations, then weight rows) as twelve leading words in the
+# The token matvec kernel takes what its first loads need (activations, then weight rows) as thirteen leading words in the
 # same way.
 EXTRA = {"msq_moe.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=2"],
-         "msq_matvec.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=12"],
+         "msq_matvec.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=13"],
          "msq_router.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=6"],  # x, W, dim, n_exp of the fused router: 11.1 -> 10.8 us
          "msq_matmul.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=14"]}  # the fused matmul's arguments: 2-3 % at 64 / 128 tokens
 

@@ -357,7 +357,7 @@ __device__ __forceinline__ void copy_words16(uint32_t* dst, const uint32_t* src,
 }
 
 
-// floor(a / b) for a < 4096 and 0 < b <= 64 (or a < 512 and b <= 256: at least 1 / 512 away, error below 1 / 65536) in four instructions instead of the forty of an integer division (wave
+// floor(a / b) for a < 4096 and 0 < b <= 64 in four instructions instead of the forty of an integer division (wave
 // counts and rows of a chunk): (a + 0.5) / b lies at least 1 / 128 away from every integer, and the float product is
 // within 1 / 1024 of it.
 __device__ __forceinline__ uint32_t small_div(uint32_t a, uint32_t b) {

@@ -265,12 +265,15 @@ bool tok_serves_single(int t, int rows, int cols, const MvShape& s, const MsqMvC
 // the fewest waves per row. One group, a number of rows that divides, a row's units a multiple of 8 (several tokens: two rows, 16).
 // Measured, rows one by one (512 and 5120 columns, and all of 7168: in pairs at most) / packed: Q6_K 32768 rows of 256 columns 2.0 times
 // the speed, 512 7.57 / 6.05 us, 768 10.84 / 7.39, 1280 11.64 / 10.57, 1536 12.13 / 10.87, 129280x5120 113.2 / 99.8, 1536x7168 6.41 / 6.10;
-// Q8_0 32768x512 7.01 / 5.93, 2304x5120 6.67 / 6.52; over 8000 random matrices of the K-quants, Q8_0, BF16 and F32 0.97 to 2.1. More than two
+// Q8_0 32768x512 7.01 / 5.93, 2304x5120 6.67 / 6.52; over 19000 random matrices of the K-quants, Q8_0, BF16 and F32 0.96 to 2.1, below 0.975 in
+// one of a thousand (under a norm Q6_K 2304x11000 and 2816x7500, Q5_K 1536x15000, and Q6_K pairs of 512 columns from the caches). More than two
 // rows for an eighth fewer waves or less gain nothing (3328 columns 0.96 to 1.06), nor do five waves a workgroup where there are
-// not four packed rows for each (2304x2304 0.95), nor rows of 2304 columns below 6 MB (0.94 to 0.97); the codebook formats, bound by their
-// lookups, lose 1 % and keep the one-row form. MSQ_MV_PAIR = 0 / 2: never / every format.
+// not four packed rows for each (2304x2304 0.95), nor rows of 2304 columns below 6 MB (0.94 to 0.97), nor four short rows of Q8_0 where
+// they make the waves' runs two long and pairs would make them three (512 columns, 8193 to 12288 rows 0.95 to 0.97, on either side 1.01 to
+// 1.03); the codebook formats, bound by their lookups, lose 1 % and keep the one-row form. MSQ_MV_PAIR = 0 / 2: never / every format.
 // Under a fused norm likewise, but for Q8_0 below 20 MB (2560, 4608, 5120 and 7168 columns, one by one over in pairs: 6 to 18 MB
-// 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04). A row's bits are the same packed or not, so the rule is free to differ.
+// 0.97 to 1.02 and once 1.07, 22 to 45 MB 1.00 to 1.04) and Q5_K rows of 2304 and 2816 columns below 12 MB (0.95 to 0.98). A row's bits are
+// the same packed or not, so the rule is free to differ.
 //
 // Five waves a workgroup leave the SIMDs unequal work: K-quants take two of them per CU from 16 MB on (2560 and 5120 columns, one / two:
 // 12 MB 0.95 to 1.03, 16 MB 1.02 to 1.06, 26 MB 1.10 to 1.17, 44 MB 1.17 to 1.24), under a norm of two trips from 26 MB on (1.03 to
@@ -282,13 +285,16 @@ int packed_rows(const MvArgs& a, MvShape& s) {
   const int u = (int)(a.cols / D::UNIT), cus = device_info().cus;
   constexpr bool q8 = std::is_same_v<D, DecQ8_0>, kq = std::is_same_v<D, DecQ6KQ> || std::is_same_v<D, DecQ5KQ>;
   auto waves = [&](int p) { return (p * u + 63) / 64; };
+  const double bytes8 = q8 ? 20e6 : u < 64 ? 0. : a.norm_w && std::is_same_v<D, DecQ5KQ> ? 12e6 : 6e6;  // sums of eight lanes from here on
   int pack = 1;
   if (s.iters == 1 && s.free_shape && (D::LDS_WORDS == 0 || env_pair == 2) && env_pair != 0 && a.rows_per_group >= a.rows &&
       !(a.norm_w && q8 && bytes < 20e6) && u % (T == 1 && D::LDS_WORDS == 0 ? 8 : 16) == 0)
-    for (int p = 2; p <= (T == 1 ? 8 : 2); p *= 2)
-      if (a.rows % p == 0 && waves(p) <= 8 && (u % 16 == 0 || bytes >= (q8 ? 20e6 : u < 64 ? 0. : 6e6)) && waves(p) * pack < waves(pack) * p &&
+    for (int p = 2; p <= (T == 1 ? 8 : 2); p *= 2) {
+      if (q8 && p == 4 && waves(4) == 1 && (long)a.rows > 32L * cus && (long)a.rows <= 48L * cus) break;  // (eight waves a workgroup, one a CU)
+      if (a.rows % p == 0 && waves(p) <= 8 && (u % 16 == 0 || bytes >= bytes8) && waves(p) * pack < waves(pack) * p &&
           (p == 2 || (8 * waves(p) < 7 * p * waves(1) && (waves(p) != 5 || (long)a.rows >= 4L * p * cus))))
         pack = p;
+    }
   if (kq && s.own_per_cu && pack > 1 && waves(pack) == 5 && bytes >= (a.norm_w ? 26e6 : 16e6) &&
       !(a.norm_w && norm_of_tok<D>(a.cols, bytes) == kNormOneTrip))
     s.per_cu = 2;
@@ -303,8 +309,6 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   const double bytes = (double)a.rows * a.row_bytes;
   const int pack = packed_rows<D, T>(a, s), u = (int)(a.cols / D::UNIT);
   if (pack > 1) {
-    a.pack = pack;
-    a.pack_units = u;
     a.rows /= pack;
     a.rows_per_group = a.rows;
     a.row_bytes *= pack;
@@ -313,7 +317,7 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
     const long wgs = std::max<long>(1, s.per_cu * device_info().cus / (((long)ta.n + T - 1) / T));
     s.rpw = (int)std::min<long>(32, std::max<long>(1, (a.rows + wgs * s.rw - 1) / (wgs * s.rw)));
   }
-  const bool sums8 = pack > 1 && a.pack_units % 16;
+  const bool sums8 = pack > 1 && u % 16;
   const int threads = 64 * s.rw * s.ks;
   const int tile_rows = s.rw * s.rpw;
   a.units = pack * (a.cols / D::UNIT);
@@ -345,7 +349,7 @@ int launch_mv_tok(hipStream_t st, const MvShape& s_, const MvTokArgs& ta_) {
   }
   auto launch = [&](auto kernel, dim3 grid) {
     allow_large_lds(kernel, lds);
-    hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a.W, a.rows, a.row_bytes, a.units, a.ks, a.rpw, a.ntiles, a.rows_per_group, a.x, a.cols, ta);
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), lds, st, a.W, a.rows, a.row_bytes, a.units, a.ks, a.rpw, a.ntiles, a.rows_per_group, a.x, a.cols, (uint32_t)threads, ta);
   };
   // persistent workgroups, one per CU over all token groups (two for a large matrix: MvShape::per_cu)
   // A fused norm's prologue of one trip leaves Q5_K, Q6_K rows in registers (144) and two units of F32 no room for a second one:

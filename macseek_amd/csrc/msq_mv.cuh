@@ -32,7 +32,6 @@ struct MvArgs {
   // (xlds_words(cols) words), and whether the plain kernels stage at all (rows too long for LDS are read directly)
   uint32_t xs_off;
   uint32_t stage_x;
-  uint32_t pack, pack_units;  // token kernel, PACK: rows of the matrix in a launched row, units of each
   uint32_t w_off;     // word offset in dynamic LDS of the waves' weight-row buffers (token kernel, one token of a block format)
 };
 
@@ -534,13 +533,13 @@ __device__ __forceinline__ void wait_rows_n(int n) {
 template <class D, int ITERS, int T, int NORM = kNormNone, bool SW = false, int PACK = 0>
 __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t rows_, uint32_t row_bytes_, uint32_t units_, uint32_t ks_,
                                                      uint32_t rpw_, uint32_t ntiles_, uint32_t rows_per_group_, const float* x_,
-                                                     uint32_t cols_, const MvTokArgs ta) {
+                                                     uint32_t cols_, uint32_t threads_, const MvTokArgs ta) {
   constexpr bool STAGE = tok_stages_x<D, T>();
   constexpr bool STAGE_W = SW && tok_stages_w<D, ITERS, T>();  // weight rows through LDS: the launch's choice (large matrices)
   constexpr int WL = STAGE_W ? (int)wspan_loads<D>() : 1;
-  // What the first loads need comes as leading arguments (W_ .. cols_: the fields of the same names in ta.m, delivered
-  // in scalar registers with the wave when the file is built with kernel-argument preload) and is used under those
-  // names below; the rest is read from the argument block.
+  // What the first loads need comes as leading arguments (W_ .. cols_: the fields of the same names in ta.m, and threads_, which is
+  // blockDim.x, whose place behind the argument block is a trip to memory away), delivered in scalar registers with the wave when
+  // the file is built with kernel-argument preload, and is used under those names below; the rest is read from the argument block.
   const MvArgs& a = ta.m;
   extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
   // the codebook table is a static array: its LDS address is a compile-time constant, which saves the addition of a base
@@ -549,7 +548,7 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
   constexpr uint32_t SUMS = PACK == 8 ? 8 : 4;  // of a wave: 8 or 16 lanes each
   float* part = (float*)smem;  // [row of tile][ks][SUMS][T]
 
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, nwaves = blockDim.x >> 6;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, nwaves = threads_ >> 6;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   // (the quotients come from the vector unit: brought back to scalar registers, the wave's row offsets are scalar too)
   const uint32_t KS = ks_, rw = (uint32_t)__builtin_amdgcn_readfirstlane((int)small_div(wave, KS)), ks = wave - rw * KS;
@@ -565,13 +564,13 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
   [[maybe_unused]] bool early = false;
   if constexpr (EARLY_X) {
     const uint32_t n4 = cols_ >> 2;
-    early = blockIdx.y == 0 && rows_per_group_ >= rows_ && n4 <= XK * blockDim.x;
+    early = blockIdx.y == 0 && rows_per_group_ >= rows_ && n4 <= XK * threads_;
     if (early) {
 #pragma unroll
-      for (int k = 0; k < XK; k++) xe[k] = ((const u32x4*)x_)[min(tid + k * blockDim.x, n4 - 1u)];
+      for (int k = 0; k < XK; k++) xe[k] = ((const u32x4*)x_)[min(tid + k * threads_, n4 - 1u)];
     }
   }
-  D::fill_lds(tbl, (int)tid, (int)blockDim.x);
+  D::fill_lds(tbl, (int)tid, (int)threads_);
 
   uint32_t unit[ITERS];
   bool valid[ITERS];
@@ -581,9 +580,18 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
     valid[i] = u < units_;
     unit[i] = valid[i] ? u : units_ - 1;  // idle lanes shadow the last unit; their result is dropped
   }
+  // PACK: the units of one of the rows, and how many rows (as a power of two) there are, from what came in registers: read from the argument
+  // block they are a trip to memory ahead of the sums (this and threads_: Q8_0 9424x512 4.39 -> 4.19 us, Q6_K 32768x1280 9.89 -> 9.59)
+  [[maybe_unused]] const uint32_t pu = cols_ / D::UNIT, sh = units_ >= 8u * pu ? 3u : units_ >= 4u * pu ? 2u : 1u;
   uint32_t xu[ITERS];  // the unit of the activations that goes with unit[i] (every row of a packed one: the same columns again)
 #pragma unroll
-  for (int i = 0; i < ITERS; i++) xu[i] = PACK ? unit[i] - a.pack_units * small_div(unit[i], a.pack_units) : unit[i];
+  for (int i = 0; i < ITERS; i++) {
+    xu[i] = unit[i];
+    if constexpr (PACK) {  // (mod pu: below zero wraps to a large number)
+#pragma unroll
+      for (uint32_t m = 4u; m > 0u; m >>= 1) xu[i] = min(xu[i], xu[i] - m * pu);
+    }
+  }
   typename D::X xr[T][ITERS];
   uint32_t cur_group = 0xFFFFFFFFu;
   float* xs = (float*)(smem + a.xs_off);
@@ -676,7 +684,7 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
         if (early && cur_group == 0xFFFFFFFFu) {  // (group 0, token 0: the row requested at the top)
 #pragma unroll
           for (int k = 0; k < XK; k++) {
-            const uint32_t i = tid + k * blockDim.x;
+            const uint32_t i = tid + k * threads_;
             if (i < (cols_ >> 2)) *(u32x4*)(xs + 4u * i + (i >> 3) * 4u) = xe[k];
           }
           __syncthreads();
@@ -703,7 +711,7 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
             const float* src[G];
 #pragma unroll
             for (int k = 0; k < G; k++) src[k] = x_of(t + k);
-            stage_x_rows<G>(xs, src, G, roww, cols_, tid, blockDim.x);
+            stage_x_rows<G>(xs, src, G, roww, cols_, tid, threads_);
             __syncthreads();
           }
 #pragma unroll
@@ -772,19 +780,19 @@ __global__ __launch_bounds__(512) void mv_tok_kernel(const uint8_t* W_, uint32_t
     for (; j0 + NR < rpw_; j0 += NR) round.template operator()<true>(j0);
     round.template operator()<false>(j0);
     __syncthreads();
-    if constexpr (PACK) {  // packed row r / pack, its sums pack_units / PACK of each row
-      const uint32_t G = a.pack_units / PACK, sh = (uint32_t)__builtin_ctz(a.pack), n = tile_rows << sh;
-      for (uint32_t idx = tid; idx < n * T; idx += blockDim.x) {
+    if constexpr (PACK) {  // packed row r >> sh, its sums pu / PACK of each row
+      const uint32_t G = pu / PACK, n = tile_rows << sh;
+      for (uint32_t idx = tid; idx < n * T; idx += threads_) {
         const uint32_t r = T == 1 ? idx : idx % n, t = T == 1 ? 0u : idx / n, row = (tile_row0 << sh) + r;
         if (row < rows_ << sh && t0 + t < ta.n) {
-          const float* sums = part + ((r >> sh) * SUMS * KS + (r & (a.pack - 1u)) * G) * T + t;
+          const float* sums = part + ((r >> sh) * SUMS * KS + (r & ((1u << sh) - 1u)) * G) * T + t;
           const float s = PACK == 8 ? sum_pairs_in_order(sums, G) : sum_in_order(sums, G, T);  // (eight lanes: one token)
           float* y = a.y + (size_t)(t0 + t) * ta.y_stride + row;
           *y = a.accumulate ? *y + s : s;
         }
       }
     } else
-    for (uint32_t idx = tid; idx < tile_rows * T; idx += blockDim.x) {
+    for (uint32_t idx = tid; idx < tile_rows * T; idx += threads_) {
       const uint32_t r = idx % tile_rows, t = idx / tile_rows, row = tile_row0 + r;  // consecutive lanes: consecutive rows
       if (row < rows_ && t0 + t < ta.n) {
         const float s = sum_in_order(part + r * 4 * KS * T + t, 4 * KS, T);

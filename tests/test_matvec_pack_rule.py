@@ -12,6 +12,9 @@ CASES = [  # (type, rows, cols, norm): (rows as one, workgroups per CU); 0 rows:
     ((O.Q6_K, 4096, 5120, 0), (2, 2)), ((O.Q6_K, 3000, 5120, 0), (2, 1)), ((O.Q6_K, 4097, 5120, 0), (1, 1)), ((O.Q6_K, 4096, 5120, 1), (2, 1)),
     ((O.Q5_K, 6144, 2304, 0), (4, 1)), ((O.Q5_K, 3000, 2304, 0), (1, 1)), ((O.Q8_0, 20000, 1280, 0), (8, 1)), ((O.Q8_0, 8192, 1280, 0), (1, 1)),
     ((O.Q8_0, 4096, 5120, 1), (2, 1)), ((O.Q8_0, 2304, 5120, 1), (1, 1)), ((O.BF16, 512, 1280, 0), (0, 0)),
+    ((O.Q8_0, 8192, 512, 0), (4, 1)), ((O.Q8_0, 8196, 512, 0), (2, 1)), ((O.Q8_0, 12288, 512, 0), (2, 1)), ((O.Q8_0, 12292, 512, 0), (4, 1)),
+    ((O.Q6_K, 8196, 512, 0), (4, 1)), ((O.Q5_K, 7000, 2304, 1), (1, 1)), ((O.Q5_K, 7600, 2304, 1), (4, 1)), ((O.Q5_K, 7000, 2304, 0), (4, 1)),
+    ((O.Q6_K, 7000, 2304, 1), (4, 1)),
 ]
 
 
