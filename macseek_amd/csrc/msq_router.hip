@@ -87,20 +87,19 @@ __device__ __forceinline__ void select6(float (&key)[kMaxEpl], const double (&sc
   }
 }
 
-// A workgroup of up to eight waves selects the top six of one token, one expert a thread (key -inf: none, or not comparable) and writes ids
-// and weights; after(any): by one thread, behind the barrier; any (WAITS): a thread came with `missing`, which makes all six weights NaN.
+// A workgroup of `waves` waves, up to eight, selects the top six of one token, one expert a thread (key -inf: none, or not comparable) and writes ids
+// and weights; after(): by one thread, behind the barrier.
 // Selection in two levels: each wave picks the six best of its 64 experts, one a lane, and leaves them in LDS; wave 0 picks
 // the six best of those 48. The six best overall are among the six best of their waves, and "greater key, then lower expert
 // id" is a total order: experts, and the candidates that a wave leaves, stand in the lanes in the order of their ids where keys
 // are equal, so the first lane with the greatest key is the choice. NaN and -inf are never chosen.
-template <bool WAITS, class After>
-__device__ __forceinline__ void select6_of_block(float key, double sc, bool missing, uint32_t tid, float route_scale, int* __restrict__ ids,
+template <class After>
+__device__ __forceinline__ void select6_of_block(float key, double sc, uint32_t tid, uint32_t waves, float route_scale, int* __restrict__ ids,
                                                float* __restrict__ wts, After after) {
   constexpr uint32_t WAVES = 8;
   __shared__ float c_key[WAVES * kTopK];
   __shared__ int c_id[WAVES * kTopK];
   __shared__ double c_sc[WAVES * kTopK];
-  [[maybe_unused]] __shared__ uint32_t c_missing[WAVES];
   const uint32_t lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
 #pragma unroll
   for (int k = 0; k < kTopK; k++) {
@@ -114,22 +113,16 @@ __device__ __forceinline__ void select6_of_block(float key, double sc, bool miss
       key = -INFINITY;
     }
   }
-  if constexpr (WAITS) {
-    const uint64_t lacks = __builtin_amdgcn_ballot_w64(missing);
-    if (lane == 0) c_missing[wave] = lacks != 0;
-  }
   __syncthreads();
   if (wave != 0) return;
-  bool any = false;
-  if constexpr (WAITS) any = __builtin_amdgcn_ballot_w64(lane < (blockDim.x >> 6) && c_missing[lane & (WAVES - 1u)] != 0) != 0;
-  if (lane == 0) after(any);
-  const uint32_t candidates = (blockDim.x >> 6) * kTopK;
+  if (lane == 0) after();
+  const uint32_t candidates = waves * kTopK;
   float ck = lane < candidates ? c_key[lane] : -INFINITY;
   const int ce = lane < candidates ? c_id[lane] : 0;
   const uint64_t cs = lane < candidates ? __builtin_bit_cast(uint64_t, c_sc[lane]) : 0;
   int sel_e[kTopK];
   double sel_s[kTopK];
-  double sum = any ? __builtin_nan("") : 0.0;  // the six scores are added in selection order, as the reference adds them
+  double sum = 0.0;  // the six scores are added in selection order, as the reference adds them
 #pragma unroll
   for (int k = 0; k < kTopK; k++) {
     const float m = wave_max_f(ck);
@@ -183,7 +176,7 @@ __global__ __launch_bounds__(512) void router_topk_wide_kernel(const float* __re
     score_key(logits[(size_t)t * n_exp + tid], bias[tid], sc, key);
     if (!(key > -INFINITY)) key = -INFINITY;
   }
-  select6_of_block<false>(key, sc, false, tid, route_scale, ids + (size_t)t * kTopK, wts + (size_t)t * kTopK, [](bool) {});
+  select6_of_block(key, sc, tid, (n_exp + 63u) >> 6, route_scale, ids + (size_t)t * kTopK, wts + (size_t)t * kTopK, [] {});
 }
 
 // Decode: logits = W[n_exp][dim] . x[dim] and the selection in one launch. A workgroup is eight waves, four to an expert's row,
@@ -200,7 +193,7 @@ __global__ __launch_bounds__(512) void router_topk_wide_kernel(const float* __re
 // of the launch, gives up after `polls` reads (kRouterPolls: seconds). Then a workgroup may still be to come that reads the number
 // only after it has been counted up, and its record would pass for one of the next call. So a call that gave up leaves
 // kRouterGaveUp in place of its number: records written under it name no call (0), and this call and all that follow return six NaN
-// weights, until the scratch is zeroed.
+// weights, until the scratch is zeroed. (Should six keys of +inf stand ahead of the missing ones, the choice does not depend on these.)
 constexpr uint32_t kRouterPolls = 1u << 22;
 constexpr uint32_t kRouterGaveUp = 0xFFFFFFFFu;  // (as a number, the last before counting starts again at 1: never left by a call that ended well)
 template <int QT, uint32_t U>
@@ -262,7 +255,6 @@ __global__ __launch_bounds__(512) void router_fused_kernel(const float* __restri
   }
   float key = -INFINITY;
   double sc = 0.0;
-  bool missing = false;
   if (tid < n_exp) {
     const float b = bias[tid];
     uint64_t r = 0;
@@ -270,14 +262,18 @@ __global__ __launch_bounds__(512) void router_fused_kernel(const float* __restri
       r = __hip_atomic_load(recs + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if ((uint32_t)(r >> 32) == number) break;
     }
-    missing = (uint32_t)(r >> 32) != number || number == 0u;
-    const float logit = missing ? __builtin_nanf("") : __builtin_bit_cast(float, (uint32_t)r);
-    score_key(logit, b, sc, key);
+    score_key(__builtin_bit_cast(float, (uint32_t)r), b, sc, key);
     if (!(key > -INFINITY)) key = -INFINITY;
+    if ((uint32_t)(r >> 32) != number || number == 0u) {  // no logit: ahead of every other key, with a score that makes all six weights NaN
+      key = INFINITY;
+      sc = __builtin_nan("");
+      __hip_atomic_store(call, kRouterGaveUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // ahead of the barrier, and so of the number
+    }
   }
-  select6_of_block<true>(key, sc, missing, tid, route_scale, ids, wts, [&](bool any) {
-    const uint32_t left = any ? kRouterGaveUp : number == kRouterGaveUp ? 0u : number;
-    __hip_atomic_store(call, left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  select6_of_block(key, sc, tid, WAVES, route_scale, ids, wts, [&] {  // (the mark is the greatest number: it stays)
+    if (number != kRouterGaveUp) __hip_atomic_fetch_max(call, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else atomicCAS(call, number - 1u, 0u);
   });
 }
 
