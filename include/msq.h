@@ -127,11 +127,13 @@ int msq_f32_to_f16(void* stream, const MsqBuffer* X, const MsqBuffer* X16, size_
 /* reference: ms::q::encode_matmul_h (quant.hpp:43-45, quant.mm:193-238). Prefill matmul
  * Y[n x rows] (+)= X16[n x x_stride] . W^T, X16 fp16 (x_stride = cols if 0), Y F32, any n >= 1, cols % 128 == 0.
  * Weights are rounded to fp16 and products accumulate in fp32, the reference's numerics (quant.hpp:36-39).
- * Calls of little work over Q5_K, Q6_K, IQ4_NL, IQ1_S and IQ2_XXS take a few-token kernel in blocks of sixteen tokens, which
+ * Calls of little work over Q5_K, Q6_K, IQ4_NL, IQ1_S and IQ2_XXS take a few-token kernel in blocks of sixteen or 32 tokens, which
  * allocates nothing and uses no buffer of the library: 17 to 2048 tokens (eight per CU), 257 to 4096 columns, at most 8192
  * rows, and at most 48 pieces of 16 rows x 256 columns x 16 tokens per CU (64 up to 256 tokens and 2048 rows; 32, and 4096
- * rows, up to 512 columns; up to 32 tokens beyond 4096 rows of more than 1024 columns), X on a 16-byte boundary (X16: 8-byte,
- * its stride a multiple of 4). It is left out while MSQ_MM_FUSED_MAX is set, and behind the second fused kernel while one of its bounds
+ * rows, up to 512 columns; up to 32 tokens beyond 4096 rows of more than 1024 columns); and of up to 256 tokens more, mostly those of
+ * 1280 to 8192 columns and 17 to 64 tokens, of any number of rows up to 80 pieces of 16 rows x 256 columns x 32 tokens per CU (which
+ * of them depends on the type and was measured: msq_rows.hip). X on a 16-byte boundary (X16: 8-byte, its stride a multiple of 4).
+ * It is left out while MSQ_MM_FUSED_MAX is set, and behind the second fused kernel while one of its bounds
  * (MSQ_MM_TILE_MIN / _MAX / _ELEMS) is.
  * Others up to 128 tokens (256 on matrices of at most 2048 rows and on Q6_K / Q5_K; MSQ_MM_FUSED_MAX=N in the environment: up
  * to N) are served by a fused kernel: nothing is allocated and the call only enqueues. When the matrix has few tiles K
@@ -273,8 +275,8 @@ size_t msq_moe_prefill_scratch_bytes(int total_entries, int n_tokens, int n_exp,
  * the matrix instructions as fp16 like the reference's tiles (IQ1_S / IQ2_XXS: the sub-block scale is rounded to fp16 and
  * its product with the grid value is rounded again, where the reference rounds the fp32 product once; a Q6_K / Q8_0 shared
  * expert keeps exact payloads and fp32 scales). The call only enqueues
- * (no host copy, no wait, no allocation) and can be captured in a HIP graph. With a shared expert its launches are
- * forked onto a stream that the library owns (one per device, created by msq_init() or by the
+ * (no host copy, no wait, no allocation) and can be captured in a HIP graph. With a shared expert its launches (but for a Q6_K /
+ * Q8_0 expert over up to 112 tokens, whose few-token kernel mostly stays on the caller's stream) are forked onto a stream that the library owns (one per device, created by msq_init() or by the
  * first call outside a capture) and joined back before the reduction, all through events, so the caller
  * sees the ordering of a single stream (MSQ_MOEP_ONE_STREAM=1 in the environment turns the fork off); `offs` (host memory) is read at call time and
  * travels to the device inside kernel arguments. The result is bit-identical from run to run. n_tokens <= 0 returns MSQ_OK and

@@ -263,9 +263,9 @@ bool tok_serves_single(int t, int rows, int cols, const MvShape& s, const MsqMvC
 
 // Rows whose units do not fill whole waves: two, four or eight rows are launched as one (mv_tok_kernel, PACK), as few as leave
 // the fewest waves per row. One group, a number of rows that divides, a row's units a multiple of 8 (several tokens: two rows, 16).
-// Measured, rows one by one (512 and 5120 columns, and all of 7168: in pairs at most) / packed: Q6_K 32768 rows of 256 columns 2.0 times
-// the speed, 512 7.57 / 6.05 us, 768 10.84 / 7.39, 1280 11.64 / 10.57, 1536 12.13 / 10.87, 129280x5120 113.2 / 99.8, 1536x7168 6.41 / 6.10;
-// Q8_0 32768x512 7.01 / 5.93, 2304x5120 6.67 / 6.52; over 19000 random matrices of the K-quants, Q8_0, BF16 and F32 0.96 to 2.1, below 0.975 in
+// Measured with weights beyond the caches, rows one by one / packed: Q6_K 32768 rows of 256 columns 10.8 / 5.4 us, 512 10.3 / 6.2 (in pairs
+// 7.6), 768 10.4 / 7.5, 1280 11.9 / 10.6, 1536 12.0 / 11.5, 129280x5120 108.3 / 99.1, 1536x7168 6.27 / 5.94; Q8_0 32768x512 9.1 / 7.2,
+// 2304x5120 6.37 / 6.29; against pairs at most over 19000 random matrices of the K-quants, Q8_0, BF16 and F32 0.96 to 2.1, below 0.975 in
 // one of a thousand (under a norm Q6_K 2304x11000 and 2816x7500, Q5_K 1536x15000, and Q6_K pairs of 512 columns from the caches). More than two
 // rows for an eighth fewer waves or less gain nothing (3328 columns 0.96 to 1.06), nor do five waves a workgroup where there are
 // not four packed rows for each (2304x2304 0.95), nor rows of 2304 columns below 6 MB (0.94 to 0.97), nor four short rows of Q8_0 where

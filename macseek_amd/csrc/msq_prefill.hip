@@ -141,7 +141,7 @@ int launch_block_t(hipStream_t st, PfBlkArgs a, uint32_t n6, uint32_t n3, uint32
 constexpr int kPfQueueTokens = 2 * kPfBigTokens;
 // The shared expert of a K-quant / Q8_0 type through the few-token kernel (msq_rows.cuh), on the caller's stream? The tile kernel's 128 x 128
 // tiles are a chain of 150 us however few the tokens, and the fork to a second stream costs 14 us by itself; but they run beside the routed
-// experts, and the few-token kernel's 36 us (37 tokens) to 80 us (112) come behind them. Time before / after, Q6_K and Q8_0 alike, 384 IQ1_S
+// experts, and the few-token kernel's launches (36 us at 37 tokens) come behind them. Time before / after, Q6_K and Q8_0 alike, 384 IQ1_S
 // experts: 5120x2304 at 2 tokens 186 / 119, 16 307 / 280, 37 517 / 502, 64 650 / 606, 100 761 / 761, 150 (the tile kernel ahead) 992 / 978;
 // Q6_K 7168x2048 at 64 703 / 694, 100 918 / 889, 150 1171 / 1190 (Q8_0 of 7168 columns does not fit the LDS); 2560x1024 at 100 252 / 229, 150
 // 347 / 338. 94 to 242 experts in use 0.98 to 1.3 times the former speed at 37 to 112 tokens. Fewer of them leave compute units to the tile

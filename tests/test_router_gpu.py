@@ -149,15 +149,15 @@ def test_router_fused_vs_oracle(dev, wtype, dim):
 
 @pytest.mark.parametrize("n_exp", [64, 128, 384, 512])
 def test_router_fused_ties_expert_counts_and_nan(dev, n_exp):
-    """The fused router selects in two levels (each wave of the last workgroup from its quarter of the experts, then one
-    wave from the 24 survivors): exact ties inside a lane's pair of experts, across lanes and across quarters must go to
-    the lower expert id, fewer than six comparable keys give expert 0 with weight 0, for every supported expert count."""
+    """The fused router selects in two levels (each wave of the last workgroup from its 64 experts, one a lane, then one
+    wave from the six that each leaves): exact ties across lanes and across waves must go to the lower expert id, fewer
+    than six comparable keys give expert 0 with weight 0, for every supported expert count."""
     dim = 256
     rng = np.random.default_rng(n_exp)
     W = (rng.standard_normal((n_exp, dim)) * 0.05).astype(np.float32)
     q4 = n_exp // 4
-    # identical rows: same logit, same bias -> same key. Pairs (e, e + 64) share a lane when the quarter has 128
-    # experts; (e, e + q4) sit in different quarters; runs of equal rows sit in neighbouring lanes
+    # identical rows: same logit, same bias -> same key. (e, e + 64) and, from 256 experts on, (e, e + q4) are lanes of
+    # different waves; runs of equal rows sit in neighbouring lanes
     W[3 + q4] = W[3]
     W[7 + 2 * q4] = W[7]
     W[10:14] = W[10]
@@ -246,7 +246,7 @@ def test_route_lists_over_waves_and_rounds(dev, n, n_exp):
     assert np.array_equal(L.t_slot_of.cpu().numpy()[: 6 * n], slot)
 
 
-# rows of as many vectors a lane as one trip to memory takes, one vector more, and the kernels of ten and twelve
+# rows of 512, 640 and 768 vectors, a quarter to each of four waves, and of one vector more
 @pytest.mark.parametrize("wtype,dim", [(q.QType.BF16, d) for d in (4096, 4104, 5120, 5128, 6144, 6152)] + [(q.QType.F32, d) for d in (2048, 2056, 2560, 2568, 3072, 3080)])
 def test_router_fused_row_lengths(dev, wtype, dim):
     test_router_fused_vs_oracle(dev, wtype, dim)
@@ -293,3 +293,18 @@ def test_router_fused_that_gave_up_shows_it(dev):
             i, v = call()
             assert i == ids0 and torch.equal(v, w0)
     assert int(number) == 2
+
+
+@pytest.mark.parametrize("n_exp", [128, 384, 512])
+def test_router_fused_ties_on_either_side_of_a_wave(dev, n_exp):
+    # experts 60 to 67 are one row, the last four of a wave of 64 and the first four of the next, ahead of all others: the six lowest ids
+    dim = 512
+    W = O.randn(n_exp * dim, n_exp, 0.01).reshape(n_exp, dim)
+    x = O.randn(dim, 8)
+    W[60:68] = (x / np.linalg.norm(x)).astype(np.float32)
+    s, e = arch.Scratch.create(n_exp), q.Enc()
+    ids, w = torch.full((6,), -1, dtype=torch.int32, device=dev), torch.zeros(6, device=dev)
+    arch.encode_router_fused(e, q.Buffer.of(up(x)), q.Buffer.of(up(W.reshape(-1))), q.Buffer.of(up(np.zeros(n_exp, np.float32))), q.Buffer.of(ids),
+                             q.Buffer.of(w), s, dim)
+    e.wait()
+    assert ids.tolist() == [60, 61, 62, 63, 64, 65] and bool((w == w[0]).all()) and float(w[0]) > 0
